@@ -23,10 +23,11 @@
 //
 // Rows are expanded edge-balanced: a workgroup takes a tile of the list, scans the row lengths in
 // LDS and deals the tile's edge slots out one per thread, so a thread's critical path is one edge
-// rather than one row. Rows longer than `light` are cut into chunks that whole waves expand: in the
-// walk and the pull after a barrier of their own, in the relax phase at the start of the next
-// iteration. Per-iteration list counters live in rings of three slots, so a relax iteration needs
-// one barrier. Workgroups exchange data only through agent-scope
+// rather than one row. Rows longer than `light` are cut into chunks that whole waves of the grid
+// expand after a split barrier (a workgroup arrives when its chunks are listed and goes on with its
+// tile). Whoever lists a vertex looks at its row's length, so a phase over a list without long rows
+// has no chunks and one barrier; the barrier brings the lists' lengths. Per-iteration list counters
+// live in rings of three slots. Workgroups exchange data only through agent-scope
 // atomics and loads/stores that bypass the non-coherent caches, so the grid barrier itself needs
 // no cache write-back or invalidation (the distance-only unpack, which reads plain stores of
 // other workgroups, uses the fenced barrier).
@@ -57,6 +58,20 @@ constexpr int kRelaxNarrow = 128; ///< a near frontier of at most this many vert
 /// local level that reaches a bushy part of the graph would otherwise keep the grid waiting on one
 /// workgroup: measured on RMAT-22, one local relax iteration of 124 us where the others took 12).
 constexpr int kLocalEdgeBudget = 8192;
+/// Rows of more edges are cut into chunks of kChunkEdges, one wave each, instead of lying in one
+/// workgroup's tile, where the grid would wait for that workgroup. A repair's frontier holds few
+/// vertices per workgroup, so one row of a few thousand edges is most of its tile (1M-operation
+/// batches on RMAT-23: the six wide relax iterations kept an average workgroup busy for 18-36 us
+/// and the last one for 97-136); below 1024 edges the split barrier that chunks need costs more than
+/// they even out (RMAT-22 batches of 100,000: engine 239 us at 1024, 248 at 768, 255 at 512). The
+/// walk's edges are cheaper, and chunks keep a round to one level: 2048 (58 us of the walk, as at
+/// 4096, but 114 us against 149 on RMAT-23; 8192: 72 and 209 us). A solve's tiles hold up to 1024
+/// rows, and short ones balance best: RMAT-22 2.9 ms at 64-128 edges, 3.0 at 256, 3.3 at 1024, 4.1
+/// at 2048 and above.
+constexpr int kLightRelax = 1024;
+constexpr int kLightWalk = 2048;
+constexpr int kLightSolve = 128;
+constexpr int kChunkEdges = 256;
 constexpr int kLocalGenerations = 1600000000;  ///< no local relax iteration starts past this generation
 
 struct control {
@@ -139,7 +154,8 @@ struct engine_params {
   int64_t chunk_cap;
   control* ctl;
   grid_sync_state* bar;
-  int32_t light;
+  int32_t light;       ///< rows of more edges are cut into chunks (pull and relax)
+  int32_t light_walk;  ///< and in the subtree walk
   int32_t chunk_edges;
   unsigned long long barrier_ticks;  ///< longest wait at a grid barrier (s_memrealtime ticks)
   const int* hold;  ///< null, or a flag of the apply queued ahead: nonzero, the run does nothing
@@ -161,7 +177,12 @@ constexpr int kStage = 2048;  ///< entries a workgroup stages per list between f
 /// go to the list directly.
 struct stage_shared {
   int count[3];
+  int ready[3];  ///< entries of the flush under way
   int base[3];
+  /// entries this workgroup put on lists 0 and 1 since it last told the grid, and how many of the
+  /// vertices it listed for expansion have rows past `light`
+  unsigned int sent[2];
+  int sent_long;
   int item[3][kStage];
   int* list2;     ///< list 2 is always the unpack's list (engine_params::touched)
   int* counter2;  ///< and its counter
@@ -171,35 +192,72 @@ struct stage_shared {
 DYNG_DEV void stage_append(stage_shared& S, int k, bool pred, int32_t v, int* list, int* counter) {
   const u64 mask = __ballot(pred);
   if (mask == 0) return;  // uniform per wave
-  const int leader = __ffsll(static_cast<long long>(mask)) - 1;
+  const int leader = uniform(__ffsll(static_cast<long long>(mask)) - 1);
   int b = 0;
   if (lane() == leader) b = atomicAdd(&S.count[k], __popcll(mask));
-  b = __shfl(b, leader);
+  b = from_lane(b, leader);
   const int slot = b + __popcll(mask & lanes_below());
   if (pred && slot < kStage) S.item[k][slot] = v;
   append(list, counter, pred && slot >= kStage, v);
 }
 
-/// Publish the staged entries of list 0, of list 1 when list1 is not null, and of list 2 (the
+/// Threads 0-2, when every staged entry is in LDS: reserve the places of list k's staged entries
+/// and empty the stage. Entries past the stage's capacity are on the list already.
+DYNG_DEV int stage_reserve(stage_shared& S, int k, int* counter) {
+  const int all = S.count[k];
+  const int cnt = counter != nullptr ? min(all, kStage) : 0;
+  S.count[k] = 0;
+  S.ready[k] = cnt;
+  if (k < 2) S.sent[k] += static_cast<unsigned int>(all);
+  return cnt > 0 ? atomicAdd(counter, cnt) : 0;
+}
+
+/// Copy the reserved entries to their places (every thread, after a workgroup barrier).
+DYNG_DEV void stage_copy(stage_shared& S, int* list0, int* list1) {
+  for (int k = 0; k < 3; ++k) {
+    int* list = k == 0 ? list0 : k == 1 ? list1 : S.list2;
+    const int cnt = S.ready[k], b = S.base[k];
+    for (int i = threadIdx.x; i < cnt; i += blockDim.x) st(&list[b + i], S.item[k][i]);
+  }
+}
+
+/// Publish the staged entries of list 0, of list 1 when its counter is not null, and of list 2 (the
 /// unpack's list). Every thread of the workgroup calls it; the stage is empty afterwards.
 DYNG_DEV void stage_flush(stage_shared& S, int* list0, int* counter0, int* list1 = nullptr, int* counter1 = nullptr) {
   __syncthreads();  // every staged entry is in LDS
   if (threadIdx.x < 3) {
     const int k = threadIdx.x;
-    int* counter = k == 0 ? counter0 : k == 1 ? counter1 : S.counter2;
-    const int cnt = counter != nullptr ? min(S.count[k], kStage) : 0;
-    S.count[k] = cnt;
-    S.base[k] = cnt > 0 ? atomicAdd(counter, cnt) : 0;
+    S.base[k] = stage_reserve(S, k, k == 0 ? counter0 : k == 1 ? counter1 : S.counter2);
   }
   __syncthreads();
-  for (int k = 0; k < 3; ++k) {
-    int* list = k == 0 ? list0 : k == 1 ? list1 : S.list2;
-    const int cnt = S.count[k], b = S.base[k];
-    for (int i = threadIdx.x; i < cnt; i += blockDim.x) st(&list[b + i], S.item[k][i]);
+  stage_copy(S, list0, list1);
+  __syncthreads();  // the copy has read the stage before the next append
+}
+
+/// The same, while waiting for round `round` of the grid barrier, at which this workgroup has
+/// arrived: the reservations' round trip and the poll's are one. The copy may still be under way in
+/// other waves when it returns: a workgroup barrier before the next append.
+DYNG_DEV grid_found stage_flush_wait(stage_shared& S, int* list0, int* counter0, int* list1, int* counter1,
+                                     grid_sync_state* bar, unsigned int round, unsigned long long limit) {
+  __shared__ grid_found found;
+  __syncthreads();  // every staged entry is in LDS
+  if (threadIdx.x < 3) {
+    const int k = threadIdx.x;
+    const int base = stage_reserve(S, k, k == 0 ? counter0 : k == 1 ? counter1 : S.counter2);
+    if (k == 0) found = grid_poll(bar, round, limit);  // its first load goes out behind the reservations
+    S.base[k] = base;
   }
-  __syncthreads();  // every thread has read count and base
-  if (threadIdx.x < 3) S.count[threadIdx.x] = 0;
-  __syncthreads();  // the reset lands before the next stage_append
+  __syncthreads();
+  stage_copy(S, list0, list1);
+  return grid_found{uniform(found.ok), uniform(found.published), uniform(found.marked)};
+}
+
+/// Note the lanes that list a vertex with a row past `light` for expansion (every active lane calls
+/// it): the next expansion of a list without any needs no chunks and no split barrier.
+DYNG_DEV void note_long(stage_shared& S, bool is_long) {
+  const u64 mask = __ballot(is_long);
+  if (mask == 0) return;
+  if (lane() == __ffsll(static_cast<long long>(mask)) - 1) atomicAdd(&S.sent_long, __popcll(mask));
 }
 
 /// Claim v for the list of generation `generation` (the stamp exchange): true when this call
@@ -225,65 +283,40 @@ DYNG_DEV int4 ld_chunk(const int4* ch) {
 }
 
 
-/// Four stamps at once, as two agent-scope 8-byte loads.
-DYNG_DEV int4 ld_int4(const int4* q4) {
-  const u64* q = reinterpret_cast<const u64*>(q4);
-  const u64 a = ld(&q[0]), b = ld(&q[1]);
-  return make_int4(static_cast<int32_t>(static_cast<uint32_t>(a)), static_cast<int32_t>(static_cast<uint32_t>(a >> 32)),
-                   static_cast<int32_t>(static_cast<uint32_t>(b)), static_cast<int32_t>(static_cast<uint32_t>(b >> 32)));
-}
-
-/// Cut the row [begin, begin + len) of vertex v into chunks of `chunk` edges (one wave each).
-DYNG_DEV void emit_chunks_to(const engine_params& p, int4* out, int64_t cap, int* counter, int32_t v, int32_t begin,
-                              int32_t len) {
-  const int pieces = (len + p.chunk_edges - 1) / p.chunk_edges;
-  const int base = atomicAdd(counter, pieces);
-  for (int c = 0; c < pieces; ++c) {
-    if (base + c >= cap) {
-      atomicOr(&p.ctl->error_bits, DYNG_HIP_DEVICE_ERROR_CAPACITY);
-      return;
-    }
-    const int b = begin + c * p.chunk_edges;
-    const int e = min(begin + len, b + p.chunk_edges);
-    st_chunk(&out[base + c], v, b, e);
-  }
-}
-DYNG_DEV void emit_chunks(const engine_params& p, int* counter, int32_t v, int32_t begin, int32_t len) {
-  emit_chunks_to(p, p.chunks, p.chunk_cap, counter, v, begin, len);
-}
-
 /// The workgroup's view of one tile of a vertex list: per item the first edge slot of its rows in
-/// the tile (exclusive prefix of the lengths), the row offset, the vertex and a 64-bit word.
+/// the tile (exclusive prefix of the lengths), the row offset, the vertex and a 64-bit word; for
+/// tiles with long rows also the first chunk of each and its length.
 struct tile_shared {
   int start[kBlock + 1];
   int off[kBlock];
   int vert[kBlock];
   u64 word[kBlock];
-  int scan[kWaves + 1];
+  int chunk_start[kBlock + 1];
+  int len[kBlock];
+  int chunk_base;
+  int scan[2][kWaves + 1];
 };
 
-/// Exclusive prefix sum of x over the workgroup; `total` gets the sum. Every thread calls it.
-DYNG_DEV int block_scan(tile_shared& L, int x, int& total) {
-  int v = x;
-  for (int off = 1; off < 64; off <<= 1) {
-    const int y = __shfl_up(v, off);
-    if (lane() >= off) v += y;
-  }
-  const int w = static_cast<int>(threadIdx.x) >> 6;
-  if (lane() == 63) L.scan[w] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int i = 0; i < kWaves; ++i) {
-      const int t = L.scan[i];
-      L.scan[i] = run;
-      run += t;
-    }
-    L.scan[kWaves] = run;
+/// Exclusive prefix sums of x and of y over the workgroup; `total_x` and `total_y` get the sums.
+/// y is zero in most waves (the chunks of long rows), which then skip its scan. Every thread
+/// calls it; returns x's prefix, `before_y` is y's.
+DYNG_DEV int block_scan2(tile_shared& L, int x, int y, int& total_x, int& total_y, int& before_y) {
+  const int v = wave_scan(x);
+  const int z = __ballot(y != 0) != 0 ? wave_scan(y) : 0;
+  const int w = uniform(static_cast<int>(threadIdx.x) >> 6);
+  if (lane() == 63) {
+    L.scan[0][w] = v;
+    L.scan[1][w] = z;
   }
   __syncthreads();
-  total = L.scan[kWaves];
-  return L.scan[w] + v - x;
+  // every wave scans the waves' sums itself: one LDS read and a row scan, no second barrier
+  static_assert(kWaves == 16, "the waves' sums fill a row of 16 lanes");
+  const int sx = L.scan[0][lane() & 15], sy = L.scan[1][lane() & 15];
+  const int ax = row_scan(sx), ay = row_scan(sy);
+  total_x = from_lane(ax, 15);
+  total_y = from_lane(ay, 15);
+  before_y = from_lane(ay - sy, w) + z - y;
+  return from_lane(ax - sx, w) + v - x;
 }
 
 /// Edge slots a lane takes per step of an expansion: their loads are issued together (each slot's
@@ -291,21 +324,58 @@ DYNG_DEV int block_scan(tile_shared& L, int x, int& total) {
 /// instead of one per slot.
 constexpr int kSlots = 1;
 
+/// Steps of a long tile between two looks at how full the append stage is (see expand_tile).
+constexpr int kCheckSteps = 4;
+
+/// The last of the `cnt` items whose first slot (or chunk) is <= e: the one that holds e, given
+/// that some item does.
+DYNG_DEV int item_of(const int* start, int cnt, int e) {
+  int lo = 0, hi = cnt;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (start[mid] <= e) {
+      lo = mid;
+    } else {
+      hi = mid;
+    }
+  }
+  return lo;
+}
+
+/// Where a phase's long rows go: their chunks, and the chunks this workgroup published there.
+struct chunk_sink {
+  int4* list;
+  int64_t cap;
+  int* counter;   ///< reserves places in the list
+  int light;      ///< rows of more edges are cut into chunks (INT32_MAX: none, the phase has no chunks)
+  int published;  ///< uniform over the workgroup
+};
+
 /// Edge-balanced expansion of one tile of `cnt` items (cnt <= kBlock): `load(i, v, off, len,
-/// word)` fills thread i's item (i < cnt; len 0: nothing to expand, e.g. a long row sent to the
-/// chunk list), and the edge slots of the tile's rows are dealt out to the workgroup's threads,
-/// kSlots slots per thread per step (slot j of a step kBlock apart from slot j - 1, so each j is
-/// one coalesced run per wave): `edges(act, item, slot)` runs with every lane of a wave, on arrays
-/// of kSlots (act false on padding). `done(valid, item)` runs on every thread after the tile's
-/// edges. Every thread of the workgroup calls it.
-template <class Load, class Edges, class Done>
-DYNG_DEV void expand_tile(tile_shared& L, int cnt, Load load, Edges edges, Done done) {
+/// word)` fills thread i's item (i < cnt; len 0: nothing to expand). Rows of more than
+/// `out.light` edges are cut into chunks, written to the chunk list by the whole workgroup (one reservation
+/// per tile); `ready()` runs on every thread when they are all published, before the tile's own
+/// edges. The edge slots of the other rows are dealt out to the workgroup's threads, kSlots slots
+/// per thread per step (slot j of a step kBlock apart from slot j - 1, so each j is one coalesced
+/// run per wave): `edges(act, item, slot)` runs with every lane of a wave, on arrays of kSlots
+/// (act false on padding); every kCheckSteps steps of a long tile `check()` runs on every thread
+/// (to publish staged appends before the stage overflows). `done(valid, item)` runs on every
+/// thread after the tile's edges. Returns the edges expanded here. Every thread of the workgroup
+/// calls it.
+template <class Load, class Ready, class Edges, class Check, class Done>
+DYNG_DEV int expand_tile(const engine_params& p, tile_shared& L, chunk_sink& out, int cnt, Load load, Ready ready,
+                         Edges edges, Check check, Done done) {
   const int i = static_cast<int>(threadIdx.x);
   int32_t v = -1, off = 0, len = 0;
   u64 word = packed_inf;
   if (i < cnt) load(i, v, off, len, word);
-  int total = 0;
-  const int start = block_scan(L, len, total);
+  int pieces = 0, short_len = len;
+  if (len > out.light) {
+    pieces = (len + p.chunk_edges - 1) / p.chunk_edges;
+    short_len = 0;
+  }
+  int total = 0, chunks = 0, first_chunk = 0;
+  const int start = block_scan2(L, short_len, pieces, total, chunks, first_chunk);
   if (i < cnt) {
     L.start[i] = start;
     L.off[i] = off;
@@ -313,52 +383,90 @@ DYNG_DEV void expand_tile(tile_shared& L, int cnt, Load load, Edges edges, Done 
     L.word[i] = word;
   }
   if (i == 0) L.start[cnt] = total;
-  __syncthreads();
-  for (int base = i - lane(); base < total; base += kSlots * kBlock) {
-    bool act[kSlots];
-    int item[kSlots], slot[kSlots];
-#pragma unroll
-    for (int j = 0; j < kSlots; ++j) {
-      const int e = base + j * kBlock + lane();
-      act[j] = e < total;
-      int lo = 0;
-      if (act[j]) {
-        int hi = cnt;  // the last item whose first slot is <= e (its row holds e)
-        while (hi - lo > 1) {
-          const int mid = (lo + hi) >> 1;
-          if (L.start[mid] <= e) {
-            lo = mid;
-          } else {
-            hi = mid;
-          }
-        }
-      }
-      item[j] = lo;
-      slot[j] = act[j] ? L.off[lo] + (e - L.start[lo]) : 0;
+  if (chunks > 0) {  // uniform
+    if (i < cnt) {
+      L.chunk_start[i] = first_chunk;
+      L.len[i] = len;
     }
-    edges(act, item, slot);
+    if (i == 0) {
+      L.chunk_start[cnt] = chunks;
+      L.chunk_base = atomicAdd(out.counter, chunks);
+    }
+    __syncthreads();
+    for (int q = i; q < chunks; q += kBlock) {
+      const int row = item_of(L.chunk_start, cnt, q);
+      const int64_t at = static_cast<int64_t>(L.chunk_base) + q;
+      if (at >= out.cap) {
+        atomicOr(&p.ctl->error_bits, DYNG_HIP_DEVICE_ERROR_CAPACITY);
+        break;
+      }
+      const int32_t b = L.off[row] + (q - L.chunk_start[row]) * p.chunk_edges;
+      st_chunk(&out.list[at], L.vert[row], b, min(L.off[row] + L.len[row], b + p.chunk_edges));
+    }
+    out.published += chunks;
+    __builtin_amdgcn_s_waitcnt(0);  // the wave's entries are out before ready() tells of them
+  }
+  __syncthreads();
+  ready();
+  const int wave_base = i - lane();
+  int steps = 0;
+  for (int t = 0; t < total; t += kSlots * kBlock) {
+    const int base = t + wave_base;
+    if (base < total) {
+      bool act[kSlots];
+      int item[kSlots], slot[kSlots];
+#pragma unroll
+      for (int j = 0; j < kSlots; ++j) {
+        const int e = base + j * kBlock + lane();
+        act[j] = e < total;
+        const int lo = act[j] ? item_of(L.start, cnt, e) : 0;
+        item[j] = lo;
+        slot[j] = act[j] ? L.off[lo] + (e - L.start[lo]) : 0;
+      }
+      edges(act, item, slot);
+    }
+    if (++steps == kCheckSteps && t + kSlots * kBlock < total) {  // uniform
+      steps = 0;
+      check();
+    }
   }
   __syncthreads();
   done(i < cnt, i);
   __syncthreads();
+  return total;
 }
 
-/// Edge-balanced expansion of list items [0, count): the items are cut into one tile per
-/// workgroup (up to kBlock items), each expanded by expand_tile with `load(index, ...)` given the
-/// item's index in the list, and `flush()` runs on every thread of the workgroup after each tile
-/// (to publish staged appends). Uniform per workgroup: every thread calls it.
-template <class Load, class Edges, class Done, class Flush>
-DYNG_DEV void tile_rows(tile_shared& L, int count, Load load, Edges edges, Done done, Flush flush) {
+/// Edge-balanced expansion of list items [0, count): every workgroup takes the same number of
+/// tiles of the same size (at most kBlock items; a last tile that only some workgroups have would
+/// keep the others waiting), each expanded by expand_tile with `load(index, ...)` given the item's
+/// index in the list. `between()` runs on every thread of the workgroup between two tiles (to
+/// publish staged appends). With round `round` of the grid barrier given (not 0), the workgroup
+/// arrives at it when the chunks of its last tile are published. Returns the edges this workgroup expanded. Uniform per
+/// workgroup: every thread calls it.
+template <class Load, class Edges, class Check, class Done, class Between>
+DYNG_DEV int tile_rows(const engine_params& p, tile_shared& L, chunk_sink& out, unsigned int round, int count, Load load,
+                       Edges edges, Check check, Done done, Between between) {
   const int G = static_cast<int>(gridDim.x);
-  const int ts = min(kBlock, max(1, (count + G - 1) / G));
-  for (long long t0 = static_cast<long long>(blockIdx.x) * ts; t0 < count; t0 += static_cast<long long>(G) * ts) {
+  const int share = max(1, (count + G - 1) / G);
+  const int tiles = (share + kBlock - 1) / kBlock;
+  const int ts = (share + tiles - 1) / tiles;
+  const long long stride = static_cast<long long>(G) * ts;
+  long long t0 = static_cast<long long>(blockIdx.x) * ts;
+  int expanded = 0;
+  if (t0 >= count && round != 0 && threadIdx.x == 0) grid_arrive(p.bar, round, 0);
+  for (; t0 < count; t0 += stride) {
     const int cnt = static_cast<int>(min(static_cast<long long>(ts), count - t0));
     const int first = static_cast<int>(t0);
-    expand_tile(
-        L, cnt, [&](int i, int32_t& v, int32_t& off, int32_t& len, u64& word) { load(first + i, v, off, len, word); },
-        edges, done);
-    flush();
+    const bool last = t0 + stride >= count;
+    expanded += expand_tile(
+        p, L, out, cnt, [&](int i, int32_t& v, int32_t& off, int32_t& len, u64& word) { load(first + i, v, off, len, word); },
+        [&] {
+          if (last && round != 0 && threadIdx.x == 0) grid_arrive(p.bar, round, static_cast<unsigned int>(out.published));
+        },
+        edges, check, done);
+    if (!last) between();
   }
+  return expanded;
 }
 
 /// w's word changed in this run without its distance falling (a lower parent id at the same
@@ -373,8 +481,10 @@ DYNG_DEV bool mark_changed(const engine_params& p, int32_t w) { return atomicMax
 /// below the truth and only costs an atomic): the candidate word joins the next near list or the
 /// far pile when it lowered w's word. Returns the lists to append w to.
 DYNG_DEV void relax_decide(const engine_params& p, bool active, int32_t u, u64 du, int32_t w, int32_t wt, u64 seen,
-                           u64 threshold, int generation, unsigned long long* improved, bool& to_near,
-                           bool& to_far, bool& first) {
+                           u64 threshold, int generation, bool& lowered, bool& to_near, bool& to_far, bool& first,
+                           bool& is_long) {
+  lowered = false;
+  is_long = false;
   to_near = false;
   to_far = false;
   first = false;
@@ -383,16 +493,18 @@ DYNG_DEV void relax_decide(const engine_params& p, bool active, int32_t u, u64 d
     if (nd <= p.max_distance) {
       const u64 cand = p.pk.pack(nd, u);
       if (cand < seen) {
+        const int len = p.out_meta[w].y;  // in flight together with the minimum
         const u64 old = atomicMin(&p.packed[w], cand);
         // Any lowered word joins a list, also one lowered only to a lower parent id at the same
         // distance (fused.cuh:341-362 lists only a lower distance): the extra expansion is rare
         // and offers nothing new, and being claimed stamps the vertex for the unpack.
         if (cand < old) {
-          atomicAdd(improved, 1ULL);
+          lowered = true;
           // both flags as values (a store through a reference chosen by the branch would keep
           // them in scratch memory); a far vertex is stamped when it leaves the far pile
           const bool near = nd < threshold;
           to_near = near && claim_first(p, w, generation, first);
+          is_long = to_near && len > p.light;
           to_far = !near && atomicExch(&p.in_far[w], 1) == 0;
         }
       }
@@ -420,7 +532,9 @@ struct near_sink {
 };
 
 /// kSlots relaxations per lane: the row entries first, then the words they point at, then the
-/// atomics and the list appends. Every lane of the wave calls it.
+/// atomics and the list appends. Every lane of the wave calls it. A solve from the sources unpacks
+/// every vertex, so it keeps no list of the touched ones.
+template <bool kSolve>
 DYNG_DEV void relax_slots(const engine_params& p, const bool (&act)[kSlots], const int32_t (&u)[kSlots],
                           const u64 (&du)[kSlots], const int (&slot)[kSlots], u64 threshold, int generation,
                           stage_shared& S, int* next, int* next_count, int* far, int* far_count,
@@ -440,11 +554,15 @@ DYNG_DEV void relax_slots(const engine_params& p, const bool (&act)[kSlots], con
   }
 #pragma unroll
   for (int j = 0; j < kSlots; ++j) {
-    bool to_near, to_far, first;
-    relax_decide(p, live[j], u[j], du[j], w[j], wt[j], seen[j], threshold, generation, improved, to_near, to_far,
-                 first);
+    bool lowered, to_near, to_far, first, is_long;
+    relax_decide(p, live[j], u[j], du[j], w[j], wt[j], seen[j], threshold, generation, lowered, to_near, to_far, first,
+                 is_long);
+    const u64 better = __ballot(lowered);
+    if (better == 0) continue;  // uniform per wave: nothing to count or to append
+    if (lane() == 0) atomicAdd(improved, static_cast<unsigned long long>(__popcll(better)));
+    note_long(S, is_long);
     bool to_list = to_near;
-    if (to_near && sink.local != nullptr) {
+    if (to_near && !is_long && sink.local != nullptr) {
       const int at = atomicAdd(&sink.local->count[sink.q], 1);
       if (at < kBlock) {
         sink.local->item[sink.q][at] = w[j];
@@ -454,31 +572,50 @@ DYNG_DEV void relax_slots(const engine_params& p, const bool (&act)[kSlots], con
     if (to_list && sink.listed != nullptr) to_list = atomicExch(&sink.listed[w[j]], sink.tag) != sink.tag;
     stage_append(S, 0, to_list, w[j], next, next_count);
     stage_append(S, 1, to_far, w[j], far, far_count);
-    stage_append(S, 2, first, w[j], S.list2, S.counter2);
+    if (!kSolve) stage_append(S, 2, first, w[j], S.list2, S.counter2);
   }
 }
 
-/// Chunks of long rows, one wave per chunk: `edges(act, u, slot)` with every lane of the wave, on
-/// arrays of kSlots slots (64 apart).
-template <class Edges>
-DYNG_DEV void chunk_rows(const engine_params& p, int nchunks, Edges edges) {
-  const int wave = static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) / 64);
-  const int waves = static_cast<int>((gridDim.x * blockDim.x) / 64);
-  for (int c = wave; c < nchunks; c += waves) {
-    const int4 ch = ld_chunk(&p.chunks[c]);
-    for (int b = ch.y; b < ch.z; b += 64 * kSlots) {
-      bool act[kSlots];
-      int32_t u[kSlots];
-      int slot[kSlots];
+/// The published chunks of long rows, spread over the waves of the grid (consecutive chunks to
+/// different workgroups); while there are few, a chunk is cut into up to four parts, so that a few
+/// long rows still reach every workgroup. `begin(v, edges)` runs with every lane of a wave before
+/// its chunk (the edges of the part it takes), `edges(act, u, slot)` for every 64 slots, on arrays
+/// of kSlots slots (64 apart), `end(v)` after it, and `check()` on every thread of the workgroup
+/// after each round of chunks.
+template <class Begin, class Edges, class End, class Check>
+DYNG_DEV void chunk_rows(const engine_params& p, const int4* chunks, int nchunks, Begin begin, Edges edges, End end,
+                         Check check) {
+  const int G = static_cast<int>(gridDim.x);
+  const int waves = G * kWaves;
+  const int parts = nchunks * 4 <= waves ? 4 : nchunks * 2 <= waves ? 2 : 1;
+  const int span = (p.chunk_edges + parts * 64 - 1) / (parts * 64) * 64;  // slots of a part, whole waves of them
+  const int units = nchunks * parts;
+  const int wave = static_cast<int>(threadIdx.x / 64) * G + static_cast<int>(blockIdx.x);
+  for (int q0 = 0; q0 < units; q0 += waves) {  // uniform over the grid
+    const int q = q0 + wave;
+    if (q < units) {
+      const int4 ch = ld_chunk(&chunks[q / parts]);
+      const int first = ch.y + (q % parts) * span;
+      const int last = min(ch.z, first + span);
+      if (first < last) {
+        begin(ch.x, last - first);
+        for (int b = first; b < last; b += 64 * kSlots) {
+          bool act[kSlots];
+          int32_t u[kSlots];
+          int slot[kSlots];
 #pragma unroll
-      for (int j = 0; j < kSlots; ++j) {
-        const int e = b + j * 64 + lane();
-        act[j] = e < ch.z;
-        u[j] = ch.x;
-        slot[j] = act[j] ? e : 0;
+          for (int j = 0; j < kSlots; ++j) {
+            const int e = b + j * 64 + lane();
+            act[j] = e < last;
+            u[j] = ch.x;
+            slot[j] = act[j] ? e : 0;
+          }
+          edges(act, u, slot);
+        }
+        end(ch.x);
       }
-      edges(act, u, slot);
     }
+    check();
   }
 }
 
@@ -549,26 +686,60 @@ DYNG_DEV void pull_commit(const engine_params& p, bool pred, int32_t v, u64 best
       }
     }
   }
+  note_long(S, add && p.out_meta[v].y > p.light);
   stage_append(S, 0, add, v, p.frontier, counter);
   stage_append(S, 2, first, v, S.list2, S.counter2);
+  if (__ballot(low != packed_inf) == 0) return;  // uniform per wave
   low = wave_min(low);
-  if (lane() == 0 && low != packed_inf) atomicMin(minimum, low);
+  if (lane() == 0) atomicMin(minimum, low);
 }
 
 }  // namespace
 
-/// Leave the kernel when the grid barrier gave up (see grid_barrier); uniform per workgroup.
-/// DYNG_GRID_SYNC separates phases whose shared data is only touched with agent-scope
-/// operations; DYNG_GRID_SYNC_FENCED also orders plain loads and stores.
-#define DYNG_GRID_SYNC_AS(fenced)                                                   \
-  do {                                                                              \
-    if (!grid_barrier<fenced>(p.bar, p.barrier_ticks)) {                            \
+/// Leave the kernel when a grid wait gave up (see grid_barrier); uniform per workgroup.
+/// DYNG_GRID_SYNC separates phases whose shared data is only touched with agent-scope operations;
+/// DYNG_GRID_SYNC_FENCED also orders plain loads and stores; DYNG_GRID_SYNC_SENT(list, total, longs)
+/// also gives the entries all workgroups put on a list since the last one, and whether a vertex
+/// listed for expansion has a row past `light`.
+#define DYNG_GRID_LEAVE_UNLESS(ok)                                                   \
+  do {                                                                               \
+    if (!(ok)) {                                                                     \
       if (threadIdx.x == 0) atomicOr(&c->error_bits, DYNG_HIP_DEVICE_ERROR_TIMEOUT); \
-      return;                                                                       \
-    }                                                                               \
+      return;                                                                        \
+    }                                                                                \
   } while (0)
-#define DYNG_GRID_SYNC() DYNG_GRID_SYNC_AS(false)
-#define DYNG_GRID_SYNC_FENCED() DYNG_GRID_SYNC_AS(true)
+#define DYNG_GRID_SYNC_AS(fenced, list, found)                                           \
+  ++round;                                                                               \
+  const grid_found found = grid_barrier<fenced>(p.bar, round, p.barrier_ticks, [&] {     \
+    grid_arrive(p.bar, round, S.sent[list], S.sent_long != 0);                           \
+    S.sent[0] = S.sent[1] = 0;                                                           \
+    S.sent_long = 0;                                                                     \
+  });                                                                                    \
+  DYNG_GRID_LEAVE_UNLESS(found.ok)
+#define DYNG_GRID_SYNC()                  \
+  do {                                    \
+    DYNG_GRID_SYNC_AS(false, 0, found_);  \
+  } while (0)
+#define DYNG_GRID_SYNC_FENCED()           \
+  do {                                    \
+    DYNG_GRID_SYNC_AS(true, 0, found_);   \
+  } while (0)
+#define DYNG_GRID_SYNC_SENT(list, total, longs) \
+  do {                                          \
+    DYNG_GRID_SYNC_AS(false, list, found_);     \
+    total = found_.published;                   \
+    longs = found_.marked != 0;                 \
+  } while (0)
+/// Publish the staged entries and wait until every workgroup has published the long rows' chunks of
+/// this phase; `nchunks` gets their number (uniform over the grid).
+#define DYNG_FLUSH_AND_CHUNKS_WAIT(nchunks, list0, counter0, list1, counter1)                              \
+  do {                                                                                                     \
+    ++round;                                                                                               \
+    const grid_found found_ =                                                                              \
+        stage_flush_wait(S, list0, counter0, list1, counter1, p.bar, round, p.barrier_ticks);              \
+    DYNG_GRID_LEAVE_UNLESS(found_.ok);                                                                     \
+    nchunks = static_cast<int>(min(static_cast<int64_t>(found_.published), chunk_cap));                    \
+  } while (0)
 
 /// Clear the grid barrier (a kernel, not a memset, so the launch can live in a hipGraph).
 /// Before each run (one workgroup): the barrier state and the control block zeroed, the control
@@ -587,12 +758,12 @@ __global__ void k_reset_barrier(grid_sync_state* bar, control* ctl) {
   }
 }
 
-/// Two builds of the persistent kernel: kWaves = 8 waves per SIMD keeps it at 64 VGPRs, so two
-/// 1024-thread workgroups fit a CU (solves from the sources), at the price of 17 VGPRs spilled to
-/// scratch; kWaves = 4 gives it 128 (it takes 85, nothing spilled) for grids of one workgroup per
-/// CU (repairs).
-template <int kWaves>
-__global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_params p) {
+/// The builds of the persistent kernel. kPerSimd = 8 waves per SIMD keeps it at 64 VGPRs, so two
+/// 1024-thread workgroups fit a CU (solves from the sources); kPerSimd = 4 gives it 128, for grids
+/// of one workgroup per CU (repairs). kSolve: from the sources (compute, recompute), else the
+/// repair of a tree: two kernels, so that neither carries the other's registers.
+template <int kPerSimd, bool kSolve>
+__global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_params p) {
   // queued right behind an apply whose merges were held back: nothing to do (uniform)
   if (p.hold != nullptr && *p.hold != 0) {
     if (blockIdx.x == 0 && threadIdx.x == 0) p.ctl->held = 1;
@@ -607,6 +778,8 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
   if (threadIdx.x < 5) counts[threadIdx.x] = 0;
   if (threadIdx.x < 3) S.count[threadIdx.x] = 0;
   if (threadIdx.x == 0) {
+    S.sent[0] = S.sent[1] = 0;
+    S.sent_long = 0;
     S.list2 = p.touched;
     S.counter2 = &p.ctl->touched_count;
   }
@@ -622,11 +795,14 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
   control* c = p.ctl;
   int generation = p.generation;
   int frontier_count = 0;
+  bool long_near = true;  // the next relax iteration's list holds a vertex with a row past `light`
   int step = 0, cstep = 0;  // ring positions (uniform across the grid)
+  unsigned int round = 0;  // of the grid barrier (uniform over the grid)
+  const int64_t chunk_cap = p.chunk_cap / 2;  // one phase's chunks: at most slots / 16 + n
   unsigned long long jump_items = 0;
   if (tid == 0) c->t_phase[0] = __builtin_amdgcn_s_memrealtime();
 
-  if (p.from_scratch) {
+  if constexpr (kSolve) {
     if (p.source >= 0) {
       for (int v = tid; v < n; v += threads) st(&p.packed[v], v == p.source ? p.pk.pack(0, -1) : packed_inf);
       if (tid == 0) st(&p.frontier[0], p.source);
@@ -673,11 +849,16 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
         v = p.ins_dst[j];
         changed = v >= 0 && p.ins_inc[j * p.inc_stride + p.inc_k] != 0;
       }
-      const bool root = changed && p.parents[v] == u && atomicExch(&p.flag[v], 1) == 0;
+      const bool cut = changed && p.parents[v] == u;
+      const int len = cut ? p.out_meta[v].y : 0;  // in flight together with the exchange
+      const bool root = cut && atomicExch(&p.flag[v], 1) == 0;
       if (root) st(&p.stamp[v], generation + 1);
+      note_long(S, root && len > p.light_walk);
       append(p.cand, &c->cand_count, root, v);
     }
-    DYNG_GRID_SYNC();
+    bool long_front = false;  // the frontier holds a vertex with a row past `light`
+    [[maybe_unused]] int sent = 0;
+    DYNG_GRID_SYNC_SENT(0, sent, long_front);
     if (tid == 0) c->t_phase[4] = __builtin_amdgcn_s_memrealtime();
     if (ld(&c->overflow) != 0) return;  // uniform: the host reports invalid_input
     const int roots = uniform(ld(&c->cand_count));
@@ -685,6 +866,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
     int inv = roots;  // the invalidated vertices: cand[0, inv)
     bool jump = work && p.check_cycles;
     int jump_slot = 0;  // the first ring slot pointer jumping counts in (a slot already zero)
+    int earlier = 0;    // flagged vertices in the candidate list that cand_count does not count
     if (work && !p.check_cycles && roots > 0) {
       // ---- B (tree from this engine): the subtrees under the roots, down the tree edges
       // (parent[w] == u for an out-edge (u, w)); every tree edge of the old tree is an edge of
@@ -699,16 +881,19 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
       // enough for the chunk list) is the next round's frontier, after a grid barrier. Every flagged vertex joins the
       // candidate list after the roots. A walk still going after kWalkRounds rounds (a deep tree)
       // is finished by pointer jumping ----
-      // the frontier: a range [lo, hi) of the candidate list while rounds walk one level (the
-      // level's children are appended right after it), then a list of its own
+      // the frontier: a range of the candidate list while rounds walk one level (the level's
+      // children are appended right after it), then a list of its own. A one-level round counts
+      // its children in a ring slot and places them from `found` on (the vertices flagged before
+      // it), which every workgroup knows; cand_count, whose reader would race the next round's
+      // appends there, stays at `roots` until the local rounds, whose places follow from it
       const int* front = p.cand;
       int front_count = roots;
-      int lo = 0, hi = roots;
+      int found = roots;
       int rounds = 0;
       // kSlots out-edges (u, w) per lane: the entries, then parent[w] (the tree is read-only
       // here), then the flag claims of the tree children (rare: one in-edge of each child)
       auto claim_children = [&](const bool (&act)[kSlots], const int32_t (&u)[kSlots], const int (&slot)[kSlots],
-                                int32_t (&w)[kSlots], bool (&add)[kSlots]) {
+                                int32_t (&w)[kSlots], bool (&add)[kSlots], bool (&is_long)[kSlots]) {
         int32_t par[kSlots];
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) w[j] = act[j] ? p.out_nbr[slot[j]] : -1;  // dead entries are negative
@@ -716,48 +901,64 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
         for (int j = 0; j < kSlots; ++j) par[j] = w[j] >= 0 ? p.parents[w[j]] : -2;
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) {
-          add[j] = w[j] >= 0 && par[j] == u[j] && atomicExch(&p.flag[w[j]], 1) == 0;
+          const bool child = w[j] >= 0 && par[j] == u[j];
+          const int len = child ? p.out_meta[w[j]].y : 0;  // in flight together with the exchange
+          add[j] = child && atomicExch(&p.flag[w[j]], 1) == 0;
           if (add[j]) st(&p.stamp[w[j]], generation + 1);
+          is_long[j] = add[j] && len > p.light_walk;
+          note_long(S, is_long[j]);
         }
       };
-      auto row_of = [&](int32_t v, int32_t& off, int32_t& len, int* chunk_count) {
+      auto row_of = [&](int32_t v, int32_t& off, int32_t& len) {
         const int2 mt = p.out_meta[v];
-        if (mt.y <= p.light) {
-          off = mt.x;
-          len = mt.y;
-        } else {
-          emit_chunks(p, chunk_count, v, mt.x, mt.y);
-        }
+        off = mt.x;
+        len = mt.y;
       };
       while (front_count > 0 && rounds < kWalkRounds) {
         // the first rounds walk one level each (a bushy tree's levels spread over the grid); the
-        // rest kWalkLocal levels each (a deep tree's narrow levels walked without barriers)
-        const bool local = rounds >= kWalkGlobal;
+        // rest kWalkLocal levels each (a deep tree's narrow levels walked without barriers), but
+        // one level over a frontier with long rows, whose chunks the whole grid walks
+        const bool early = rounds < kWalkGlobal;
+        const bool one_level = early || long_front;
         int* spill = (rounds & 1) ? p.near_b : p.near_a;
         int* spill_count = &c->ring_jump[rounds % 3];
         int* chunk_count = &c->ring_chunk[cstep % 3];
         if (tid == 0) {
           st(&c->ring_jump[(rounds + 1) % 3], 0);
-          st(&c->ring_chunk[(cstep + 1) % 3], 0);
+          if (long_front) st(&c->ring_chunk[(cstep + 1) % 3], 0);
         }
         ++rounds;
-        if (!local) {
+        chunk_sink long_rows{p.chunks, chunk_cap, chunk_count, long_front ? p.light_walk : INT32_MAX, 0};
+        int* flagged = early ? p.cand + found : p.cand + (found - roots);
+        int* flagged_count = early ? spill_count : &c->cand_count;
+        int* deeper_count = early ? nullptr : spill_count;
+        auto publish = [&] { stage_flush(S, flagged, flagged_count, spill, deeper_count); };
+        auto check = [&] {
+          __syncthreads();
+          const bool full = S.count[0] > kStage / 4 || S.count[1] > kStage / 4;
+          __syncthreads();  // everybody has read the counts before the next append
+          if (full) publish();
+        };
+        if (one_level) {
           tile_rows(
-              L, front_count,
+              p, L, long_rows, long_front ? round + 1 : 0, front_count,
               [&](int idx, int32_t& v, int32_t& off, int32_t& len, u64&) {
                 v = ld(&front[idx]);
-                row_of(v, off, len, chunk_count);
+                row_of(v, off, len);
               },
               [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
                 int32_t u[kSlots], w[kSlots];
-                bool add[kSlots];
+                bool add[kSlots], is_long[kSlots];
 #pragma unroll
                 for (int j = 0; j < kSlots; ++j) u[j] = act[j] ? L.vert[item[j]] : -1;
-                claim_children(act, u, slot, w, add);
+                claim_children(act, u, slot, w, add, is_long);
 #pragma unroll
-                for (int j = 0; j < kSlots; ++j) stage_append(S, 0, add[j], w[j], p.cand, &c->cand_count);
+                for (int j = 0; j < kSlots; ++j) {
+                  stage_append(S, 0, add[j], w[j], flagged, flagged_count);
+                  stage_append(S, 1, !early && add[j], w[j], spill, spill_count);
+                }
               },
-              [&](bool, int) {}, [&] { stage_flush(S, p.cand, &c->cand_count); });
+              check, [&](bool, int) {}, publish);
         } else {
           const int G = static_cast<int>(gridDim.x);
           const int ts = min(kBlock, max(1, (front_count + G - 1) / G));
@@ -775,36 +976,36 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
             for (int level = 0; level < kWalkLocal && spent < kLocalEdgeBudget; ++level) {
               const int items = W.count[q];  // uniform: LDS after a workgroup barrier
               if (items == 0) break;
-              expand_tile(
-                  L, items,
+              spent += expand_tile(
+                  p, L, long_rows, items,
                   [&](int i, int32_t& v, int32_t& off, int32_t& len, u64&) {
                     v = W.item[q][i];
-                    row_of(v, off, len, chunk_count);
+                    row_of(v, off, len);
                   },
+                  [] {},
                   [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
                     int32_t u[kSlots], w[kSlots];
-                    bool add[kSlots];
+                    bool add[kSlots], is_long[kSlots];
 #pragma unroll
                     for (int j = 0; j < kSlots; ++j) u[j] = act[j] ? L.vert[item[j]] : -1;
-                    claim_children(act, u, slot, w, add);
+                    claim_children(act, u, slot, w, add, is_long);
 #pragma unroll
                     for (int j = 0; j < kSlots; ++j) {
                       // the child joins the next local level, or the next round's frontier when
-                      // the level is full
-                      const int at = add[j] ? atomicAdd(&W.count[q ^ 1], 1) : 0;
-                      if (add[j] && at < kBlock) W.item[q ^ 1][at] = w[j];
-                      stage_append(S, 0, add[j], w[j], p.cand, &c->cand_count);
+                      // the level is full or its row is long
+                      const int at = add[j] && !is_long[j] ? atomicAdd(&W.count[q ^ 1], 1) : kBlock;
+                      if (at < kBlock) W.item[q ^ 1][at] = w[j];
+                      stage_append(S, 0, add[j], w[j], flagged, flagged_count);
                       stage_append(S, 1, add[j] && at >= kBlock, w[j], spill, spill_count);
                     }
                   },
-                  [&](bool, int) {});
-              spent += L.start[items];  // the level's edges (LDS after the expansion's barrier: uniform)
+                  check, [&](bool, int) {});
               if (threadIdx.x == 0) {
                 W.count[q] = 0;
                 W.count[q ^ 1] = min(W.count[q ^ 1], kBlock);
               }
               if (S.count[0] > kStage / 2 || S.count[1] > kStage / 2) {
-                stage_flush(S, p.cand, &c->cand_count, spill, spill_count);  // uniform: LDS after a barrier
+                publish();  // uniform: LDS after a barrier
               }
               __syncthreads();
               q ^= 1;
@@ -815,43 +1016,45 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
               const int i = base + lane();
               stage_append(S, 1, i < left, i < left ? W.item[q][i] : -1, spill, spill_count);
             }
-            stage_flush(S, p.cand, &c->cand_count, spill, spill_count);
+            check();  // and a workgroup barrier before the next tile's levels
           }
         }
-        DYNG_GRID_SYNC();
-        // long rows: their chunks, by every workgroup; the children join the next frontier
-        const int nchunks = uniform(static_cast<int>(min(static_cast<int64_t>(ld(chunk_count)), p.chunk_cap)));
-        ++cstep;
-        if (nchunks > 0) {
-          chunk_rows(p, nchunks, [&](const bool (&act)[kSlots], const int32_t (&u)[kSlots], const int (&slot)[kSlots]) {
-            int32_t w[kSlots];
-            bool add[kSlots];
-            claim_children(act, u, slot, w, add);
+        // long rows: their chunks, by every wave of the grid; the children join the next frontier
+        if (long_front) {
+          int nchunks = 0;
+          DYNG_FLUSH_AND_CHUNKS_WAIT(nchunks, flagged, flagged_count, spill, deeper_count);
+          ++cstep;
+          __syncthreads();  // the flush has read the stage
+          chunk_rows(
+              p, p.chunks, nchunks, [](int32_t, int) {},
+              [&](const bool (&act)[kSlots], const int32_t (&u)[kSlots], const int (&slot)[kSlots]) {
+                int32_t w[kSlots];
+                bool add[kSlots], is_long[kSlots];
+                claim_children(act, u, slot, w, add, is_long);
 #pragma unroll
-            for (int j = 0; j < kSlots; ++j) {
-              stage_append(S, 0, add[j], w[j], p.cand, &c->cand_count);
-              stage_append(S, 1, local && add[j], w[j], spill, spill_count);
-            }
-          });
-          stage_flush(S, p.cand, &c->cand_count, spill, spill_count);
-          DYNG_GRID_SYNC();
+                for (int j = 0; j < kSlots; ++j) {
+                  stage_append(S, 0, add[j], w[j], flagged, flagged_count);
+                  stage_append(S, 1, !early && add[j], w[j], spill, spill_count);
+                }
+              },
+              [](int32_t) {}, check);
         }
-        if (!local) {
+        publish();
+        DYNG_GRID_SYNC_SENT(early ? 0 : 1, front_count, long_front);  // the children, or the next round's own list
+        if (early) {
           // the next round starts from this level's children, right after it in the list
-          lo = hi;
-          hi = uniform(ld(&c->cand_count));
-          front = p.cand + lo;
-          front_count = hi - lo;
+          front = p.cand + found;
+          found += front_count;
         } else {
           front = spill;
-          front_count = uniform(ld(spill_count));
         }
       }
       if (tid == 0) st(&c->rounds, rounds);
-      hi = uniform(ld(&c->cand_count));  // every flagged vertex (no append after the barrier)
-      jump_items = hi;
+      earlier = found - roots;
+      const int all = earlier + uniform(ld(&c->cand_count));  // every flagged vertex (no append after the barrier)
+      jump_items = all;
       if (front_count > 0) {
-        // deep: pointer jumping from every vertex flagged so far (they are cand[0, hi)). Its
+        // deep: pointer jumping from every vertex flagged so far (they are cand[0, all)). Its
         // rounds continue the ring where the walk stopped: slot `rounds % 3` was cleared during
         // the last round and nobody reads it, while the last round's count may still be unread
         // by slower workgroups and must not be touched here.
@@ -860,7 +1063,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
         jump = true;
         jump_slot = rounds;
       } else {
-        inv = hi;
+        inv = all;
       }
     }
     if (jump) {
@@ -899,9 +1102,9 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
               }
             }
           }
-          stage_append(S, 0, flagged, v, p.cand, &c->cand_count);
+          stage_append(S, 0, flagged, v, p.cand + earlier, &c->cand_count);
           stage_append(S, 1, keep, v, out, out_count);
-          stage_flush(S, p.cand, &c->cand_count, out, out_count);
+          stage_flush(S, p.cand + earlier, &c->cand_count, out, out_count);
         }
         DYNG_GRID_SYNC();
         count = uniform(ld(out_count));
@@ -912,7 +1115,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
         if (tid == 0) atomicOr(&c->error_bits, DYNG_HIP_DEVICE_ERROR_PARENT_CYCLE);
         return;  // uniform
       }
-      inv = uniform(ld(&c->cand_count));  // nothing appends to it after the last round's barrier
+      inv = earlier + uniform(ld(&c->cand_count));  // nothing appends to it after the last round's barrier
     }
     // ---- C: invalidate the flagged vertices (stamped when flagged) and claim the insertion
     // heads that are not invalidated, in one phase ----
@@ -922,6 +1125,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
       const int32_t v = ld(&p.cand[i]);
       st(&p.flag[v], 0);
       st(&p.packed[v], packed_inf);
+      note_long(S, p.in_meta[v].y > p.light);
     }
     if (tid == 0) st(&c->invalidated, inv);
     // A tree from outside: the insertion heads that are not invalidated pull over all their
@@ -935,10 +1139,12 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
         v = p.ins_dst[i];
         add = v >= 0 && v != p.source && claim_first(p, v, generation, first);
       }
+      note_long(S, add && p.in_meta[v].y > p.light);
       append(p.cand + inv, &c->heads_count, add, v);
       append(p.touched, &c->touched_count, first, v);
     }
-    DYNG_GRID_SYNC();
+    bool long_pull = false;  // a candidate of the pull has an in-row past `light`
+    DYNG_GRID_SYNC_SENT(0, sent, long_pull);
     // ---- D: pull ----
     ++generation;
     const int cands = inv + uniform(ld(&c->heads_count));
@@ -948,7 +1154,13 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
       c->pull_vertices = cands + (p.check_cycles ? 0 : p.num_ins);
     }
     int* chunk_count = &c->ring_chunk[cstep % 3];
-    if (tid == 0) st(&c->ring_chunk[(cstep + 1) % 3], 0);
+    if (tid == 0 && long_pull) st(&c->ring_chunk[(cstep + 1) % 3], 0);
+    auto check = [&] {
+      __syncthreads();
+      const bool full = S.count[0] > kStage / 4 || S.count[2] > kStage / 4;
+      __syncthreads();  // everybody has read the counts before the next append
+      if (full) stage_flush(S, p.frontier, &c->frontier_count);
+    };
     if (!p.check_cycles) {
       // The engine's own tree is canonical: for a head v that was not invalidated, every in-edge
       // that was there before the batch and not reweighted offers at least v's old word (no
@@ -968,21 +1180,17 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
         }
         pull_commit(p, best != packed_inf, v, best, generation, S, &c->frontier_count, &c->min_frontier);
       }
-      stage_flush(S, p.frontier, &c->frontier_count);
+      check();
     }
-    tile_rows(
-        L, cands,
+    chunk_sink long_rows{p.chunks, chunk_cap, chunk_count, long_pull ? p.light : INT32_MAX, 0};
+    const int pulled = tile_rows(
+        p, L, long_rows, long_pull ? round + 1 : 0, cands,
         [&](int idx, int32_t& v, int32_t& off, int32_t& len, u64& word) {
           v = ld(&p.cand[idx]);
           const int2 mt = p.in_meta[v];
           word = packed_inf;  // the best offer so far
-          if (mt.y <= p.light) {
-            off = mt.x;
-            len = mt.y;
-            atomicAdd(pull_edges, static_cast<unsigned long long>(mt.y));
-          } else {
-            emit_chunks(p, chunk_count, v, mt.x, mt.y);
-          }
+          off = mt.x;
+          len = mt.y;
         },
         [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
           int32_t u[kSlots], wt[kSlots];
@@ -1000,53 +1208,48 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
             if (act[j] && o < L.word[item[j]]) atomicMin(&L.word[item[j]], o);
           }
         },
+        check,
         [&](bool valid, int item) {
           pull_commit(p, valid, valid ? L.vert[item] : -1, valid ? L.word[item] : packed_inf, generation, S,
                       &c->frontier_count, &c->min_frontier);
         },
         [&] { stage_flush(S, p.frontier, &c->frontier_count); });
-    DYNG_GRID_SYNC();
-    const int nchunks = uniform(static_cast<int>(min(static_cast<int64_t>(ld(chunk_count)), p.chunk_cap)));
-    ++cstep;
-    if (nchunks > 0) {
-      const int wave = tid / 64;
-      const int waves = threads / 64;
-      for (int q = wave; q < nchunks; q += waves) {
-        const int4 ch = ld_chunk(&p.chunks[q]);
-        u64 best = packed_inf;
-        for (int e = ch.y + lane(); e < ch.z; e += 64) {
-          const u64 o = pull_offer(p, p.in_nbr[e], p.in_w[e]);
-          best = o < best ? o : best;
-        }
-        if (lane() == 0) atomicAdd(pull_edges, static_cast<unsigned long long>(ch.z - ch.y));
-        best = wave_min(best);
-        if (lane() == 0) {
-          const u64 current = ld(&p.packed[ch.x]);
-          if (best < current) {
-            const u64 old = atomicMin(&p.packed[ch.x], best);
-            bool first = false;
-            if (best < old && p.pk.distance(best) == p.pk.distance(old)) first = mark_changed(p, ch.x);
-            if (p.pk.distance(best) < p.pk.distance(old)) {
-              atomicMin(&c->min_frontier, p.pk.distance(best));
-              if (claim_first(p, ch.x, generation, first)) {
-                const int slot = atomicAdd(&c->frontier_count, 1);
-                st(&p.frontier[slot], ch.x);
-              }
+    if (threadIdx.x == 0) atomicAdd(pull_edges, static_cast<unsigned long long>(pulled));
+    if (long_pull) {
+      // long rows: each chunk's best offer, by every wave of the grid
+      int nchunks = 0;
+      DYNG_FLUSH_AND_CHUNKS_WAIT(nchunks, p.frontier, &c->frontier_count, nullptr, nullptr);
+      ++cstep;
+      __syncthreads();  // the flush has read the stage
+      u64 best = packed_inf;
+      chunk_rows(
+          p, p.chunks, nchunks,
+          [&](int32_t, int edges) {
+            best = packed_inf;
+            if (lane() == 0) atomicAdd(pull_edges, static_cast<unsigned long long>(edges));
+          },
+          [&](const bool (&act)[kSlots], const int32_t (&)[kSlots], const int (&slot)[kSlots]) {
+#pragma unroll
+            for (int j = 0; j < kSlots; ++j) {
+              const u64 o = act[j] ? pull_offer(p, p.in_nbr[slot[j]], p.in_w[slot[j]]) : packed_inf;
+              best = o < best ? o : best;
             }
-            if (first) st(&p.touched[atomicAdd(&c->touched_count, 1)], ch.x);
-          }
-        }
-      }
-      DYNG_GRID_SYNC();
+          },
+          [&](int32_t v) {
+            best = wave_min(best);
+            pull_commit(p, lane() == 0, v, best, generation, S, &c->frontier_count, &c->min_frontier);
+          },
+          check);
     }
-    frontier_count = uniform(ld(&c->frontier_count));
+    stage_flush(S, p.frontier, &c->frontier_count);
+    DYNG_GRID_SYNC_SENT(0, frontier_count, long_near);
   }
 
   // ---- E: near-far propagation (the frontier's smallest distance came with the pull, or is the
   // source's 0) ----
   if (tid == 0) c->t_phase[2] = __builtin_amdgcn_s_memrealtime();
   u64 local = packed_inf;
-  const u64 smallest = p.from_scratch ? 0 : uniform(ld(&c->min_frontier));
+  const u64 smallest = kSolve ? 0 : uniform(ld(&c->min_frontier));
   u64 threshold = (smallest == packed_inf ? 0 : smallest) + p.delta;
   int* current = p.near_a;
   int* next = p.near_b;
@@ -1061,7 +1264,6 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
   int near_count = frontier_count;
   int iterations = 0, epochs = 0;
   long long pushes = 0;
-  int pending = 0;  // chunks of long rows the previous relax iteration left for the next one
   // every relax iteration expands a vertex whose distance fell since its last expansion; a run
   // past this bound is a bug: stop with an internal error instead of spinning
   const long long guard = 4LL * n + 100000;
@@ -1070,42 +1272,38 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
       if (tid == 0) atomicOr(&c->error_bits, DYNG_HIP_DEVICE_ERROR_INTERNAL);
       break;
     }
-    if (near_count > 0 || pending > 0) {
-      // -- one relax iteration, one grid barrier: rows up to `light` edges edge-balanced per
-      // workgroup; a longer row is cut into chunks of chunk_edges, which every wave of the grid
-      // relaxes at the start of the next iteration, before its tile (the chunks of iteration k
-      // and k + 1 sit in the two halves of the chunk list; a vertex a chunk improves is claimed
-      // with the next iteration's generation and expanded one iteration later, and the fixed
-      // point, so the tree, is the same). After the first kRelaxGlobal iterations of a repair, an
-      // iteration over a narrow near frontier lets each workgroup relax its share for up to
-      // kRelaxLocal rounds on its own: the vertices it claims go to its next local level (LDS)
-      // rather than to the next near list, each round claiming with a generation of its own
-      // (generation0 + round * workgroups + workgroup), so a vertex improved after a workgroup
-      // expanded it is claimed again and expanded again (every improvement is expanded, as in a
-      // global iteration; the fixed point, and so the tree, is the same). A level past LDS and
-      // the last level go to the next near list, once per vertex (the `ancestor` array, free in
-      // this phase, tags them with the iteration). The deep, narrow repairs of a high-diameter
-      // graph take hundreds of iterations; each global one costs a grid barrier and a list round
-      // trip --
-      // (a local iteration takes workgroups * kRelaxLocal generations: past kLocalGenerations
-      // the iterations stay global, one generation each, so a run of millions of levels cannot
-      // carry the stamps past INT32_MAX). An iteration with chunks to relax is global.
-      const bool local = !p.from_scratch && iterations >= kRelaxGlobal && pending == 0 &&
+    if (near_count > 0) {
+      // -- one relax iteration: rows up to `light` edges edge-balanced per workgroup; a longer row
+      // is cut into chunks of chunk_edges, which every wave of the grid relaxes once the split
+      // barrier says they are all published (each workgroup arrives there before it expands its
+      // own rows, so the wait is over when it gets there), then the grid barrier. One hub row in a
+      // tile would keep the grid waiting on its workgroup otherwise. Whoever lists a vertex looks
+      // at its row's length, so an iteration without long rows takes one barrier. After the first
+      // kRelaxGlobal iterations, an iteration over a narrow near frontier without long rows lets
+      // each workgroup relax its share for up to kRelaxLocal rounds on its own: the vertices it
+      // claims go to its next local level (LDS) rather than to the next near list, each round
+      // claiming with a generation of its own (generation0 + round * workgroups + workgroup), so a
+      // vertex improved after a workgroup expanded it is claimed again and expanded again (every
+      // improvement is expanded, as in a global iteration; the fixed point, and so the tree, is the
+      // same). A long row, a level past LDS and the last level go to the next near list, once per
+      // vertex (the `ancestor` array, free in this phase, tags them with the iteration). The deep,
+      // narrow frontiers of a high-diameter graph take hundreds of iterations; each global one
+      // costs a grid barrier and a list round trip (a local iteration takes workgroups *
+      // kRelaxLocal generations: past kLocalGenerations the iterations stay global, one generation
+      // each, so a run of millions of levels cannot carry the stamps past INT32_MAX).
+      const bool local = !long_near && iterations >= kRelaxGlobal &&
                          near_count <= static_cast<int>(gridDim.x) * kRelaxNarrow && generation < kLocalGenerations;
       ++iterations;
       pushes += near_count;
       const int gen0 = generation + 1;
-      // a global iteration claims with one generation; a local one reserves one per workgroup
-      // and round
+      // a global iteration claims with one generation; a local one reserves one per workgroup and
+      // round
       generation += local ? static_cast<int>(gridDim.x) * kRelaxLocal : 1;
       int* next_count = &c->ring_near[step % 3];
       int* chunk_count = &c->ring_chunk[cstep % 3];
-      const int64_t chunk_half = p.chunk_cap / 2;
-      int4* chunk_out = p.chunks + (cstep & 1) * chunk_half;               // this iteration's chunks
-      const int4* chunk_in = p.chunks + ((cstep + 1) & 1) * chunk_half;    // the previous one's
       if (tid == 0) {
         st(&c->ring_near[(step + 1) % 3], 0);
-        st(&c->ring_chunk[(cstep + 1) % 3], 0);
+        if (long_near) st(&c->ring_chunk[(cstep + 1) % 3], 0);
       }
       int* far_list = far_of(fb);
       int* far_counter = &c->far_count[fb];
@@ -1113,6 +1311,13 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
       const int* cur = seeding ? seed : current;
       seed = nullptr;
       const int tag = local ? -2 - generation : 0;  // a local iteration's list tag: below every vertex id and -1
+      chunk_sink long_rows{p.chunks, chunk_cap, chunk_count, long_near ? p.light : INT32_MAX, 0};
+      auto check = [&] {
+        __syncthreads();
+        const bool full = S.count[0] > kStage / 4 || S.count[1] > kStage / 4 || S.count[2] > kStage / 4;
+        __syncthreads();  // everybody has read the counts before the next append
+        if (full) stage_flush(S, next, next_count, far_list, far_counter);
+      };
       auto load_row = [&](int32_t v, int32_t& off, int32_t& len, u64& word) {
         const int2 mt = p.out_meta[v];  // issued together with the word's load
         word = ld(&p.packed[v]);
@@ -1122,65 +1327,34 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
           stage_append(S, 1, atomicExch(&p.in_far[v], 1) == 0, v, far_list, far_counter);
           return;
         }
-        if (mt.y <= p.light) {
-          off = mt.x;
-          len = mt.y;
-          atomicAdd(relax_edges, static_cast<unsigned long long>(mt.y));
-        } else {
-          emit_chunks_to(p, chunk_out, chunk_half, chunk_count, v, mt.x, mt.y);
-        }
+        off = mt.x;
+        len = mt.y;
       };
-      if (pending > 0) {
-        // the previous iteration's chunks: one wave per chunk, grid-wide, then a flush (a tile
-        // may not follow)
-        const near_sink sink{nullptr, 0, nullptr, 0};
-        const int wave = tid / 64;
-        const int waves = threads / 64;
-        for (int q = wave; q < pending; q += waves) {
-          const int4 ch = ld_chunk(&chunk_in[q]);
-          const int32_t u = ch.x;
-          const u64 word = ld(&p.packed[u]);
-          const u64 du = p.pk.distance(word);
-          if (lane() == 0) atomicAdd(relax_edges, static_cast<unsigned long long>(ch.z - ch.y));
-          for (int b = ch.y; b < ch.z; b += 64 * kSlots) {
-            bool act[kSlots];
-            int32_t uu[kSlots];
-            u64 dd[kSlots];
-            int slot[kSlots];
+      auto relax_tile = [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots], int gen,
+                            const near_sink& sink) {
+        int32_t u[kSlots];
+        u64 du[kSlots];
 #pragma unroll
-            for (int j = 0; j < kSlots; ++j) {
-              const int e = b + j * 64 + lane();
-              act[j] = word != packed_inf && e < ch.z;
-              uu[j] = u;
-              dd[j] = du;
-              slot[j] = act[j] ? e : 0;
-            }
-            relax_slots(p, act, uu, dd, slot, threshold, generation, S, next, next_count, far_list, far_counter,
-                        relax_improved, sink);
-          }
+        for (int j = 0; j < kSlots; ++j) {
+          u[j] = act[j] ? L.vert[item[j]] : 0;
+          du[j] = act[j] ? p.pk.distance(L.word[item[j]]) : 0;
         }
-        stage_flush(S, next, next_count, far_list, far_counter);
-      }
+        relax_slots<kSolve>(p, act, u, du, slot, threshold, gen, S, next, next_count, far_list, far_counter,
+                            relax_improved, sink);
+      };
+      int expanded = 0;  // edges of the rows this workgroup expanded itself
       if (!local) {
         const near_sink sink{nullptr, 0, nullptr, 0};
-        tile_rows(
-            L, near_count,
+        expanded = tile_rows(
+            p, L, long_rows, long_near ? round + 1 : 0, near_count,
             [&](int idx, int32_t& v, int32_t& off, int32_t& len, u64& word) {
               v = ld(&cur[idx]);
               load_row(v, off, len, word);
             },
             [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
-              int32_t u[kSlots];
-              u64 du[kSlots];
-#pragma unroll
-              for (int j = 0; j < kSlots; ++j) {
-                u[j] = act[j] ? L.vert[item[j]] : 0;
-                du[j] = act[j] ? p.pk.distance(L.word[item[j]]) : 0;
-              }
-              relax_slots(p, act, u, du, slot, threshold, generation, S, next, next_count, far_list, far_counter,
-                          relax_improved, sink);
+              relax_tile(act, item, slot, generation, sink);
             },
-            [&](bool, int) {}, [&] { stage_flush(S, next, next_count, far_list, far_counter); });
+            check, [&](bool, int) {}, [&] { stage_flush(S, next, next_count, far_list, far_counter); });
       } else {
         const int G = static_cast<int>(gridDim.x);
         const int ts = min(kBlock, max(1, (near_count + G - 1) / G));
@@ -1201,25 +1375,17 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
             if (round > 0 && threadIdx.x == 0) *local_pushes += static_cast<unsigned long long>(items);
             const int gen = gen0 + round * G + static_cast<int>(blockIdx.x);
             const near_sink sink{&W, q ^ 1, p.ancestor, tag};
-            expand_tile(
-                L, items,
+            spent += expand_tile(
+                p, L, long_rows, items,
                 [&](int i, int32_t& v, int32_t& off, int32_t& len, u64& word) {
                   v = W.item[q][i];
                   load_row(v, off, len, word);
                 },
+                [] {},
                 [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
-                  int32_t u[kSlots];
-                  u64 du[kSlots];
-#pragma unroll
-                  for (int j = 0; j < kSlots; ++j) {
-                    u[j] = act[j] ? L.vert[item[j]] : 0;
-                    du[j] = act[j] ? p.pk.distance(L.word[item[j]]) : 0;
-                  }
-                  relax_slots(p, act, u, du, slot, threshold, gen, S, next, next_count, far_list, far_counter,
-                              relax_improved, sink);
+                  relax_tile(act, item, slot, gen, sink);
                 },
-                [&](bool, int) {});
-            spent += L.start[items];  // the round's edges (LDS after the expansion's barrier: uniform)
+                check, [&](bool, int) {});
             if (threadIdx.x == 0) {
               W.count[q] = 0;
               W.count[q ^ 1] = min(W.count[q ^ 1], kBlock);
@@ -1230,6 +1396,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
             __syncthreads();
             q ^= 1;
           }
+          expanded += spent;
           // the level the last round left: the next near list, once per vertex
           const int left = W.count[q];
           for (int base = static_cast<int>(threadIdx.x) - lane(); base < left; base += kBlock) {
@@ -1238,13 +1405,40 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
             const bool add = i < left && atomicExch(&p.ancestor[v], tag) != tag;
             stage_append(S, 0, add, v, next, next_count);
           }
-          stage_flush(S, next, next_count, far_list, far_counter);
+          check();  // and a workgroup barrier before the next tile's levels
         }
       }
-      DYNG_GRID_SYNC();
-      pending = uniform(static_cast<int>(min(static_cast<int64_t>(ld(chunk_count)), chunk_half)));
-      ++cstep;
-      near_count = uniform(ld(next_count));
+      if (threadIdx.x == 0) atomicAdd(relax_edges, static_cast<unsigned long long>(expanded));
+      if (long_near) {
+        // the long rows' chunks
+        int nchunks = 0;
+        DYNG_FLUSH_AND_CHUNKS_WAIT(nchunks, next, next_count, far_list, far_counter);
+        ++cstep;
+        __syncthreads();  // the flush has read the stage
+        const near_sink sink{nullptr, 0, nullptr, 0};
+        u64 word = packed_inf, du = 0;
+        chunk_rows(
+            p, p.chunks, nchunks,
+            [&](int32_t v, int edges) {
+              word = ld(&p.packed[v]);
+              du = p.pk.distance(word);
+              if (lane() == 0) atomicAdd(relax_edges, static_cast<unsigned long long>(edges));
+            },
+            [&](const bool (&act)[kSlots], const int32_t (&u)[kSlots], const int (&slot)[kSlots]) {
+              bool on[kSlots];
+              u64 dd[kSlots];
+#pragma unroll
+              for (int j = 0; j < kSlots; ++j) {
+                on[j] = act[j] && word != packed_inf;
+                dd[j] = du;
+              }
+              relax_slots<kSolve>(p, on, u, dd, slot, threshold, generation, S, next, next_count, far_list, far_counter,
+                                  relax_improved, sink);
+            },
+            [](int32_t) {}, check);
+      }
+      stage_flush(S, next, next_count, far_list, far_counter);
+      DYNG_GRID_SYNC_SENT(0, near_count, long_near);
       ++step;
       int* t = current;
       current = next;
@@ -1283,13 +1477,13 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
         to_near = near && claim_first(p, v, generation, first);
         keep = !near;
       }
+      note_long(S, to_near && p.out_meta[v].y > p.light);
       stage_append(S, 0, to_near, v, current, split_count);
       stage_append(S, 1, keep, v, far_of(fb ^ 1), &c->far_count[fb ^ 1]);
       stage_append(S, 2, first, v, S.list2, S.counter2);
     }
     stage_flush(S, current, split_count, far_of(fb ^ 1), &c->far_count[fb ^ 1]);
-    DYNG_GRID_SYNC();
-    near_count = uniform(ld(split_count));
+    DYNG_GRID_SYNC_SENT(0, near_count, long_near);
     ++step;
     if (tid == 0) st(&c->far_count[fb], 0);
     fb ^= 1;
@@ -1316,7 +1510,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
         ++changed;
       }
     };
-    if (p.from_scratch) {
+    if constexpr (kSolve) {
       for (int v = tid; v < n; v += threads) unpack(v);
     } else {
       // the invalidated vertices (cand[0, invalidated)) and the vertices whose first stamp of
@@ -1378,6 +1572,9 @@ __global__ void __launch_bounds__(kBlock, kWaves) sssp_fused_kernel(engine_param
 #undef DYNG_GRID_SYNC
 #undef DYNG_GRID_SYNC_FENCED
 #undef DYNG_GRID_SYNC_AS
+#undef DYNG_GRID_SYNC_SENT
+#undef DYNG_FLUSH_AND_CHUNKS_WAIT
+#undef DYNG_GRID_LEAVE_UNLESS
 
 }  // namespace dyng_hip
 
@@ -1414,7 +1611,7 @@ struct dyng_hip_workspace {
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
   hipGraphNode_t graph_kernel = nullptr;
-  bool graph_narrow = false;  ///< which build the graph's kernel node launches
+  void (*graph_build)(dyng_hip::engine_params) = nullptr;  ///< the build the graph's kernel node launches
   ~dyng_hip_workspace() {
     if (graph_exec != nullptr) (void)hipGraphExecDestroy(graph_exec);
     if (graph != nullptr) (void)hipGraphDestroy(graph);
@@ -1429,8 +1626,19 @@ namespace {
 
 /// The build of the persistent kernel a grid takes: the 128-VGPR one when the grid fits at its
 /// occupancy (one workgroup per CU), else the 64-VGPR one.
-const void* fused_kernel(bool narrow) {
-  return narrow ? reinterpret_cast<const void*>(sssp_fused_kernel<4>) : reinterpret_cast<const void*>(sssp_fused_kernel<8>);
+using fused_fn = void (*)(engine_params);
+fused_fn fused_kernel(bool narrow, bool solve) {
+  if (solve) return narrow ? sssp_fused_kernel<4, true> : sssp_fused_kernel<8, true>;
+  return narrow ? sssp_fused_kernel<4, false> : sssp_fused_kernel<8, false>;
+}
+/// Workgroups per CU of the 64-VGPR (or the 128-VGPR, `narrow`) builds: what both fit.
+int resident_per_cu(bool narrow) {
+  int fit[2] = {0, 0};
+  for (int solve = 0; solve < 2; ++solve) {
+    DYNG_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &fit[solve], reinterpret_cast<const void*>(fused_kernel(narrow, solve != 0)), kBlock, 0));
+  }
+  return std::min(fit[0], fit[1]);
 }
 bool narrow_grid(int blocks, int occupancy_narrow, int cu_count) {
   return occupancy_narrow >= 1 && blocks <= occupancy_narrow * cu_count;
@@ -1473,8 +1681,8 @@ void ws_reserve(dyng_hip_workspace* ws, int64_t n, int64_t slots, hipStream_t s)
   ws->bar.reserve(1);
   if (ws->cu_count == 0) {
     DYNG_HIP_TRY(hipDeviceGetAttribute(&ws->cu_count, hipDeviceAttributeMultiprocessorCount, ws->device));
-    DYNG_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&ws->occupancy, fused_kernel(false), kBlock, 0));
-    DYNG_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&ws->occupancy_narrow, fused_kernel(true), kBlock, 0));
+    ws->occupancy = resident_per_cu(false);
+    ws->occupancy_narrow = resident_per_cu(true);
     if (ws->occupancy < 1) fail(DYNG_HIP_NOT_SUPPORTED, "dyng: sssp: the persistent kernel does not fit on a CU");
   }
 }
@@ -1575,11 +1783,9 @@ void engine_setup(const dyng_hip_sssp_run* run, bool update, engine_params& p, i
   p.max_rounds = rounds + 1;
   p.distances = reinterpret_cast<long long*>(run->distances);
   p.parents = run->parents;
-  // rows up to 8192 edges in a repair's tiles (4096 measured 6 % slower on RMAT-22 repairs: more
-  // rows waited a relax iteration as chunks), up to 4096 in a solve's (its wide frontiers balance
-  // better with the long rows in chunks: 8192 measured 5.9 -> 8.7 ms on RMAT-22)
-  p.light = run->tuning.light_degree > 0 ? run->tuning.light_degree : (p.from_scratch ? 4096 : 8192);
-  p.chunk_edges = run->tuning.chunk_edges > 0 ? std::max(16, run->tuning.chunk_edges) : 256;
+  p.light = run->tuning.light_degree > 0 ? run->tuning.light_degree : (p.from_scratch ? kLightSolve : kLightRelax);
+  p.light_walk = run->tuning.light_degree > 0 ? run->tuning.light_degree : kLightWalk;
+  p.chunk_edges = run->tuning.chunk_edges > 0 ? std::max(16, run->tuning.chunk_edges) : kChunkEdges;
   // the real-time counter runs at 100 MHz: 100 ticks per microsecond
   timeout_us = run->tuning.barrier_timeout_us > 0   ? run->tuning.barrier_timeout_us
                : run->tuning.barrier_timeout_us == 0 ? 4000000
@@ -1725,7 +1931,7 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
                                    ws->frontier.p, ws->near_a.p, ws->near_b.p, ws->far_a.p, ws->far_b.p,
                                    ws->touched.p, ws->chunks.p, ws->chunk_cap, ws->ctl.p, ws->bar.p});
   const int blocks = grid_blocks(run->tuning, ws->occupancy, ws->cu_count, p.from_scratch != 0);
-  const bool narrow = narrow_grid(blocks, ws->occupancy_narrow, ws->cu_count);
+  const fused_fn kernel = fused_kernel(narrow_grid(blocks, ws->occupancy_narrow, ws->cu_count), p.from_scratch != 0);
   control* hc = ws->host_ctl.p;
   std::memset(hc, 0, sizeof(control));
   hc->min_frontier = packed_inf;
@@ -1738,14 +1944,14 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
   void* args[] = {&p};
   if (run->tuning.launch == DYNG_HIP_LAUNCH_GRAPH) {
     hipKernelNodeParams kp{};
-    kp.func = const_cast<void*>(fused_kernel(narrow));
+    kp.func = reinterpret_cast<void*>(kernel);
     kp.gridDim = dim3(blocks);
     kp.blockDim = dim3(kBlock);
     kp.sharedMemBytes = 0;
     kp.kernelParams = args;
     kp.extra = nullptr;
-    if (ws->graph_exec != nullptr && ws->graph_narrow != narrow) {
-      // the other build of the kernel: the graph is built again around it
+    if (ws->graph_exec != nullptr && ws->graph_build != kernel) {
+      // another build of the kernel: the graph is built again around it
       DYNG_HIP_TRY(hipGraphExecDestroy(ws->graph_exec));
       DYNG_HIP_TRY(hipGraphDestroy(ws->graph));
       ws->graph_exec = nullptr;
@@ -1753,7 +1959,7 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
     }
     if (ws->graph_exec == nullptr) {
       // built once per workspace: the control block, the barrier and the events never move
-      ws->graph_narrow = narrow;
+      ws->graph_build = kernel;
       DYNG_HIP_TRY(hipGraphCreate(&ws->graph, 0));
       hipGraphNode_t reset, start, stop, down;
       grid_sync_state* bar = ws->bar.p;
@@ -1778,11 +1984,7 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
   } else {
     hipLaunchKernelGGL(k_reset_barrier, dim3(1), dim3(64), 0, s, ws->bar.p, ws->ctl.p);
     DYNG_HIP_TRY(hipEventRecord(ws->ev_start, s));
-    if (narrow) {
-      hipLaunchKernelGGL(sssp_fused_kernel<4>, dim3(blocks), dim3(kBlock), 0, s, p);
-    } else {
-      hipLaunchKernelGGL(sssp_fused_kernel<8>, dim3(blocks), dim3(kBlock), 0, s, p);
-    }
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, s, p);
     DYNG_HIP_TRY(hipGetLastError());
     DYNG_HIP_TRY(hipEventRecord(ws->ev_stop, s));
     DYNG_HIP_TRY(hipMemcpyAsync(hc, ws->ctl.p, sizeof(control), hipMemcpyDeviceToHost, s));
@@ -1955,8 +2157,8 @@ noalloc_device& noalloc_for(int device, hipStream_t s) {
                                      hipGetErrorString(e));
   }
   DYNG_HIP_TRY(hipDeviceGetAttribute(&st.cu_count, hipDeviceAttributeMultiprocessorCount, device));
-  DYNG_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&st.occupancy, fused_kernel(false), kBlock, 0));
-  DYNG_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&st.occupancy_narrow, fused_kernel(true), kBlock, 0));
+  st.occupancy = resident_per_cu(false);
+  st.occupancy_narrow = resident_per_cu(true);
   if (st.occupancy < 1) fail(DYNG_HIP_NOT_SUPPORTED, "dyng: sssp: the persistent kernel does not fit on a CU");
   clear_scratch(ptr, DYNG_HIP_NOALLOC_SCRATCH_BYTES, s);
   DYNG_HIP_TRY(hipStreamSynchronize(s));
@@ -2017,11 +2219,8 @@ void run_engine_noalloc(const dyng_hip_sssp_run* run, hipStream_t s, dyng_hip_co
                                    reinterpret_cast<grid_sync_state*>(base + L.bar)});
   const int blocks = grid_blocks(run->tuning, st.occupancy, st.cu_count, p.from_scratch != 0);
   hipLaunchKernelGGL(k_reset_barrier, dim3(1), dim3(64), 0, s, p.bar, p.ctl);
-  if (narrow_grid(blocks, st.occupancy_narrow, st.cu_count)) {
-    hipLaunchKernelGGL(sssp_fused_kernel<4>, dim3(blocks), dim3(kBlock), 0, s, p);
-  } else {
-    hipLaunchKernelGGL(sssp_fused_kernel<8>, dim3(blocks), dim3(kBlock), 0, s, p);
-  }
+  const fused_fn kernel = fused_kernel(narrow_grid(blocks, st.occupancy_narrow, st.cu_count), p.from_scratch != 0);
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, s, p);
   DYNG_HIP_TRY(hipGetLastError());
   control* hc = &st.host_ctl;
   DYNG_HIP_TRY(hipMemcpyAsync(hc, p.ctl, sizeof(control), hipMemcpyDeviceToHost, s));
