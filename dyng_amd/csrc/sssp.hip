@@ -482,9 +482,9 @@ DYNG_DEV bool mark_changed(const engine_params& p, int32_t w) { return atomicMax
 /// far pile when it lowered w's word. Returns the lists to append w to.
 DYNG_DEV void relax_decide(const engine_params& p, bool active, int32_t u, u64 du, int32_t w, int32_t wt, u64 seen,
                            u64 threshold, int generation, bool& lowered, bool& to_near, bool& to_far, bool& first,
-                           bool& is_long) {
+                           int2& row) {
   lowered = false;
-  is_long = false;
+  row = make_int2(0, 0);
   to_near = false;
   to_far = false;
   first = false;
@@ -493,7 +493,7 @@ DYNG_DEV void relax_decide(const engine_params& p, bool active, int32_t u, u64 d
     if (nd <= p.max_distance) {
       const u64 cand = p.pk.pack(nd, u);
       if (cand < seen) {
-        const int len = p.out_meta[w].y;  // in flight together with the minimum
+        row = p.out_meta[w];  // in flight together with the minimum
         const u64 old = atomicMin(&p.packed[w], cand);
         // Any lowered word joins a list, also one lowered only to a lower parent id at the same
         // distance (fused.cuh:341-362 lists only a lower distance): the extra expansion is rare
@@ -504,7 +504,6 @@ DYNG_DEV void relax_decide(const engine_params& p, bool active, int32_t u, u64 d
           // them in scratch memory); a far vertex is stamped when it leaves the far pile
           const bool near = nd < threshold;
           to_near = near && claim_first(p, w, generation, first);
-          is_long = to_near && len > p.light;
           to_far = !near && atomicExch(&p.in_far[w], 1) == 0;
         }
       }
@@ -513,10 +512,13 @@ DYNG_DEV void relax_decide(const engine_params& p, bool active, int32_t u, u64 d
 }
 
 /// The subtree walk's and the local relax rounds' levels in LDS: two levels of up to kBlock
-/// vertices.
+/// vertices, each with its row {offset, length}, which whoever claims a vertex loads beside the
+/// claim: a level starts with the row entries, not with a round trip for the rows (the 1001^2 grid's
+/// solve, 9 epochs of narrow local rounds: 1.38 -> 1.29 ms).
 struct walk_shared {
   int count[2];
   int item[2][kBlock];
+  int2 row[2][kBlock];
 };
 
 /// Where a relax step sends the vertices it claimed for the near frontier. In a global iteration
@@ -554,18 +556,21 @@ DYNG_DEV void relax_slots(const engine_params& p, const bool (&act)[kSlots], con
   }
 #pragma unroll
   for (int j = 0; j < kSlots; ++j) {
-    bool lowered, to_near, to_far, first, is_long;
+    bool lowered, to_near, to_far, first;
+    int2 row;
     relax_decide(p, live[j], u[j], du[j], w[j], wt[j], seen[j], threshold, generation, lowered, to_near, to_far, first,
-                 is_long);
+                 row);
     const u64 better = __ballot(lowered);
     if (better == 0) continue;  // uniform per wave: nothing to count or to append
     if (lane() == 0) atomicAdd(improved, static_cast<unsigned long long>(__popcll(better)));
+    const bool is_long = to_near && row.y > p.light;
     note_long(S, is_long);
     bool to_list = to_near;
     if (to_near && !is_long && sink.local != nullptr) {
       const int at = atomicAdd(&sink.local->count[sink.q], 1);
       if (at < kBlock) {
         sink.local->item[sink.q][at] = w[j];
+        sink.local->row[sink.q][at] = row;
         to_list = false;
       }
     }
@@ -893,7 +898,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
       // kSlots out-edges (u, w) per lane: the entries, then parent[w] (the tree is read-only
       // here), then the flag claims of the tree children (rare: one in-edge of each child)
       auto claim_children = [&](const bool (&act)[kSlots], const int32_t (&u)[kSlots], const int (&slot)[kSlots],
-                                int32_t (&w)[kSlots], bool (&add)[kSlots], bool (&is_long)[kSlots]) {
+                                int32_t (&w)[kSlots], bool (&add)[kSlots], int2 (&row)[kSlots]) {
         int32_t par[kSlots];
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) w[j] = act[j] ? p.out_nbr[slot[j]] : -1;  // dead entries are negative
@@ -902,17 +907,11 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
 #pragma unroll
         for (int j = 0; j < kSlots; ++j) {
           const bool child = w[j] >= 0 && par[j] == u[j];
-          const int len = child ? p.out_meta[w[j]].y : 0;  // in flight together with the exchange
+          row[j] = child ? p.out_meta[w[j]] : make_int2(0, 0);  // in flight together with the exchange
           add[j] = child && atomicExch(&p.flag[w[j]], 1) == 0;
           if (add[j]) st(&p.stamp[w[j]], generation + 1);
-          is_long[j] = add[j] && len > p.light_walk;
-          note_long(S, is_long[j]);
+          note_long(S, add[j] && row[j].y > p.light_walk);
         }
-      };
-      auto row_of = [&](int32_t v, int32_t& off, int32_t& len) {
-        const int2 mt = p.out_meta[v];
-        off = mt.x;
-        len = mt.y;
       };
       while (front_count > 0 && rounds < kWalkRounds) {
         // the first rounds walk one level each (a bushy tree's levels spread over the grid); the
@@ -944,14 +943,17 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
               p, L, long_rows, long_front ? round + 1 : 0, front_count,
               [&](int idx, int32_t& v, int32_t& off, int32_t& len, u64&) {
                 v = ld(&front[idx]);
-                row_of(v, off, len);
+                const int2 mt = p.out_meta[v];
+                off = mt.x;
+                len = mt.y;
               },
               [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
                 int32_t u[kSlots], w[kSlots];
-                bool add[kSlots], is_long[kSlots];
+                bool add[kSlots];
+                int2 row[kSlots];
 #pragma unroll
                 for (int j = 0; j < kSlots; ++j) u[j] = act[j] ? L.vert[item[j]] : -1;
-                claim_children(act, u, slot, w, add, is_long);
+                claim_children(act, u, slot, w, add, row);
 #pragma unroll
                 for (int j = 0; j < kSlots; ++j) {
                   stage_append(S, 0, add[j], w[j], flagged, flagged_count);
@@ -965,7 +967,11 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
           for (long long t0 = static_cast<long long>(blockIdx.x) * ts; t0 < front_count;
                t0 += static_cast<long long>(G) * ts) {
             const int cnt = static_cast<int>(min(static_cast<long long>(ts), front_count - t0));
-            if (static_cast<int>(threadIdx.x) < cnt) W.item[0][threadIdx.x] = ld(&front[t0 + threadIdx.x]);
+            if (static_cast<int>(threadIdx.x) < cnt) {
+              const int32_t v = ld(&front[t0 + threadIdx.x]);
+              W.item[0][threadIdx.x] = v;
+              W.row[0][threadIdx.x] = p.out_meta[v];
+            }
             if (threadIdx.x == 0) {
               W.count[0] = cnt;
               W.count[1] = 0;
@@ -980,21 +986,26 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
                   p, L, long_rows, items,
                   [&](int i, int32_t& v, int32_t& off, int32_t& len, u64&) {
                     v = W.item[q][i];
-                    row_of(v, off, len);
+                    off = W.row[q][i].x;
+                    len = W.row[q][i].y;
                   },
                   [] {},
                   [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
                     int32_t u[kSlots], w[kSlots];
-                    bool add[kSlots], is_long[kSlots];
+                    bool add[kSlots];
+                int2 row[kSlots];
 #pragma unroll
                     for (int j = 0; j < kSlots; ++j) u[j] = act[j] ? L.vert[item[j]] : -1;
-                    claim_children(act, u, slot, w, add, is_long);
+                    claim_children(act, u, slot, w, add, row);
 #pragma unroll
                     for (int j = 0; j < kSlots; ++j) {
                       // the child joins the next local level, or the next round's frontier when
                       // the level is full or its row is long
-                      const int at = add[j] && !is_long[j] ? atomicAdd(&W.count[q ^ 1], 1) : kBlock;
-                      if (at < kBlock) W.item[q ^ 1][at] = w[j];
+                      const int at = add[j] && row[j].y <= p.light_walk ? atomicAdd(&W.count[q ^ 1], 1) : kBlock;
+                      if (at < kBlock) {
+                        W.item[q ^ 1][at] = w[j];
+                        W.row[q ^ 1][at] = row[j];
+                      }
                       stage_append(S, 0, add[j], w[j], flagged, flagged_count);
                       stage_append(S, 1, add[j] && at >= kBlock, w[j], spill, spill_count);
                     }
@@ -1029,8 +1040,9 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
               p, p.chunks, nchunks, [](int32_t, int) {},
               [&](const bool (&act)[kSlots], const int32_t (&u)[kSlots], const int (&slot)[kSlots]) {
                 int32_t w[kSlots];
-                bool add[kSlots], is_long[kSlots];
-                claim_children(act, u, slot, w, add, is_long);
+                bool add[kSlots];
+                int2 row[kSlots];
+                claim_children(act, u, slot, w, add, row);
 #pragma unroll
                 for (int j = 0; j < kSlots; ++j) {
                   stage_append(S, 0, add[j], w[j], flagged, flagged_count);
@@ -1361,7 +1373,11 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
         for (long long t0 = static_cast<long long>(blockIdx.x) * ts; t0 < near_count;
              t0 += static_cast<long long>(G) * ts) {
           const int cnt = static_cast<int>(min(static_cast<long long>(ts), near_count - t0));
-          if (static_cast<int>(threadIdx.x) < cnt) W.item[0][threadIdx.x] = ld(&cur[t0 + threadIdx.x]);
+          if (static_cast<int>(threadIdx.x) < cnt) {
+            const int32_t v = ld(&cur[t0 + threadIdx.x]);
+            W.item[0][threadIdx.x] = v;
+            W.row[0][threadIdx.x] = p.out_meta[v];
+          }
           if (threadIdx.x == 0) {
             W.count[0] = cnt;
             W.count[1] = 0;
@@ -1377,13 +1393,25 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
             const near_sink sink{&W, q ^ 1, p.ancestor, tag};
             spent += expand_tile(
                 p, L, long_rows, items,
-                [&](int i, int32_t& v, int32_t& off, int32_t& len, u64& word) {
+                [&](int i, int32_t& v, int32_t& off, int32_t& len, u64&) {
                   v = W.item[q][i];
-                  load_row(v, off, len, word);
+                  off = W.row[q][i].x;
+                  len = W.row[q][i].y;
                 },
                 [] {},
                 [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
-                  relax_tile(act, item, slot, gen, sink);
+                  // each lane reads its tail's word beside its row entry (one round trip for both);
+                  // a tail without a distance would offer nothing (weights are >= 1)
+                  int32_t u[kSlots];
+                  u64 du[kSlots];
+#pragma unroll
+                  for (int j = 0; j < kSlots; ++j) {
+                    u[j] = act[j] ? L.vert[item[j]] : 0;
+                    const u64 word = act[j] ? ld(&p.packed[u[j]]) : packed_inf;
+                    du[j] = word == packed_inf ? p.max_distance : p.pk.distance(word);
+                  }
+                  relax_slots<kSolve>(p, act, u, du, slot, threshold, gen, S, next, next_count, far_list, far_counter,
+                                      relax_improved, sink);
                 },
                 check, [&](bool, int) {});
             if (threadIdx.x == 0) {
