@@ -8,7 +8,7 @@
 //      n vertices). A tree this engine produced is walked top-down instead along its tree edges
 //      (out-edges (u, w) with parent[w] == u), touching only the invalidated region: each
 //      workgroup walks its tile of the frontier down several levels on its own (levels in LDS)
-//      between grid barriers; a walk deeper than kWalkRounds such rounds hands its unfinished
+//      between grid barriers; a walk deeper than walk_rounds such rounds hands its unfinished
 //      part to pointer jumping. A tree handed in from outside keeps pointer jumping (over
 //      compacted lists of the vertices still jumping), which also detects parent cycles.
 //   C  invalidate (word INF, stamp), then the insertion heads (fused.cuh:236-256).
@@ -49,7 +49,14 @@ constexpr int kBlock = 1024;  ///< 16 waves per workgroup; 8 waves/SIMD fit two 
 constexpr int kWaves = kBlock / 64;
 constexpr int kWalkGlobal = 2;   ///< first rounds of the subtree walk: one level each
 constexpr int kWalkLocal = 16;   ///< later rounds: levels a workgroup walks on its own between grid barriers
-constexpr int kWalkRounds = kWalkGlobal + 8;  ///< grid rounds of the walk before pointer jumping takes over
+/// Grid rounds of the subtree walk before pointer jumping takes over: kWalkRounds and one more per
+/// kWalkRoundVertices vertices. A local round of 16 narrow levels takes about 38 us; pointer jumping
+/// reads every vertex a few times (1.87 ms over the 4096^2 grid's 16.8 M, about 0.11 ns per vertex
+/// and 0.1 ms of rounds), so the walk may spend about that before it gives up. With ten rounds for
+/// every size the grid's deep subtrees handed over (walk phase 1.35 ms on average); with 64 they
+/// finish in 11.5 rounds on average (0.59 ms).
+constexpr int kWalkRounds = kWalkGlobal + 8;
+constexpr int kWalkRoundVertices = 300000;
 constexpr int kRelaxGlobal = 2;  ///< relax iterations of a repair before local rounds may start
 constexpr int kRelaxLocal = 16;  ///< local rounds of a workgroup in one relax iteration
 constexpr int kRelaxNarrow = 128; ///< a near frontier of at most this many vertices per workgroup is narrow
@@ -133,7 +140,8 @@ struct engine_params {
   packing pk;
   u64 max_distance;
   u64 delta;
-  int32_t max_rounds;
+  int32_t max_rounds;   ///< of pointer jumping
+  int32_t walk_rounds;  ///< of the subtree walk before it
   int32_t generation;
   long long* distances;
   int32_t* parents;
@@ -884,7 +892,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
       // narrow levels of a deep tree: the 4096^2 grid's walk 2.0 -> 0.4 ms). What a workgroup did
       // not reach (a level past the cap or past the LDS queue, and the children of rows long
       // enough for the chunk list) is the next round's frontier, after a grid barrier. Every flagged vertex joins the
-      // candidate list after the roots. A walk still going after kWalkRounds rounds (a deep tree)
+      // candidate list after the roots. A walk still going after walk_rounds rounds (a deep tree)
       // is finished by pointer jumping ----
       // the frontier: a range of the candidate list while rounds walk one level (the level's
       // children are appended right after it), then a list of its own. A one-level round counts
@@ -913,7 +921,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
           note_long(S, add[j] && row[j].y > p.light_walk);
         }
       };
-      while (front_count > 0 && rounds < kWalkRounds) {
+      while (front_count > 0 && rounds < p.walk_rounds) {
         // the first rounds walk one level each (a bushy tree's levels spread over the grid); the
         // rest kWalkLocal levels each (a deep tree's narrow levels walked without barriers), but
         // one level over a frontier with long rows, whose chunks the whole grid walks
@@ -1809,6 +1817,7 @@ void engine_setup(const dyng_hip_sssp_run* run, bool update, engine_params& p, i
   int rounds = 0;
   while ((1LL << rounds) < static_cast<long long>(n)) ++rounds;
   p.max_rounds = rounds + 1;
+  p.walk_rounds = kWalkRounds + static_cast<int32_t>(n / kWalkRoundVertices);
   p.distances = reinterpret_cast<long long*>(run->distances);
   p.parents = run->parents;
   p.light = run->tuning.light_degree > 0 ? run->tuning.light_degree : (p.from_scratch ? kLightSolve : kLightRelax);
