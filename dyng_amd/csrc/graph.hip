@@ -581,6 +581,8 @@ struct out_pair_params {
   const u64* keys;
   const uint32_t* vals;
   int64_t N;
+  int64_t stride;  ///< of the weight columns of pend_w and of the iop arrays
+  int64_t at;      ///< place of keys[0] among all the sorted operations
   int vbits;
   int K;
   int64_t n_before;  ///< rows that existed before the batch (classification)
@@ -619,12 +621,15 @@ struct run_pair {
   int bl, lb, ub, tl, tu;
 };
 
+/// One probe per round: a batch's operations search different rows, so each probe is a line of its own,
+/// and the lines are what bounds a large batch's pairing (1,000,000 operations on RMAT-23: 510 us with
+/// one probe per round, 552 with three, 600 with seven; 100,000 on RMAT-22: 112, 119 and 134).
 DYNG_DEV run_pair find_runs(const int32_t* row, int base_len, int len, int32_t v) {
   run_pair r;
   r.bl = base_len;
-  r.lb = row_lower_bound(row, 0, base_len, v);
+  r.lb = row_lower_bound<1>(row, 0, base_len, v);
   r.ub = row_upper_bound_from(row, r.lb, base_len, v);
-  r.tl = row_lower_bound(row, base_len, len, v);
+  r.tl = row_lower_bound<1>(row, base_len, len, v);
   r.tu = row_upper_bound_from(row, r.tl, len, v);
   return r;
 }
@@ -675,15 +680,30 @@ __global__ void __launch_bounds__(kBlock) k_check_pairs(op_layout L, const u64* 
 }
 
 /// Record where row r's operations start and end in the sorted keys (row = key >> vbits).
-DYNG_DEV void mark_row_range(const u64* keys, int64_t i, int64_t N, int vbits, int32_t* row_a, int32_t* row_b) {
+DYNG_DEV void mark_row_range(const u64* keys, int64_t i, int64_t N, int64_t at, int vbits, int32_t* row_a,
+                             int32_t* row_b) {
   const u64 key = keys[i];
   const u64 r = key >> vbits;
-  if (i == 0 || (keys[i - 1] >> vbits) != r) row_a[r] = static_cast<int32_t>(i);
-  if (i + 1 == N || (keys[i + 1] >> vbits) != r) row_b[r] = static_cast<int32_t>(i + 1);
+  if (i == 0 || (keys[i - 1] >> vbits) != r) row_a[r] = static_cast<int32_t>(at + i);
+  if (i + 1 == N || (keys[i + 1] >> vbits) != r) row_b[r] = static_cast<int32_t>(at + i + 1);
+}
+
+/// A row whose entries change: marked for the plan of its group (`kGrouped`: one workgroup holds all
+/// the row's operations), or listed.
+template <bool kGrouped>
+DYNG_DEV void touch_row(bool structural, int32_t r, int32_t* mark, int mark_gen, int* touched_count, int32_t* touched) {
+  if (kGrouped) {
+    if (structural) mark[r] = mark_gen;
+    return;
+  }
+  const bool first_touch = structural && atomicExch(&mark[r], mark_gen) != mark_gen;
+  const int t = wave_append(touched_count, first_touch);
+  if (first_touch) touched[t] = r;
 }
 
 /// The out-row pass of thread i (every thread of the workgroup calls it: it ends with the
 /// workgroup's counter reduction).
+template <int kThreads, bool kGrouped>
 DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
   unsigned long long c_ins = 0, c_upd = 0, c_del = 0, c_ign_del = 0, c_ign_ins = 0;
   // weight sum and count-at-maximum deltas of columns 0..3 (named, not an array: a private
@@ -697,7 +717,7 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
   }
   if (i < p.N) {
     const u64 key = p.keys[i];
-    if (key != kNoKey) mark_row_range(p.keys, i, p.N, p.vbits, p.row_a, p.row_b);
+    if (key != kNoKey) mark_row_range(p.keys, i, p.N, p.at, p.vbits, p.row_a, p.row_b);
     if (key == kNoKey) {
       p.pend_alive[i] = 0;
       p.kill[i] = 0;
@@ -770,7 +790,7 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
             }
             for (int k = 0; k < K; ++k) {
               const int32_t wo = p.w[k * p.slot_cap + mt.x + old_hit];
-              p.iop_wold[k * p.N + e] = wo;
+              p.iop_wold[k * p.stride + e] = wo;
               account(k, wo, 0, true, false);
             }
             p.iop_type[e] = kInDelete;
@@ -779,8 +799,8 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
           } else if (pend_hit >= 0) {
             p.pend_alive[pend_hit] = 0;
             for (int k = 0; k < K; ++k) {
-              const int32_t wo = p.pend_w[k * p.N + pend_hit];
-              p.iop_wold[k * p.N + e] = wo;
+              const int32_t wo = p.pend_w[k * p.stride + pend_hit];
+              p.iop_wold[k * p.stride + e] = wo;
               account(k, wo, 0, true, false);
             }
             p.iop_type[e] = kInDelete;
@@ -797,11 +817,11 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
               if (old_hit >= 0 && old_hit == init_hit && first_mod < 0) first_mod = e;
               for (int k = 0; k < K; ++k) {
                 const int32_t wn = p.ins_w[bj * K + k];
-                int32_t* slot = old_hit >= 0 ? &p.w[k * p.slot_cap + mt.x + old_hit] : &p.pend_w[k * p.N + pend_hit];
+                int32_t* slot = old_hit >= 0 ? &p.w[k * p.slot_cap + mt.x + old_hit] : &p.pend_w[k * p.stride + pend_hit];
                 const int32_t wo = *slot;
                 *slot = wn;
-                p.iop_wold[k * p.N + e] = wo;
-                p.iop_wnew[k * p.N + e] = wn;
+                p.iop_wold[k * p.stride + e] = wo;
+                p.iop_wnew[k * p.stride + e] = wn;
                 account(k, wo, wn, true, true);
               }
               p.iop_type[e] = kInModify;
@@ -811,8 +831,8 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
             p.pend_alive[q] = 1;
             for (int k = 0; k < K; ++k) {
               const int32_t wn = p.ins_w[bj * K + k];
-              p.pend_w[k * p.N + q] = wn;
-              p.iop_wnew[k * p.N + e] = wn;
+              p.pend_w[k * p.stride + q] = wn;
+              p.iop_wnew[k * p.stride + e] = wn;
               account(k, 0, wn, false, true);
             }
             p.iop_type[e] = kInInsert;
@@ -832,7 +852,7 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
         }
         if (wf == nullptr) {
           for (int64_t x = i; x < j; ++x) {
-            if (p.pend_alive[x]) { wf = p.pend_w + x; wf_stride = p.N; break; }
+            if (p.pend_alive[x]) { wf = p.pend_w + x; wf_stride = p.stride; break; }
           }
         }
         if (wf != nullptr) {
@@ -841,7 +861,7 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
             if (p.L.is_del(e)) continue;
             const int64_t loc = p.L.local(e);
             for (int k = 0; k < K; ++k) {
-              const int32_t orig = first_mod >= 0 ? p.iop_wold[k * p.N + first_mod] : p.w[k * p.slot_cap + mt.x + init_hit];
+              const int32_t orig = first_mod >= 0 ? p.iop_wold[k * p.stride + first_mod] : p.w[k * p.slot_cap + mt.x + init_hit];
               p.e_inc[loc * K + k] = wf[k * wf_stride] > orig ? 1 : 0;
             }
           }
@@ -858,7 +878,7 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
           wf_stride = p.slot_cap;
         } else {
           for (int64_t x = i; x < j; ++x) {
-            if (p.pend_alive[x]) { wf = p.pend_w + x; wf_stride = p.N; break; }
+            if (p.pend_alive[x]) { wf = p.pend_w + x; wf_stride = p.stride; break; }
           }
         }
         for (int64_t q = i; q < j; ++q) {
@@ -868,50 +888,56 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
           for (int k = 0; k < K; ++k) p.e_fw[loc * K + k] = wf != nullptr ? wf[k * wf_stride] : -1;
         }
       }
-      const bool first_touch = structural && atomicExch(&p.mark[u], p.mark_gen) != p.mark_gen;
-      const int t = wave_append(&p.ctl->touched_out, first_touch);
-      if (first_touch) p.touched[t] = u;
+      touch_row<kGrouped>(structural, u, p.mark, p.mark_gen, &p.ctl->touched_out, p.touched);
     }
   }
-  // the workgroup's counters in one pass: wave sums by shuffles, one barrier, then thread 0 adds
-  // the waves' sums and bumps the device counters (13 values)
+  // the workgroup's counters in one pass: wave sums by lane-to-lane moves (a count fits 32 bits; a
+  // weight sum goes in three parts, modulo 2^64), one barrier, then a thread per counter adds the
+  // waves' sums
   constexpr int kSums = 13;
-  u64 sum[kSums] = {c_ins, c_upd, c_del, c_ign_del, c_ign_ins,
-                    static_cast<u64>(ds0), static_cast<u64>(ds1), static_cast<u64>(ds2), static_cast<u64>(ds3),
-                    static_cast<u64>(dc0), static_cast<u64>(dc1), static_cast<u64>(dc2), static_cast<u64>(dc3)};
-  __shared__ u64 part[kBlock / 64][kSums];
-#pragma unroll
-  for (int q = 0; q < kSums; ++q) {
-    for (int off = 32; off > 0; off >>= 1) sum[q] += static_cast<u64>(__shfl_xor(sum[q], off));
-  }
-  if (lane() == 0) {
-#pragma unroll
-    for (int q = 0; q < kSums; ++q) part[threadIdx.x / 64][q] = sum[q];
+  __shared__ u64 part[kThreads / 64][kSums];
+  const int w = static_cast<int>(threadIdx.x) / 64;
+  auto count_sum = [&](int q, long long x) {
+    const int t = wave_scan(static_cast<int>(x));
+    if (lane() == 63) part[w][q] = static_cast<u64>(static_cast<long long>(t));
+  };
+  auto weight_sum = [&](int q, long long x) {
+    const int lo = wave_scan(static_cast<int>(x & 0xffff)), mid = wave_scan(static_cast<int>((x >> 16) & 0xffff)),
+              hi = wave_scan(static_cast<int>(x >> 32));
+    if (lane() == 63) {
+      part[w][q] = static_cast<u64>(lo) + (static_cast<u64>(mid) << 16) + (static_cast<u64>(static_cast<uint32_t>(hi)) << 32);
+    }
+  };
+  count_sum(0, static_cast<long long>(c_ins));
+  count_sum(1, static_cast<long long>(c_upd));
+  count_sum(2, static_cast<long long>(c_del));
+  count_sum(3, static_cast<long long>(c_ign_del));
+  count_sum(4, static_cast<long long>(c_ign_ins));
+  weight_sum(5, ds0);
+  count_sum(9, dc0);
+  if (K > 1) {
+    weight_sum(6, ds1);
+    weight_sum(7, ds2);
+    weight_sum(8, ds3);
+    count_sum(10, dc1);
+    count_sum(11, dc2);
+    count_sum(12, dc3);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < kSums; ++q) {
-      u64 t = part[0][q];
-      for (int wv = 1; wv < kBlock / 64; ++wv) t += part[wv][q];
-      sum[q] = t;
-    }
-    if (sum[0]) atomicAdd(&p.ctl->inserted_edges, sum[0]);
-    if (sum[1]) atomicAdd(&p.ctl->updated_edges, sum[1]);
-    if (sum[2]) atomicAdd(&p.ctl->deleted_edges, sum[2]);
-    if (sum[3]) atomicAdd(&p.ctl->ignored_deletions, sum[3]);
-    if (sum[4]) atomicAdd(&p.ctl->ignored_insertions, sum[4]);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (k >= K) break;
-      if (sum[5 + k]) atomicAdd(reinterpret_cast<unsigned long long*>(&p.ctl->col_dsum[k]), sum[5 + k]);
-      if (sum[9 + k]) atomicAdd(reinterpret_cast<unsigned long long*>(&p.ctl->col_dcount[k]), sum[9 + k]);
-    }
+  const int q = static_cast<int>(threadIdx.x);
+  if (q < kSums && (q < 5 || ((q - 5) & 3) < K)) {
+    u64 t = 0;
+    for (int wv = 0; wv < kThreads / 64; ++wv) t += part[wv][q];
+    u64* to = &p.ctl->inserted_edges + q;  // inserted, updated, deleted, ignored deletions
+    if (q == 4) to = &p.ctl->ignored_insertions;
+    if (q >= 5) to = reinterpret_cast<u64*>(&p.ctl->col_dsum[q - 5]);
+    if (q >= 9) to = reinterpret_cast<u64*>(&p.ctl->col_dcount[q - 9]);
+    if (t != 0) atomicAdd(to, t);
   }
 }
 
 __global__ void __launch_bounds__(kBlock) k_out_pairs(out_pair_params p) {
-  out_pairs(p, blockIdx.x * int64_t{blockDim.x} + threadIdx.x);
+  out_pairs<kBlock, false>(p, blockIdx.x * int64_t{blockDim.x} + threadIdx.x);
 }
 
 struct in_pair_params {
@@ -921,6 +947,8 @@ struct in_pair_params {
   const u64* keys;  ///< sorted in-operation keys (v << b | u)
   const uint32_t* vals;  ///< out-operation position of each
   int64_t N;
+  int64_t stride;  ///< of the weight columns of pend_w and of the iop arrays
+  int64_t at;      ///< place of keys[0] among all the sorted operations
   int vbits;
   int K;
   const int32_t* iop_type;
@@ -943,8 +971,10 @@ struct in_pair_params {
   apply_control* ctl;
 };
 
-__global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
-  const int64_t i = blockIdx.x * int64_t{blockDim.x} + threadIdx.x;
+/// The in-row pass of a graph with parallel edges, thread i: each operation's effect as the out-row
+/// pass recorded it.
+template <bool kGrouped>
+DYNG_DEV void in_pairs(const in_pair_params& p, int64_t i) {
   if (i == p.N) {
     p.pend_alive[i] = 0;
     p.kill[i] = 0;
@@ -956,7 +986,7 @@ __global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
     p.kill[i] = 0;
     return;
   }
-  mark_row_range(p.keys, i, p.N, p.vbits, p.row_a, p.row_b);
+  mark_row_range(p.keys, i, p.N, p.at, p.vbits, p.row_a, p.row_b);
   if (i > 0 && p.keys[i - 1] == key) return;
   int64_t j = i + 1;
   while (j < p.N && p.keys[j] == key) ++j;
@@ -976,7 +1006,7 @@ __global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
     if (type == kInNone) continue;  // ignored by the out-row pass
     if (type == kInInsert) {
       p.pend_alive[q] = 1;
-      for (int k = 0; k < K; ++k) p.pend_w[k * p.N + q] = p.iop_wnew[k * p.N + o];
+      for (int k = 0; k < K; ++k) p.pend_w[k * p.stride + q] = p.iop_wnew[k * p.stride + o];
       structural = true;
       continue;
     }
@@ -987,7 +1017,7 @@ __global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
       if (x >= rr.tu) break;
       if (row[x] < 0) continue;
       bool same = true;
-      for (int k = 0; k < K && same; ++k) same = p.w[k * p.slot_cap + mt.x + x] == p.iop_wold[k * p.N + o];
+      for (int k = 0; k < K && same; ++k) same = p.w[k * p.slot_cap + mt.x + x] == p.iop_wold[k * p.stride + o];
       if (same) old_hit = x;
     }
     int64_t pend_hit = -1;
@@ -995,7 +1025,7 @@ __global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
       for (int64_t x = i; x < q && pend_hit < 0; ++x) {
         if (!p.pend_alive[x]) continue;
         bool same = true;
-        for (int k = 0; k < K && same; ++k) same = p.pend_w[k * p.N + x] == p.iop_wold[k * p.N + o];
+        for (int k = 0; k < K && same; ++k) same = p.pend_w[k * p.stride + x] == p.iop_wold[k * p.stride + o];
         if (same) pend_hit = x;
       }
     }
@@ -1017,14 +1047,16 @@ __global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
       }
     } else {
       for (int k = 0; k < K; ++k) {
-        const int32_t wn = p.iop_wnew[k * p.N + o];
-        if (old_hit >= 0) p.w[k * p.slot_cap + mt.x + old_hit] = wn; else p.pend_w[k * p.N + pend_hit] = wn;
+        const int32_t wn = p.iop_wnew[k * p.stride + o];
+        if (old_hit >= 0) p.w[k * p.slot_cap + mt.x + old_hit] = wn; else p.pend_w[k * p.stride + pend_hit] = wn;
       }
     }
   }
-  const bool first_touch = structural && atomicExch(&p.mark[v], p.mark_gen) != p.mark_gen;
-  const int t = wave_append(&p.ctl->touched_in, first_touch);
-  if (first_touch) p.touched[t] = v;
+  touch_row<kGrouped>(structural, v, p.mark, p.mark_gen, &p.ctl->touched_in, p.touched);
+}
+
+__global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
+  in_pairs<false>(p, blockIdx.x * int64_t{blockDim.x} + threadIdx.x);
 }
 
 /// The in-row pass of a simple graph, thread i. A simple graph holds at most one alive (u, v), and
@@ -1034,6 +1066,7 @@ __global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
 /// reaches the same decisions and weights without that pass's results: both passes run in one
 /// launch (k_pairs_simple). With parallel edges the copy an operation takes is matched by weight
 /// to the out-row's (k_in_pairs, after k_out_pairs).
+template <bool kGrouped>
 DYNG_DEV void in_pairs_simple(const in_pair_params& p, int64_t i) {
   if (i == p.N) {
     p.pend_alive[i] = 0;
@@ -1046,7 +1079,7 @@ DYNG_DEV void in_pairs_simple(const in_pair_params& p, int64_t i) {
     p.kill[i] = 0;
     return;
   }
-  mark_row_range(p.keys, i, p.N, p.vbits, p.row_a, p.row_b);
+  mark_row_range(p.keys, i, p.N, p.at, p.vbits, p.row_a, p.row_b);
   if (i > 0 && p.keys[i - 1] == key) return;
   int64_t j = i + 1;
   while (j < p.N && p.keys[j] == key) ++j;
@@ -1099,19 +1132,17 @@ DYNG_DEV void in_pairs_simple(const in_pair_params& p, int64_t i) {
         if (p.upsert) {
           for (int k = 0; k < K; ++k) {
             const int32_t wn = p.ins_w[bj * K + k];
-            if (old_hit >= 0) p.w[k * p.slot_cap + mt.x + old_hit] = wn; else p.pend_w[k * p.N + pend_hit] = wn;
+            if (old_hit >= 0) p.w[k * p.slot_cap + mt.x + old_hit] = wn; else p.pend_w[k * p.stride + pend_hit] = wn;
           }
         }
       } else {
         p.pend_alive[q] = 1;
-        for (int k = 0; k < K; ++k) p.pend_w[k * p.N + q] = p.ins_w[bj * K + k];
+        for (int k = 0; k < K; ++k) p.pend_w[k * p.stride + q] = p.ins_w[bj * K + k];
         structural = true;
       }
     }
   }
-  const bool first_touch = structural && atomicExch(&p.mark[v], p.mark_gen) != p.mark_gen;
-  const int t = wave_append(&p.ctl->touched_in, first_touch);
-  if (first_touch) p.touched[t] = v;
+  touch_row<kGrouped>(structural, v, p.mark, p.mark_gen, &p.ctl->touched_in, p.touched);
 }
 
 /// Both pairing passes of a simple graph in one launch: workgroups [0, split) the out-rows,
@@ -1119,9 +1150,9 @@ DYNG_DEV void in_pairs_simple(const in_pair_params& p, int64_t i) {
 __global__ void __launch_bounds__(kBlock) k_pairs_simple(out_pair_params po, in_pair_params pi, int split) {
   const int b = static_cast<int>(blockIdx.x);
   if (b < split) {
-    out_pairs(po, b * int64_t{blockDim.x} + threadIdx.x);
+    out_pairs<kBlock, false>(po, b * int64_t{blockDim.x} + threadIdx.x);
   } else {
-    in_pairs_simple(pi, (b - split) * int64_t{blockDim.x} + threadIdx.x);
+    in_pairs_simple<false>(pi, (b - split) * int64_t{blockDim.x} + threadIdx.x);
   }
 }
 
@@ -1158,12 +1189,18 @@ struct merge_params {
   long long* need_stage;
   int* error_bits;
   double headroom;
-  const int* hold;  ///< null, or a flag that makes the merge do nothing (see k_merge_gate)
 };
 
 /// The in-place tail merges of one mode for both stores in one launch: workgroups [0, split)
 /// merge out-rows, the others in-rows. The two stores share nothing these merges write (the error
 /// bits aside, which they set atomically), so the halves run side by side.
+/// The merges of both stores in one launch: a workgroup's role and store by its place in the grid.
+struct merge_roles {
+  merge_params side[2];
+  int groups[4];        ///< workgroups per role and store: first role's out-rows, in-rows, second role's out-rows, in-rows
+  apply_control* gate;  ///< null, or where the first launch's workgroups find whether the merges fit (merges_fit)
+};
+
 struct merge_sides {
   merge_params side[2];
   int split;
@@ -1176,10 +1213,10 @@ DYNG_DEV void for_side(const merge_sides& m, Body&& body) {
   const int b = static_cast<int>(blockIdx.x);
   const bool in = b >= m.split;
   const merge_params p = in ? m.side[1] : m.side[0];
-  if (p.hold != nullptr && *p.hold != 0) return;  // uniform: the gate held the merges back
   body(p, in ? b - m.split : b, in ? static_cast<int>(gridDim.x) - m.split : m.split);
 }
 
+constexpr int kTailsBlock = 256;   ///< threads of a workgroup that merges short tails (a thread's needs 162 registers)
 constexpr int kMergeBlock = 1024;  ///< threads of a merge workgroup
 constexpr int kMergeWaves = kMergeBlock / 64;
 constexpr int kMergeSeg = 2048;    ///< operations of one row a workgroup stages in LDS
@@ -1221,18 +1258,19 @@ struct row_plan {
   int new_len;  ///< full merge: the rewritten row's length
 };
 
-DYNG_DEV row_plan plan_row(const merge_params& p, int32_t u, int2 mt, int64_t a, int64_t b) {
+/// `dead`: the dead entries of the row's base run.
+DYNG_DEV row_plan plan_row(const merge_params& p, int32_t u, int2 mt, int64_t a, int64_t b, int dead) {
   row_plan r;
   r.base_len = p.base[u];
   r.tail_len = mt.y - r.base_len;
   r.pending = p.pend_prefix[b] - p.pend_prefix[a];
   r.alive_tail = r.tail_len - (p.kill_prefix[b] - p.kill_prefix[a]);
-  r.alive_base = r.base_len - p.dead[u];
+  r.alive_base = r.base_len - dead;
   r.new_tail = r.alive_tail + r.pending;
   r.new_len = r.alive_base + r.new_tail;
   const int nops = static_cast<int>(b - a);
   const bool tail_ok = r.new_tail <= tail_limit(r.base_len) && r.base_len + r.new_tail <= p.cap[u] &&
-                       p.dead[u] <= dead_limit(r.base_len);
+                       dead <= dead_limit(r.base_len);
   if (tail_ok && r.tail_len <= kLaneTail && nops <= kLaneOps) {
     r.mode = kTailLane;
   } else if (tail_ok && r.tail_len <= kMergeSmall && nops <= 64) {
@@ -1252,52 +1290,67 @@ DYNG_DEV row_plan plan_row(const merge_params& p, int32_t u, int2 mt, int64_t a,
 /// addresses every workgroup hits).
 constexpr int kPlanBlock = 1024;
 
-DYNG_DEV void merge_plan(const merge_params& p, int block) {
-  __shared__ int wave_offset[kPlanBlock / 64][kModes];
-  __shared__ int base[kModes];
-  __shared__ long long part[kPlanBlock / 64];
-  const int count = *p.touched_count;
-  const int t = block * kPlanBlock + threadIdx.x;
+/// Plan one row per thread (u < 0: none) and append it to its mode's list. Every thread of the
+/// workgroup calls it. kGrouped: the row's dead entries were counted in this kernel (by device-scope
+/// atomics, so they are read at that scope), and the row joins the touched list here.
+template <int kThreads, bool kGrouped>
+DYNG_DEV void plan_rows(const merge_params& p, int32_t u, int* touched_count, int32_t* touched) {
+  constexpr int kLists = kModes + (kGrouped ? 1 : 0);
+  __shared__ int wave_offset[kThreads / 64][kModes + 1];
+  __shared__ int base[kModes + 1];
+  __shared__ long long part[kThreads / 64];
   const int w = threadIdx.x / 64;
   long long reloc = 0, stage = 0;
   int mode = -1;
-  int32_t u = -1;
-  if (t < count) {
-    u = p.touched[t];
+  if (u >= 0) {
     const int2 mt = p.meta[u];
-    const row_plan r = plan_row(p, u, mt, p.row_a[u], p.row_b[u]);
+    const row_plan r = plan_row(p, u, mt, p.row_a[u], p.row_b[u], kGrouped ? ld(&p.dead[u]) : p.dead[u]);
     mode = r.mode;
     if (r.mode == kFull) {
       stage = r.alive_base + r.alive_tail;
       if (r.new_len > p.cap[u]) reloc = grown_cap(r.new_len, p.headroom);
     }
   }
-  int rank = 0;  // among the wave's rows of the same mode
+  int rank = 0, row_rank = 0;  // among the wave's rows of the same mode, and among all its rows
 #pragma unroll
-  for (int m = 0; m < kModes; ++m) {
-    const u64 b = __ballot(mode == m);
-    if (mode == m) rank = __popcll(b & lanes_below());
+  for (int m = 0; m < kLists; ++m) {
+    const u64 b = __ballot(m == kModes ? mode >= 0 : mode == m);
+    if (m == kModes) {
+      row_rank = __popcll(b & lanes_below());
+    } else if (mode == m) {
+      rank = __popcll(b & lanes_below());
+    }
     if (lane() == 0) wave_offset[w][m] = __popcll(b);
   }
   __syncthreads();
-  if (threadIdx.x < kModes) {
+  if (threadIdx.x < kLists) {
     const int m = threadIdx.x;
     int run = 0;
-    for (int i = 0; i < kPlanBlock / 64; ++i) {
+    for (int i = 0; i < kThreads / 64; ++i) {
       const int c = wave_offset[i][m];
       wave_offset[i][m] = run;
       run += c;
     }
-    base[m] = run > 0 ? atomicAdd(&p.list_count[m], run) : 0;
+    base[m] = run > 0 ? atomicAdd(m == kModes ? touched_count : &p.list_count[m], run) : 0;
   }
   __syncthreads();
-  if (mode >= 0) p.lists[mode * (p.N + 1) + base[mode] + wave_offset[w][mode] + rank] = u;
+  if (mode >= 0) {
+    p.lists[mode * (p.N + 1) + base[mode] + wave_offset[w][mode] + rank] = u;
+    if (kGrouped) touched[base[kModes] + wave_offset[w][kModes] + row_rank] = u;
+  }
+  if (__syncthreads_or(mode == kFull ? 1 : 0) == 0) return;  // the sums are zero
   reloc = block_reduce(reloc, part, op_sum{});
   stage = block_reduce(stage, part, op_sum{});
   if (threadIdx.x == 0) {
     if (reloc) atomicAdd(reinterpret_cast<unsigned long long*>(p.need_reloc), static_cast<unsigned long long>(reloc));
     if (stage) atomicAdd(reinterpret_cast<unsigned long long*>(p.need_stage), static_cast<unsigned long long>(stage));
   }
+}
+
+DYNG_DEV void merge_plan(const merge_params& p, int block) {
+  const int count = *p.touched_count;
+  const int t = block * kPlanBlock + threadIdx.x;
+  plan_rows<kPlanBlock, false>(p, t < count ? p.touched[t] : -1, nullptr, nullptr);
 }
 
 __global__ void __launch_bounds__(kPlanBlock) k_merge_plan(merge_sides m) {
@@ -1307,15 +1360,362 @@ __global__ void __launch_bounds__(kPlanBlock) k_merge_plan(merge_sides m) {
 /// Slots a relocating merge leaves free at the arena's tail (the host's plan keeps the same).
 constexpr long long kArenaMargin = 1024;
 
-/// After a plan that the host does not read back: whether the merges fit as planned (the
-/// arenas' free tails take the relocations, the staging arena the full merges) and no error came
-/// first. If not, `hold` makes the merges and the engine run behind them do nothing, and the host
-/// plans again after its synchronization. One thread.
-__global__ void k_merge_gate(apply_control* c, long long slot_cap_out, long long slot_cap_in, long long stage_cap) {
-  const bool fits = c->error_bits == 0 && c->need_reloc_out + kArenaMargin <= slot_cap_out - c->tail_out &&
-                    c->need_reloc_in + kArenaMargin <= slot_cap_in - c->tail_in &&
-                    c->need_stage_out <= stage_cap && c->need_stage_in <= stage_cap;
-  c->hold = fits ? 0 : 1;
+/// After a plan that the host does not read back: whether the merges fit as planned (the arenas'
+/// free tails take the relocations, the staging arena both stores' full merges) and nothing came
+/// first that stops them.
+DYNG_DEV bool merges_fit(const apply_control* c, long long slot_cap_out, long long slot_cap_in, long long stage_cap) {
+  return c->miss == 0 && c->error_bits == 0 && c->need_reloc_out + kArenaMargin <= slot_cap_out - c->tail_out &&
+         c->need_reloc_in + kArenaMargin <= slot_cap_in - c->tail_in &&
+         c->need_stage_out + c->need_stage_in <= stage_cap;
+}
+
+// ---------------------------------------------------------------------------------------------
+// The grouped apply: operations scattered into groups of whole rows, then everything up to the merge
+// plan of a group's rows in one workgroup
+// ---------------------------------------------------------------------------------------------
+
+/// A batch's operations need not be sorted as a whole: the pairing needs each (u, v) together in
+/// batch order, the merges each row's operations together by neighbour. So the rows are hashed into
+/// groups of about 256-512 operations per direction (an odd multiplier modulo 2^vbits is a
+/// bijection, its top bits the group), one launch scatters the operations into their groups, and in
+/// the next one workgroup per group sorts its operations in LDS, pairs them with their rows, scans
+/// their flags and plans its rows' merges. That replaces a device-wide sort (75 us of block sort and
+/// eight merge passes for a batch of 100,000 on RMAT-22, 269 us of radix passes for 1,000,000 on
+/// RMAT-23), the untagging, the pairing, two scan launches and the plan: two launches for ten to
+/// seventeen, nothing between them through memory but the operations.
+constexpr int kGroupBlock = 256;
+/// Operations per group and direction (the groups hold 1 to 2 times this), by how many groups there are:
+/// few while processors are idle (2^7 groups per direction give every one of the 256 a workgroup),
+/// more up to the workgroups it holds at once (2^9), and beyond that what the front's reservations and
+/// the per-group work favour. 2,000 arcs of an undirected 64 K graph: 25 us with 32 each, 43 with
+/// 128; 100,000 operations on RMAT-22: 103 us with 128, 110 with 256; 1,000,000 on RMAT-23: 515 us with
+/// 256, 550 to 590 with 128.
+constexpr int kGroupBitsFew = 7, kGroupOpsFew = 32;
+constexpr int kGroupBitsSome = 9, kGroupOpsSome = 128;
+constexpr int kGroupOps = 256;
+constexpr int64_t kGroupMost = int64_t{1} << 22;  ///< operations of a batch (1024 per group)
+constexpr int kGroupCap = 4096;   ///< most a group takes; one row with more operations sends the batch to the sort
+constexpr int kGroupPause = 15;   ///< batches sorted device-wide after one that a group could not take
+constexpr int kGroupBits = 12;    ///< at most 2^12 groups per direction
+constexpr uint32_t kGroupHash = 0x9E3779B1u;
+
+/// Why the grouped apply did nothing (apply_control::miss).
+enum { kMissFull = 1 };
+
+/// What the control block starts an apply with, and the group counters to clear. A launch with these
+/// in its arguments in place of a copy from host memory: one launch clears both.
+struct begin_params {
+  long long tail_out, tail_in;
+  long long col_max[max_weights];
+  int* counts;
+  int num_counts;
+};
+__global__ void __launch_bounds__(1024) k_begin(apply_control* c, begin_params b) {
+  static_assert(sizeof(apply_control) % sizeof(int) == 0);
+  for (int i = threadIdx.x; i < static_cast<int>(sizeof(apply_control) / sizeof(int)); i += blockDim.x) {
+    reinterpret_cast<int*>(c)[i] = 0;
+  }
+  for (int i = threadIdx.x; i < b.num_counts; i += blockDim.x) b.counts[i] = 0;
+  __syncthreads();  // the words are cleared
+  if (threadIdx.x < max_weights) c->col_max[threadIdx.x] = b.col_max[threadIdx.x];
+  if (threadIdx.x == 0) {
+    c->tail_out = b.tail_out;
+    c->tail_in = b.tail_in;
+    c->first_error = kNoError;
+  }
+}
+
+struct front_params {
+  op_layout L;
+  const int32_t *ins_src, *ins_dst, *del_src, *del_dst;
+  int directed, drop_self_loops;
+  int64_t n_after;
+  int vbits, ebits, lb, K;
+  int groups;
+  u64* entries;  ///< kGroupCap per group: out-row groups, then in-row groups
+  int* counts;
+  int32_t *e_del_src, *e_del_dst, *e_ins_src, *e_ins_dst;
+  uint8_t* e_inc;
+  int32_t* e_fw;
+  apply_control* ctl;
+};
+
+/// One arc of the batch: operation e of the layout. False when it is dropped (a self-loop, the
+/// second arc of a directed graph, a deletion naming a vertex that does not exist).
+struct front_op {
+  bool del, dropped, ignored;
+  int64_t loc;
+  int32_t u, v;
+};
+DYNG_DEV bool front_decode(const front_params& f, int64_t e, front_op& o) {
+  o.del = f.L.is_del(e);
+  o.loc = f.L.local(e);
+  const int64_t j = o.loc / f.L.stride;
+  const int r = static_cast<int>(o.loc % f.L.stride);
+  const int32_t u0 = o.del ? f.del_src[j] : f.ins_src[j];
+  const int32_t v0 = o.del ? f.del_dst[j] : f.ins_dst[j];
+  o.u = r ? v0 : u0;
+  o.v = r ? u0 : v0;
+  bool valid = !(r == 1 && (f.directed || u0 == v0));
+  o.dropped = valid && u0 == v0 && f.drop_self_loops;
+  valid = valid && !o.dropped;
+  o.ignored = valid && o.del && (o.u >= f.n_after || o.v >= f.n_after);
+  return valid && !o.ignored;
+}
+
+/// The effective operation lists, and each operation's out- and in-key in its group. A workgroup
+/// counts its operations per group in LDS and reserves their places with one atomic per group it
+/// touches (the counters of all groups share a few cache lines). kOps operations per thread.
+template <int kOps>
+__global__ void __launch_bounds__(1024) k_group_front(front_params f) {
+  __shared__ int hist[2 << kGroupBits];
+  const int all = 2 * f.groups;
+  for (int b = threadIdx.x; b < all; b += blockDim.x) hist[b] = 0;
+  __syncthreads();
+  const int64_t total = (f.L.num_first + f.L.num_second) * f.L.stride;
+  const int64_t e0 = (int64_t{blockIdx.x} * kOps) * blockDim.x + threadIdx.x;
+  const uint32_t mask = static_cast<uint32_t>((u64{1} << f.vbits) - 1);
+  const int low = f.vbits - f.lb;  // bits of a hashed row below its group's
+  int rank[2][kOps];
+  unsigned long long dropped = 0, ignored = 0;
+#pragma unroll
+  for (int j = 0; j < kOps; ++j) {
+    const int64_t e = e0 + int64_t{j} * blockDim.x;
+    front_op o{};
+    const bool valid = e < total && front_decode(f, e, o);
+    dropped += __popcll(__ballot(e < total && o.dropped));
+    ignored += __popcll(__ballot(e < total && o.ignored));
+    if (e < total) {
+      if (o.del) {
+        f.e_del_src[o.loc] = valid ? o.u : -1;
+        f.e_del_dst[o.loc] = valid ? o.v : -1;
+      } else {
+        f.e_ins_src[o.loc] = valid ? o.u : -1;
+        f.e_ins_dst[o.loc] = valid ? o.v : -1;
+        for (int k = 0; k < f.K; ++k) f.e_inc[o.loc * f.K + k] = 0;
+        if (f.e_fw != nullptr) {
+          for (int k = 0; k < f.K; ++k) f.e_fw[o.loc * f.K + k] = -1;
+        }
+      }
+    }
+    rank[0][j] = rank[1][j] = -1;
+    if (valid) {
+      const uint32_t hu = (static_cast<uint32_t>(o.u) * kGroupHash) & mask;
+      const uint32_t hv = (static_cast<uint32_t>(o.v) * kGroupHash) & mask;
+      rank[0][j] = atomicAdd(&hist[hu >> low], 1);
+      rank[1][j] = atomicAdd(&hist[f.groups + static_cast<int>(hv >> low)], 1);
+    }
+  }
+  if (lane() == 0) {
+    if (dropped) atomicAdd(&f.ctl->dropped_self_loops, dropped);
+    if (ignored) atomicAdd(&f.ctl->ignored_deletions, ignored);
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < all; b += blockDim.x) {
+    if (hist[b] > 0) {
+      const int mine = hist[b];
+      hist[b] = atomicAdd(&f.counts[b], mine);
+      if (hist[b] + mine > kGroupCap) atomicOr(&f.ctl->miss, kMissFull);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kOps; ++j) {
+    if (rank[0][j] < 0) continue;
+    const int64_t e = e0 + int64_t{j} * blockDim.x;
+    front_op o;
+    (void)front_decode(f, e, o);
+    const uint32_t hu = (static_cast<uint32_t>(o.u) * kGroupHash) & mask;
+    const uint32_t hv = (static_cast<uint32_t>(o.v) * kGroupHash) & mask;
+    const u64 below = (u64{1} << low) - 1;
+    const int gu = static_cast<int>(hu >> low), gv = f.groups + static_cast<int>(hv >> low);
+    const int at_u = hist[gu] + rank[0][j], at_v = hist[gv] + rank[1][j];
+    if (at_u < kGroupCap) {
+      f.entries[int64_t{gu} * kGroupCap + at_u] =
+          ((((hu & below) << f.vbits) | static_cast<u64>(o.v)) << f.ebits) | static_cast<u64>(e);
+    }
+    if (at_v < kGroupCap) {
+      f.entries[int64_t{gv} * kGroupCap + at_v] =
+          ((((hv & below) << f.vbits) | static_cast<u64>(o.u)) << f.ebits) | static_cast<u64>(e);
+    }
+  }
+}
+
+/// Entries below x in 64 sorted words of LDS.
+DYNG_DEV int segment_rank(const u64* S, u64 x) {
+  int at = 0;
+#pragma unroll
+  for (int step = 32; step > 0; step >>= 1) at += S[at + step - 1] < x ? step : 0;
+  return at + (S[at] < x ? 1 : 0);
+}
+
+/// Sort the `count` words of src (distinct, below 2^63): place(rank, word) for each. Every wave
+/// ranks 64 words at a time among themselves (each lane counts the smaller ones, broadcast from
+/// register to register) and leaves them sorted in S; then a word's rank is the sum of its ranks in
+/// all the sorted segments, searched independently of each other. 256 words: about 1 us, where a bitonic
+/// sort's 36 dependent LDS steps take 9. Every thread of the workgroup calls it.
+template <class Place>
+DYNG_DEV void group_sort(const u64* src, int count, u64* S, Place place) {
+  const int segments = (count + 63) / 64;
+  const int wave = uniform(static_cast<int>(threadIdx.x) / 64);
+  for (int s = wave; s < segments; s += kGroupBlock / 64) {
+    const int i = s * 64 + lane();
+    const u64 x = i < count ? src[i] : ~u64{0} - 63 + lane();
+    const int lo = static_cast<int>(x), hi = static_cast<int>(x >> 32);
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+      const u64 y = (static_cast<u64>(static_cast<uint32_t>(__builtin_amdgcn_readlane(hi, j))) << 32) |
+                    static_cast<uint32_t>(__builtin_amdgcn_readlane(lo, j));
+      rank += y < x ? 1 : 0;
+    }
+    S[s * 64 + rank] = x;
+  }
+  __syncthreads();
+  for (int s = wave; s < segments; s += kGroupBlock / 64) {
+    const u64 x = S[s * 64 + lane()];
+    int rank = lane();
+    if (segments > 1) {
+      rank = 0;
+#pragma unroll 4
+      for (int t = 0; t < segments; ++t) rank += segment_rank(S + t * 64, x);
+    }
+    if (s * 64 + lane() < count) place(rank, x);  // the fillers sort behind the last segment's words
+  }
+}
+
+struct group_params {
+  const u64* entries;
+  const int* counts;
+  int groups, vbits, ebits, lb;
+  uint32_t inverse;  ///< of kGroupHash modulo 2^32
+  u64* keys;         ///< sorted operations: out-rows [0, P), in-rows [P, 2P)
+  uint32_t* vals;
+  int64_t P;         ///< operations plus one place per group
+  out_pair_params out;
+  in_pair_params in;
+  merge_params merge_out, merge_in;
+  int32_t *pend_prefix_out, *kill_prefix_out, *pend_prefix_in, *kill_prefix_in;
+  apply_control* ctl;
+};
+
+enum { kGroupsBoth = 0, kGroupsOut = 1, kGroupsIn = 2 };
+
+/// One group per workgroup: its operations sorted by (row, neighbour, batch order), paired with
+/// their rows, their pending and killed flags scanned (a row's operations are in one group, and
+/// only differences within a row are used), and its rows' merges planned. kGroupsBoth: a simple
+/// graph's out-rows and in-rows side by side; else one direction (with parallel edges the in-row
+/// pass reads what the out-row pass recorded).
+template <int kWhich>
+__global__ void __launch_bounds__(kGroupBlock, 4) k_group_pairs(group_params g) {
+  __shared__ u64 S[kGroupCap];
+  __shared__ int part[kGroupBlock / 64];
+  __shared__ int2 sums[kGroupBlock / 64];
+  if (g.ctl->miss != 0) return;  // uniform
+  const int tid = static_cast<int>(threadIdx.x);
+  const bool in = kWhich == kGroupsIn || (kWhich == kGroupsBoth && static_cast<int>(blockIdx.x) >= g.groups);
+  const int q = static_cast<int>(blockIdx.x) - (kWhich == kGroupsBoth && in ? g.groups : 0);
+  const int* counts = g.counts + (in ? g.groups : 0);
+  const int count = uniform(counts[q]);
+  if (count == 0) return;  // uniform
+  int before = 0;
+  for (int b = tid; b < q; b += kGroupBlock) before += counts[b];
+  const int64_t at = uniform(block_reduce(before, part, op_sum{})) + q;
+  const u64* src = g.entries + int64_t{(in ? g.groups : 0) + q} * kGroupCap;
+  u64* keys = g.keys + (in ? g.P : 0) + at;
+  uint32_t* vals = g.vals + (in ? g.P : 0) + at;
+  const int low = g.vbits - g.lb;
+  const u64 vmask = (u64{1} << g.vbits) - 1, emask = (u64{1} << g.ebits) - 1;
+  auto row_of = [&](u64 x) -> u64 {
+    const uint32_t h = static_cast<uint32_t>((static_cast<u64>(q) << low) | (x >> (g.vbits + g.ebits)));
+    return (h * g.inverse) & static_cast<uint32_t>(vmask);
+  };
+  group_sort(src, count, S, [&](int i, u64 x) {
+    keys[i] = (row_of(x) << g.vbits) | ((x >> g.ebits) & vmask);
+    vals[i] = static_cast<uint32_t>(x & emask);
+  });
+  __syncthreads();  // the group's operations are in memory for the whole workgroup
+  int32_t *pend_alive, *kill, *pend_prefix, *kill_prefix;
+  if (!in) {
+    out_pair_params p = g.out;
+    p.keys = keys;
+    p.vals = vals;
+    p.N = count;
+    p.at = at;
+    p.pend_alive += at;
+    p.kill += at;
+    p.pend_w += at;
+    for (int t = 0; t < count; t += kGroupBlock) {
+      out_pairs<kGroupBlock, true>(p, t + tid);
+      __syncthreads();  // its sums are read
+    }
+    pend_alive = p.pend_alive;
+    kill = p.kill;
+    pend_prefix = g.pend_prefix_out + at;
+    kill_prefix = g.kill_prefix_out + at;
+  } else {
+    in_pair_params p = g.in;
+    p.keys = keys;
+    p.vals = vals;
+    p.N = count;
+    p.at = at;
+    p.pend_alive += at;
+    p.kill += at;
+    p.pend_w += at;
+    for (int t = 0; t < count; t += kGroupBlock) {
+      if (kWhich == kGroupsIn) {
+        in_pairs<true>(p, t + tid);
+      } else {
+        in_pairs_simple<true>(p, t + tid);
+      }
+    }
+    pend_alive = p.pend_alive;
+    kill = p.kill;
+    pend_prefix = g.pend_prefix_in + at;
+    kill_prefix = g.kill_prefix_in + at;
+  }
+  __syncthreads();  // the flags are written
+  int carry_p = 0, carry_k = 0;
+  for (int t = 0; t < count; t += kGroupBlock) {
+    const int i = t + tid;
+    const int xp = i < count ? pend_alive[i] : 0, xk = i < count ? kill[i] : 0;
+    const int sp = wave_scan(xp), sk = wave_scan(xk);
+    __syncthreads();
+    if (lane() == 63) sums[tid / 64] = make_int2(sp, sk);
+    __syncthreads();
+    int bp = carry_p, bk = carry_k;
+    for (int w = 0; w < kGroupBlock / 64; ++w) {
+      const int2 x = sums[w];
+      if (w < tid / 64) {
+        bp += x.x;
+        bk += x.y;
+      }
+      carry_p += x.x;
+      carry_k += x.y;
+    }
+    if (i < count) {
+      pend_prefix[i] = bp + sp - xp;
+      kill_prefix[i] = bk + sk - xk;
+    }
+  }
+  if (tid == 0) {
+    pend_prefix[count] = carry_p;
+    kill_prefix[count] = carry_k;
+  }
+  __syncthreads();  // the prefixes, the rows' ranges and marks are written
+  const merge_params& m = in ? g.merge_in : g.merge_out;
+  const int32_t* mark = in ? g.in.mark : g.out.mark;
+  const int gen = g.out.mark_gen;
+  for (int t = 0; t < count; t += kGroupBlock) {
+    const int i = t + tid;
+    int32_t u = -1;
+    if (i < count) {
+      const u64 r = keys[i] >> g.vbits;
+      if ((i == 0 || keys[i - 1] >> g.vbits != r) && mark[r] == gen) u = static_cast<int32_t>(r);
+    }
+    plan_rows<kGroupBlock, true>(m, u, in ? &g.ctl->touched_in : &g.ctl->touched_out, in ? g.in.touched : g.out.touched);
+    __syncthreads();  // plan_rows' arrays are free again
+  }
 }
 
 /// One thread per row whose tail holds at most kLaneTail entries and that has at most kLaneOps
@@ -1401,11 +1801,6 @@ DYNG_DEV void tail_lane(const merge_params& p, int block, int blocks) {
     }
     p.meta[u] = make_int2(mt.x, bl + alive + pending);
   }
-}
-
-template <int KW>
-__global__ void __launch_bounds__(256) k_tail_lane(merge_sides m) {
-  for_side(m, [](const merge_params& p, int block, int blocks) { tail_lane<KW>(p, block, blocks); });
 }
 
 /// One wave per row whose tail is short (at most kMergeSmall entries, 64 operations): the tail
@@ -1498,8 +1893,20 @@ DYNG_DEV void tail_wave(const merge_params& p, int block, int blocks) {
   }
 }
 
-__global__ void __launch_bounds__(kMergeBlock) k_tail_wave(merge_sides m) {
-  for_side(m, [](const merge_params& p, int block, int blocks) { tail_wave(p, block, blocks); });
+/// The tails short enough for a wave or a thread each, of both stores. Without a plan read back by the
+/// host every workgroup looks for itself whether the merges fit; if not, nothing is merged and the
+/// first workgroup says so (`hold`) to the launch and any engine run queued behind. One launch where
+/// three (the check, the lanes', the waves') took 10 us for a batch of 10.
+template <int KW>
+__global__ void __launch_bounds__(kTailsBlock) k_tails(merge_roles m) {
+  if (m.gate != nullptr && !merges_fit(m.gate, m.side[0].slot_cap, m.side[1].slot_cap, m.side[0].stage_cap)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) m.gate->hold = 1;
+    return;
+  }
+  int b = static_cast<int>(blockIdx.x), role = 0;
+  while (role < 3 && b >= m.groups[role]) b -= m.groups[role++];
+  const merge_params& p = m.side[role & 1];
+  if (role < 2) tail_wave(p, b, m.groups[role]); else tail_lane<KW>(p, b, m.groups[role]);
 }
 
 /// One workgroup per row whose tail needs more than a wave (up to kTailMax entries, kMergeSeg
@@ -1604,10 +2011,6 @@ DYNG_DEV void tail_block(const merge_params& p, int block, int blocks) {
   }
 }
 
-__global__ void __launch_bounds__(kMergeBlock) k_tail_block(merge_sides m) {
-  for_side(m, [](const merge_params& p, int block, int blocks) { tail_block(p, block, blocks); });
-}
-
 /// Count of the entries of a sorted run in global memory that are < v (or <= v when `upper`).
 DYNG_DEV int global_bound(const int32_t* a, int len, int32_t v, bool upper) {
   int lo = 0, hi = len;
@@ -1646,32 +2049,32 @@ DYNG_DEV int compact_alive(const merge_params& p, int64_t src, int len, int64_t 
   return carry;
 }
 
-/// One workgroup per row rewritten whole (its tail or dead entries outgrew their limits, or the
+/// One workgroup per row rewritten whole, staging from `stage_from` on (its tail or dead
+/// entries outgrew their limits, or the
 /// row its capacity): the alive base (A) and the alive tail (B) are compacted into the staging
 /// arena, then A, B and the pending entries (C) are merged into one base run, in place or at the
 /// tail of the arena. An entry's place is its index in its run plus the entries of the other two
 /// runs before it: A before B before C among equal neighbours.
-__global__ void __launch_bounds__(kMergeBlock) k_full_merge(merge_params p) {
+DYNG_DEV void full_merge(const merge_params& p, int block, int blocks, long long stage_from) {
   __shared__ int32_t s_v[kMergeSeg];
   __shared__ int32_t s_pp[kMergeSeg + 1];
   __shared__ int32_t s_b[kTailMax];
   __shared__ int s_tot[kMergeWaves];
   __shared__ long long s_stage, s_dest;
   __shared__ int s_newcap;
-  if (p.hold != nullptr && *p.hold != 0) return;  // uniform: the gate held the merges back
   const int count = p.list_count[kFull];
   const int32_t* list = p.lists + kFull * (p.N + 1);
   const u64 mask = (1ULL << p.vbits) - 1;
   const int tid = static_cast<int>(threadIdx.x);
   const int K = p.K;
-  for (int t = blockIdx.x; t < count; t += gridDim.x) {
+  for (int t = block; t < count; t += blocks) {
     const int32_t u = list[t];
     const int2 mt = p.meta[u];
     const int64_t a = p.row_a[u], b = p.row_b[u];
     const int nops = static_cast<int>(b - a);
-    const row_plan r = plan_row(p, u, mt, a, b);
+    const row_plan r = plan_row(p, u, mt, a, b, p.dead[u]);
     if (tid == 0) {
-      s_stage = static_cast<long long>(atomicAdd(reinterpret_cast<unsigned long long*>(p.stage_used),
+      s_stage = stage_from + static_cast<long long>(atomicAdd(reinterpret_cast<unsigned long long*>(p.stage_used),
                                                  static_cast<unsigned long long>(r.alive_base + r.alive_tail)));
       s_newcap = p.cap[u];
       s_dest = mt.x;
@@ -1748,6 +2151,20 @@ __global__ void __launch_bounds__(kMergeBlock) k_full_merge(merge_params p) {
       p.cap[u] = s_newcap;
     }
     __syncthreads();
+  }
+}
+
+/// The rows that take a workgroup each, of both stores: tails, then whole rows. The in-rows stage behind
+/// what the plan says the out-rows take. One launch where three took 11 us for a batch of 10.
+__global__ void __launch_bounds__(kMergeBlock) k_rows(merge_roles m) {
+  if (m.gate != nullptr && m.gate->hold != 0) return;  // uniform: the merges did not fit
+  int b = static_cast<int>(blockIdx.x), role = 0;
+  while (role < 3 && b >= m.groups[role]) b -= m.groups[role++];
+  const merge_params& p = m.side[role & 1];
+  if (role < 2) {
+    tail_block(p, b, m.groups[role]);
+  } else {
+    full_merge(p, b, m.groups[role], role == 3 ? *m.side[0].need_stage : 0);
   }
 }
 
@@ -2216,7 +2633,7 @@ void scan_batch(dyng_hip_graph* g, const dyng_hip_batch* b, hipStream_t s, batch
 }
 
 /// The merge parameters of one row store for a batch of N operations (keys of `vbits` bits).
-merge_params merge_setup(dyng_hip_graph* g, bool outs, int64_t N, int vbits, const int* hold) {
+merge_params merge_setup(dyng_hip_graph* g, bool outs, int64_t N, int vbits) {
   apply_control* dc = g->ctl.p;
   row_store& rs = outs ? g->out : g->in;
   merge_params mp{};
@@ -2252,29 +2669,47 @@ merge_params merge_setup(dyng_hip_graph* g, bool outs, int64_t N, int vbits, con
   mp.need_stage = outs ? &dc->need_stage_out : &dc->need_stage_in;
   mp.error_bits = &dc->error_bits;
   mp.headroom = g->props.headroom;
-  mp.hold = hold;
   return mp;
 }
 
 unsigned plan_groups(int64_t N) { return static_cast<unsigned>((N + kPlanBlock - 1) / kPlanBlock); }  // rows <= N
 
-/// Launch the tail merges of one mode for both stores: `groups` workgroups per store.
-void launch_tails(void (*kernel)(merge_sides), merge_sides ms, int out_groups, int in_groups, int block,
-                  hipStream_t s) {
-  if (out_groups + in_groups == 0) return;
-  ms.split = out_groups;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(out_groups + in_groups)), dim3(block), 0, s, ms);
+/// Launch the merges: `rows` of each store's per mode (an upper bound, the merges loop over what the
+/// plan listed), `cap` limiting the workgroups per role and store.
+void launch_merges(dyng_hip_graph* g, int64_t P, int vbits, const int* out_rows, const int* in_rows, bool gated,
+                   const int (&cap)[kModes], hipStream_t s) {
+  merge_roles m{};
+  m.side[0] = merge_setup(g, true, P, vbits);
+  m.side[1] = merge_setup(g, false, P, vbits);
+  m.gate = gated ? g->ctl.p : nullptr;
+  auto groups = [&](int rows, int per_group, int mode) { return std::min((rows + per_group - 1) / per_group, cap[mode]); };
+  auto launch = [&](void (*kernel)(merge_roles), int mode0, int per0, int mode1, int per1, int threads) {
+    m.groups[0] = groups(out_rows[mode0], per0, mode0);
+    m.groups[1] = groups(in_rows[mode0], per0, mode0);
+    m.groups[2] = groups(out_rows[mode1], per1, mode1);
+    m.groups[3] = groups(in_rows[mode1], per1, mode1);
+    const int all = m.groups[0] + m.groups[1] + m.groups[2] + m.groups[3];
+    if (all > 0) hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(all)), dim3(threads), 0, s, m);
+    DYNG_HIP_TRY(hipGetLastError());
+  };
+  mark_stage(g, 10, s);
+  launch(g->K == 1 ? k_tails<1> : k_tails<kRegWeights>, kTailWave, kTailsBlock / 64, kTailLane, kTailsBlock, kTailsBlock);
+  mark_stage(g, 11, s);
+  launch(k_rows, kTailBlock, 1, kFull, 1, kMergeBlock);
+  mark_stage(g, 12, s);
 }
 
 /// The merge plan and the merges with the plan read back first: the launches sized from it, the
-/// arenas compacted and the staging arena grown as it needs. `replan`: a plan already ran (its
-/// counts are cleared first).
-void merges_exact(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s, dyng_hip_apply_summary* out, bool replan) {
+/// arenas compacted and the staging arena grown as it needs. kPlanAgain: a plan already ran (its
+/// counts are cleared first); kPlanDone: it is the one to use.
+enum plan_state { kPlanNone, kPlanAgain, kPlanDone };
+void merges_exact(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s, dyng_hip_apply_summary* out, plan_state state) {
   apply_control* hc = g->host_ctl.p;
   apply_control* dc = g->ctl.p;
   const int K = g->K;
   for (int attempt = 0;; ++attempt) {
-    if (attempt > 0 || replan) {
+    const bool planned = attempt == 0 && state == kPlanDone;
+    if (attempt > 0 || state == kPlanAgain) {
       // planning again: clear what the last plan counted (the first plan of a batch finds them
       // zero, as the control block was uploaded zeroed at the start of the apply)
       hc->need_reloc_out = hc->need_reloc_in = hc->need_stage_out = hc->need_stage_in = 0;
@@ -2284,16 +2719,18 @@ void merges_exact(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s, dyng_h
       DYNG_HIP_TRY(hipMemcpyAsync(dc->modes_out, hc->modes_out, 2 * sizeof(hc->modes_out), hipMemcpyHostToDevice,
                                   s));
     }
-    merge_sides plan{};  // both stores' plans in one launch: out-rows first
-    plan.side[0] = merge_setup(g, true, N, vbits, nullptr);
-    plan.side[1] = merge_setup(g, false, N, vbits, nullptr);
-    plan.split = static_cast<int>(plan_groups(N));
-    hipLaunchKernelGGL(k_merge_plan, dim3(2 * plan_groups(N)), dim3(kPlanBlock), 0, s, plan);
-    DYNG_HIP_TRY(hipGetLastError());
+    if (!planned) {
+      merge_sides plan{};  // both stores' plans in one launch: out-rows first
+      plan.side[0] = merge_setup(g, true, N, vbits);
+      plan.side[1] = merge_setup(g, false, N, vbits);
+      plan.split = static_cast<int>(plan_groups(N));
+      hipLaunchKernelGGL(k_merge_plan, dim3(2 * plan_groups(N)), dim3(kPlanBlock), 0, s, plan);
+      DYNG_HIP_TRY(hipGetLastError());
+    }
     DYNG_HIP_TRY(hipMemcpyAsync(hc, dc, sizeof(apply_control), hipMemcpyDeviceToHost, s));
     DYNG_HIP_TRY(hipStreamSynchronize(s));
     if (out) out->host_plans += 1;
-    if (hc->error_bits != 0) return;  // reported by the caller
+    if (hc->error_bits != 0 || hc->miss != 0) return;  // the caller's to report, or to sort and plan
     bool compacted = false;
     for (int side = 0; side < 2; ++side) {
       row_store& rs = side == 0 ? g->out : g->in;
@@ -2313,72 +2750,33 @@ void merges_exact(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s, dyng_h
     DYNG_HIP_TRY(hipMemcpyAsync(&dc->tail_out, &hc->tail_out, 2 * sizeof(long long), hipMemcpyHostToDevice, s));
     DYNG_HIP_TRY(hipMemcpyAsync(&dc->garbage_out, &hc->garbage_out, 2 * sizeof(long long), hipMemcpyHostToDevice, s));
   }
-  const int64_t stage_need = std::max(hc->need_stage_out, hc->need_stage_in);
+  const int64_t stage_need = hc->need_stage_out + hc->need_stage_in;
   if (stage_need > g->stage_cap) {
     g->stage_cap = stage_need + stage_need / 4 + 4096;
     g->stage_nbr.reserve(g->stage_cap);
     g->stage_w.reserve(g->stage_cap * K);
   }
-  mark_stage(g, 10, s);
-  // the in-place tail merges: one launch per mode for both stores (out-rows in the first
-  // workgroups, in-rows in the rest), grids from the plan
-  merge_sides ms{};
-  ms.side[0] = merge_setup(g, true, N, vbits, nullptr);
-  ms.side[1] = merge_setup(g, false, N, vbits, nullptr);
-  auto groups = [](int rows, int per_group, int cap) { return std::min((rows + per_group - 1) / per_group, cap); };
-  launch_tails(g->K == 1 ? k_tail_lane<1> : k_tail_lane<kRegWeights>, ms, groups(hc->modes_out[kTailLane], 256, 8192),
-               groups(hc->modes_in[kTailLane], 256, 8192), 256, s);
-  launch_tails(k_tail_wave, ms, groups(hc->modes_out[kTailWave], kMergeWaves, 8192),
-               groups(hc->modes_in[kTailWave], kMergeWaves, 8192), kMergeBlock, s);
-  launch_tails(k_tail_block, ms, groups(hc->modes_out[kTailBlock], 1, 4096), groups(hc->modes_in[kTailBlock], 1, 4096),
-               kMergeBlock, s);
-  DYNG_HIP_TRY(hipGetLastError());
-  mark_stage(g, 11, s);
-  // whole rows through the staging arena, which both stores use: one store at a time
-  for (int side = 0; side < 2; ++side) {
-    const int rows = side == 0 ? hc->modes_out[kFull] : hc->modes_in[kFull];
-    if (rows > 0) {
-      hipLaunchKernelGGL(k_full_merge, dim3(static_cast<unsigned>(std::min(rows, 4096))), dim3(kMergeBlock), 0, s,
-                         ms.side[side]);
-    }
-  }
-  DYNG_HIP_TRY(hipGetLastError());
-  mark_stage(g, 12, s);
+  launch_merges(g, N, vbits, hc->modes_out, hc->modes_in, false, {32768, 4096, 4096, 8192}, s);
 }
 
-/// The merge plan and the merges queued together for a small batch, with no read-back in between:
-/// a gate on the device checks that the arenas take what the plan asks (k_merge_gate) and holds
-/// the merges back otherwise; the grids are sized for the batch (every touched row is one of its
-/// at most N + 1 rows per store) and the merges loop over the rows the plan listed.
+/// The merges of a small batch queued behind its plan, with no read-back in between: the device
+/// checks that the arenas take what the plan asks (merges_fit) and holds the merges back otherwise; the grids are sized for the batch (every touched row is one of its at most N + 1 rows
+/// per store) and the merges loop over the rows the plan listed.
+void merges_queued(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s) {
+  int rows[kModes];
+  std::fill(rows, rows + kModes, static_cast<int>(N + 1));
+  launch_merges(g, N, vbits, rows, rows, true, {1024, 256, 256, 1024}, s);
+}
+
+/// The merge plan and the merges queued together (see merges_queued).
 void merges_speculative(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s) {
-  apply_control* dc = g->ctl.p;
-  const int* hold = &dc->hold;
   merge_sides plan{};
-  plan.side[0] = merge_setup(g, true, N, vbits, nullptr);
-  plan.side[1] = merge_setup(g, false, N, vbits, nullptr);
+  plan.side[0] = merge_setup(g, true, N, vbits);
+  plan.side[1] = merge_setup(g, false, N, vbits);
   plan.split = static_cast<int>(plan_groups(N));
   hipLaunchKernelGGL(k_merge_plan, dim3(2 * plan_groups(N)), dim3(kPlanBlock), 0, s, plan);
-  hipLaunchKernelGGL(k_merge_gate, dim3(1), dim3(1), 0, s, dc, static_cast<long long>(g->out.slot_cap),
-                     static_cast<long long>(g->in.slot_cap), static_cast<long long>(g->stage_cap));
   DYNG_HIP_TRY(hipGetLastError());
-  mark_stage(g, 10, s);
-  merge_sides ms{};
-  ms.side[0] = merge_setup(g, true, N, vbits, hold);
-  ms.side[1] = merge_setup(g, false, N, vbits, hold);
-  const int rows = static_cast<int>(N + 1);
-  const int lane = std::min((rows + 255) / 256, 1024);
-  const int wave = std::min((rows + kMergeWaves - 1) / kMergeWaves, 512);
-  const int block = std::min(rows, 256);
-  launch_tails(g->K == 1 ? k_tail_lane<1> : k_tail_lane<kRegWeights>, ms, lane, lane, 256, s);
-  launch_tails(k_tail_wave, ms, wave, wave, kMergeBlock, s);
-  launch_tails(k_tail_block, ms, block, block, kMergeBlock, s);
-  DYNG_HIP_TRY(hipGetLastError());
-  mark_stage(g, 11, s);
-  for (int side = 0; side < 2; ++side) {
-    hipLaunchKernelGGL(k_full_merge, dim3(static_cast<unsigned>(block)), dim3(kMergeBlock), 0, s, ms.side[side]);
-  }
-  DYNG_HIP_TRY(hipGetLastError());
-  mark_stage(g, 12, s);
+  merges_queued(g, N, vbits, s);
 }
 
 /// Throw the invalid-argument error of the offending operation of rank `rank` (k_check_pairs):
@@ -2410,6 +2808,310 @@ void merges_speculative(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s) 
                                : " names an existing edge and batch_semantics::on_existing_insert is error"));
 }
 
+/// The control block at the start of an apply: counters, tails, the column targets; the first
+/// `num_counts` group counters cleared.
+void begin_apply(dyng_hip_graph* g, const batch_scan& sc, int num_counts, hipStream_t s) {
+  begin_params b{};
+  b.tail_out = g->out.tail;
+  b.tail_in = g->in.tail;
+  for (int k = 0; k < g->K; ++k) b.col_max[k] = std::max<int64_t>(g->wmax[k], sc.wmax[k]);
+  b.counts = g->group_counts.p;
+  b.num_counts = num_counts;
+  hipLaunchKernelGGL(k_begin, dim3(1), dim3(1024), 0, s, g->ctl.p, b);
+  DYNG_HIP_TRY(hipGetLastError());
+}
+
+/// Per-operation scratch for P places in sorted order.
+void reserve_ops(dyng_hip_graph* g, int64_t P) {
+  const int K = g->K;
+  g->keys_b.reserve(2 * P);  // out-row keys, then in-row keys
+  g->vals_b.reserve(2 * P);
+  g->pend_alive.reserve(P + 1);
+  g->kill.reserve(P + 1);
+  g->pend_prefix.reserve(P + 1);
+  g->kill_prefix.reserve(P + 1);
+  g->pend_w.reserve(P * K);
+  g->iop_type.reserve(P);
+  g->iop_wold.reserve(P * K);
+  g->iop_wnew.reserve(P * K);
+  g->ipend_alive.reserve(P + 1);
+  g->ikill.reserve(P + 1);
+  g->ipend_prefix.reserve(P + 1);
+  g->ikill_prefix.reserve(P + 1);
+  g->ipend_w.reserve(P * K);
+  g->merge_lists.reserve(2 * kModes * (P + 1));
+}
+
+/// Groups per direction for N operations, as a power of two's exponent.
+int group_bits(int64_t N, int vbits) {
+  int lb = 0;
+  while (lb < kGroupBits && lb < vbits) {
+    const int ops = lb < kGroupBitsFew ? kGroupOpsFew : lb < kGroupBitsSome ? kGroupOpsSome : kGroupOps;
+    if ((N / ops) >> (lb + 1) == 0) break;
+    ++lb;
+  }
+  return lb;
+}
+
+int op_bits(int64_t N) {
+  int b = 1;
+  while ((int64_t{1} << b) < N) ++b;
+  return b;
+}
+
+/// Whether a batch takes the grouped apply: an operation's row within its group, neighbour and
+/// batch place fit a word (less its top bit), the groups hold it on average, and no error mode wants
+/// the operations checked before anything changes (k_check_pairs reads them in the order of the rows).
+bool group_eligible(const dyng_hip_graph* g, int64_t N, int vbits, int lb) {
+  return N > 0 && N <= kGroupMost && 2 * vbits - lb + op_bits(N) <= 63 &&
+         g->props.on_missing_delete != 1 && g->props.on_existing_insert != 1;
+}
+
+out_pair_params out_setup(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, int64_t N, int64_t P, int vbits,
+                          int64_t n_before) {
+  out_pair_params op{};
+  op.L = L;
+  op.keys = g->keys_b.p;
+  op.vals = g->vals_b.p;
+  op.N = N;
+  op.stride = P;
+  op.vbits = vbits;
+  op.K = g->K;
+  op.n_before = n_before;
+  op.upsert = g->props.on_existing_insert == 0 ? 1 : 0;
+  op.ins_w = sc.ins_w;
+  op.meta = g->out.meta.p;
+  op.base = g->out.base.p;
+  op.dead = g->out.dead.p;
+  op.nbr = g->out.nbr.p;
+  op.w = g->out.w.p;
+  op.slot_cap = g->out.slot_cap;
+  op.pend_alive = g->pend_alive.p;
+  op.kill = g->kill.p;
+  op.pend_w = g->pend_w.p;
+  op.e_inc = g->ins_inc.p;
+  op.e_fw = g->props.allow_parallel ? nullptr : g->ins_fw.p;
+  op.iop_type = g->iop_type.p;
+  op.iop_wold = g->iop_wold.p;
+  op.iop_wnew = g->iop_wnew.p;
+  op.mark = g->mark_out.p;
+  op.mark_gen = g->mark_generation;
+  op.touched = g->touched_out.p;
+  op.row_a = g->row_a_out.p;
+  op.row_b = g->row_b_out.p;
+  op.ctl = g->ctl.p;
+  return op;
+}
+
+in_pair_params in_setup(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, int64_t N, int64_t P, int vbits) {
+  in_pair_params ip{};
+  ip.L = L;
+  ip.ins_w = sc.ins_w;
+  ip.upsert = g->props.on_existing_insert == 0 ? 1 : 0;
+  ip.keys = g->keys_b.p + P;
+  ip.vals = g->vals_b.p + P;
+  ip.N = N;
+  ip.stride = P;
+  ip.vbits = vbits;
+  ip.K = g->K;
+  ip.iop_type = g->iop_type.p;
+  ip.iop_wold = g->iop_wold.p;
+  ip.iop_wnew = g->iop_wnew.p;
+  ip.meta = g->in.meta.p;
+  ip.base = g->in.base.p;
+  ip.dead = g->in.dead.p;
+  ip.nbr = g->in.nbr.p;
+  ip.w = g->in.w.p;
+  ip.slot_cap = g->in.slot_cap;
+  ip.pend_alive = g->ipend_alive.p;
+  ip.kill = g->ikill.p;
+  ip.pend_w = g->ipend_w.p;
+  ip.mark = g->mark_in.p;
+  ip.mark_gen = g->mark_generation;
+  ip.touched = g->touched_in.p;
+  ip.row_a = g->row_a_in.p;
+  ip.row_b = g->row_b_in.p;
+  ip.ctl = g->ctl.p;
+  return ip;
+}
+
+op_layout layout_of(const dyng_hip_graph* g, const batch_scan& sc) {
+  op_layout L;
+  L.first_is_del = g->props.deletions_first ? 1 : 0;
+  L.num_first = L.first_is_del ? sc.num_del : sc.num_ins;
+  L.num_second = L.first_is_del ? sc.num_ins : sc.num_del;
+  L.stride = g->props.directed ? 1 : 2;
+  return L;
+}
+
+/// The rows' update behind a device-wide sort of the operations: the error modes, batches past the
+/// groups' limits, and batches with more operations on one row than a group takes.
+void rows_sorted(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, int64_t N, int vbits, int64_t n_before,
+                 hipStream_t s, dyng_hip_apply_summary* out, hipEvent_t wait, apply_pending& ap) {
+  apply_control* hc = g->host_ctl.p;
+  apply_control* dc = g->ctl.p;
+  const int K = g->K;
+  const int64_t n_after = sc.n_after;
+  const int32_t *ins_src = sc.ins_src, *ins_dst = sc.ins_dst, *del_src = sc.del_src, *del_dst = sc.del_dst;
+  g->keys_a.reserve(2 * N);
+  g->vals_a.reserve(2 * N);
+  mark_stage(g, 2, s);
+  hipLaunchKernelGGL(k_make_ops, dim3(blocks_for(N)), dim3(kBlock), 0, s, L, ins_src, ins_dst, del_src, del_dst,
+                     g->props.directed, g->props.on_self_loop == 1 ? 1 : 0, n_after, vbits, g->keys_a.p,
+                     g->vals_a.p, g->del_src.p, g->del_dst.p, g->ins_src.p, g->ins_dst.p, g->ins_inc.p,
+                     g->props.allow_parallel ? nullptr : g->ins_fw.p, K, g->props.on_missing_delete == 1 ? 1 : 0,
+                     dc);
+  DYNG_HIP_TRY(hipGetLastError());
+  mark_stage(g, 3, s);
+  // one stable sort of both directions' keys (2N of them, 2 * vbits + 1 bits): one sort of 2N
+  // keys costs little more than one of N, since rocPRIM's small-size path is launch-bound
+  sort_pairs(g->sort_tmp, g->keys_a.p, g->keys_b.p, g->vals_a.p, g->vals_b.p, 2 * N, 2 * vbits + 1, s);
+  hipLaunchKernelGGL(k_untag, dim3(std::min<unsigned>(blocks_for(2 * N), 1024)), dim3(kBlock), 0, s, g->keys_b.p,
+                     2 * N, vbits);
+  if (g->props.on_missing_delete == 1 || g->props.on_existing_insert == 1) {
+    // the error modes: every operation checked before anything changes (one more launch and
+    // synchronization, only in these modes)
+    hipLaunchKernelGGL(k_check_pairs, dim3(blocks_for(N)), dim3(kBlock), 0, s, L, g->keys_b.p, g->vals_b.p, N,
+                       vbits, n_before, g->out.meta.p, g->out.base.p, g->out.nbr.p,
+                       g->props.on_missing_delete == 1 ? 1 : 0, g->props.on_existing_insert == 1 ? 1 : 0, dc);
+    DYNG_HIP_TRY(hipGetLastError());
+    DYNG_HIP_TRY(hipMemcpyAsync(&hc->first_error, &dc->first_error, sizeof(hc->first_error),
+                                hipMemcpyDeviceToHost, s));
+    DYNG_HIP_TRY(hipStreamSynchronize(s));
+    if (hc->first_error != kNoError) report_batch_error(g, sc, L, hc->first_error, s);
+  }
+  mark_stage(g, 4, s);
+  const out_pair_params op = out_setup(g, sc, L, N, N, vbits, n_before);
+  const in_pair_params ip = in_setup(g, sc, L, N, N, vbits);
+  const unsigned pair_groups = blocks_for(N + 1);
+  if (!g->props.allow_parallel) {
+    // a simple graph: the in-row pass replays the operations itself, in the same launch
+    mark_stage(g, 5, s);
+    hipLaunchKernelGGL(k_pairs_simple, dim3(2 * pair_groups), dim3(kBlock), 0, s, op, ip,
+                       static_cast<int>(pair_groups));
+    DYNG_HIP_TRY(hipGetLastError());
+    mark_stage(g, 6, s);
+    mark_stage(g, 7, s);
+  } else {
+    mark_stage(g, 5, s);
+    hipLaunchKernelGGL(k_out_pairs, dim3(pair_groups), dim3(kBlock), 0, s, op);
+    DYNG_HIP_TRY(hipGetLastError());
+    mark_stage(g, 6, s);
+    mark_stage(g, 7, s);
+    hipLaunchKernelGGL(k_in_pairs, dim3(pair_groups), dim3(kBlock), 0, s, ip);
+    DYNG_HIP_TRY(hipGetLastError());
+  }
+  mark_stage(g, 8, s);
+  exclusive_scan4(g->scan_tmp, g->pend_alive.p, g->kill.p, g->ipend_alive.p, g->ikill.p, g->pend_prefix.p,
+                  g->kill_prefix.p, g->ipend_prefix.p, g->ikill_prefix.p, N + 1, s);
+  mark_stage(g, 9, s);
+  // ---- plan the merges: each row's mode, and the staging and tail slots they take ----
+  g->merge_lists.reserve(2 * kModes * (N + 1));
+  if (wait != nullptr) DYNG_HIP_TRY(hipStreamWaitEvent(s, wait, 0));  // before the rows change
+  ap.speculative = N <= kSpeculativeOps;
+  if (ap.speculative) {
+    merges_speculative(g, N, vbits, s);
+  } else {
+    merges_exact(g, N, vbits, s, out, kPlanNone);
+  }
+}
+
+/// A batch whose groups could not take it (more operations on one row than a group's room) again
+/// behind the device-wide sort; nothing changed yet. The graph's next batches go there directly: a
+/// stream with such a batch has more of them, and each would pay for the attempt.
+void resort(dyng_hip_graph* g, const batch_scan& sc, int64_t n_before, hipStream_t s, dyng_hip_apply_summary* out,
+            apply_pending& ap) {
+  g->group_pause = kGroupPause;
+  begin_apply(g, sc, 0, s);
+  ap.P = ap.N;
+  rows_sorted(g, sc, layout_of(g, sc), ap.N, ap.vbits, n_before, s, out, ap.wait, ap);
+}
+
+/// The rows' update by groups (see k_group_front).
+void rows_grouped(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, int64_t N, int64_t P, int vbits, int lb,
+                  int64_t n_before, hipStream_t s, dyng_hip_apply_summary* out, hipEvent_t wait, apply_pending& ap) {
+  apply_control* dc = g->ctl.p;
+  const int groups = 1 << lb;
+  mark_stage(g, 2, s);
+  front_params f{};
+  f.L = L;
+  f.ins_src = sc.ins_src;
+  f.ins_dst = sc.ins_dst;
+  f.del_src = sc.del_src;
+  f.del_dst = sc.del_dst;
+  f.directed = g->props.directed;
+  f.drop_self_loops = g->props.on_self_loop == 1 ? 1 : 0;
+  f.n_after = sc.n_after;
+  f.vbits = vbits;
+  f.ebits = op_bits(N);
+  f.lb = lb;
+  f.K = g->K;
+  f.groups = groups;
+  f.entries = g->group_entries.p;
+  f.counts = g->group_counts.p;
+  f.e_del_src = g->del_src.p;
+  f.e_del_dst = g->del_dst.p;
+  f.e_ins_src = g->ins_src.p;
+  f.e_ins_dst = g->ins_dst.p;
+  f.e_inc = g->ins_inc.p;
+  f.e_fw = g->props.allow_parallel ? nullptr : g->ins_fw.p;
+  f.ctl = dc;
+  // one operation per thread while that fills the chip at most once; eight above, so that a
+  // workgroup reserves a group's places for several operations at a time
+  if (N <= 256 * 1024) {
+    hipLaunchKernelGGL(k_group_front<1>, dim3(blocks_for(N, 1024)), dim3(1024), 0, s, f);
+  } else {
+    hipLaunchKernelGGL(k_group_front<8>, dim3(blocks_for(N, 8 * 1024)), dim3(1024), 0, s, f);
+  }
+  DYNG_HIP_TRY(hipGetLastError());
+  mark_stage(g, 3, s);
+  mark_stage(g, 4, s);
+  group_params gp{};
+  gp.entries = g->group_entries.p;
+  gp.counts = g->group_counts.p;
+  gp.groups = groups;
+  gp.vbits = vbits;
+  gp.ebits = f.ebits;
+  gp.lb = lb;
+  uint32_t inverse = kGroupHash;  // Newton's iteration: right modulo 2^3, then 2^6, ... 2^48
+  for (int i = 0; i < 4; ++i) inverse *= 2u - kGroupHash * inverse;
+  gp.inverse = inverse;
+  gp.keys = g->keys_b.p;
+  gp.vals = g->vals_b.p;
+  gp.P = P;
+  gp.out = out_setup(g, sc, L, N, P, vbits, n_before);
+  gp.in = in_setup(g, sc, L, N, P, vbits);
+  gp.merge_out = merge_setup(g, true, P, vbits);
+  gp.merge_in = merge_setup(g, false, P, vbits);
+  gp.pend_prefix_out = g->pend_prefix.p;
+  gp.kill_prefix_out = g->kill_prefix.p;
+  gp.pend_prefix_in = g->ipend_prefix.p;
+  gp.kill_prefix_in = g->ikill_prefix.p;
+  gp.ctl = dc;
+  mark_stage(g, 5, s);
+  if (!g->props.allow_parallel) {
+    hipLaunchKernelGGL(k_group_pairs<kGroupsBoth>, dim3(static_cast<unsigned>(2 * groups)), dim3(kGroupBlock), 0, s, gp);
+    mark_stage(g, 6, s);
+    mark_stage(g, 7, s);
+  } else {
+    hipLaunchKernelGGL(k_group_pairs<kGroupsOut>, dim3(static_cast<unsigned>(groups)), dim3(kGroupBlock), 0, s, gp);
+    mark_stage(g, 6, s);
+    mark_stage(g, 7, s);
+    hipLaunchKernelGGL(k_group_pairs<kGroupsIn>, dim3(static_cast<unsigned>(groups)), dim3(kGroupBlock), 0, s, gp);
+  }
+  DYNG_HIP_TRY(hipGetLastError());
+  mark_stage(g, 8, s);
+  mark_stage(g, 9, s);
+  ap.speculative = N <= kSpeculativeOps;
+  if (wait != nullptr) DYNG_HIP_TRY(hipStreamWaitEvent(s, wait, 0));  // before the rows change
+  if (ap.speculative) {
+    merges_queued(g, P, vbits, s);
+    return;
+  }
+  merges_exact(g, P, vbits, s, out, kPlanDone);
+  if (g->host_ctl.p->miss != 0) resort(g, sc, n_before, s, out, ap);
+}
+
 apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t s, dyng_hip_apply_summary* out,
                            hipEvent_t wait) {
   const int K = g->K;
@@ -2427,8 +3129,6 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
   g->last.n = g->n;
   g->last.num_ins = sc.num_ins;
   const int64_t num_ins = sc.num_ins, num_del = sc.num_del;
-  const int32_t *ins_src = sc.ins_src, *ins_dst = sc.ins_dst, *ins_w = sc.ins_w, *del_src = sc.del_src,
-                *del_dst = sc.del_dst;
   const int64_t n_after = sc.n_after;
   apply_control* hc = g->host_ctl.p;
   const int64_t n_before = g->n;
@@ -2444,11 +3144,7 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
   ap.N = N;
   ap.vbits = vbits;
   ap.wait = wait;
-  op_layout L;
-  L.first_is_del = g->props.deletions_first ? 1 : 0;
-  L.num_first = L.first_is_del ? num_del : num_ins;
-  L.num_second = L.first_is_del ? num_ins : num_del;
-  L.stride = stride;
+  const op_layout L = layout_of(g, sc);
   g->num_del_slots = num_del * stride;
   g->num_ins_slots = num_ins * stride;
   g->del_src.reserve(g->num_del_slots);
@@ -2457,25 +3153,18 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
   g->ins_dst.reserve(g->num_ins_slots);
   g->ins_inc.reserve(g->num_ins_slots * K);
   if (!g->props.allow_parallel) g->ins_fw.reserve(g->num_ins_slots * K);
-  g->keys_a.reserve(2 * N);  // out-row keys, then in-row keys
-  g->keys_b.reserve(2 * N);
-  g->vals_a.reserve(2 * N);
-  g->vals_b.reserve(2 * N);
-  g->pend_alive.reserve(N + 1);
-  g->kill.reserve(N + 1);
-  g->pend_prefix.reserve(N + 1);
-  g->kill_prefix.reserve(N + 1);
-  g->pend_w.reserve(N * K);
-  g->iop_type.reserve(N);
-  g->iop_wold.reserve(N * K);
-  g->iop_wnew.reserve(N * K);
-  g->ipend_alive.reserve(N + 1);
-  g->ikill.reserve(N + 1);
-  g->ipend_prefix.reserve(N + 1);
-  g->ikill_prefix.reserve(N + 1);
-  g->ipend_w.reserve(N * K);
-  g->touched_out.reserve(N + 1);
-  g->touched_in.reserve(N + 1);
+  // P: places of the sorted operations (the grouped apply leaves one behind each group)
+  const int lb = group_bits(N, vbits);
+  const bool grouped = group_eligible(g, N, vbits, lb) && g->group_pause == 0;
+  if (g->group_pause > 0) g->group_pause -= 1;
+  const int64_t P = ap.P = grouped ? N + (int64_t{1} << lb) : N;
+  if (grouped) {
+    g->group_entries.reserve((size_t{2} << lb) * kGroupCap);
+    g->group_counts.reserve(size_t{2} << lb);
+  }
+  reserve_ops(g, P);
+  g->touched_out.reserve(P + 1);
+  g->touched_in.reserve(P + 1);
   g->row_a_out.reserve(g->n_cap);
   g->row_b_out.reserve(g->n_cap);
   g->row_a_in.reserve(g->n_cap);
@@ -2485,129 +3174,13 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
     fill<int32_t>(g->mark_in.p, g->n_cap, 0, s);
     g->mark_generation = 1;
   }
-  // ---- control block: counters, tails, the column targets ----
-  std::memset(hc, 0, sizeof(apply_control));
-  hc->first_error = kNoError;
-  for (int k = 0; k < K; ++k) hc->col_max[k] = std::max<int64_t>(g->wmax[k], sc.wmax[k]);
-  hc->tail_out = g->out.tail;
-  hc->tail_in = g->in.tail;
-  DYNG_HIP_TRY(hipMemcpyAsync(g->ctl.p, hc, sizeof(apply_control), hipMemcpyHostToDevice, s));
+  begin_apply(g, sc, grouped ? 2 << lb : 0, s);
   apply_control* dc = g->ctl.p;
   if (N > 0) {
-    mark_stage(g, 2, s);
-    hipLaunchKernelGGL(k_make_ops, dim3(blocks_for(N)), dim3(kBlock), 0, s, L, ins_src, ins_dst, del_src, del_dst,
-                       g->props.directed, g->props.on_self_loop == 1 ? 1 : 0, n_after, vbits, g->keys_a.p,
-                       g->vals_a.p, g->del_src.p, g->del_dst.p, g->ins_src.p, g->ins_dst.p, g->ins_inc.p,
-                       g->props.allow_parallel ? nullptr : g->ins_fw.p, K, g->props.on_missing_delete == 1 ? 1 : 0,
-                       dc);
-    DYNG_HIP_TRY(hipGetLastError());
-    mark_stage(g, 3, s);
-    // one stable sort of both directions' keys (2N of them, 2 * vbits + 1 bits): one sort of 2N
-    // keys costs little more than one of N, since rocPRIM's small-size path is launch-bound
-    sort_pairs(g->sort_tmp, g->keys_a.p, g->keys_b.p, g->vals_a.p, g->vals_b.p, 2 * N, 2 * vbits + 1, s);
-    hipLaunchKernelGGL(k_untag, dim3(std::min<unsigned>(blocks_for(2 * N), 1024)), dim3(kBlock), 0, s, g->keys_b.p,
-                       2 * N, vbits);
-    if (g->props.on_missing_delete == 1 || g->props.on_existing_insert == 1) {
-      // the error modes: every operation checked before anything changes (one more launch and
-      // synchronization, only in these modes)
-      hipLaunchKernelGGL(k_check_pairs, dim3(blocks_for(N)), dim3(kBlock), 0, s, L, g->keys_b.p, g->vals_b.p, N,
-                         vbits, n_before, g->out.meta.p, g->out.base.p, g->out.nbr.p,
-                         g->props.on_missing_delete == 1 ? 1 : 0, g->props.on_existing_insert == 1 ? 1 : 0, dc);
-      DYNG_HIP_TRY(hipGetLastError());
-      DYNG_HIP_TRY(hipMemcpyAsync(&hc->first_error, &dc->first_error, sizeof(hc->first_error),
-                                  hipMemcpyDeviceToHost, s));
-      DYNG_HIP_TRY(hipStreamSynchronize(s));
-      if (hc->first_error != kNoError) report_batch_error(g, sc, L, hc->first_error, s);
-    }
-    mark_stage(g, 4, s);
-    out_pair_params op{};
-    op.L = L;
-    op.keys = g->keys_b.p;
-    op.vals = g->vals_b.p;
-    op.N = N;
-    op.vbits = vbits;
-    op.K = K;
-    op.n_before = n_before;
-    op.upsert = g->props.on_existing_insert == 0 ? 1 : 0;
-    op.ins_w = ins_w;
-    op.meta = g->out.meta.p;
-    op.base = g->out.base.p;
-    op.dead = g->out.dead.p;
-    op.nbr = g->out.nbr.p;
-    op.w = g->out.w.p;
-    op.slot_cap = g->out.slot_cap;
-    op.pend_alive = g->pend_alive.p;
-    op.kill = g->kill.p;
-    op.pend_w = g->pend_w.p;
-    op.e_inc = g->ins_inc.p;
-    op.e_fw = g->props.allow_parallel ? nullptr : g->ins_fw.p;
-    op.iop_type = g->iop_type.p;
-    op.iop_wold = g->iop_wold.p;
-    op.iop_wnew = g->iop_wnew.p;
-    op.mark = g->mark_out.p;
-    op.mark_gen = g->mark_generation;
-    op.touched = g->touched_out.p;
-    op.row_a = g->row_a_out.p;
-    op.row_b = g->row_b_out.p;
-    op.ctl = dc;
-    // ---- the in-rows' operations (they do not read the out-rows) ----
-    in_pair_params ip{};
-    ip.L = L;
-    ip.ins_w = ins_w;
-    ip.upsert = op.upsert;
-    ip.keys = g->keys_b.p + N;
-    ip.vals = g->vals_b.p + N;
-    ip.N = N;
-    ip.vbits = vbits;
-    ip.K = K;
-    ip.iop_type = g->iop_type.p;
-    ip.iop_wold = g->iop_wold.p;
-    ip.iop_wnew = g->iop_wnew.p;
-    ip.meta = g->in.meta.p;
-    ip.base = g->in.base.p;
-    ip.dead = g->in.dead.p;
-    ip.nbr = g->in.nbr.p;
-    ip.w = g->in.w.p;
-    ip.slot_cap = g->in.slot_cap;
-    ip.pend_alive = g->ipend_alive.p;
-    ip.kill = g->ikill.p;
-    ip.pend_w = g->ipend_w.p;
-    ip.mark = g->mark_in.p;
-    ip.mark_gen = g->mark_generation;
-    ip.touched = g->touched_in.p;
-    ip.row_a = g->row_a_in.p;
-    ip.row_b = g->row_b_in.p;
-    ip.ctl = dc;
-    const unsigned pair_groups = blocks_for(N + 1);
-    if (!g->props.allow_parallel) {
-      // a simple graph: the in-row pass replays the operations itself, in the same launch
-      mark_stage(g, 5, s);
-      hipLaunchKernelGGL(k_pairs_simple, dim3(2 * pair_groups), dim3(kBlock), 0, s, op, ip,
-                         static_cast<int>(pair_groups));
-      DYNG_HIP_TRY(hipGetLastError());
-      mark_stage(g, 6, s);
-      mark_stage(g, 7, s);
+    if (grouped) {
+      rows_grouped(g, sc, L, N, P, vbits, lb, n_before, s, out, wait, ap);
     } else {
-      mark_stage(g, 5, s);
-      hipLaunchKernelGGL(k_out_pairs, dim3(pair_groups), dim3(kBlock), 0, s, op);
-      DYNG_HIP_TRY(hipGetLastError());
-      mark_stage(g, 6, s);
-      mark_stage(g, 7, s);
-      hipLaunchKernelGGL(k_in_pairs, dim3(pair_groups), dim3(kBlock), 0, s, ip);
-      DYNG_HIP_TRY(hipGetLastError());
-    }
-    mark_stage(g, 8, s);
-    exclusive_scan4(g->scan_tmp, g->pend_alive.p, g->kill.p, g->ipend_alive.p, g->ikill.p, g->pend_prefix.p,
-                    g->kill_prefix.p, g->ipend_prefix.p, g->ikill_prefix.p, N + 1, s);
-    mark_stage(g, 9, s);
-    // ---- plan the merges: each row's mode, and the staging and tail slots they take ----
-    g->merge_lists.reserve(2 * kModes * (N + 1));
-    if (wait != nullptr) DYNG_HIP_TRY(hipStreamWaitEvent(s, wait, 0));  // before the rows change
-    ap.speculative = N <= kSpeculativeOps;
-    if (ap.speculative) {
-      merges_speculative(g, N, vbits, s);
-    } else {
-      merges_exact(g, N, vbits, s, out, false);
+      rows_sorted(g, sc, L, N, vbits, n_before, s, out, wait, ap);
     }
   }
   if (wait != nullptr) DYNG_HIP_TRY(hipStreamWaitEvent(s, wait, 0));
@@ -2625,13 +3198,19 @@ void apply_finish(dyng_hip_graph* g, const batch_scan& sc, apply_pending& ap, hi
   const int64_t n_before = ap.n_before;
   const int64_t n_after = g->n;
   DYNG_HIP_TRY(hipStreamSynchronize(s));
+  if (hc->miss != 0 && hc->error_bits == 0) {
+    resort(g, sc, n_before, s, out, ap);
+    DYNG_HIP_TRY(hipMemcpyAsync(hc, dc, sizeof(apply_control), hipMemcpyDeviceToHost, s));
+    DYNG_HIP_TRY(hipStreamSynchronize(s));
+    ap.replanned = true;
+  }
   if (ap.speculative && hc->hold != 0 && hc->error_bits == 0) {
     // the arenas could not take the merges as the device planned them: plan again with the
     // host's compaction and staging growth (nothing was merged; the rows are as the pairing left
     // them)
     hc->hold = 0;
     DYNG_HIP_TRY(hipMemcpyAsync(&dc->hold, &hc->hold, sizeof(int), hipMemcpyHostToDevice, s));
-    merges_exact(g, ap.N, ap.vbits, s, out, true);
+    merges_exact(g, ap.P, ap.vbits, s, out, kPlanAgain);
     if (ap.wait != nullptr) DYNG_HIP_TRY(hipStreamWaitEvent(s, ap.wait, 0));
     DYNG_HIP_TRY(hipMemcpyAsync(hc, dc, sizeof(apply_control), hipMemcpyDeviceToHost, s));
     DYNG_HIP_TRY(hipStreamSynchronize(s));

@@ -180,9 +180,10 @@ struct apply_control {
   unsigned long long first_error;
   /// nonzero: the merges were queued without the host reading the plan, and the arenas could
   /// not take them as planned (or an error came first): the merges and any engine run queued
-  /// behind them did nothing, and the host plans again (k_merge_gate)
+  /// behind them did nothing, and the host plans again (merges_fit)
   int hold;
-  int pad1;
+  /// nonzero: the grouped apply did nothing (k_group_front says why); the host sorts the batch
+  int miss;
 };
 
 /// What the batch scan found (before anything changes) and where the batch is on the device.
@@ -272,6 +273,7 @@ struct apply_pending {
   bool speculative = false;
   bool replanned = false;
   int64_t n_before = 0, N = 0;
+  int64_t P = 0;               ///< places of the operations in sorted order
   int vbits = 0;
   hipEvent_t wait = nullptr;
 };
@@ -318,6 +320,9 @@ struct dyng_hip_graph {
   dyng_hip::dbuf<unsigned long long> keys_a, keys_b;  ///< the apply's sort: out-row keys, then in-row keys
   dyng_hip::dbuf<uint32_t> vals_a, vals_b;
   dyng_hip::dbuf<unsigned char> sort_tmp, scan_tmp;
+  dyng_hip::dbuf<unsigned long long> group_entries;  ///< the grouped apply's operations, a fixed room per group
+  dyng_hip::dbuf<int> group_counts;
+  int group_pause = 0;  ///< batches left that are sorted device-wide (see resort)
   dyng_hip::dbuf<int32_t> pend_alive, kill, pend_prefix, kill_prefix, pend_w;
   dyng_hip::dbuf<int32_t> ipend_alive, ikill, ipend_prefix, ikill_prefix, ipend_w;
   dyng_hip::dbuf<int32_t> iop_type, iop_wold, iop_wnew;

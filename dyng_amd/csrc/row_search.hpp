@@ -25,14 +25,15 @@ struct alignas(16) row_quad {
 /// wave's lanes usually search different rows, so each instruction fetches up to 64 lines). A
 /// word that holds an entry of [lo, hi) lies in the same page as that entry, so no load reaches
 /// memory the row's allocation does not map.
+template <int kProbes = 7>
 DYNG_ROW_SEARCH_FN int row_lower_bound(const int32_t* a, int lo, int hi, int32_t v) {
   while (hi - lo > 16) {  // the answer lies in [lo, hi]
-    const int step = (hi - lo) >> 3;
-    int below = 0;  // probes lo + k * step (k = 1..7) whose neighbour is < v: a prefix of them
+    const int step = (hi - lo) / (kProbes + 1);
+    int below = 0;  // probes lo + k * step (k = 1..kProbes) whose neighbour is < v: a prefix of them
 #pragma unroll
-    for (int k = 1; k <= 7; ++k) below += (a[lo + k * step] & 0x7fffffff) < v ? 1 : 0;
+    for (int k = 1; k <= kProbes; ++k) below += (a[lo + k * step] & 0x7fffffff) < v ? 1 : 0;
     const int next_lo = below == 0 ? lo : lo + below * step + 1;
-    hi = below == 7 ? hi : lo + (below + 1) * step;
+    hi = below == kProbes ? hi : lo + (below + 1) * step;
     lo = next_lo;
   }
   if (lo >= hi) return lo;
