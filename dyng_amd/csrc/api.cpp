@@ -310,7 +310,7 @@ void repair_core(dyng_hip_graph* g, dyng_hip_result* r, int64_t delta, int64_t m
     DYNG_HIP_TRY(hipEventRecord(ev.a, s));
     r->tree_token = 0;
     // queued right behind the apply when it is in flight: one synchronization for both
-    engine_pending pend = engine_launch(&run, true, s, inflight != nullptr ? apply_hold(g) : nullptr);
+    engine_pending pend = engine_launch(&run, true, s, inflight != nullptr ? inflight->ap : nullptr);
     DYNG_HIP_TRY(hipEventRecord(ev.b, s));
     if (inflight != nullptr) {
       try {

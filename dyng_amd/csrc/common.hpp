@@ -78,7 +78,20 @@ DYNG_DEV int wave_scan(int v) {
   return v;
 }
 
-/// The same within each row of 16 lanes.
+/// Fold `f` over the wave by the same six moves: the last lane has the result (a lane without a
+/// source folds its own value in again, so f(x, x) must be x).
+template <class F>
+DYNG_DEV int wave_fold(int v, F f) {
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));
+  v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));
+  return v;
+}
+
+/// The same sums within each row of 16 lanes.
 DYNG_DEV int row_scan(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
   v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);

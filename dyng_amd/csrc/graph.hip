@@ -405,76 +405,97 @@ __global__ void k_column_summary(const int2* meta, const int32_t* nbr, const int
 // ---------------------------------------------------------------------------------------------
 
 /// Batch scan (before anything changes): id range, self-loops, weight range per objective. The
-/// insertions and deletions are read in one loop (their loads in flight together); each
-/// workgroup reduces its nine values in one pass (wave shuffles, one barrier) and adds them to
-/// the control block with one atomic per value: the launch is 64 workgroups of 1024 threads, so
-/// few workgroups queue on those nine addresses, which share a cache line.
+/// insertions and deletions are read in one loop (their loads in flight together); each workgroup
+/// folds its values by lane-to-lane moves and one barrier and writes them to pinned host memory, where
+/// the host folds the workgroups': no control block sent up, no copy back. A batch of 10: 11 us of
+/// shuffles and atomics between two copies of 4 us each before.
 constexpr int kScanBlock = 1024;
+constexpr int64_t kGatherBytes = int64_t{1} << 20;  ///< host batches up to this many bytes go as one copy from pinned memory
+constexpr int kScanColumns = 4;  ///< weight columns per pass of the batch scan
 __global__ void __launch_bounds__(kScanBlock) k_batch_scan(const int32_t* ins_src, const int32_t* ins_dst,
                                                             const int32_t* ins_w, int64_t num_ins,
                                                             const int32_t* del_src, const int32_t* del_dst,
-                                                            int64_t num_del, int K, apply_control* ctl) {
-  long long mn = INT32_MAX, mx = -1, sl_i = 0, sl_d = 0, wmin = INT32_MAX;
-  long long lmax0 = 0, lmax1 = 0, lmax2 = 0, lmax3 = 0;  // named: a private array would sit in scratch
+                                                            int64_t num_del, int K, scan_part* parts) {
+  constexpr int kVals = 4 + 2 * kScanColumns;
+  __shared__ int part[kScanBlock / 64][kVals];
   const int64_t stride = int64_t{gridDim.x} * blockDim.x;
-  const int64_t total = num_ins > num_del ? num_ins : num_del;
-  for (int64_t i = blockIdx.x * int64_t{blockDim.x} + threadIdx.x; i < total; i += stride) {
-    const bool ins = i < num_ins, del = i < num_del;
-    const int32_t u = ins ? ins_src[i] : 0, v = ins ? ins_dst[i] : 0;
-    const int32_t du = del ? del_src[i] : 0, dv = del ? del_dst[i] : 0;
-    if (ins) {
-      mn = min(mn, static_cast<long long>(min(u, v)));
-      mx = max(mx, static_cast<long long>(max(u, v)));
-      sl_i += u == v ? 1 : 0;
-      for (int k = 0; k < K; ++k) {
-        const int32_t x = ins_w[i * K + k];
-        wmin = min(wmin, static_cast<long long>(x));
-        if (k == 0) lmax0 = max(lmax0, static_cast<long long>(x));
-        else if (k == 1) lmax1 = max(lmax1, static_cast<long long>(x));
-        else if (k == 2) lmax2 = max(lmax2, static_cast<long long>(x));
-        else if (k == 3) lmax3 = max(lmax3, static_cast<long long>(x));
-        else atomicMax(&ctl->batch_wmax[k], x);
-        if (x < 1) atomicMin(&ctl->batch_wmin[k], x);  // rare: the objective checks are the host's
+  const int64_t first = blockIdx.x * int64_t{blockDim.x} + threadIdx.x;
+  scan_part& to = parts[blockIdx.x];
+  for (int k0 = 0; k0 == 0 || k0 < K; k0 += kScanColumns) {
+    int mn = INT32_MAX, mx = -1, sl_i = 0, sl_d = 0;
+    int top[kScanColumns], low[kScanColumns];
+#pragma unroll
+    for (int c = 0; c < kScanColumns; ++c) {
+      top[c] = 0;
+      low[c] = 1;
+    }
+    const int64_t total = k0 == 0 && num_del > num_ins ? num_del : num_ins;
+    for (int64_t i = first; i < total; i += stride) {
+      const bool ins = i < num_ins, del = k0 == 0 && i < num_del;
+      int32_t u = 0, v = 0, du = 0, dv = 0, x[kScanColumns];
+      if (ins && k0 == 0) {
+        u = ins_src[i];
+        v = ins_dst[i];
+      }
+      if (del) {
+        du = del_src[i];
+        dv = del_dst[i];
+      }
+#pragma unroll
+      for (int c = 0; c < kScanColumns; ++c) x[c] = ins && k0 + c < K ? ins_w[i * K + k0 + c] : 1;
+      if (ins && k0 == 0) {
+        mn = min(mn, min(u, v));
+        mx = max(mx, max(u, v));
+        sl_i += u == v ? 1 : 0;
+      }
+      if (del) {
+        mn = min(mn, min(du, dv));
+        sl_d += du == dv ? 1 : 0;
+      }
+#pragma unroll
+      for (int c = 0; c < kScanColumns; ++c) {
+        if (ins && k0 + c < K) top[c] = max(top[c], x[c]);
+        low[c] = min(low[c], x[c]);
       }
     }
-    if (del) {
-      mn = min(mn, static_cast<long long>(min(du, dv)));
-      sl_d += du == dv ? 1 : 0;
+    // the last lane has the wave's, then a thread per value the workgroup's
+    auto least = [](int a, int b) { return min(a, b); };
+    auto most = [](int a, int b) { return max(a, b); };
+    mn = wave_fold(mn, least);
+    mx = wave_fold(mx, most);
+    sl_i = wave_scan(sl_i);
+    sl_d = wave_scan(sl_d);
+#pragma unroll
+    for (int c = 0; c < kScanColumns; ++c) {
+      top[c] = wave_fold(top[c], most);
+      low[c] = wave_fold(low[c], least);
     }
-  }
-  constexpr int kVals = 9;
-  long long val[kVals] = {mn, mx, sl_i, sl_d, wmin, lmax0, lmax1, lmax2, lmax3};
-  auto combine = [](int q, long long a, long long b) -> long long {
-    if (q == 0 || q == 4) return b < a ? b : a;  // minima
-    if (q == 2 || q == 3) return a + b;          // counts
-    return b > a ? b : a;                        // maxima
-  };
+    if (k0 > 0) __syncthreads();  // the last pass's values are read
+    if (lane() == 63) {
+      int* mine = part[threadIdx.x / 64];
+      mine[0] = mn;
+      mine[1] = mx;
+      mine[2] = sl_i;
+      mine[3] = sl_d;
 #pragma unroll
-  for (int q = 0; q < kVals; ++q) {
-    for (int off = 32; off > 0; off >>= 1) val[q] = combine(q, val[q], static_cast<long long>(__shfl_xor(val[q], off)));
-  }
-  __shared__ long long part[kScanBlock / 64][kVals];
-  if (lane() == 0) {
-#pragma unroll
-    for (int q = 0; q < kVals; ++q) part[threadIdx.x / 64][q] = val[q];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int waves = static_cast<int>(blockDim.x / 64);
-#pragma unroll
-    for (int q = 0; q < kVals; ++q) {
-      long long t = part[0][q];
-      for (int w = 1; w < waves; ++w) t = combine(q, t, part[w][q]);
-      val[q] = t;
+      for (int c = 0; c < kScanColumns; ++c) {
+        mine[4 + c] = top[c];
+        mine[4 + kScanColumns + c] = low[c];
+      }
     }
-    if (val[0] != INT32_MAX) atomicMin(&ctl->min_id, static_cast<int>(val[0]));
-    if (val[1] >= 0) atomicMax(&ctl->max_id, static_cast<int>(val[1]));
-    if (val[2]) atomicAdd(&ctl->self_loops_ins, static_cast<int>(val[2]));
-    if (val[3]) atomicAdd(&ctl->self_loops_del, static_cast<int>(val[3]));
-    if (val[4] != INT32_MAX) atomicMin(&ctl->min_weight, static_cast<int>(val[4]));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (k < K && val[5 + k] > 0) atomicMax(&ctl->batch_wmax[k], static_cast<int>(val[5 + k]));
+    __syncthreads();
+    const int q = static_cast<int>(threadIdx.x);
+    if (q < kVals) {
+      const bool column = q >= 4;
+      const int c = k0 + ((q - 4) & (kScanColumns - 1));
+      const bool is_max = q == 1 || (column && q < 4 + kScanColumns), is_sum = q == 2 || q == 3;
+      int t = part[0][q];
+      for (int w = 1; w < kScanBlock / 64; ++w) {
+        const int x = part[w][q];
+        t = is_sum ? t + x : is_max ? max(t, x) : min(t, x);
+      }
+      if (!column && k0 == 0) to.id[q] = t;
+      if (column && c < K) (is_max ? to.wmax : to.wmin)[c] = t;
     }
   }
 }
@@ -2565,56 +2586,72 @@ void scan_batch(dyng_hip_graph* g, const dyng_hip_batch* b, hipStream_t s, batch
   const int32_t *ins_src = b->ins_src, *ins_dst = b->ins_dst, *ins_w = b->ins_w, *del_src = b->del_src,
                 *del_dst = b->del_dst;
   if (!b->on_device) {
-    g->b_ins_src.reserve(num_ins);
-    g->b_ins_dst.reserve(num_ins);
-    g->b_ins_w.reserve(num_ins * K);
-    g->b_del_src.reserve(num_del);
-    g->b_del_dst.reserve(num_del);
-    if (num_ins > 0) {
-      DYNG_HIP_TRY(hipMemcpyAsync(g->b_ins_src.p, ins_src, num_ins * 4, hipMemcpyHostToDevice, s));
-      DYNG_HIP_TRY(hipMemcpyAsync(g->b_ins_dst.p, ins_dst, num_ins * 4, hipMemcpyHostToDevice, s));
-      DYNG_HIP_TRY(hipMemcpyAsync(g->b_ins_w.p, ins_w, num_ins * K * 4, hipMemcpyHostToDevice, s));
+    // one device buffer, each array from a 256-byte boundary on
+    const int32_t* from[5] = {ins_src, ins_dst, ins_w, del_src, del_dst};
+    const int64_t count[5] = {num_ins, num_ins, num_ins * K, num_del, num_del};
+    int64_t at[5], total = 0;
+    for (int i = 0; i < 5; ++i) {
+      at[i] = total;
+      total += (count[i] + 63) / 64 * 64;
     }
-    if (num_del > 0) {
-      DYNG_HIP_TRY(hipMemcpyAsync(g->b_del_src.p, del_src, num_del * 4, hipMemcpyHostToDevice, s));
-      DYNG_HIP_TRY(hipMemcpyAsync(g->b_del_dst.p, del_dst, num_del * 4, hipMemcpyHostToDevice, s));
+    g->b_batch.reserve(total);
+    if (total * 4 <= kGatherBytes) {
+      // a small batch: gathered in pinned memory (the last batch's copy ended before its scan was read)
+      // and sent as one copy. Five copies from pageable memory took 23 us of a batch of 1,000.
+      g->host_batch.reserve(static_cast<size_t>(total) * 4);
+      for (int i = 0; i < 5; ++i) {
+        if (count[i] > 0) std::memcpy(g->host_batch.p + at[i] * 4, from[i], static_cast<size_t>(count[i]) * 4);
+      }
+      if (total > 0) DYNG_HIP_TRY(hipMemcpyAsync(g->b_batch.p, g->host_batch.p, total * 4, hipMemcpyHostToDevice, s));
+    } else {
+      for (int i = 0; i < 5; ++i) {
+        if (count[i] > 0) DYNG_HIP_TRY(hipMemcpyAsync(g->b_batch.p + at[i], from[i], count[i] * 4, hipMemcpyHostToDevice, s));
+      }
     }
-    ins_src = g->b_ins_src.p;
-    ins_dst = g->b_ins_dst.p;
-    ins_w = g->b_ins_w.p;
-    del_src = g->b_del_src.p;
-    del_dst = g->b_del_dst.p;
+    ins_src = g->b_batch.p + at[0];
+    ins_dst = g->b_batch.p + at[1];
+    ins_w = g->b_batch.p + at[2];
+    del_src = g->b_batch.p + at[3];
+    del_dst = g->b_batch.p + at[4];
   }
-  apply_control* hc = g->host_ctl.p;
   // ---- scan the batch (ids, self-loops, weights) before anything changes ----
-  std::memset(hc, 0, sizeof(apply_control));
-  hc->min_id = INT32_MAX;
-  hc->max_id = -1;
-  hc->min_weight = INT32_MAX;
-  for (int k = 0; k < max_weights; ++k) hc->batch_wmin[k] = 1;
-  DYNG_HIP_TRY(hipMemcpyAsync(g->ctl.p, hc, sizeof(apply_control), hipMemcpyHostToDevice, s));
-  if (num_ins + num_del > 0) {
-    hipLaunchKernelGGL(k_batch_scan, dim3(std::min<unsigned>(blocks_for(std::max(num_ins, num_del), kScanBlock), 64)),
-                       dim3(kScanBlock), 0, s, ins_src, ins_dst, ins_w, num_ins, del_src, del_dst, num_del, K, g->ctl.p);
+  int min_id = INT32_MAX, max_id = -1, self_loops = 0;
+  sc.wmax.assign(K, 0);
+  sc.wmin.assign(K, 1);
+  if (num_ins + num_del == 0) {
+    mark_stage(g, 1, s);
+  } else {
+    const int blocks = static_cast<int>(std::min<unsigned>(blocks_for(std::max(num_ins, num_del), kScanBlock), kScanParts));
+    scan_part* parts = g->host_scan.p->part;
+    hipLaunchKernelGGL(k_batch_scan, dim3(static_cast<unsigned>(blocks)), dim3(kScanBlock), 0, s, ins_src, ins_dst, ins_w,
+                       num_ins, del_src, del_dst, num_del, K, parts);
     DYNG_HIP_TRY(hipGetLastError());
+    mark_stage(g, 1, s);
+    DYNG_HIP_TRY(hipStreamSynchronize(s));
+    for (int b = 0; b < blocks; ++b) {
+      min_id = std::min(min_id, parts[b].id[0]);
+      max_id = std::max(max_id, parts[b].id[1]);
+      self_loops += parts[b].id[2] != 0 || parts[b].id[3] != 0 ? 1 : 0;
+      for (int k = 0; k < K; ++k) {
+        sc.wmax[k] = std::max<int64_t>(sc.wmax[k], parts[b].wmax[k]);
+        sc.wmin[k] = std::min<int64_t>(sc.wmin[k], parts[b].wmin[k]);
+      }
+    }
   }
-  mark_stage(g, 1, s);
-  DYNG_HIP_TRY(hipMemcpyAsync(hc, g->ctl.p, sizeof(apply_control), hipMemcpyDeviceToHost, s));
-  DYNG_HIP_TRY(hipStreamSynchronize(s));
-  if (hc->min_id < 0) fail(DYNG_HIP_INVALID_ARGUMENT, "dyng: the batch names a negative vertex id");
-  if (g->props.on_self_loop == 2 && hc->self_loops_ins + hc->self_loops_del > 0) {
+  if (min_id < 0) fail(DYNG_HIP_INVALID_ARGUMENT, "dyng: the batch names a negative vertex id");
+  if (g->props.on_self_loop == 2 && self_loops > 0) {
     fail(DYNG_HIP_INVALID_ARGUMENT, "dyng: the batch has a self-loop and on_self_loop is error");
   }
   int64_t n_after = g->n;
-  if (hc->max_id >= 0) {
-    if (!g->props.allow_vertex_growth && hc->max_id >= g->n) {
+  if (max_id >= 0) {
+    if (!g->props.allow_vertex_growth && max_id >= g->n) {
       fail(DYNG_HIP_INVALID_ARGUMENT, "dyng: an insertion names a vertex >= " + std::to_string(g->n) +
                                           " and allow_vertex_growth is false");
     }
-    if (hc->max_id >= INT32_MAX - 1) fail(DYNG_HIP_INVALID_ARGUMENT, "dyng: an insertion names the largest vertex id");
+    if (max_id >= INT32_MAX - 1) fail(DYNG_HIP_INVALID_ARGUMENT, "dyng: an insertion names the largest vertex id");
     // a self-loop insertion that is dropped does not grow the vertex set; keep the rule simple by
     // growing only for kept insertions (the scan covers them all; drop is rare)
-    n_after = std::max<int64_t>(n_after, static_cast<int64_t>(hc->max_id) + 1);
+    n_after = std::max<int64_t>(n_after, static_cast<int64_t>(max_id) + 1);
   }
   sc.n_after = n_after;
   sc.num_ins = num_ins;
@@ -2624,12 +2661,6 @@ void scan_batch(dyng_hip_graph* g, const dyng_hip_batch* b, hipStream_t s, batch
   sc.ins_w = ins_w;
   sc.del_src = del_src;
   sc.del_dst = del_dst;
-  sc.wmax.assign(K, 0);
-  sc.wmin.assign(K, 1);
-  for (int k = 0; k < K; ++k) {
-    sc.wmax[k] = num_ins > 0 ? hc->batch_wmax[k] : 0;
-    sc.wmin[k] = hc->batch_wmin[k];
-  }
 }
 
 /// The merge parameters of one row store for a batch of N operations (keys of `vbits` bits).
@@ -3130,7 +3161,6 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
   g->last.num_ins = sc.num_ins;
   const int64_t num_ins = sc.num_ins, num_del = sc.num_del;
   const int64_t n_after = sc.n_after;
-  apply_control* hc = g->host_ctl.p;
   const int64_t n_before = g->n;
   const int stride = g->props.directed ? 1 : 2;
   const int64_t N = (num_ins + num_del) * stride;
@@ -3175,7 +3205,6 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
     g->mark_generation = 1;
   }
   begin_apply(g, sc, grouped ? 2 << lb : 0, s);
-  apply_control* dc = g->ctl.p;
   if (N > 0) {
     if (grouped) {
       rows_grouped(g, sc, L, N, P, vbits, lb, n_before, s, out, wait, ap);
@@ -3184,7 +3213,6 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
     }
   }
   if (wait != nullptr) DYNG_HIP_TRY(hipStreamWaitEvent(s, wait, 0));
-  DYNG_HIP_TRY(hipMemcpyAsync(hc, dc, sizeof(apply_control), hipMemcpyDeviceToHost, s));
   // from here on the graph has the batch's vertices (work queued behind reads them)
   g->n = n_after;
   return ap;
@@ -3197,6 +3225,7 @@ void apply_finish(dyng_hip_graph* g, const batch_scan& sc, apply_pending& ap, hi
   apply_control* dc = g->ctl.p;
   const int64_t n_before = ap.n_before;
   const int64_t n_after = g->n;
+  if (!ap.published) DYNG_HIP_TRY(hipMemcpyAsync(hc, dc, sizeof(apply_control), hipMemcpyDeviceToHost, s));
   DYNG_HIP_TRY(hipStreamSynchronize(s));
   if (hc->miss != 0 && hc->error_bits == 0) {
     resort(g, sc, n_before, s, out, ap);
@@ -3262,7 +3291,6 @@ void apply_scanned(dyng_hip_graph* g, const batch_scan& sc, hipStream_t s, dyng_
   apply_finish(g, sc, ap, s, out);
 }
 
-const int* apply_hold(const dyng_hip_graph* g) { return &g->ctl.p->hold; }
 
 }  // namespace dyng_hip
 

@@ -127,6 +127,34 @@ struct pinned {
   pinned& operator=(const pinned&) = delete;
 };
 
+/// Pinned host memory that grows (contents not kept), freed with its owner.
+struct pinned_bytes {
+  unsigned char* p = nullptr;
+  size_t size = 0;
+  void reserve(size_t bytes) {
+    if (bytes <= size) return;
+    size_t want = size_t{1} << 16;
+    while (want < bytes) want *= 2;
+    release();
+    void* q = nullptr;
+    if (hipHostMalloc(&q, want, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      throw status_error(DYNG_HIP_OUT_OF_MEMORY, "dyng: out of pinned host memory");
+    }
+    p = static_cast<unsigned char*>(q);
+    size = want;
+  }
+  void release() {
+    if (p != nullptr) (void)hipHostFree(p);
+    p = nullptr;
+    size = 0;
+  }
+  pinned_bytes() = default;
+  ~pinned_bytes() { release(); }
+  pinned_bytes(const pinned_bytes&) = delete;
+  pinned_bytes& operator=(const pinned_bytes&) = delete;
+};
+
 /// One direction of the device graph: per-vertex {offset, length} and capacity, and the slot
 /// arena (neighbour ids, then num_weights weight columns of slot_cap entries each).
 ///
@@ -160,18 +188,10 @@ struct apply_control {
   long long tail_out, tail_in;        ///< arena tails (atomic bump allocation)
   long long stage_out, stage_in;      ///< staging slots used
   long long garbage_out, garbage_in;  ///< slots left behind by relocations
-  // batch scan
-  int min_id;
-  int max_id;
-  int self_loops_ins, self_loops_del;
-  int min_weight;
-  int pad0;
   // column summaries: target max per objective (set by the host), deltas (device)
   long long col_max[max_weights];
   long long col_dsum[max_weights];
   long long col_dcount[max_weights];
-  int batch_wmax[max_weights];
-  int batch_wmin[max_weights];
   long long col_bad[max_weights];  ///< weights below 1 per column (column summary)
   // merge plan: tail slots of the relocating rows, staging slots of the staged rows
   long long need_reloc_out, need_reloc_in, need_stage_out, need_stage_in;
@@ -184,6 +204,18 @@ struct apply_control {
   int hold;
   /// nonzero: the grouped apply did nothing (k_group_front says why); the host sorts the batch
   int miss;
+};
+
+/// What a workgroup of the batch scan found, written to pinned host memory: least and largest id, self-loop
+/// insertions and deletions, and per objective the largest weight (0 if none is larger) and the smallest
+/// (1 if none is smaller).
+struct scan_part {
+  int id[4];
+  int wmax[max_weights], wmin[max_weights];
+};
+constexpr int kScanParts = 64;
+struct scan_parts {
+  scan_part part[kScanParts];
 };
 
 /// What the batch scan found (before anything changes) and where the batch is on the device.
@@ -206,6 +238,7 @@ void scan_batch(dyng_hip_graph* g, const dyng_hip_batch* b, hipStream_t s, batch
 /// dyng_hip_sssp_update / _compute are the two back to back. Runs on one device are queued on one
 /// stream, one after another: two persistent launches resident together gave wrong trees on
 /// MI355X (the kernel keeps a little per-lane state in scratch memory), so runs never overlap.
+struct apply_pending;
 struct engine_pending {
   dyng_hip_workspace* ws = nullptr;
   hipStream_t s = nullptr;
@@ -217,13 +250,13 @@ struct engine_pending {
   int64_t n = 0;
   int64_t timeout_us = 0;
   int64_t* distances = nullptr;
-  bool held = false;  ///< set by engine_finish: the run did nothing (see engine_launch's `hold`)
+  bool held = false;  ///< set by engine_finish: the run did nothing (see engine_launch's `ahead`)
   dyng_hip_counters counters{};
 };
-/// `hold`: queued behind apply_launch, the apply's
-/// apply_hold flag: when the apply's merges were held back the run does nothing, and
+/// `ahead`: queued behind this apply_launch: the run's first launch also hands the apply's control block
+/// to the host, and when the apply's merges were held back the run does nothing, and
 /// engine_finish sets `held` (the caller launches it again after apply_finish).
-engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStream_t s, const int* hold = nullptr);
+engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStream_t s, apply_pending* ahead = nullptr);
 void engine_finish(engine_pending& pend, dyng_hip_counters* out);
 /// The scheduler's pick for a scanned batch on G_t: features, BF16 inference, argmin (one sync).
 int mlp_choose(dyng_hip_mlp* m, const dyng_hip_graph* g, const batch_scan& sc, const int32_t* parents, int64_t n_tree,
@@ -264,7 +297,7 @@ void apply_scanned(dyng_hip_graph* g, const batch_scan& sc, hipStream_t s, dyng_
                    hipEvent_t wait = nullptr);
 /// The apply in two halves: apply_launch queues the device work (the graph's vertex count is
 /// n_after from then on; for a batch of up to kSpeculativeOps operations the merges are queued
-/// without reading the merge plan back, guarded by a device flag, apply_hold) and the control
+/// without reading the merge plan back, guarded by a device flag) and the control
 /// block's read-back; work queued on the stream after it sees the applied rows. apply_finish
 /// waits for the stream, plans and merges again from the host if the guard held the merges
 /// back (then `replanned` is set: engine runs queued in between did nothing), reports errors
@@ -272,6 +305,7 @@ void apply_scanned(dyng_hip_graph* g, const batch_scan& sc, hipStream_t s, dyng_
 struct apply_pending {
   bool speculative = false;
   bool replanned = false;
+  bool published = false;  ///< the control block reaches the host with an engine run queued behind (engine_launch)
   int64_t n_before = 0, N = 0;
   int64_t P = 0;               ///< places of the operations in sorted order
   int vbits = 0;
@@ -282,8 +316,6 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
                            hipEvent_t wait = nullptr);
 void apply_finish(dyng_hip_graph* g, const batch_scan& sc, apply_pending& ap, hipStream_t s,
                   dyng_hip_apply_summary* out);
-/// The device flag an engine run queued between apply_launch and apply_finish checks first.
-const int* apply_hold(const dyng_hip_graph* g);
 }  // namespace dyng_hip
 
 /// The device graph behind the dyng_hip_graph handle.
@@ -332,9 +364,11 @@ struct dyng_hip_graph {
   dyng_hip::dbuf<int32_t> stage_nbr, stage_w;
   int64_t stage_cap = 0;
   int mark_generation = 0;
-  dyng_hip::dbuf<int32_t> b_ins_src, b_ins_dst, b_ins_w, b_del_src, b_del_dst;
+  dyng_hip::dbuf<int32_t> b_batch;     ///< a host batch's arrays on the device, one after another
+  dyng_hip::pinned_bytes host_batch;   ///< where a small one is gathered for a single copy
   dyng_hip::dbuf<dyng_hip::apply_control> ctl;
   dyng_hip::pinned<dyng_hip::apply_control> host_ctl;
+  dyng_hip::pinned<dyng_hip::scan_parts> host_scan;
   /// events at the apply's stage boundaries (0-1 batch scan, 2-12 the update of the rows)
   hipEvent_t apply_ev[13] = {};
   bool apply_ev_recorded = false;

@@ -110,6 +110,7 @@ struct control {
   unsigned long long pull_vertices;
   unsigned long long t_phase[8];  ///< s_memrealtime ticks: start, pull, near-far, unpack, after A, B, C, end
   unsigned int error_bits;
+  unsigned int finished;  ///< workgroups that ended the run; all of them: the block was published to the host
 };
 
 struct engine_params {
@@ -167,6 +168,7 @@ struct engine_params {
   int32_t chunk_edges;
   unsigned long long barrier_ticks;  ///< longest wait at a grid barrier (s_memrealtime ticks)
   const int* hold;  ///< null, or a flag of the apply queued ahead: nonzero, the run does nothing
+  control* publish; ///< null, or where in pinned host memory the control block goes when the run ends
 };
 
 /// Append v to a list when pred (wave-aggregated reservation).
@@ -757,8 +759,13 @@ DYNG_DEV void pull_commit(const engine_params& p, bool pred, int32_t v, u64 best
 /// Clear the grid barrier (a kernel, not a memset, so the launch can live in a hipGraph).
 /// Before each run (one workgroup): the barrier state and the control block zeroed, the control
 /// block's minima at INF (a kernel rather than a host copy: it costs the stream no blit).
+constexpr int kResetBlock = 256;
 static_assert(sizeof(control) % 8 == 0 && sizeof(grid_sync_state) % 8 == 0, "reset in 8-byte words");
-__global__ void k_reset_barrier(grid_sync_state* bar, control* ctl) {
+/// The apply queued ahead of a run has ended when this starts: `words` 4-byte words of its control
+/// block go to pinned host memory here, in place of a copy of their own.
+__global__ void __launch_bounds__(kResetBlock) k_reset_barrier(grid_sync_state* bar, control* ctl, const int* from, int* to,
+                                                                 int words) {
+  for (int i = threadIdx.x; i < words; i += blockDim.x) to[i] = from[i];
   unsigned long long* w = reinterpret_cast<unsigned long long*>(bar);
   for (unsigned int i = threadIdx.x; i < sizeof(grid_sync_state) / 8; i += blockDim.x) w[i] = 0;
   unsigned long long* c = reinterpret_cast<unsigned long long*>(ctl);
@@ -813,7 +820,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
   unsigned int round = 0;  // of the grid barrier (uniform over the grid)
   const int64_t chunk_cap = p.chunk_cap / 2;  // one phase's chunks: at most slots / 16 + n
   unsigned long long jump_items = 0;
-  if (tid == 0) c->t_phase[0] = __builtin_amdgcn_s_memrealtime();
+  if (tid == 0) st(&c->t_phase[0], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
 
   if constexpr (kSolve) {
     if (p.source >= 0) {
@@ -872,7 +879,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
     bool long_front = false;  // the frontier holds a vertex with a row past `light`
     [[maybe_unused]] int sent = 0;
     DYNG_GRID_SYNC_SENT(0, sent, long_front);
-    if (tid == 0) c->t_phase[4] = __builtin_amdgcn_s_memrealtime();
+    if (tid == 0) st(&c->t_phase[4], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
     if (ld(&c->overflow) != 0) return;  // uniform: the host reports invalid_input
     const int roots = uniform(ld(&c->cand_count));
     const bool work = p.num_del + p.num_ins > 0;
@@ -1139,7 +1146,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
     }
     // ---- C: invalidate the flagged vertices (stamped when flagged) and claim the insertion
     // heads that are not invalidated, in one phase ----
-    if (tid == 0) c->t_phase[5] = __builtin_amdgcn_s_memrealtime();
+    if (tid == 0) st(&c->t_phase[5], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
     ++generation;
     for (int i = tid; i < inv; i += threads) {
       const int32_t v = ld(&p.cand[i]);
@@ -1169,9 +1176,9 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
     ++generation;
     const int cands = inv + uniform(ld(&c->heads_count));
     if (tid == 0) {
-      c->t_phase[1] = __builtin_amdgcn_s_memrealtime();
-      c->jump_items = jump_items;
-      c->pull_vertices = cands + (p.check_cycles ? 0 : p.num_ins);
+      st(&c->t_phase[1], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
+      st(&c->jump_items, static_cast<u64>(jump_items));
+      st(&c->pull_vertices, static_cast<u64>(cands + (p.check_cycles ? 0 : p.num_ins)));
     }
     int* chunk_count = &c->ring_chunk[cstep % 3];
     if (tid == 0 && long_pull) st(&c->ring_chunk[(cstep + 1) % 3], 0);
@@ -1267,7 +1274,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
 
   // ---- E: near-far propagation (the frontier's smallest distance came with the pull, or is the
   // source's 0) ----
-  if (tid == 0) c->t_phase[2] = __builtin_amdgcn_s_memrealtime();
+  if (tid == 0) st(&c->t_phase[2], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
   u64 local = packed_inf;
   const u64 smallest = kSolve ? 0 : uniform(ld(&c->min_frontier));
   u64 threshold = (smallest == packed_inf ? 0 : smallest) + p.delta;
@@ -1526,7 +1533,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
   }
 
   // ---- F: unpack ----
-  if (tid == 0) c->t_phase[3] = __builtin_amdgcn_s_memrealtime();
+  if (tid == 0) st(&c->t_phase[3], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
   unsigned long long changed = 0;
   if (p.pk.bits > 0) {
     // A repair changed only words of vertices it stamped (see mark_changed); every other word
@@ -1597,11 +1604,26 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
     if (*local_pushes) atomicAdd(reinterpret_cast<unsigned long long*>(&c->pushes), *local_pushes);
   }
   if (tid == 0) {
-    c->t_phase[7] = __builtin_amdgcn_s_memrealtime();
-    c->iterations = iterations;
-    c->epochs = epochs;
+    st(&c->t_phase[7], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
+    st(&c->iterations, iterations);
+    st(&c->epochs, epochs);
     atomicAdd(reinterpret_cast<unsigned long long*>(&c->pushes), static_cast<unsigned long long>(pushes));
-    c->generation = generation;
+    st(&c->generation, generation);
+  }
+  if (p.publish == nullptr) return;  // uniform
+  // The last workgroup to get here hands the control block to the host: every store and addition to
+  // it was made at device scope and has completed before its workgroup's arrival. A copy queued
+  // behind the kernel cost 5 to 10 us of every run.
+  __shared__ int last;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x == 0) last = atomicAdd(&c->finished, 1u) == gridDim.x - 1 ? 1 : 0;
+  __syncthreads();
+  if (last) {
+    constexpr int kWords = sizeof(control) / 8;
+    if (threadIdx.x < kWords) {
+      reinterpret_cast<u64*>(p.publish)[threadIdx.x] = ld(reinterpret_cast<const u64*>(c) + threadIdx.x);
+    }
   }
 }
 
@@ -1646,6 +1668,7 @@ struct dyng_hip_workspace {
   /// download), built once and replayed with the kernel node's arguments updated
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
+  hipGraphNode_t graph_reset = nullptr;
   hipGraphNode_t graph_kernel = nullptr;
   void (*graph_build)(dyng_hip::engine_params) = nullptr;  ///< the build the graph's kernel node launches
   ~dyng_hip_workspace() {
@@ -1923,7 +1946,7 @@ void read_counters(const control* hc, bool update, int bits, int blocks, dyng_hi
 
 }  // namespace
 
-engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStream_t s, const int* hold) {
+engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStream_t s, apply_pending* ahead) {
   if (run == nullptr || run->graph == nullptr || run->workspace == nullptr) {
     fail(DYNG_HIP_INVALID_ARGUMENT, "dyng: sssp run: graph and workspace are required");
   }
@@ -1946,7 +1969,7 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
   engine_params p{};
   int64_t timeout_us = 0;
   engine_setup(run, update, p, timeout_us);
-  p.hold = hold;
+  p.hold = ahead != nullptr ? &g->ctl.p->hold : nullptr;
   ws_reserve(ws, n, std::max(g->out.slot_cap, g->in.slot_cap), s);
   if (ws->generation > INT32_MAX / 2) {
     // stamps and the relax phase's list tags (-2 - generation, in `ancestor`) restart
@@ -1974,6 +1997,10 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
   hc->min_frontier = packed_inf;
   hc->minimum[0] = packed_inf;
   hc->minimum[1] = packed_inf;
+  p.publish = hc;
+  const int* from = ahead != nullptr ? reinterpret_cast<const int*>(g->ctl.p) : nullptr;
+  int* to = ahead != nullptr ? reinterpret_cast<int*>(g->host_ctl.p) : nullptr;
+  const int words = ahead != nullptr ? static_cast<int>(sizeof(apply_control) / sizeof(int)) : 0;
   if (ws->ev_start == nullptr) {
     DYNG_HIP_TRY(hipEventCreate(&ws->ev_start));
     DYNG_HIP_TRY(hipEventCreate(&ws->ev_stop));
@@ -1987,6 +2014,14 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
     kp.sharedMemBytes = 0;
     kp.kernelParams = args;
     kp.extra = nullptr;
+    grid_sync_state* bar = ws->bar.p;
+    control* ctl = ws->ctl.p;
+    void* reset_args[] = {&bar, &ctl, &from, &to, const_cast<int*>(&words)};
+    hipKernelNodeParams rp{};
+    rp.func = reinterpret_cast<void*>(k_reset_barrier);
+    rp.gridDim = dim3(1);
+    rp.blockDim = dim3(kResetBlock);
+    rp.kernelParams = reset_args;
     if (ws->graph_exec != nullptr && ws->graph_build != kernel) {
       // another build of the kernel: the graph is built again around it
       DYNG_HIP_TRY(hipGraphExecDestroy(ws->graph_exec));
@@ -1998,34 +2033,26 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
       // built once per workspace: the control block, the barrier and the events never move
       ws->graph_build = kernel;
       DYNG_HIP_TRY(hipGraphCreate(&ws->graph, 0));
-      hipGraphNode_t reset, start, stop, down;
-      grid_sync_state* bar = ws->bar.p;
-      control* ctl = ws->ctl.p;
-      void* reset_args[] = {&bar, &ctl};
-      hipKernelNodeParams rp{};
-      rp.func = reinterpret_cast<void*>(k_reset_barrier);
-      rp.gridDim = dim3(1);
-      rp.blockDim = dim3(64);
-      rp.kernelParams = reset_args;
-      DYNG_HIP_TRY(hipGraphAddKernelNode(&reset, ws->graph, nullptr, 0, &rp));
-      DYNG_HIP_TRY(hipGraphAddEventRecordNode(&start, ws->graph, &reset, 1, ws->ev_start));
+      hipGraphNode_t start, stop;
+      DYNG_HIP_TRY(hipGraphAddKernelNode(&ws->graph_reset, ws->graph, nullptr, 0, &rp));
+      DYNG_HIP_TRY(hipGraphAddEventRecordNode(&start, ws->graph, &ws->graph_reset, 1, ws->ev_start));
       DYNG_HIP_TRY(hipGraphAddKernelNode(&ws->graph_kernel, ws->graph, &start, 1, &kp));
       DYNG_HIP_TRY(hipGraphAddEventRecordNode(&stop, ws->graph, &ws->graph_kernel, 1, ws->ev_stop));
-      DYNG_HIP_TRY(hipGraphAddMemcpyNode1D(&down, ws->graph, &stop, 1, hc, ws->ctl.p, sizeof(control),
-                                           hipMemcpyDeviceToHost));
       DYNG_HIP_TRY(hipGraphInstantiate(&ws->graph_exec, ws->graph, nullptr, nullptr, 0));
     } else {
+      DYNG_HIP_TRY(hipGraphExecKernelNodeSetParams(ws->graph_exec, ws->graph_reset, &rp));
       DYNG_HIP_TRY(hipGraphExecKernelNodeSetParams(ws->graph_exec, ws->graph_kernel, &kp));
     }
     DYNG_HIP_TRY(hipGraphLaunch(ws->graph_exec, s));
   } else {
-    hipLaunchKernelGGL(k_reset_barrier, dim3(1), dim3(64), 0, s, ws->bar.p, ws->ctl.p);
+    hipLaunchKernelGGL(k_reset_barrier, dim3(1), dim3(kResetBlock), 0, s, ws->bar.p, ws->ctl.p, from, to, words);
+    DYNG_HIP_TRY(hipGetLastError());
     DYNG_HIP_TRY(hipEventRecord(ws->ev_start, s));
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, s, p);
     DYNG_HIP_TRY(hipGetLastError());
     DYNG_HIP_TRY(hipEventRecord(ws->ev_stop, s));
-    DYNG_HIP_TRY(hipMemcpyAsync(hc, ws->ctl.p, sizeof(control), hipMemcpyDeviceToHost, s));
   }
+  if (ahead != nullptr) ahead->published = true;
   pend.launched = true;
   pend.bits = p.pk.bits;
   pend.blocks = blocks;
@@ -2047,6 +2074,10 @@ void engine_finish(engine_pending& pend, dyng_hip_counters* out) {
   const int64_t timeout_us = pend.timeout_us;
   control* hc = ws->host_ctl.p;
   DYNG_HIP_TRY(hipStreamSynchronize(s));
+  if (hc->finished == 0) {  // held back, or stopped early: the block was not published
+    DYNG_HIP_TRY(hipMemcpyAsync(hc, ws->ctl.p, sizeof(control), hipMemcpyDeviceToHost, s));
+    DYNG_HIP_TRY(hipStreamSynchronize(s));
+  }
   if (hc->held != 0) {
     // nothing ran (the apply ahead of the run was held back): the caller runs it again
     pend.held = true;
@@ -2255,7 +2286,8 @@ void run_engine_noalloc(const dyng_hip_sssp_run* run, hipStream_t s, dyng_hip_co
                                    L.chunk_cap, reinterpret_cast<control*>(base + L.ctl),
                                    reinterpret_cast<grid_sync_state*>(base + L.bar)});
   const int blocks = grid_blocks(run->tuning, st.occupancy, st.cu_count, p.from_scratch != 0);
-  hipLaunchKernelGGL(k_reset_barrier, dim3(1), dim3(64), 0, s, p.bar, p.ctl);
+  hipLaunchKernelGGL(k_reset_barrier, dim3(1), dim3(kResetBlock), 0, s, p.bar, p.ctl, static_cast<const int*>(nullptr),
+                     static_cast<int*>(nullptr), 0);
   const fused_fn kernel = fused_kernel(narrow_grid(blocks, st.occupancy_narrow, st.cu_count), p.from_scratch != 0);
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, s, p);
   DYNG_HIP_TRY(hipGetLastError());
