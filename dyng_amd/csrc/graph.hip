@@ -603,7 +603,6 @@ struct out_pair_params {
   const uint32_t* vals;
   int64_t N;
   int64_t stride;  ///< of the weight columns of pend_w and of the iop arrays
-  int64_t at;      ///< place of keys[0] among all the sorted operations
   int vbits;
   int K;
   int64_t n_before;  ///< rows that existed before the batch (classification)
@@ -628,7 +627,8 @@ struct out_pair_params {
   int32_t* iop_wnew;
   int32_t* mark;
   int mark_gen;
-  int32_t* touched;
+  int4* touched;  ///< rows whose entries change: row, and its operations (-1: in row_a and row_b)
+  int32_t* flag;  ///< grouped: per operation, whether its pair changes the row's entries
   int32_t* row_a;  ///< per vertex: first operation of its row in the sorted keys
   int32_t* row_b;  ///< per vertex: one past its last operation
   apply_control* ctl;
@@ -701,25 +701,24 @@ __global__ void __launch_bounds__(kBlock) k_check_pairs(op_layout L, const u64* 
 }
 
 /// Record where row r's operations start and end in the sorted keys (row = key >> vbits).
-DYNG_DEV void mark_row_range(const u64* keys, int64_t i, int64_t N, int64_t at, int vbits, int32_t* row_a,
-                             int32_t* row_b) {
+DYNG_DEV void mark_row_range(const u64* keys, int64_t i, int64_t N, int vbits, int32_t* row_a, int32_t* row_b) {
   const u64 key = keys[i];
   const u64 r = key >> vbits;
-  if (i == 0 || (keys[i - 1] >> vbits) != r) row_a[r] = static_cast<int32_t>(at + i);
-  if (i + 1 == N || (keys[i + 1] >> vbits) != r) row_b[r] = static_cast<int32_t>(at + i + 1);
+  if (i == 0 || (keys[i - 1] >> vbits) != r) row_a[r] = static_cast<int32_t>(i);
+  if (i + 1 == N || (keys[i + 1] >> vbits) != r) row_b[r] = static_cast<int32_t>(i + 1);
 }
 
-/// A row whose entries change: marked for the plan of its group (`kGrouped`: one workgroup holds all
-/// the row's operations), or listed.
-template <bool kGrouped>
-DYNG_DEV void touch_row(bool structural, int32_t r, int32_t* mark, int mark_gen, int* touched_count, int32_t* touched) {
+/// A pair whose operations change its row's entries: flagged for the plan of the row's group
+/// (`kGrouped`: one workgroup holds all the row's operations), or the row listed.
+template <bool kGrouped, class Params>
+DYNG_DEV void touch_row(const Params& p, bool structural, int64_t i, int32_t r, int* touched_count) {
   if (kGrouped) {
-    if (structural) mark[r] = mark_gen;
+    if (structural) p.flag[i] = 1;
     return;
   }
-  const bool first_touch = structural && atomicExch(&mark[r], mark_gen) != mark_gen;
+  const bool first_touch = structural && atomicExch(&p.mark[r], p.mark_gen) != p.mark_gen;
   const int t = wave_append(touched_count, first_touch);
-  if (first_touch) touched[t] = r;
+  if (first_touch) p.touched[t] = make_int4(r, -1, -1, 0);
 }
 
 /// The out-row pass of thread i (every thread of the workgroup calls it: it ends with the
@@ -738,7 +737,7 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
   }
   if (i < p.N) {
     const u64 key = p.keys[i];
-    if (key != kNoKey) mark_row_range(p.keys, i, p.N, p.at, p.vbits, p.row_a, p.row_b);
+    if (!kGrouped && key != kNoKey) mark_row_range(p.keys, i, p.N, p.vbits, p.row_a, p.row_b);
     if (key == kNoKey) {
       p.pend_alive[i] = 0;
       p.kill[i] = 0;
@@ -909,7 +908,7 @@ DYNG_DEV void out_pairs(const out_pair_params& p, int64_t i) {
           for (int k = 0; k < K; ++k) p.e_fw[loc * K + k] = wf != nullptr ? wf[k * wf_stride] : -1;
         }
       }
-      touch_row<kGrouped>(structural, u, p.mark, p.mark_gen, &p.ctl->touched_out, p.touched);
+      touch_row<kGrouped>(p, structural, i, u, &p.ctl->touched_out);
     }
   }
   // the workgroup's counters in one pass: wave sums by lane-to-lane moves (a count fits 32 bits; a
@@ -969,7 +968,6 @@ struct in_pair_params {
   const uint32_t* vals;  ///< out-operation position of each
   int64_t N;
   int64_t stride;  ///< of the weight columns of pend_w and of the iop arrays
-  int64_t at;      ///< place of keys[0] among all the sorted operations
   int vbits;
   int K;
   const int32_t* iop_type;
@@ -986,7 +984,8 @@ struct in_pair_params {
   int32_t* pend_w;
   int32_t* mark;
   int mark_gen;
-  int32_t* touched;
+  int4* touched;  ///< rows whose entries change: row, and its operations (-1: in row_a and row_b)
+  int32_t* flag;  ///< grouped: per operation, whether its pair changes the row's entries
   int32_t* row_a;
   int32_t* row_b;
   apply_control* ctl;
@@ -1007,7 +1006,7 @@ DYNG_DEV void in_pairs(const in_pair_params& p, int64_t i) {
     p.kill[i] = 0;
     return;
   }
-  mark_row_range(p.keys, i, p.N, p.at, p.vbits, p.row_a, p.row_b);
+  if (!kGrouped) mark_row_range(p.keys, i, p.N, p.vbits, p.row_a, p.row_b);
   if (i > 0 && p.keys[i - 1] == key) return;
   int64_t j = i + 1;
   while (j < p.N && p.keys[j] == key) ++j;
@@ -1073,7 +1072,7 @@ DYNG_DEV void in_pairs(const in_pair_params& p, int64_t i) {
       }
     }
   }
-  touch_row<kGrouped>(structural, v, p.mark, p.mark_gen, &p.ctl->touched_in, p.touched);
+  touch_row<kGrouped>(p, structural, i, v, &p.ctl->touched_in);
 }
 
 __global__ void __launch_bounds__(kBlock) k_in_pairs(in_pair_params p) {
@@ -1100,7 +1099,7 @@ DYNG_DEV void in_pairs_simple(const in_pair_params& p, int64_t i) {
     p.kill[i] = 0;
     return;
   }
-  mark_row_range(p.keys, i, p.N, p.at, p.vbits, p.row_a, p.row_b);
+  if (!kGrouped) mark_row_range(p.keys, i, p.N, p.vbits, p.row_a, p.row_b);
   if (i > 0 && p.keys[i - 1] == key) return;
   int64_t j = i + 1;
   while (j < p.N && p.keys[j] == key) ++j;
@@ -1163,7 +1162,7 @@ DYNG_DEV void in_pairs_simple(const in_pair_params& p, int64_t i) {
       }
     }
   }
-  touch_row<kGrouped>(structural, v, p.mark, p.mark_gen, &p.ctl->touched_in, p.touched);
+  touch_row<kGrouped>(p, structural, i, v, &p.ctl->touched_in);
 }
 
 /// Both pairing passes of a simple graph in one launch: workgroups [0, split) the out-rows,
@@ -1193,10 +1192,11 @@ struct merge_params {
   const int32_t* pend_prefix;
   const int32_t* kill_prefix;  ///< prefix of the tail entries each operation killed
   const int32_t* pend_w;
-  const int32_t* touched;
+  const int4* touched;
   const int* touched_count;
-  const int32_t* row_a;  ///< the row's operations: keys[row_a[u], row_b[u])
-  const int32_t* row_b;
+  int32_t* row_a;  ///< the row's operations: keys[row_a[u], row_b[u])
+  int32_t* row_b;
+  int4* lane_rows;  ///< rows of the threads' list, two words each: see plan_rows
   int32_t* lists;        ///< the merge plan: kModes lists of rows, N + 1 entries each
   int* list_count;       ///< rows per list
   int32_t* stage_nbr;
@@ -1279,19 +1279,26 @@ struct row_plan {
   int new_len;  ///< full merge: the rewritten row's length
 };
 
-/// `dead`: the dead entries of the row's base run.
-DYNG_DEV row_plan plan_row(const merge_params& p, int32_t u, int2 mt, int64_t a, int64_t b, int dead) {
+/// What a row's plan is made from: its place, base run, capacity and dead base entries, and its
+/// operations [a, b) with the pending entries and the killed tail entries among them.
+struct row_facts {
+  int2 mt;
+  int32_t base, cap, dead;
+  int32_t a, b, pending, killed;
+};
+
+DYNG_DEV row_plan plan_row(const row_facts& f) {
   row_plan r;
-  r.base_len = p.base[u];
-  r.tail_len = mt.y - r.base_len;
-  r.pending = p.pend_prefix[b] - p.pend_prefix[a];
-  r.alive_tail = r.tail_len - (p.kill_prefix[b] - p.kill_prefix[a]);
-  r.alive_base = r.base_len - dead;
+  r.base_len = f.base;
+  r.tail_len = f.mt.y - r.base_len;
+  r.pending = f.pending;
+  r.alive_tail = r.tail_len - f.killed;
+  r.alive_base = r.base_len - f.dead;
   r.new_tail = r.alive_tail + r.pending;
   r.new_len = r.alive_base + r.new_tail;
-  const int nops = static_cast<int>(b - a);
-  const bool tail_ok = r.new_tail <= tail_limit(r.base_len) && r.base_len + r.new_tail <= p.cap[u] &&
-                       dead <= dead_limit(r.base_len);
+  const int nops = f.b - f.a;
+  const bool tail_ok = r.new_tail <= tail_limit(r.base_len) && r.base_len + r.new_tail <= f.cap &&
+                       f.dead <= dead_limit(r.base_len);
   if (tail_ok && r.tail_len <= kLaneTail && nops <= kLaneOps) {
     r.mode = kTailLane;
   } else if (tail_ok && r.tail_len <= kMergeSmall && nops <= 64) {
@@ -1304,6 +1311,20 @@ DYNG_DEV row_plan plan_row(const merge_params& p, int32_t u, int2 mt, int64_t a,
   return r;
 }
 
+/// A row's facts as the pairing and the scans left them in memory.
+DYNG_DEV row_facts read_facts(const merge_params& p, int32_t u, int32_t a, int32_t b) {
+  row_facts f;
+  f.mt = p.meta[u];
+  f.base = p.base[u];
+  f.cap = p.cap[u];
+  f.dead = p.dead[u];
+  f.a = a;
+  f.b = b;
+  f.pending = p.pend_prefix[b] - p.pend_prefix[a];
+  f.killed = p.kill_prefix[b] - p.kill_prefix[a];
+  return f;
+}
+
 /// Before the merges: each touched row's mode (appended to its list) and, for full merges, the
 /// staging slots (its alive entries) and the tail slots (a row that outgrew its capacity), so the
 /// host can compact or grow first and no row is refused. One row per thread; the lists are
@@ -1311,30 +1332,31 @@ DYNG_DEV row_plan plan_row(const merge_params& p, int32_t u, int2 mt, int64_t a,
 /// addresses every workgroup hits).
 constexpr int kPlanBlock = 1024;
 
-/// Plan one row per thread (u < 0: none) and append it to its mode's list. Every thread of the
-/// workgroup calls it. kGrouped: the row's dead entries were counted in this kernel (by device-scope
-/// atomics, so they are read at that scope), and the row joins the touched list here.
-template <int kThreads, bool kGrouped>
-DYNG_DEV void plan_rows(const merge_params& p, int32_t u, int* touched_count, int32_t* touched) {
-  constexpr int kLists = kModes + (kGrouped ? 1 : 0);
+/// Plan one row per thread (u < 0: none) and append it to its mode's list: a row for one thread with
+/// all its merge needs (row, place, base length, tail length; first operation, operations), so that the
+/// merge reads them in a row instead of five arrays by vertex (1,000,000 operations on RMAT-23:
+/// see k_tails), the others by their number, their operations in row_a and row_b. Every thread of the
+/// workgroup calls it. `touched`: where the row joins the touched rows (null: it is one already).
+template <int kThreads>
+DYNG_DEV void plan_rows(const merge_params& p, int32_t u, const row_facts& f, int* touched_count, int4* touched) {
   __shared__ int wave_offset[kThreads / 64][kModes + 1];
   __shared__ int base[kModes + 1];
   __shared__ long long part[kThreads / 64];
+  const int lists = kModes + (touched != nullptr ? 1 : 0);
   const int w = threadIdx.x / 64;
   long long reloc = 0, stage = 0;
   int mode = -1;
   if (u >= 0) {
-    const int2 mt = p.meta[u];
-    const row_plan r = plan_row(p, u, mt, p.row_a[u], p.row_b[u], kGrouped ? ld(&p.dead[u]) : p.dead[u]);
+    const row_plan r = plan_row(f);
     mode = r.mode;
     if (r.mode == kFull) {
       stage = r.alive_base + r.alive_tail;
-      if (r.new_len > p.cap[u]) reloc = grown_cap(r.new_len, p.headroom);
+      if (r.new_len > f.cap) reloc = grown_cap(r.new_len, p.headroom);
     }
   }
   int rank = 0, row_rank = 0;  // among the wave's rows of the same mode, and among all its rows
 #pragma unroll
-  for (int m = 0; m < kLists; ++m) {
+  for (int m = 0; m <= kModes; ++m) {
     const u64 b = __ballot(m == kModes ? mode >= 0 : mode == m);
     if (m == kModes) {
       row_rank = __popcll(b & lanes_below());
@@ -1344,7 +1366,7 @@ DYNG_DEV void plan_rows(const merge_params& p, int32_t u, int* touched_count, in
     if (lane() == 0) wave_offset[w][m] = __popcll(b);
   }
   __syncthreads();
-  if (threadIdx.x < kLists) {
+  if (static_cast<int>(threadIdx.x) < lists) {
     const int m = threadIdx.x;
     int run = 0;
     for (int i = 0; i < kThreads / 64; ++i) {
@@ -1356,8 +1378,16 @@ DYNG_DEV void plan_rows(const merge_params& p, int32_t u, int* touched_count, in
   }
   __syncthreads();
   if (mode >= 0) {
-    p.lists[mode * (p.N + 1) + base[mode] + wave_offset[w][mode] + rank] = u;
-    if (kGrouped) touched[base[kModes] + wave_offset[w][kModes] + row_rank] = u;
+    const int64_t place = base[mode] + wave_offset[w][mode] + rank;
+    if (mode == kTailLane) {
+      p.lane_rows[2 * place] = make_int4(u, f.mt.x, f.base, f.mt.y - f.base);
+      p.lane_rows[2 * place + 1] = make_int4(f.a, f.b - f.a, 0, 0);
+    } else {
+      p.lists[mode * (p.N + 1) + place] = u;
+      p.row_a[u] = f.a;
+      p.row_b[u] = f.b;
+    }
+    if (touched != nullptr) touched[base[kModes] + wave_offset[w][kModes] + row_rank] = make_int4(u, f.a, f.b, 0);
   }
   if (__syncthreads_or(mode == kFull ? 1 : 0) == 0) return;  // the sums are zero
   reloc = block_reduce(reloc, part, op_sum{});
@@ -1371,7 +1401,14 @@ DYNG_DEV void plan_rows(const merge_params& p, int32_t u, int* touched_count, in
 DYNG_DEV void merge_plan(const merge_params& p, int block) {
   const int count = *p.touched_count;
   const int t = block * kPlanBlock + threadIdx.x;
-  plan_rows<kPlanBlock, false>(p, t < count ? p.touched[t] : -1, nullptr, nullptr);
+  row_facts f{};
+  int32_t u = -1;
+  if (t < count) {
+    const int4 x = p.touched[t];
+    u = x.x;
+    f = read_facts(p, u, x.y >= 0 ? x.y : p.row_a[u], x.y >= 0 ? x.z : p.row_b[u]);
+  }
+  plan_rows<kPlanBlock>(p, u, f, nullptr, nullptr);
 }
 
 __global__ void __launch_bounds__(kPlanBlock) k_merge_plan(merge_sides m) {
@@ -1416,6 +1453,7 @@ constexpr int kGroupBitsSome = 9, kGroupOpsSome = 128;
 constexpr int kGroupOps = 256;
 constexpr int64_t kGroupMost = int64_t{1} << 22;  ///< operations of a batch (1024 per group)
 constexpr int kGroupCap = 4096;   ///< most a group takes; one row with more operations sends the batch to the sort
+constexpr int kGroupLds = 1024;   ///< a group with fewer operations keeps them in LDS: 8 KB sorted segments, 28 KB of the rest
 constexpr int kGroupPause = 15;   ///< batches sorted device-wide after one that a group could not take
 constexpr int kGroupBits = 12;    ///< at most 2^12 groups per direction
 constexpr uint32_t kGroupHash = 0x9E3779B1u;
@@ -1623,65 +1661,83 @@ struct group_params {
 enum { kGroupsBoth = 0, kGroupsOut = 1, kGroupsIn = 2 };
 
 /// One group per workgroup: its operations sorted by (row, neighbour, batch order), paired with
-/// their rows, their pending and killed flags scanned (a row's operations are in one group, and
-/// only differences within a row are used), and its rows' merges planned. kGroupsBoth: a simple
-/// graph's out-rows and in-rows side by side; else one direction (with parallel edges the in-row
-/// pass reads what the out-row pass recorded).
+/// their rows, their flags scanned (a row's operations are in one group, and only differences within
+/// a row are used), and its rows' merges planned. kGroupsBoth: a simple graph's out-rows and in-rows
+/// side by side; else one direction (with parallel edges the in-row pass reads what the out-row pass
+/// recorded). What bounds it is the chain of dependent reads, so the sorted operations, their flags and
+/// the scans stay in LDS (a group of more than kGroupLds keeps them in memory), a row's plan takes
+/// what it needs of them from there, and its operations are found there and not by vertex in memory.
 template <int kWhich>
 __global__ void __launch_bounds__(kGroupBlock, 4) k_group_pairs(group_params g) {
   __shared__ u64 S[kGroupCap];
   __shared__ int part[kGroupBlock / 64];
-  __shared__ int2 sums[kGroupBlock / 64];
-  if (g.ctl->miss != 0) return;  // uniform
+  __shared__ int3 sums[kGroupBlock / 64];
   const int tid = static_cast<int>(threadIdx.x);
   const bool in = kWhich == kGroupsIn || (kWhich == kGroupsBoth && static_cast<int>(blockIdx.x) >= g.groups);
   const int q = static_cast<int>(blockIdx.x) - (kWhich == kGroupsBoth && in ? g.groups : 0);
   const int* counts = g.counts + (in ? g.groups : 0);
-  const int count = uniform(counts[q]);
-  if (count == 0) return;  // uniform
+  const int missed = g.ctl->miss, here = counts[q];
   int before = 0;
   for (int b = tid; b < q; b += kGroupBlock) before += counts[b];
-  const int64_t at = uniform(block_reduce(before, part, op_sum{})) + q;
+  const int count = uniform(here);
+  if (missed != 0 || count == 0) return;  // uniform
+  before = wave_scan(before);
+  if (lane() == 63) part[tid / 64] = before;
+  const bool lds = count < kGroupLds;
   const u64* src = g.entries + int64_t{(in ? g.groups : 0) + q} * kGroupCap;
-  u64* keys = g.keys + (in ? g.P : 0) + at;
-  uint32_t* vals = g.vals + (in ? g.P : 0) + at;
   const int low = g.vbits - g.lb;
   const u64 vmask = (u64{1} << g.vbits) - 1, emask = (u64{1} << g.ebits) - 1;
-  auto row_of = [&](u64 x) -> u64 {
-    const uint32_t h = static_cast<uint32_t>((static_cast<u64>(q) << low) | (x >> (g.vbits + g.ebits)));
-    return (h * g.inverse) & static_cast<uint32_t>(vmask);
-  };
+  int64_t at = q;
+  u64* keys = S + kGroupLds;
+  uint32_t* vals = reinterpret_cast<uint32_t*>(S + 2 * kGroupLds);
+  if (!lds) {
+    __syncthreads();
+    for (int w = 0; w < kGroupBlock / 64; ++w) at += uniform(part[w]);
+    keys = g.keys + (in ? g.P : 0) + at;
+    vals = g.vals + (in ? g.P : 0) + at;
+  }
   group_sort(src, count, S, [&](int i, u64 x) {
-    keys[i] = (row_of(x) << g.vbits) | ((x >> g.ebits) & vmask);
+    const uint32_t h = static_cast<uint32_t>((static_cast<u64>(q) << low) | (x >> (g.vbits + g.ebits)));
+    const u64 row = (h * g.inverse) & static_cast<uint32_t>(vmask);
+    keys[i] = (row << g.vbits) | ((x >> g.ebits) & vmask);
     vals[i] = static_cast<uint32_t>(x & emask);
   });
-  __syncthreads();  // the group's operations are in memory for the whole workgroup
-  int32_t *pend_alive, *kill, *pend_prefix, *kill_prefix;
+  if (lds) {
+    for (int w = 0; w < kGroupBlock / 64; ++w) at += uniform(part[w]);  // behind group_sort's barrier
+  }
+  // per operation: pending, killed tail entry, changed row; scanned in place, and the killed ones
+  // where the sort's words were
+  int32_t* const out_alive = (in ? g.in.pend_alive : g.out.pend_alive) + at;
+  int32_t* const out_pend = (in ? g.pend_prefix_in : g.pend_prefix_out) + at;
+  int32_t* const out_kill = (in ? g.kill_prefix_in : g.kill_prefix_out) + at;
+  int32_t* const ints = reinterpret_cast<int32_t*>(S + 2 * kGroupLds + kGroupLds / 2);
+  int32_t* const alive = lds ? ints : out_alive;
+  int32_t* const killed = lds ? ints + kGroupLds : (in ? g.in.kill : g.out.kill) + at;  // then changed rows before
+  int32_t* const flag = lds ? ints + 2 * kGroupLds : out_pend;                           // then pending before
+  int32_t* const killed_before = lds ? reinterpret_cast<int32_t*>(S) : out_kill;
+  for (int i = tid; i < count; i += kGroupBlock) flag[i] = 0;
+  __syncthreads();  // the sorted operations and the cleared flags are there for the whole workgroup
   if (!in) {
     out_pair_params p = g.out;
     p.keys = keys;
     p.vals = vals;
     p.N = count;
-    p.at = at;
-    p.pend_alive += at;
-    p.kill += at;
+    p.pend_alive = alive;
+    p.kill = killed;
+    p.flag = flag;
     p.pend_w += at;
     for (int t = 0; t < count; t += kGroupBlock) {
       out_pairs<kGroupBlock, true>(p, t + tid);
       __syncthreads();  // its sums are read
     }
-    pend_alive = p.pend_alive;
-    kill = p.kill;
-    pend_prefix = g.pend_prefix_out + at;
-    kill_prefix = g.kill_prefix_out + at;
   } else {
     in_pair_params p = g.in;
     p.keys = keys;
     p.vals = vals;
     p.N = count;
-    p.at = at;
-    p.pend_alive += at;
-    p.kill += at;
+    p.pend_alive = alive;
+    p.kill = killed;
+    p.flag = flag;
     p.pend_w += at;
     for (int t = 0; t < count; t += kGroupBlock) {
       if (kWhich == kGroupsIn) {
@@ -1690,51 +1746,77 @@ __global__ void __launch_bounds__(kGroupBlock, 4) k_group_pairs(group_params g) 
         in_pairs_simple<true>(p, t + tid);
       }
     }
-    pend_alive = p.pend_alive;
-    kill = p.kill;
-    pend_prefix = g.pend_prefix_in + at;
-    kill_prefix = g.kill_prefix_in + at;
   }
   __syncthreads();  // the flags are written
-  int carry_p = 0, carry_k = 0;
+  int3 carry = make_int3(0, 0, 0);
   for (int t = 0; t < count; t += kGroupBlock) {
     const int i = t + tid;
-    const int xp = i < count ? pend_alive[i] : 0, xk = i < count ? kill[i] : 0;
-    const int sp = wave_scan(xp), sk = wave_scan(xk);
+    const int xp = i < count ? alive[i] : 0, xk = i < count ? killed[i] : 0, xf = i < count ? flag[i] : 0;
+    const int sp = wave_scan(xp), sk = wave_scan(xk), sf = wave_scan(xf);
     __syncthreads();
-    if (lane() == 63) sums[tid / 64] = make_int2(sp, sk);
+    if (lane() == 63) sums[tid / 64] = make_int3(sp, sk, sf);
     __syncthreads();
-    int bp = carry_p, bk = carry_k;
+    int3 b = carry;
     for (int w = 0; w < kGroupBlock / 64; ++w) {
-      const int2 x = sums[w];
+      const int3 x = sums[w];
       if (w < tid / 64) {
-        bp += x.x;
-        bk += x.y;
+        b.x += x.x;
+        b.y += x.y;
+        b.z += x.z;
       }
-      carry_p += x.x;
-      carry_k += x.y;
+      carry.x += x.x;
+      carry.y += x.y;
+      carry.z += x.z;
     }
     if (i < count) {
-      pend_prefix[i] = bp + sp - xp;
-      kill_prefix[i] = bk + sk - xk;
+      flag[i] = b.x + sp - xp;
+      killed_before[i] = b.y + sk - xk;
+      killed[i] = b.z + sf - xf;
+      if (lds) {
+        g.keys[(in ? g.P : 0) + at + i] = keys[i];
+        out_alive[i] = xp;
+        out_pend[i] = b.x + sp - xp;
+        out_kill[i] = b.y + sk - xk;
+      }
     }
   }
   if (tid == 0) {
-    pend_prefix[count] = carry_p;
-    kill_prefix[count] = carry_k;
+    flag[count] = out_pend[count] = carry.x;
+    killed_before[count] = out_kill[count] = carry.y;
+    killed[count] = carry.z;
   }
-  __syncthreads();  // the prefixes, the rows' ranges and marks are written
+  __syncthreads();
   const merge_params& m = in ? g.merge_in : g.merge_out;
-  const int32_t* mark = in ? g.in.mark : g.out.mark;
-  const int gen = g.out.mark_gen;
   for (int t = 0; t < count; t += kGroupBlock) {
     const int i = t + tid;
     int32_t u = -1;
+    row_facts f{};
     if (i < count) {
       const u64 r = keys[i] >> g.vbits;
-      if ((i == 0 || keys[i - 1] >> g.vbits != r) && mark[r] == gen) u = static_cast<int32_t>(r);
+      if (i == 0 || keys[i - 1] >> g.vbits != r) {
+        int b = i + 1;  // the row's operations end at b
+        if (b < count && keys[b] >> g.vbits == r) {
+          int end = count;
+          ++b;
+          while (b < end) {
+            const int mid = (b + end) >> 1;
+            if (keys[mid] >> g.vbits == r) b = mid + 1; else end = mid;
+          }
+        }
+        if (killed[b] != killed[i]) {
+          u = static_cast<int32_t>(r);
+          f.mt = m.meta[u];
+          f.base = m.base[u];
+          f.cap = m.cap[u];
+          f.dead = ld(&m.dead[u]);  // counted by device-scope additions of this launch
+          f.a = static_cast<int32_t>(at + i);
+          f.b = static_cast<int32_t>(at + b);
+          f.pending = flag[b] - flag[i];
+          f.killed = killed_before[b] - killed_before[i];
+        }
+      }
     }
-    plan_rows<kGroupBlock, true>(m, u, in ? &g.ctl->touched_in : &g.ctl->touched_out, in ? g.in.touched : g.out.touched);
+    plan_rows<kGroupBlock>(m, u, f, in ? &g.ctl->touched_in : &g.ctl->touched_out, in ? g.in.touched : g.out.touched);
     __syncthreads();  // plan_rows' arrays are free again
   }
 }
@@ -1750,17 +1832,16 @@ __global__ void __launch_bounds__(kGroupBlock, 4) k_group_pairs(group_params g) 
 template <int KW>
 DYNG_DEV void tail_lane(const merge_params& p, int block, int blocks) {
   const int count = p.list_count[kTailLane];
-  const int32_t* list = p.lists + kTailLane * (p.N + 1);
   const u64 mask = (1ULL << p.vbits) - 1;
   const int K = p.K;
   for (int t = block * blockDim.x + threadIdx.x; t < count; t += blocks * blockDim.x) {
-    const int32_t u = list[t];
-    const int2 mt = p.meta[u];
-    const int64_t a = p.row_a[u];
-    const int nops = static_cast<int>(p.row_b[u] - a);
-    const int bl = p.base[u];
-    const int tl = mt.y - bl;
-    const int64_t at = mt.x + int64_t{bl};  // the tail's first slot
+    const int4 row = p.lane_rows[2 * int64_t{t}], ops = p.lane_rows[2 * int64_t{t} + 1];
+    const int32_t u = row.x;
+    const int64_t a = ops.x;
+    const int nops = ops.y;
+    const int bl = row.z;
+    const int tl = row.w;
+    const int64_t at = row.y + int64_t{bl};  // the tail's first slot
     int32_t x[kLaneTail];
 #pragma unroll
     for (int j = 0; j < kLaneTail; ++j) x[j] = j < tl ? p.nbr[at + j] : -1;
@@ -1820,7 +1901,7 @@ DYNG_DEV void tail_lane(const merge_params& p, int block, int blocks) {
         }
       }
     }
-    p.meta[u] = make_int2(mt.x, bl + alive + pending);
+    p.meta[u] = make_int2(row.y, bl + alive + pending);
   }
 }
 
@@ -2093,7 +2174,7 @@ DYNG_DEV void full_merge(const merge_params& p, int block, int blocks, long long
     const int2 mt = p.meta[u];
     const int64_t a = p.row_a[u], b = p.row_b[u];
     const int nops = static_cast<int>(b - a);
-    const row_plan r = plan_row(p, u, mt, a, b, p.dead[u]);
+    const row_plan r = plan_row(read_facts(p, u, static_cast<int32_t>(a), static_cast<int32_t>(b)));
     if (tid == 0) {
       s_stage = stage_from + static_cast<long long>(atomicAdd(reinterpret_cast<unsigned long long*>(p.stage_used),
                                                  static_cast<unsigned long long>(r.alive_base + r.alive_tail)));
@@ -2687,6 +2768,7 @@ merge_params merge_setup(dyng_hip_graph* g, bool outs, int64_t N, int vbits) {
   mp.touched_count = outs ? &dc->touched_out : &dc->touched_in;
   mp.row_a = outs ? g->row_a_out.p : g->row_a_in.p;
   mp.row_b = outs ? g->row_b_out.p : g->row_b_in.p;
+  mp.lane_rows = g->lane_rows.p + (outs ? 0 : 2 * (N + 1));
   mp.lists = g->merge_lists.p + (outs ? 0 : kModes * (N + 1));
   mp.list_count = outs ? dc->modes_out : dc->modes_in;
   mp.stage_nbr = g->stage_nbr.p;
@@ -2871,6 +2953,7 @@ void reserve_ops(dyng_hip_graph* g, int64_t P) {
   g->ikill_prefix.reserve(P + 1);
   g->ipend_w.reserve(P * K);
   g->merge_lists.reserve(2 * kModes * (P + 1));
+  g->lane_rows.reserve(4 * (P + 1));
 }
 
 /// Groups per direction for N operations, as a power of two's exponent.
@@ -3037,7 +3120,6 @@ void rows_sorted(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, in
                   g->kill_prefix.p, g->ipend_prefix.p, g->ikill_prefix.p, N + 1, s);
   mark_stage(g, 9, s);
   // ---- plan the merges: each row's mode, and the staging and tail slots they take ----
-  g->merge_lists.reserve(2 * kModes * (N + 1));
   if (wait != nullptr) DYNG_HIP_TRY(hipStreamWaitEvent(s, wait, 0));  // before the rows change
   ap.speculative = N <= kSpeculativeOps;
   if (ap.speculative) {

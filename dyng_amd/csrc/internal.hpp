@@ -358,7 +358,9 @@ struct dyng_hip_graph {
   dyng_hip::dbuf<int32_t> pend_alive, kill, pend_prefix, kill_prefix, pend_w;
   dyng_hip::dbuf<int32_t> ipend_alive, ikill, ipend_prefix, ikill_prefix, ipend_w;
   dyng_hip::dbuf<int32_t> iop_type, iop_wold, iop_wnew;
-  dyng_hip::dbuf<int32_t> touched_out, touched_in, mark_out, mark_in;
+  dyng_hip::dbuf<int4> touched_out, touched_in;
+  dyng_hip::dbuf<int4> lane_rows;  ///< the merge plan's rows of one thread each, per direction
+  dyng_hip::dbuf<int32_t> mark_out, mark_in;
   dyng_hip::dbuf<int32_t> row_a_out, row_b_out, row_a_in, row_b_in;  ///< per vertex: its operations
   dyng_hip::dbuf<int32_t> merge_lists;  ///< the merge plan's row lists, per direction and mode
   dyng_hip::dbuf<int32_t> stage_nbr, stage_w;
