@@ -1829,79 +1829,94 @@ __global__ void __launch_bounds__(kGroupBlock, 4) k_group_pairs(group_params g) 
 /// move KW columns per pass, each pass reading its columns before writing them (KW = 1 for a
 /// single weight column: 162 VGPRs instead of 186, three waves per SIMD instead of two). Old
 /// entries come first among equal neighbours, as in the wave merge below.
+template <int KW, int T, int O>
+DYNG_DEV int merge_lane(const merge_params& p, int64_t at, int tl, int64_t a, int nops) {
+  const u64 mask = (1ULL << p.vbits) - 1;
+  const int K = p.K;
+      int32_t x[T];
+  #pragma unroll
+      for (int j = 0; j < T; ++j) x[j] = j < tl ? p.nbr[at + j] : -1;
+      int32_t ov[O];
+      bool pend[O];
+  #pragma unroll
+      for (int j = 0; j < O; ++j) {
+        pend[j] = j < nops && p.pend_alive[a + j] != 0;
+        ov[j] = pend[j] ? static_cast<int32_t>(p.keys[a + j] & mask) : 0;
+      }
+      int alive = 0, pending = 0;
+      for (int k0 = 0; k0 == 0 || k0 < K; k0 += KW) {
+        int32_t wr[KW][T];
+        int32_t ow[KW][O];
+  #pragma unroll
+        for (int j = 0; j < T; ++j) {
+  #pragma unroll
+          for (int k = 0; k < KW; ++k) {
+            wr[k][j] = (j < tl && k0 + k < K) ? p.w[(k0 + k) * p.slot_cap + at + j] : 0;
+          }
+        }
+  #pragma unroll
+        for (int j = 0; j < O; ++j) {
+  #pragma unroll
+          for (int k = 0; k < KW; ++k) ow[k][j] = (pend[j] && k0 + k < K) ? p.pend_w[(k0 + k) * p.N + a + j] : 0;
+        }
+        // alive entries, at their places (the tail is sorted, dead entries carry the sign bit)
+        alive = 0;
+  #pragma unroll
+        for (int i = 0; i < T; ++i) {
+          if (x[i] >= 0) {
+            int pos = alive;
+  #pragma unroll
+            for (int j = 0; j < O; ++j) pos += (pend[j] && ov[j] < x[i]) ? 1 : 0;
+            if (k0 == 0) p.nbr[at + pos] = x[i];
+  #pragma unroll
+            for (int k = 0; k < KW; ++k) {
+              if (k0 + k < K) p.w[(k0 + k) * p.slot_cap + at + pos] = wr[k][i];
+            }
+            ++alive;
+          }
+        }
+        // pending entries (the operations are sorted by neighbour, then batch order)
+        pending = 0;
+  #pragma unroll
+        for (int j = 0; j < O; ++j) {
+          if (pend[j]) {
+            int pos = pending;
+  #pragma unroll
+            for (int i = 0; i < T; ++i) pos += (x[i] >= 0 && x[i] <= ov[j]) ? 1 : 0;
+            if (k0 == 0) p.nbr[at + pos] = ov[j];
+  #pragma unroll
+            for (int k = 0; k < KW; ++k) {
+              if (k0 + k < K) p.w[(k0 + k) * p.slot_cap + at + pos] = ow[k][j];
+            }
+            ++pending;
+          }
+        }
+      }
+  return alive + pending;
+}
+
+/// The wave's longest tail and most operations choose how many entries and operations are counted out:
+/// the full 32 x 8 is 1,500 instructions, which a small batch's few waves wait for (10 operations:
+/// 11 us, 3.4 with 8 x 2; a large batch waits for memory either way).
 template <int KW>
 DYNG_DEV void tail_lane(const merge_params& p, int block, int blocks) {
   const int count = p.list_count[kTailLane];
-  const u64 mask = (1ULL << p.vbits) - 1;
-  const int K = p.K;
   for (int t = block * blockDim.x + threadIdx.x; t < count; t += blocks * blockDim.x) {
     const int4 row = p.lane_rows[2 * int64_t{t}], ops = p.lane_rows[2 * int64_t{t} + 1];
-    const int32_t u = row.x;
     const int64_t a = ops.x;
     const int nops = ops.y;
     const int bl = row.z;
     const int tl = row.w;
     const int64_t at = row.y + int64_t{bl};  // the tail's first slot
-    int32_t x[kLaneTail];
-#pragma unroll
-    for (int j = 0; j < kLaneTail; ++j) x[j] = j < tl ? p.nbr[at + j] : -1;
-    int32_t ov[kLaneOps];
-    bool pend[kLaneOps];
-#pragma unroll
-    for (int j = 0; j < kLaneOps; ++j) {
-      pend[j] = j < nops && p.pend_alive[a + j] != 0;
-      ov[j] = pend[j] ? static_cast<int32_t>(p.keys[a + j] & mask) : 0;
+    int len;
+    if (!__any(tl > kLaneTail / 4 || nops > kLaneOps / 4)) {
+      len = merge_lane<KW, kLaneTail / 4, kLaneOps / 4>(p, at, tl, a, nops);
+    } else if (!__any(tl > kLaneTail / 2 || nops > kLaneOps / 2)) {
+      len = merge_lane<KW, kLaneTail / 2, kLaneOps / 2>(p, at, tl, a, nops);
+    } else {
+      len = merge_lane<KW, kLaneTail, kLaneOps>(p, at, tl, a, nops);
     }
-    int alive = 0, pending = 0;
-    for (int k0 = 0; k0 == 0 || k0 < K; k0 += KW) {
-      int32_t wr[KW][kLaneTail];
-      int32_t ow[KW][kLaneOps];
-#pragma unroll
-      for (int j = 0; j < kLaneTail; ++j) {
-#pragma unroll
-        for (int k = 0; k < KW; ++k) {
-          wr[k][j] = (j < tl && k0 + k < K) ? p.w[(k0 + k) * p.slot_cap + at + j] : 0;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < kLaneOps; ++j) {
-#pragma unroll
-        for (int k = 0; k < KW; ++k) ow[k][j] = (pend[j] && k0 + k < K) ? p.pend_w[(k0 + k) * p.N + a + j] : 0;
-      }
-      // alive entries, at their places (the tail is sorted, dead entries carry the sign bit)
-      alive = 0;
-#pragma unroll
-      for (int i = 0; i < kLaneTail; ++i) {
-        if (x[i] >= 0) {
-          int pos = alive;
-#pragma unroll
-          for (int j = 0; j < kLaneOps; ++j) pos += (pend[j] && ov[j] < x[i]) ? 1 : 0;
-          if (k0 == 0) p.nbr[at + pos] = x[i];
-#pragma unroll
-          for (int k = 0; k < KW; ++k) {
-            if (k0 + k < K) p.w[(k0 + k) * p.slot_cap + at + pos] = wr[k][i];
-          }
-          ++alive;
-        }
-      }
-      // pending entries (the operations are sorted by neighbour, then batch order)
-      pending = 0;
-#pragma unroll
-      for (int j = 0; j < kLaneOps; ++j) {
-        if (pend[j]) {
-          int pos = pending;
-#pragma unroll
-          for (int i = 0; i < kLaneTail; ++i) pos += (x[i] >= 0 && x[i] <= ov[j]) ? 1 : 0;
-          if (k0 == 0) p.nbr[at + pos] = ov[j];
-#pragma unroll
-          for (int k = 0; k < KW; ++k) {
-            if (k0 + k < K) p.w[(k0 + k) * p.slot_cap + at + pos] = ow[k][j];
-          }
-          ++pending;
-        }
-      }
-    }
-    p.meta[u] = make_int2(row.y, bl + alive + pending);
+    p.meta[row.x] = make_int2(row.y, bl + len);
   }
 }
 
