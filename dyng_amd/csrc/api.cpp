@@ -286,11 +286,18 @@ struct apply_in_flight {
   apply_pending* ap;
   const batch_scan* sc;
   dyng_hip_apply_summary* summary;
+  hipEvent_t began;  ///< recorded before the apply was queued
+  double* apply_ms;
 };
+
+double elapsed_ms(hipEvent_t a, hipEvent_t b) {
+  float t = 0.0f;
+  (void)hipEventElapsedTime(&t, a, b);
+  return t;
+}
 
 void repair_core(dyng_hip_graph* g, dyng_hip_result* r, int64_t delta, int64_t max_weight, hipStream_t s,
                  dyng_hip_counters& c, double& engine_ms, int choice = 0, const apply_in_flight* inflight = nullptr) {
-  event_pair ev;
   try {
     grow_result(r, g->n, s);
     std::lock_guard<std::mutex> lk(pool().lock);
@@ -307,11 +314,9 @@ void repair_core(dyng_hip_graph* g, dyng_hip_result* r, int64_t delta, int64_t m
       return run;
     };
     dyng_hip_sssp_run run = run_for();
-    DYNG_HIP_TRY(hipEventRecord(ev.a, s));
     r->tree_token = 0;
     // queued right behind the apply when it is in flight: one synchronization for both
     engine_pending pend = engine_launch(&run, true, s, inflight != nullptr ? inflight->ap : nullptr);
-    DYNG_HIP_TRY(hipEventRecord(ev.b, s));
     if (inflight != nullptr) {
       try {
         apply_finish(g, *inflight->sc, *inflight->ap, s, inflight->summary);
@@ -324,17 +329,18 @@ void repair_core(dyng_hip_graph* g, dyng_hip_result* r, int64_t delta, int64_t m
       }
     }
     engine_finish(pend, &c);
+    // the events that time the run are the workspace's, recorded around its kernel; the apply's time
+    // ends where the run's begins (each record is a packet that the stream waits at)
+    if (inflight != nullptr && pend.started != nullptr) *inflight->apply_ms = elapsed_ms(inflight->began, pend.started);
     if (pend.held) {
       // the apply's merges were planned again on the host (its arenas may have moved): the run now
       run = run_for();
-      DYNG_HIP_TRY(hipEventRecord(ev.a, s));
       pend = engine_launch(&run, true, s);
-      DYNG_HIP_TRY(hipEventRecord(ev.b, s));
       engine_finish(pend, &c);
     }
     r->tree_token = c.tree_token;
     r->last = c;
-    DYNG_HIP_TRY(hipEventSynchronize(ev.b));
+    engine_ms = c.kernel_ms;
   } catch (...) {
     r->poisoned = true;
     throw;
@@ -342,7 +348,6 @@ void repair_core(dyng_hip_graph* g, dyng_hip_result* r, int64_t delta, int64_t m
   r->version = g->version;
   r->trusted = true;
   r->engine_tree = true;
-  engine_ms = ev.ms();
 }
 
 }  // namespace
@@ -483,6 +488,7 @@ extern "C" int dyng_hip_api_update(dyng_hip_graph* g, const dyng_hip_batch* batc
     // for both; apply_finish reports the apply's errors before the engine's) ----
     event_pair ev_apply;
     dyng_hip_apply_summary summary{};
+    double apply_ms = 0.0;
     DYNG_HIP_TRY(hipEventRecord(ev_apply.a, s));
     apply_pending ap;
     try {
@@ -493,17 +499,16 @@ extern "C" int dyng_hip_api_update(dyng_hip_graph* g, const dyng_hip_batch* batc
       r->poisoned = true;  // the graph may be partly updated
       throw;
     }
-    DYNG_HIP_TRY(hipEventRecord(ev_apply.b, s));
     // ---- resume + the engine; a failure from here on poisons the result ----
     dyng_hip_counters c{};
     double engine_ms = 0.0;
-    const apply_in_flight inflight{&ap, &sc, &summary};
+    const apply_in_flight inflight{&ap, &sc, &summary, ev_apply.a, &apply_ms};
     repair_core(g, r, delta, max_weight, s, c, engine_ms, 0, &inflight);
     if (stats != nullptr) {
       std::memset(stats, 0, sizeof(*stats));
       fill_stats(stats, c);
       stats->batch = summary;
-      stats->apply_ms = ev_apply.ms();
+      stats->apply_ms = apply_ms;
       stats->engine_ms = engine_ms;
     }
   });
@@ -700,6 +705,7 @@ extern "C" int dyng_hip_api_update_scheduled(dyng_hip_graph* g, const dyng_hip_b
     // schedule (the prediction is waited for after the apply was queued) ----
     event_pair ev_apply;
     dyng_hip_apply_summary summary{};
+    double apply_ms = 0.0;
     DYNG_HIP_TRY(hipEventRecord(ev_apply.a, s));
     apply_pending ap;
     try {
@@ -710,20 +716,19 @@ extern "C" int dyng_hip_api_update_scheduled(dyng_hip_graph* g, const dyng_hip_b
       r->poisoned = true;  // the graph may be partly updated
       throw;
     }
-    DYNG_HIP_TRY(hipEventRecord(ev_apply.b, s));
     // ---- resume + the engine; a failure from here on poisons the result ----
     dyng_hip_counters c{};
     double engine_ms = 0.0;
     if (predicted != nullptr) DYNG_HIP_TRY(hipEventSynchronize(predicted));
     const int pick = mlp != nullptr ? mlp_pick(mlp) : 0;
     if (choice != nullptr) *choice = pick;
-    const apply_in_flight inflight{&ap, &sc, &summary};
+    const apply_in_flight inflight{&ap, &sc, &summary, ev_apply.a, &apply_ms};
     repair_core(g, r, delta, max_weight, s, c, engine_ms, pick, &inflight);
     if (stats != nullptr) {
       std::memset(stats, 0, sizeof(*stats));
       fill_stats(stats, c);
       stats->batch = summary;
-      stats->apply_ms = ev_apply.ms();
+      stats->apply_ms = apply_ms;
       stats->engine_ms = engine_ms;
     }
   });

@@ -250,6 +250,7 @@ struct engine_pending {
   int64_t n = 0;
   int64_t timeout_us = 0;
   int64_t* distances = nullptr;
+  hipEvent_t started = nullptr;  ///< the event recorded before the kernel (null: nothing was launched)
   bool held = false;  ///< set by engine_finish: the run did nothing (see engine_launch's `ahead`)
   dyng_hip_counters counters{};
 };

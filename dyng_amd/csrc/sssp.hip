@@ -2054,6 +2054,7 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
   }
   if (ahead != nullptr) ahead->published = true;
   pend.launched = true;
+  pend.started = ws->ev_start;
   pend.bits = p.pk.bits;
   pend.blocks = blocks;
   pend.resident = p.resident;
