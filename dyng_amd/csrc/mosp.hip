@@ -145,7 +145,7 @@ __global__ void k_fill_value(T* p, int64_t n, T v) {
 DYNG_DEV int first_alive(const int32_t* row, int bl, int len, int32_t x) {
   for (int r = 0; r < 2; ++r) {
     const int lo = r == 0 ? 0 : bl, hi = r == 0 ? bl : len;
-    for (int j = row_lower_bound(row, lo, hi, x); j < hi && (row[j] & 0x7fffffff) == x; ++j) {
+    for (int j = row_lower_bound<1>(row, lo, hi, x); j < hi && (row[j] & 0x7fffffff) == x; ++j) {
       if (row[j] >= 0) return j;
     }
   }
@@ -157,7 +157,8 @@ DYNG_DEV int first_alive(const int32_t* row, int bl, int len, int32_t x) {
 /// source starts at 0 and an unreachable vertex at INF, both with no ancestor. Without parallel
 /// edges the pair (p, v) is one edge, found in v's in-row instead (short and read in vertex
 /// order, where p's out-row may be a hub's). A tree edge that is not an edge of the graph is
-/// reported (the lowest such vertex). active[0] is set when some vertex has an ancestor.
+/// reported (the lowest such vertex). One probe per search round, as the vertices' parents' rows are
+/// different lines (see find_runs in the apply).
 struct edge_rows {
   const int2* meta;
   const int32_t* base;
@@ -167,7 +168,7 @@ struct edge_rows {
 };
 
 __global__ void k_tree_edge_costs(edge_rows out, edge_rows in, bool by_in_row, int columns, const int32_t* parents,
-                                  int32_t n, int32_t source, int64_t* acc, int32_t* jump, int* missing, int* active) {
+                                  int32_t n, int32_t source, int64_t* acc, int32_t* jump, int* missing) {
   const int32_t v = static_cast<int32_t>(blockIdx.x * blockDim.x + threadIdx.x);
   int32_t link = -1;
   if (v < n) {
@@ -199,49 +200,99 @@ __global__ void k_tree_edge_costs(edge_rows out, edge_rows in, bool by_in_row, i
     }
     jump[v] = link;
   }
-  if (__syncthreads_or(link >= 0) && threadIdx.x == 0) active[0] = 1;
 }
 
-/// Path doubling, round r: each vertex adds its ancestor's sum and jumps to the ancestor's
-/// ancestor. A round whose input has no vertex left with an ancestor does nothing; a round that
-/// runs records itself in `last` and sets active[r + 1] when some vertex still has an ancestor.
-/// A vertex's jump is -1 in the round after its sum became final (that round copies the sum to
-/// the other buffer) and -2 from then on (both buffers hold it: the round only passes the -2 on).
-__global__ void k_path_double(const int64_t* acc_in, const int32_t* jump_in, int64_t* acc_out, int32_t* jump_out,
-                              int32_t n, int columns, int round, int* active, int* last) {
-  if (active[round] == 0) return;  // uniform: every thread reads the same flag
-  bool more = false;  // some vertex of this thread still has an ancestor
-  const int64_t stride = int64_t{gridDim.x} * blockDim.x;
-  for (int64_t i = blockIdx.x * int64_t{blockDim.x} + threadIdx.x; i < n; i += stride) {
-    const int32_t v = static_cast<int32_t>(i);
-    int32_t next = -2;
-    const int32_t j = jump_in[v];
-    if (j == -1) {
-      const int64_t* a = acc_in + static_cast<int64_t>(v) * columns;
-      int64_t* o = acc_out + static_cast<int64_t>(v) * columns;
-      for (int c = 0; c < columns; ++c) o[c] = a[c];
-    } else if (j >= 0) {
-      const int64_t* a = acc_in + static_cast<int64_t>(v) * columns;
-      int64_t* o = acc_out + static_cast<int64_t>(v) * columns;
-      const int64_t* b = acc_in + static_cast<int64_t>(j) * columns;
-      for (int c = 0; c < columns; ++c) o[c] = a[c] + b[c];
-      const int32_t up = jump_in[j];
-      next = up < 0 ? -1 : up;
+/// What the path doubling tells the host (pinned memory).
+struct path_report {
+  int missing;  ///< the lowest vertex whose tree edge is not in the graph (INT32_MAX: none)
+  int ended;    ///< 1: every round ran
+};
+
+struct path_params {
+  int64_t* acc[2];   ///< sums of the even and odd rounds; acc[0] is the caller's
+  int32_t* jump[2];
+  int32_t n;
+  int columns;
+  grid_sync_state* bar;
+  unsigned long long limit;  ///< ticks a grid barrier waits at most
+  unsigned int rounds;       ///< at most: log2(n) rounded up, and one
+  const int* missing;
+  path_report* report;
+};
+
+constexpr int kPathBlock = 1024;
+constexpr int kPathSlots = 4;  ///< vertices of a thread in flight
+
+/// Clear the grid barrier and the missing vertex.
+__global__ void k_path_begin(grid_sync_state* bar, int* missing) {
+  u64* w = reinterpret_cast<u64*>(bar);
+  for (unsigned int i = threadIdx.x; i < sizeof(grid_sync_state) / 8; i += blockDim.x) w[i] = 0;
+  if (threadIdx.x == 0) *missing = INT32_MAX;
+}
+
+/// Path doubling: in each round every vertex adds its ancestor's sum and jumps to the ancestor's
+/// ancestor, until none has one. A vertex's jump is -1 in the round after its sum became final (that
+/// round copies the sum to the other buffer) and -2 from then on (both buffers hold it: a round only
+/// passes the -2 on). One launch of resident workgroups with a grid barrier per round, at which each
+/// tells how many of its vertices go on: a launch per round had to queue log2(n) + 1 of them, 21 for
+/// 2^20 vertices whose trees are 5 rounds deep, and each empty one took 7 us with its gap. The rounds
+/// read what other workgroups wrote, so those accesses are at device scope.
+__global__ void __launch_bounds__(kPathBlock) k_path_costs(path_params p) {
+  const int threads = static_cast<int>(gridDim.x) * kPathBlock;
+  const int tid = static_cast<int>(blockIdx.x) * kPathBlock + static_cast<int>(threadIdx.x);
+  int cur = 0;
+  for (unsigned int round = 1; round <= p.rounds; ++round) {
+    const int64_t* acc_in = p.acc[cur];
+    const int32_t* jump_in = p.jump[cur];
+    int64_t* acc_out = p.acc[cur ^ 1];
+    int32_t* jump_out = p.jump[cur ^ 1];
+    bool more = false;  // some vertex of this thread still has an ancestor
+    for (int64_t v0 = tid; v0 < p.n; v0 += int64_t{kPathSlots} * threads) {
+      int32_t j[kPathSlots], up[kPathSlots];
+#pragma unroll
+      for (int q = 0; q < kPathSlots; ++q) {
+        const int64_t v = v0 + int64_t{q} * threads;
+        j[q] = v < p.n ? ld(&jump_in[v]) : -2;
+      }
+#pragma unroll
+      for (int q = 0; q < kPathSlots; ++q) up[q] = j[q] >= 0 ? ld(&jump_in[j[q]]) : -2;
+      for (int c = 0; c < p.columns; ++c) {
+        int64_t a[kPathSlots], b[kPathSlots];
+#pragma unroll
+        for (int q = 0; q < kPathSlots; ++q) {
+          const int64_t v = v0 + int64_t{q} * threads;
+          a[q] = j[q] != -2 ? ld(&acc_in[v * p.columns + c]) : 0;
+          b[q] = j[q] >= 0 ? ld(&acc_in[static_cast<int64_t>(j[q]) * p.columns + c]) : 0;
+        }
+#pragma unroll
+        for (int q = 0; q < kPathSlots; ++q) {
+          const int64_t v = v0 + int64_t{q} * threads;
+          if (j[q] != -2) st(&acc_out[v * p.columns + c], a[q] + b[q]);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kPathSlots; ++q) {
+        const int64_t v = v0 + int64_t{q} * threads;
+        const int32_t next = j[q] < 0 ? -2 : up[q] < 0 ? -1 : up[q];
+        if (v < p.n) st(&jump_out[v], next);
+        more = more || next >= 0;
+      }
     }
-    jump_out[v] = next;
-    more = more || next >= 0;
+    cur ^= 1;
+    const unsigned int mine = static_cast<unsigned int>(__syncthreads_count(more ? 1 : 0));
+    const grid_found found = grid_barrier<false>(p.bar, round, p.limit, [&] { grid_arrive(p.bar, round, mine); });
+    if (!found.ok) return;  // uniform: the host finds `ended` clear
+    if (found.published == 0) break;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) *last = round;
-  if (__syncthreads_or(more) && threadIdx.x == 0) active[round + 1] = 1;
-}
-
-/// Round r writes buffer (r + 1) % 2 (buffer 0 is the caller's, which the first step wrote): the
-/// sums are in `acc` only when the last round that ran is even; then copy them home.
-__global__ void k_costs_home(const int64_t* acc, int64_t* costs, int64_t count, const int* last) {
-  const int r = *last;
-  if (r < 0 || (r & 1) == 1) return;
-  for (int64_t i = blockIdx.x * int64_t{blockDim.x} + threadIdx.x; i < count; i += int64_t{gridDim.x} * blockDim.x) {
-    costs[i] = acc[i];
+  if (cur == 1) {
+    // an odd number of rounds: the sums are in the other buffer, each vertex's written by this thread
+    for (int64_t v = tid; v < p.n; v += threads) {
+      for (int c = 0; c < p.columns; ++c) p.acc[0][v * p.columns + c] = ld(&p.acc[1][v * p.columns + c]);
+    }
+  }
+  if (tid == 0) {
+    p.report->missing = *p.missing;
+    p.report->ended = 1;
   }
 }
 
@@ -485,7 +536,10 @@ struct combined_cache {
   dbuf<unsigned long long> totals;
   dbuf<int64_t> acc;
   dbuf<int32_t> jump_a, jump_b;
-  dbuf<int> flags;  ///< missing vertex, last round, then the rounds' active flags
+  dbuf<int> missing;  ///< the path costs' lowest vertex without its tree edge
+  dbuf<grid_sync_state> bar;
+  pinned<path_report> report;
+  int cu_count = 0;
   const int2* in_meta_cleared = nullptr;  ///< the in-row meta array last cleared
 };
 
@@ -624,43 +678,39 @@ void mosp_path_costs(const dyng_hip_graph* g, const int32_t* parents, int64_t n,
                      int64_t* costs, hipStream_t s) {
   if (n == 0 || columns == 0) return;
   combined_cache& cc = cache_for(g->device);
-  int rounds = 1;
-  while ((int64_t{1} << rounds) < n) ++rounds;
-  rounds += 1;
   cc.acc.reserve(static_cast<size_t>(n) * columns);
   cc.jump_a.reserve(n);
   cc.jump_b.reserve(n);
-  cc.flags.reserve(rounds + 3);
-  // flags: [0] the lowest vertex whose tree edge is missing, [1] the last round that ran, then
-  // active[0 .. rounds]
-  std::vector<int> init(static_cast<size_t>(rounds) + 3, 0);
-  init[0] = INT32_MAX;
-  init[1] = -1;
-  DYNG_HIP_TRY(hipMemcpyAsync(cc.flags.p, init.data(), init.size() * sizeof(int), hipMemcpyHostToDevice, s));
-  int* missing = cc.flags.p;
-  int* last = cc.flags.p + 1;
-  int* active = cc.flags.p + 2;
-  // the first step writes the caller's array; the rounds then alternate between it and `acc`
-  int64_t* bufs[2] = {costs, cc.acc.p};
-  int32_t* jumps[2] = {cc.jump_a.p, cc.jump_b.p};
+  cc.missing.reserve(1);
+  cc.bar.reserve(1);
   const edge_rows out{g->out.meta.p, g->out.base.p, g->out.nbr.p, g->out.w.p, g->out.slot_cap};
   const edge_rows in{g->in.meta.p, g->in.base.p, g->in.nbr.p, g->in.w.p, g->in.slot_cap};
   const bool by_in_row = g->props.allow_parallel == 0;
+  hipLaunchKernelGGL(k_path_begin, dim3(1), dim3(64), 0, s, cc.bar.p, cc.missing.p);
   hipLaunchKernelGGL(k_tree_edge_costs, dim3(grid(n, 256)), dim3(256), 0, s, out, in, by_in_row, columns, parents,
-                     static_cast<int32_t>(n), source, bufs[0], jumps[0], missing, active);
-  int cur = 0;
-  for (int r = 0; r < rounds; ++r) {
-    // a bounded grid: a round after the last one still launches, and returns at once
-    hipLaunchKernelGGL(k_path_double, dim3(std::min(grid(n, 256), 2048u)), dim3(256), 0, s, bufs[cur], jumps[cur],
-                       bufs[cur ^ 1], jumps[cur ^ 1], static_cast<int32_t>(n), columns, r, active, last);
-    cur ^= 1;
-  }
-  hipLaunchKernelGGL(k_costs_home, dim3(std::min(grid(n * columns, 256), 8192u)), dim3(256), 0, s, cc.acc.p, costs,
-                     n * columns, last);
+                     static_cast<int32_t>(n), source, costs, cc.jump_a.p, cc.missing.p);
   DYNG_HIP_TRY(hipGetLastError());
-  int host_missing = INT32_MAX;
-  DYNG_HIP_TRY(hipMemcpyAsync(&host_missing, missing, sizeof(int), hipMemcpyDeviceToHost, s));
+  if (cc.cu_count == 0) {
+    DYNG_HIP_TRY(hipDeviceGetAttribute(&cc.cu_count, hipDeviceAttributeMultiprocessorCount, g->device));
+  }
+  path_report* report = cc.report.p;
+  report->missing = INT32_MAX;
+  report->ended = 0;
+  constexpr int64_t kTimeoutUs = 4000000;  // the engine's default for its barrier
+  unsigned int rounds = 1;
+  while ((int64_t{1} << rounds) < n) ++rounds;
+  const path_params pp{{costs, cc.acc.p}, {cc.jump_a.p, cc.jump_b.p}, static_cast<int32_t>(n), columns, cc.bar.p,
+                       static_cast<unsigned long long>(kTimeoutUs) * 100ULL, rounds + 1, cc.missing.p, report};
+  // one workgroup per processor at most, so that all are resident
+  const unsigned blocks = std::min(grid(n, kPathBlock), static_cast<unsigned>(cc.cu_count));
+  hipLaunchKernelGGL(k_path_costs, dim3(blocks), dim3(kPathBlock), 0, s, pp);
+  DYNG_HIP_TRY(hipGetLastError());
   DYNG_HIP_TRY(hipStreamSynchronize(s));
+  if (report->ended == 0) {
+    fail(DYNG_HIP_RUNTIME_ERROR, "mosp: a grid barrier wait of the path costs ran past " + std::to_string(kTimeoutUs) +
+                                     " us");
+  }
+  const int host_missing = report->missing;
   if (host_missing != INT32_MAX) {
     fail(DYNG_HIP_INVALID_ARGUMENT, "mosp: the MOSP tree edge (" + std::to_string(host_missing) +
                                         "'s parent, " + std::to_string(host_missing) +
