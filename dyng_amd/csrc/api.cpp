@@ -38,7 +38,8 @@ constexpr int64_t kInf = sssp_infinity;
 /// result at a time; an update of several results gives result i slot i % kWorkspaceSlots, so
 /// those results keep their own packed words from one update to the next (up to kWorkspaceSlots
 /// results) and kWorkspaceSlots of their runs can be queued ahead of the host.
-constexpr int kWorkspaceSlots = 4;
+/// Operations of a batch up to which the repairs of several results share a launch.
+constexpr int64_t kTeamOps = int64_t{1} << 16;
 
 struct workspace_pool {
   std::mutex lock;
@@ -602,11 +603,11 @@ extern "C" int dyng_hip_api_update_each(dyng_hip_graph* g, const dyng_hip_batch*
         first = std::current_exception();
       }
     } else {
-      // several results: result i runs on workspace slot i % kWorkspaceSlots, all of them queued
-      // on the caller's stream, kWorkspaceSlots runs ahead of the host. They run one after
-      // another: two persistent launches resident at once on MI355X gave wrong trees (each
-      // lane keeps a little state in scratch memory, which the other launch's waves corrupted),
-      // so runs never overlap
+      // several results: result i runs on workspace slot i % kWorkspaceSlots, kWorkspaceSlots of them
+      // side by side in one launch. A batch past kTeamOps keeps the processors busy by itself: its runs,
+      // and those whose tuning asks for a launch of their own, are queued one after another
+      // on the caller's stream, kWorkspaceSlots runs ahead of the host (never two launches at once: their
+      // workgroups wait for each other at grid barriers and must all be resident)
       for (int64_t i = 0; i < count; ++i) grow_result(results[i], g->n, s);
       std::lock_guard<std::mutex> lk(pool().lock);
       std::vector<engine_pending> pend(static_cast<size_t>(count));
@@ -634,19 +635,59 @@ extern "C" int dyng_hip_api_update_each(dyng_hip_graph* g, const dyng_hip_batch*
           stats[i].engine_ms = c.kernel_ms;
         }
       };
+      auto fail_result = [&](int64_t i, std::exception_ptr e) {
+        results[i]->poisoned = true;
+        if (!first) first = e;
+      };
+      std::vector<dyng_hip_sssp_run> runs(static_cast<size_t>(count));
+      std::vector<char> made(static_cast<size_t>(count), 0);
+      bool together = sc.num_ins + sc.num_del <= kTeamOps;
       for (int64_t i = 0; i < count; ++i) {
-        // a workspace holds one run at a time: the run kWorkspaceSlots back used this slot
-        if (i >= kWorkspaceSlots) finish(i - kWorkspaceSlots);
-        dyng_hip_result* r = results[i];
         try {
-          dyng_hip_sssp_run run = make_run(g, r, delta[i], max_weight[i]);
-          run.workspace = pool().get(g->device, static_cast<int>(i % kWorkspaceSlots));
-          r->tree_token = 0;
-          pend[i] = engine_launch(&run, true, s);
-          ok[i] = 1;
+          runs[i] = make_run(g, results[i], delta[i], max_weight[i]);
+          made[i] = 1;
+          together = together && engine_joins(&runs[i]);
         } catch (...) {
-          r->poisoned = true;
-          if (!first) first = std::current_exception();
+          fail_result(i, std::current_exception());
+        }
+      }
+      for (int64_t i = 0; i < count; i += together ? kWorkspaceSlots : 1) {
+        const int64_t end = std::min<int64_t>(count, together ? i + kWorkspaceSlots : i + 1);
+        const dyng_hip_sssp_run* group[kWorkspaceSlots];
+        engine_pending queued[kWorkspaceSlots];
+        std::exception_ptr errors[kWorkspaceSlots];
+        int64_t of[kWorkspaceSlots];
+        int m = 0;
+        for (int64_t j = i; j < end; ++j) {
+          // a workspace holds one run at a time: the run kWorkspaceSlots back used this slot
+          if (j >= kWorkspaceSlots) finish(j - kWorkspaceSlots);
+          if (!made[j]) continue;
+          try {
+            runs[j].workspace = pool().get(g->device, static_cast<int>(j % kWorkspaceSlots));
+            results[j]->tree_token = 0;
+            group[m] = &runs[j];
+            of[m] = j;
+            ++m;
+          } catch (...) {
+            fail_result(j, std::current_exception());
+          }
+        }
+        if (m > 1) {
+          engine_launch_teams(group, m, s, queued, errors);
+        } else if (m == 1) {
+          try {
+            queued[0] = engine_launch(group[0], true, s);
+          } catch (...) {
+            errors[0] = std::current_exception();
+          }
+        }
+        for (int q = 0; q < m; ++q) {
+          if (errors[q]) {
+            fail_result(of[q], errors[q]);
+          } else {
+            pend[of[q]] = queued[q];
+            ok[of[q]] = 1;
+          }
         }
       }
       for (int64_t i = std::max<int64_t>(0, count - kWorkspaceSlots); i < count; ++i) finish(i);

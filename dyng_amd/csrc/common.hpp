@@ -224,19 +224,26 @@ struct grid_found {
   int ok, published, marked;
 };
 
+/// A workgroup's number among the `blocks` that meet at a barrier (a launch may hold several teams, each
+/// with a barrier of its own).
+struct grid_place {
+  unsigned int block, blocks;
+};
+
 /// Arrive at round `round` (1, 2, ...), with `published` entries to tell of, some of them marked or
 /// not. One thread of the workgroup calls it, after every wave's loads and stores have completed and
 /// a workgroup barrier.
-DYNG_DEV void grid_arrive(grid_sync_state* s, unsigned int round, unsigned int published, bool marked = false) {
-  const unsigned int blocks = gridDim.x;
+DYNG_DEV void grid_arrive(grid_sync_state* s, const grid_place& at, unsigned int round, unsigned int published,
+                          bool marked = false) {
+  const unsigned int blocks = at.blocks;
   const unsigned int G = blocks < kBarrierGroups ? blocks : kBarrierGroups;
-  const unsigned int grp = blockIdx.x % G;
+  const unsigned int grp = at.block % G;
   const unsigned int members = blocks / G + (blocks % G > grp ? 1u : 0u);
   barrier_line& line = s->group[grp];
-  if (blockIdx.x < G && round > 2) {
+  if (at.block < G && round > 2) {
     const unsigned int old = (round - 2) & 3u;
     __hip_atomic_store(&line.v[old], 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (blockIdx.x == 0) __hip_atomic_store(&s->root.v[old], 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (at.block == 0) __hip_atomic_store(&s->root.v[old], 0ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   const unsigned long long mine =
       1ULL | (marked ? 1ULL << 16 : 0ULL) | (static_cast<unsigned long long>(published) << 32);
@@ -254,10 +261,10 @@ DYNG_DEV void grid_arrive(grid_sync_state* s, unsigned int round, unsigned int p
 }
 
 /// Wait for round `round`, at which this workgroup has arrived. Called by the thread that arrived.
-DYNG_DEV grid_found grid_poll(grid_sync_state* s, unsigned int round, unsigned long long limit) {
-  const unsigned int blocks = gridDim.x;
+DYNG_DEV grid_found grid_poll(grid_sync_state* s, const grid_place& at, unsigned int round, unsigned long long limit) {
+  const unsigned int blocks = at.blocks;
   const unsigned int G = blocks < kBarrierGroups ? blocks : kBarrierGroups;
-  const unsigned long long* const word = &s->group[blockIdx.x % G].release;
+  const unsigned long long* const word = &s->group[at.block % G].release;
   const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
   unsigned int polls = 0;
   for (;;) {
@@ -280,7 +287,8 @@ DYNG_DEV grid_found grid_poll(grid_sync_state* s, unsigned int round, unsigned l
 /// The whole barrier: every thread of the workgroup calls it; `arrive()` (one thread, after the
 /// workgroup barrier) is grid_arrive with what this workgroup publishes.
 template <bool Fenced, class Arrive>
-DYNG_DEV grid_found grid_barrier(grid_sync_state* s, unsigned int round, unsigned long long limit, Arrive arrive) {
+DYNG_DEV grid_found grid_barrier(grid_sync_state* s, const grid_place& at, unsigned int round, unsigned long long limit,
+                                 Arrive arrive) {
   __shared__ grid_found found;
   // every wave's loads and stores have completed (at the scope they were issued with) before the
   // arrival
@@ -289,7 +297,7 @@ DYNG_DEV grid_found grid_barrier(grid_sync_state* s, unsigned int round, unsigne
   if (threadIdx.x == 0) {
     if (Fenced) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     arrive();
-    found = grid_poll(s, round, limit);
+    found = grid_poll(s, at, round, limit);
     if (Fenced) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();

@@ -250,6 +250,7 @@ struct engine_pending {
   int64_t n = 0;
   int64_t timeout_us = 0;
   int64_t* distances = nullptr;
+  bool team = false;  ///< one of several runs in a launch (engine_launch_teams)
   hipEvent_t started = nullptr;  ///< the event recorded before the kernel (null: nothing was launched)
   bool held = false;  ///< set by engine_finish: the run did nothing (see engine_launch's `ahead`)
   dyng_hip_counters counters{};
@@ -258,6 +259,12 @@ struct engine_pending {
 /// to the host, and when the apply's merges were held back the run does nothing, and
 /// engine_finish sets `held` (the caller launches it again after apply_finish).
 engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStream_t s, apply_pending* ahead = nullptr);
+/// Up to kWorkspaceSlots repairs (of runs that engine_joins accepts, a workspace each) in one launch, side by
+/// side. A run that cannot be queued leaves its error in `errors`.
+constexpr int kWorkspaceSlots = 4;
+bool engine_joins(const dyng_hip_sssp_run* run);
+void engine_launch_teams(const dyng_hip_sssp_run* const* runs, int count, hipStream_t s, engine_pending* pends,
+                         std::exception_ptr* errors);
 void engine_finish(engine_pending& pend, dyng_hip_counters* out);
 /// The scheduler's pick for a scanned batch on G_t: features, BF16 inference, argmin (one sync).
 int mlp_choose(dyng_hip_mlp* m, const dyng_hip_graph* g, const batch_scan& sc, const int32_t* parents, int64_t n_tree,

@@ -240,6 +240,7 @@ __global__ void k_path_begin(grid_sync_state* bar, int* missing) {
 __global__ void __launch_bounds__(kPathBlock) k_path_costs(path_params p) {
   const int threads = static_cast<int>(gridDim.x) * kPathBlock;
   const int tid = static_cast<int>(blockIdx.x) * kPathBlock + static_cast<int>(threadIdx.x);
+  const grid_place at{blockIdx.x, gridDim.x};
   int cur = 0;
   for (unsigned int round = 1; round <= p.rounds; ++round) {
     const int64_t* acc_in = p.acc[cur];
@@ -280,7 +281,7 @@ __global__ void __launch_bounds__(kPathBlock) k_path_costs(path_params p) {
     }
     cur ^= 1;
     const unsigned int mine = static_cast<unsigned int>(__syncthreads_count(more ? 1 : 0));
-    const grid_found found = grid_barrier<false>(p.bar, round, p.limit, [&] { grid_arrive(p.bar, round, mine); });
+    const grid_found found = grid_barrier<false>(p.bar, at, round, p.limit, [&] { grid_arrive(p.bar, at, round, mine); });
     if (!found.ok) return;  // uniform: the host finds `ended` clear
     if (found.published == 0) break;
   }

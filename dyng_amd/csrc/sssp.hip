@@ -114,6 +114,8 @@ struct control {
 };
 
 struct engine_params {
+  int32_t first_block;  ///< the run's workgroups: [first_block, first_block + blocks) of the launch
+  int32_t blocks;
   int32_t n;
   const int2* out_meta;
   const int32_t* out_base;  ///< per vertex: the length of the row's sorted base run
@@ -170,6 +172,20 @@ struct engine_params {
   const int* hold;  ///< null, or a flag of the apply queued ahead: nonzero, the run does nothing
   control* publish; ///< null, or where in pinned host memory the control block goes when the run ends
 };
+
+/// Several runs in one launch, each on a team of workgroups with its own barrier and scratch.
+constexpr int kTeams = 4;
+struct engine_teams {
+  engine_params p[kTeams];
+  int size;  ///< workgroups of a team
+};
+static_assert(sizeof(engine_teams) <= 4096, "a kernel's arguments");
+
+/// This workgroup's number among its run's.
+DYNG_DEV int run_block(const engine_params& p) { return static_cast<int>(blockIdx.x) - p.first_block; }
+DYNG_DEV grid_place run_place(const engine_params& p) {
+  return grid_place{static_cast<unsigned int>(run_block(p)), static_cast<unsigned int>(p.blocks)};
+}
 
 /// Append v to a list when pred (wave-aggregated reservation).
 DYNG_DEV void append(int* list, int* counter, bool pred, int32_t v) {
@@ -248,13 +264,14 @@ DYNG_DEV void stage_flush(stage_shared& S, int* list0, int* counter0, int* list1
 /// arrived: the reservations' round trip and the poll's are one. The copy may still be under way in
 /// other waves when it returns: a workgroup barrier before the next append.
 DYNG_DEV grid_found stage_flush_wait(stage_shared& S, int* list0, int* counter0, int* list1, int* counter1,
-                                     grid_sync_state* bar, unsigned int round, unsigned long long limit) {
+                                     grid_sync_state* bar, const grid_place& at, unsigned int round,
+                                     unsigned long long limit) {
   __shared__ grid_found found;
   __syncthreads();  // every staged entry is in LDS
   if (threadIdx.x < 3) {
     const int k = threadIdx.x;
     const int base = stage_reserve(S, k, k == 0 ? counter0 : k == 1 ? counter1 : S.counter2);
-    if (k == 0) found = grid_poll(bar, round, limit);  // its first load goes out behind the reservations
+    if (k == 0) found = grid_poll(bar, at, round, limit);  // its first load goes out behind the reservations
     S.base[k] = base;
   }
   __syncthreads();
@@ -456,14 +473,14 @@ DYNG_DEV int expand_tile(const engine_params& p, tile_shared& L, chunk_sink& out
 template <class Load, class Edges, class Check, class Done, class Between>
 DYNG_DEV int tile_rows(const engine_params& p, tile_shared& L, chunk_sink& out, unsigned int round, int count, Load load,
                        Edges edges, Check check, Done done, Between between) {
-  const int G = static_cast<int>(gridDim.x);
+  const int G = p.blocks;
   const int share = max(1, (count + G - 1) / G);
   const int tiles = (share + kBlock - 1) / kBlock;
   const int ts = (share + tiles - 1) / tiles;
   const long long stride = static_cast<long long>(G) * ts;
-  long long t0 = static_cast<long long>(blockIdx.x) * ts;
+  long long t0 = static_cast<long long>(run_block(p)) * ts;
   int expanded = 0;
-  if (t0 >= count && round != 0 && threadIdx.x == 0) grid_arrive(p.bar, round, 0);
+  if (t0 >= count && round != 0 && threadIdx.x == 0) grid_arrive(p.bar, run_place(p), round, 0);
   for (; t0 < count; t0 += stride) {
     const int cnt = static_cast<int>(min(static_cast<long long>(ts), count - t0));
     const int first = static_cast<int>(t0);
@@ -471,7 +488,7 @@ DYNG_DEV int tile_rows(const engine_params& p, tile_shared& L, chunk_sink& out, 
     expanded += expand_tile(
         p, L, out, cnt, [&](int i, int32_t& v, int32_t& off, int32_t& len, u64& word) { load(first + i, v, off, len, word); },
         [&] {
-          if (last && round != 0 && threadIdx.x == 0) grid_arrive(p.bar, round, static_cast<unsigned int>(out.published));
+          if (last && round != 0 && threadIdx.x == 0) grid_arrive(p.bar, run_place(p), round, static_cast<unsigned int>(out.published));
         },
         edges, check, done);
     if (!last) between();
@@ -600,12 +617,12 @@ DYNG_DEV void relax_slots(const engine_params& p, const bool (&act)[kSlots], con
 template <class Begin, class Edges, class End, class Check>
 DYNG_DEV void chunk_rows(const engine_params& p, const int4* chunks, int nchunks, Begin begin, Edges edges, End end,
                          Check check) {
-  const int G = static_cast<int>(gridDim.x);
+  const int G = p.blocks;
   const int waves = G * kWaves;
   const int parts = nchunks * 4 <= waves ? 4 : nchunks * 2 <= waves ? 2 : 1;
   const int span = (p.chunk_edges + parts * 64 - 1) / (parts * 64) * 64;  // slots of a part, whole waves of them
   const int units = nchunks * parts;
-  const int wave = static_cast<int>(threadIdx.x / 64) * G + static_cast<int>(blockIdx.x);
+  const int wave = static_cast<int>(threadIdx.x / 64) * G + run_block(p);
   for (int q0 = 0; q0 < units; q0 += waves) {  // uniform over the grid
     const int q = q0 + wave;
     if (q < units) {
@@ -725,8 +742,8 @@ DYNG_DEV void pull_commit(const engine_params& p, bool pred, int32_t v, u64 best
   } while (0)
 #define DYNG_GRID_SYNC_AS(fenced, list, found)                                           \
   ++round;                                                                               \
-  const grid_found found = grid_barrier<fenced>(p.bar, round, p.barrier_ticks, [&] {     \
-    grid_arrive(p.bar, round, S.sent[list], S.sent_long != 0);                           \
+  const grid_found found = grid_barrier<fenced>(p.bar, run_place(p), round, p.barrier_ticks, [&] {     \
+    grid_arrive(p.bar, run_place(p), round, S.sent[list], S.sent_long != 0);                           \
     S.sent[0] = S.sent[1] = 0;                                                           \
     S.sent_long = 0;                                                                     \
   });                                                                                    \
@@ -751,21 +768,18 @@ DYNG_DEV void pull_commit(const engine_params& p, bool pred, int32_t v, u64 best
   do {                                                                                                     \
     ++round;                                                                                               \
     const grid_found found_ =                                                                              \
-        stage_flush_wait(S, list0, counter0, list1, counter1, p.bar, round, p.barrier_ticks);              \
+        stage_flush_wait(S, list0, counter0, list1, counter1, p.bar, run_place(p), round, p.barrier_ticks);              \
     DYNG_GRID_LEAVE_UNLESS(found_.ok);                                                                     \
     nchunks = static_cast<int>(min(static_cast<int64_t>(found_.published), chunk_cap));                    \
   } while (0)
 
-/// Clear the grid barrier (a kernel, not a memset, so the launch can live in a hipGraph).
-/// Before each run (one workgroup): the barrier state and the control block zeroed, the control
-/// block's minima at INF (a kernel rather than a host copy: it costs the stream no blit).
 constexpr int kResetBlock = 256;
 static_assert(sizeof(control) % 8 == 0 && sizeof(grid_sync_state) % 8 == 0, "reset in 8-byte words");
-/// The apply queued ahead of a run has ended when this starts: `words` 4-byte words of its control
-/// block go to pinned host memory here, in place of a copy of their own.
-__global__ void __launch_bounds__(kResetBlock) k_reset_barrier(grid_sync_state* bar, control* ctl, const int* from, int* to,
-                                                                 int words) {
-  for (int i = threadIdx.x; i < words; i += blockDim.x) to[i] = from[i];
+
+/// Before each run: the barrier state and the control block zeroed, the control block's minima at
+/// INF (a kernel, not a memset or a copy, so the launch can live in a hipGraph and costs the
+/// stream no blit). One workgroup.
+DYNG_DEV void reset_run(grid_sync_state* bar, control* ctl) {
   unsigned long long* w = reinterpret_cast<unsigned long long*>(bar);
   for (unsigned int i = threadIdx.x; i < sizeof(grid_sync_state) / 8; i += blockDim.x) w[i] = 0;
   unsigned long long* c = reinterpret_cast<unsigned long long*>(ctl);
@@ -778,15 +792,46 @@ __global__ void __launch_bounds__(kResetBlock) k_reset_barrier(grid_sync_state* 
   }
 }
 
+/// The runs of a launch of several teams, a workgroup each.
+struct reset_teams {
+  grid_sync_state* bar[kTeams];
+  control* ctl[kTeams];
+};
+__global__ void __launch_bounds__(kResetBlock) k_reset_teams(reset_teams r) { reset_run(r.bar[blockIdx.x], r.ctl[blockIdx.x]); }
+
+/// The apply queued ahead of a run has ended when this starts: `words` 4-byte words of its control
+/// block go to pinned host memory here, in place of a copy of their own.
+__global__ void __launch_bounds__(kResetBlock) k_reset_barrier(grid_sync_state* bar, control* ctl, const int* from, int* to,
+                                                                 int words) {
+  for (int i = threadIdx.x; i < words; i += blockDim.x) to[i] = from[i];
+  reset_run(bar, ctl);
+}
+
 /// The builds of the persistent kernel. kPerSimd = 8 waves per SIMD keeps it at 64 VGPRs, so two
 /// 1024-thread workgroups fit a CU (solves from the sources); kPerSimd = 4 gives it 128, for grids
 /// of one workgroup per CU (repairs). kSolve: from the sources (compute, recompute), else the
 /// repair of a tree: two kernels, so that neither carries the other's registers.
+template <bool kSolve>
+DYNG_DEV void engine_run(const engine_params& p);
+
 template <int kPerSimd, bool kSolve>
 __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_params p) {
+  engine_run<kSolve>(p);
+}
+
+/// Repairs of several trees after one batch, each on its team of workgroups, all in flight at once. A
+/// repair waits for chains of memory round trips and barriers most of its time, not for processors, so
+/// a quarter of them serves it about as fast: four trees of RMAT-20 take the time of the slowest, 170 us,
+/// where one after another took 600.
+__global__ void __launch_bounds__(kBlock, 4) sssp_teams_kernel(engine_teams t) {
+  engine_run<false>(t.p[blockIdx.x / static_cast<unsigned int>(t.size)]);
+}
+
+template <bool kSolve>
+DYNG_DEV void engine_run(const engine_params& p) {
   // queued right behind an apply whose merges were held back: nothing to do (uniform)
   if (p.hold != nullptr && *p.hold != 0) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) p.ctl->held = 1;
+    if (run_block(p) == 0 && threadIdx.x == 0) p.ctl->held = 1;
     return;
   }
   __shared__ tile_shared L;
@@ -809,8 +854,8 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
   unsigned long long* const pull_edges = &counts[2];
   unsigned long long* const affected = &counts[3];
   unsigned long long* const local_pushes = &counts[4];
-  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int threads = gridDim.x * blockDim.x;
+  const int tid = run_block(p) * kBlock + static_cast<int>(threadIdx.x);
+  const int threads = p.blocks * kBlock;
   const int n = p.n;
   control* c = p.ctl;
   int generation = p.generation;
@@ -977,9 +1022,9 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
               },
               check, [&](bool, int) {}, publish);
         } else {
-          const int G = static_cast<int>(gridDim.x);
+          const int G = p.blocks;
           const int ts = min(kBlock, max(1, (front_count + G - 1) / G));
-          for (long long t0 = static_cast<long long>(blockIdx.x) * ts; t0 < front_count;
+          for (long long t0 = static_cast<long long>(run_block(p)) * ts; t0 < front_count;
                t0 += static_cast<long long>(G) * ts) {
             const int cnt = static_cast<int>(min(static_cast<long long>(ts), front_count - t0));
             if (static_cast<int>(threadIdx.x) < cnt) {
@@ -1110,7 +1155,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
         }
         // whole workgroups per step (t0 is uniform per workgroup), so each step can publish its
         // staged appends
-        for (long long t0 = static_cast<long long>(blockIdx.x) * kBlock; t0 < count; t0 += threads) {
+        for (long long t0 = static_cast<long long>(run_block(p)) * kBlock; t0 < count; t0 += threads) {
           const int i = static_cast<int>(t0) + static_cast<int>(threadIdx.x);
           bool keep = false, flagged = false;
           int32_t v = -1;
@@ -1319,13 +1364,13 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
       // kRelaxLocal generations: past kLocalGenerations the iterations stay global, one generation
       // each, so a run of millions of levels cannot carry the stamps past INT32_MAX).
       const bool local = !long_near && iterations >= kRelaxGlobal &&
-                         near_count <= static_cast<int>(gridDim.x) * kRelaxNarrow && generation < kLocalGenerations;
+                         near_count <= p.blocks * kRelaxNarrow && generation < kLocalGenerations;
       ++iterations;
       pushes += near_count;
       const int gen0 = generation + 1;
       // a global iteration claims with one generation; a local one reserves one per workgroup and
       // round
-      generation += local ? static_cast<int>(gridDim.x) * kRelaxLocal : 1;
+      generation += local ? p.blocks * kRelaxLocal : 1;
       int* next_count = &c->ring_near[step % 3];
       int* chunk_count = &c->ring_chunk[cstep % 3];
       if (tid == 0) {
@@ -1383,9 +1428,9 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
             },
             check, [&](bool, int) {}, [&] { stage_flush(S, next, next_count, far_list, far_counter); });
       } else {
-        const int G = static_cast<int>(gridDim.x);
+        const int G = p.blocks;
         const int ts = min(kBlock, max(1, (near_count + G - 1) / G));
-        for (long long t0 = static_cast<long long>(blockIdx.x) * ts; t0 < near_count;
+        for (long long t0 = static_cast<long long>(run_block(p)) * ts; t0 < near_count;
              t0 += static_cast<long long>(G) * ts) {
           const int cnt = static_cast<int>(min(static_cast<long long>(ts), near_count - t0));
           if (static_cast<int>(threadIdx.x) < cnt) {
@@ -1404,7 +1449,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
             const int items = W.count[q];  // uniform: LDS after a workgroup barrier
             if (items == 0) break;
             if (round > 0 && threadIdx.x == 0) *local_pushes += static_cast<unsigned long long>(items);
-            const int gen = gen0 + round * G + static_cast<int>(blockIdx.x);
+            const int gen = gen0 + round * G + run_block(p);
             const near_sink sink{&W, q ^ 1, p.ancestor, tag};
             spent += expand_tile(
                 p, L, long_rows, items,
@@ -1617,7 +1662,7 @@ __global__ void __launch_bounds__(kBlock, kPerSimd) sssp_fused_kernel(engine_par
   __shared__ int last;
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (threadIdx.x == 0) last = atomicAdd(&c->finished, 1u) == gridDim.x - 1 ? 1 : 0;
+  if (threadIdx.x == 0) last = atomicAdd(&c->finished, 1u) == static_cast<unsigned int>(p.blocks) - 1 ? 1 : 0;
   __syncthreads();
   if (last) {
     constexpr int kWords = sizeof(control) / 8;
@@ -1661,7 +1706,8 @@ struct dyng_hip_workspace {
   int grid_blocks = 0;
   int cu_count = 0;
   int occupancy = 0;         ///< workgroups per CU of the 64-VGPR build
-  int occupancy_narrow = 0;  ///< and of the 128-VGPR build
+  int occupancy_narrow = 0;
+  int occupancy_teams = 0;  ///< and of the 128-VGPR build
   hipEvent_t ev_start = nullptr;
   hipEvent_t ev_stop = nullptr;
   /// the launch as a hipGraph (control upload, barrier reset, events, the kernel, control
@@ -1742,6 +1788,8 @@ void ws_reserve(dyng_hip_workspace* ws, int64_t n, int64_t slots, hipStream_t s)
     DYNG_HIP_TRY(hipDeviceGetAttribute(&ws->cu_count, hipDeviceAttributeMultiprocessorCount, ws->device));
     ws->occupancy = resident_per_cu(false);
     ws->occupancy_narrow = resident_per_cu(true);
+    DYNG_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &ws->occupancy_teams, reinterpret_cast<const void*>(sssp_teams_kernel), kBlock, 0));
     if (ws->occupancy < 1) fail(DYNG_HIP_NOT_SUPPORTED, "dyng: sssp: the persistent kernel does not fit on a CU");
   }
 }
@@ -1946,7 +1994,9 @@ void read_counters(const control* hc, bool update, int bits, int blocks, dyng_hi
 
 }  // namespace
 
-engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStream_t s, apply_pending* ahead) {
+namespace {
+
+engine_pending engine_prepare(const dyng_hip_sssp_run* run, bool update, hipStream_t s, apply_pending* ahead, engine_params& p) {
   if (run == nullptr || run->graph == nullptr || run->workspace == nullptr) {
     fail(DYNG_HIP_INVALID_ARGUMENT, "dyng: sssp run: graph and workspace are required");
   }
@@ -1966,7 +2016,6 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
     pend.launched = false;
     return pend;
   }
-  engine_params p{};
   int64_t timeout_us = 0;
   engine_setup(run, update, p, timeout_us);
   p.hold = ahead != nullptr ? &g->ctl.p->hold : nullptr;
@@ -1990,21 +2039,38 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
   attach_scratch(p, engine_scratch{ws->packed.p, ws->stamp.p, ws->in_far.p, ws->flag.p, ws->ancestor.p, ws->cand.p,
                                    ws->frontier.p, ws->near_a.p, ws->near_b.p, ws->far_a.p, ws->far_b.p,
                                    ws->touched.p, ws->chunks.p, ws->chunk_cap, ws->ctl.p, ws->bar.p});
-  const int blocks = grid_blocks(run->tuning, ws->occupancy, ws->cu_count, p.from_scratch != 0);
-  const fused_fn kernel = fused_kernel(narrow_grid(blocks, ws->occupancy_narrow, ws->cu_count), p.from_scratch != 0);
   control* hc = ws->host_ctl.p;
   std::memset(hc, 0, sizeof(control));
   hc->min_frontier = packed_inf;
   hc->minimum[0] = packed_inf;
   hc->minimum[1] = packed_inf;
   p.publish = hc;
-  const int* from = ahead != nullptr ? reinterpret_cast<const int*>(g->ctl.p) : nullptr;
-  int* to = ahead != nullptr ? reinterpret_cast<int*>(g->host_ctl.p) : nullptr;
-  const int words = ahead != nullptr ? static_cast<int>(sizeof(apply_control) / sizeof(int)) : 0;
   if (ws->ev_start == nullptr) {
     DYNG_HIP_TRY(hipEventCreate(&ws->ev_start));
     DYNG_HIP_TRY(hipEventCreate(&ws->ev_stop));
   }
+  pend.bits = p.pk.bits;
+  pend.resident = p.resident;
+  pend.timeout_us = timeout_us;
+  pend.launched = true;
+  return pend;
+}
+
+}  // namespace
+
+engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStream_t s, apply_pending* ahead) {
+  engine_params p{};
+  engine_pending pend = engine_prepare(run, update, s, ahead, p);
+  if (!pend.launched) return pend;
+  pend.launched = false;  // until it is
+  const dyng_hip_graph* g = run->graph;
+  dyng_hip_workspace* ws = run->workspace;
+  const int blocks = grid_blocks(run->tuning, ws->occupancy, ws->cu_count, p.from_scratch != 0);
+  const fused_fn kernel = fused_kernel(narrow_grid(blocks, ws->occupancy_narrow, ws->cu_count), p.from_scratch != 0);
+  p.blocks = blocks;
+  const int* from = ahead != nullptr ? reinterpret_cast<const int*>(g->ctl.p) : nullptr;
+  int* to = ahead != nullptr ? reinterpret_cast<int*>(g->host_ctl.p) : nullptr;
+  const int words = ahead != nullptr ? static_cast<int>(sizeof(apply_control) / sizeof(int)) : 0;
   void* args[] = {&p};
   if (run->tuning.launch == DYNG_HIP_LAUNCH_GRAPH) {
     hipKernelNodeParams kp{};
@@ -2055,11 +2121,52 @@ engine_pending engine_launch(const dyng_hip_sssp_run* run, bool update, hipStrea
   if (ahead != nullptr) ahead->published = true;
   pend.launched = true;
   pend.started = ws->ev_start;
-  pend.bits = p.pk.bits;
   pend.blocks = blocks;
-  pend.resident = p.resident;
-  pend.timeout_us = timeout_us;
   return pend;
+}
+
+bool engine_joins(const dyng_hip_sssp_run* run) {
+  const dyng_hip_tuning& t = run->tuning;
+  return run->graph != nullptr && run->graph->n > 0 && t.launch != DYNG_HIP_LAUNCH_GRAPH && t.grid_blocks == 0 &&
+         t.blocks_per_cu == 0 && t.recompute == 0;
+}
+
+void engine_launch_teams(const dyng_hip_sssp_run* const* runs, int count, hipStream_t s, engine_pending* pends,
+                         std::exception_ptr* errors) {
+  engine_teams t{};
+  reset_teams r{};
+  int which[kTeams], teams = 0;
+  for (int i = 0; i < count; ++i) {
+    try {
+      pends[i] = engine_prepare(runs[i], true, s, nullptr, t.p[teams]);
+      pends[i].launched = false;  // until it is
+      r.bar[teams] = runs[i]->workspace->bar.p;
+      r.ctl[teams] = runs[i]->workspace->ctl.p;
+      which[teams++] = i;
+    } catch (...) {
+      errors[i] = std::current_exception();
+    }
+  }
+  if (teams == 0) return;
+  try {
+    const dyng_hip_workspace* ws = runs[which[0]]->workspace;
+    if (ws->occupancy_teams < 1) fail(DYNG_HIP_NOT_SUPPORTED, "dyng: sssp: the persistent kernel does not fit on a CU");
+    t.size = std::max(1, ws->cu_count / teams);  // one workgroup per processor, so that all are resident
+    for (int i = 0; i < teams; ++i) {
+      t.p[i].first_block = i * t.size;
+      t.p[i].blocks = t.size;
+    }
+    hipLaunchKernelGGL(k_reset_teams, dim3(static_cast<unsigned>(teams)), dim3(kResetBlock), 0, s, r);
+    hipLaunchKernelGGL(sssp_teams_kernel, dim3(static_cast<unsigned>(teams * t.size)), dim3(kBlock), 0, s, t);
+    DYNG_HIP_TRY(hipGetLastError());
+    for (int i = 0; i < teams; ++i) {
+      pends[which[i]].launched = true;
+      pends[which[i]].team = true;
+      pends[which[i]].blocks = t.size;
+    }
+  } catch (...) {
+    for (int i = 0; i < teams; ++i) errors[which[i]] = std::current_exception();
+  }
 }
 
 void engine_finish(engine_pending& pend, dyng_hip_counters* out) {
@@ -2086,7 +2193,11 @@ void engine_finish(engine_pending& pend, dyng_hip_counters* out) {
     return;
   }
   float kernel_ms = 0.0f;
-  DYNG_HIP_TRY(hipEventElapsedTime(&kernel_ms, ws->ev_start, ws->ev_stop));
+  if (pend.team) {  // a run of several in one launch: its own clock, from its first to its last stamp
+    kernel_ms = hc->t_phase[7] >= hc->t_phase[0] ? static_cast<float>((hc->t_phase[7] - hc->t_phase[0]) * 1e-5) : 0.0f;
+  } else {
+    DYNG_HIP_TRY(hipEventElapsedTime(&kernel_ms, ws->ev_start, ws->ev_stop));
+  }
   if (hc->overflow != 0 || hc->error_bits != 0) {
     // a run that stopped early can leave flags, far marks and stamps of any later generation
     // behind in the shared workspace: clear them before any other run uses it
@@ -2290,6 +2401,7 @@ void run_engine_noalloc(const dyng_hip_sssp_run* run, hipStream_t s, dyng_hip_co
   hipLaunchKernelGGL(k_reset_barrier, dim3(1), dim3(kResetBlock), 0, s, p.bar, p.ctl, static_cast<const int*>(nullptr),
                      static_cast<int*>(nullptr), 0);
   const fused_fn kernel = fused_kernel(narrow_grid(blocks, st.occupancy_narrow, st.cu_count), p.from_scratch != 0);
+  p.blocks = blocks;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, s, p);
   DYNG_HIP_TRY(hipGetLastError());
   control* hc = &st.host_ctl;
