@@ -1,6 +1,6 @@
 """Several results repaired side by side in one launch: fewer results than teams, as many, and more (a
-second launch), different sources and weight columns, with and without parallel edges, and a batch past
-the size up to which they share a launch. Every tree and count equals the oracle's."""
+second launch), different sources and weight columns, with and without parallel edges, small and large
+batches. Every tree and count equals the oracle's."""
 
 from __future__ import annotations
 
