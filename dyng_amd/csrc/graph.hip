@@ -1491,7 +1491,8 @@ struct front_params {
   int64_t n_after;
   int vbits, ebits, lb, K;
   int groups;
-  u64* entries;  ///< kGroupCap per group: out-row groups, then in-row groups
+  int room;      ///< operations a group has room for
+  u64* entries;  ///< `room` per group: out-row groups, then in-row groups
   int* counts;
   int32_t *e_del_src, *e_del_dst, *e_ins_src, *e_ins_dst;
   uint8_t* e_inc;
@@ -1574,7 +1575,7 @@ __global__ void __launch_bounds__(1024) k_group_front(front_params f) {
     if (hist[b] > 0) {
       const int mine = hist[b];
       hist[b] = atomicAdd(&f.counts[b], mine);
-      if (hist[b] + mine > kGroupCap) atomicOr(&f.ctl->miss, kMissFull);
+      if (hist[b] + mine > f.room) atomicOr(&f.ctl->miss, kMissFull);
     }
   }
   __syncthreads();
@@ -1589,12 +1590,12 @@ __global__ void __launch_bounds__(1024) k_group_front(front_params f) {
     const u64 below = (u64{1} << low) - 1;
     const int gu = static_cast<int>(hu >> low), gv = f.groups + static_cast<int>(hv >> low);
     const int at_u = hist[gu] + rank[0][j], at_v = hist[gv] + rank[1][j];
-    if (at_u < kGroupCap) {
-      f.entries[int64_t{gu} * kGroupCap + at_u] =
+    if (at_u < f.room) {
+      f.entries[int64_t{gu} * f.room + at_u] =
           ((((hu & below) << f.vbits) | static_cast<u64>(o.v)) << f.ebits) | static_cast<u64>(e);
     }
-    if (at_v < kGroupCap) {
-      f.entries[int64_t{gv} * kGroupCap + at_v] =
+    if (at_v < f.room) {
+      f.entries[int64_t{gv} * f.room + at_v] =
           ((((hv & below) << f.vbits) | static_cast<u64>(o.u)) << f.ebits) | static_cast<u64>(e);
     }
   }
@@ -1646,7 +1647,7 @@ DYNG_DEV void group_sort(const u64* src, int count, u64* S, Place place) {
 struct group_params {
   const u64* entries;
   const int* counts;
-  int groups, vbits, ebits, lb;
+  int groups, vbits, ebits, lb, room;
   uint32_t inverse;  ///< of kGroupHash modulo 2^32
   u64* keys;         ///< sorted operations: out-rows [0, P), in-rows [P, 2P)
   uint32_t* vals;
@@ -1684,7 +1685,7 @@ __global__ void __launch_bounds__(kGroupBlock, 4) k_group_pairs(group_params g) 
   before = wave_scan(before);
   if (lane() == 63) part[tid / 64] = before;
   const bool lds = count < kGroupLds;
-  const u64* src = g.entries + int64_t{(in ? g.groups : 0) + q} * kGroupCap;
+  const u64* src = g.entries + int64_t{(in ? g.groups : 0) + q} * g.room;
   const int low = g.vbits - g.lb;
   const u64 vmask = (u64{1} << g.vbits) - 1, emask = (u64{1} << g.ebits) - 1;
   int64_t at = q;
@@ -2982,6 +2983,12 @@ int group_bits(int64_t N, int vbits) {
   return lb;
 }
 
+/// Room per group: what one takes at most, or half of it where that is still eight times its share and
+/// a graph's first batch would pay for allocating the rest (100,000 operations: 34 MB, 0.6 ms).
+int group_room(int64_t N, int lb) {
+  return lb <= kGroupBitsFew || N > (int64_t{1} << 18) ? kGroupCap : kGroupCap / 2;
+}
+
 int op_bits(int64_t N) {
   int b = 1;
   while ((int64_t{1} << b) < N) ++b;
@@ -3175,6 +3182,7 @@ void rows_grouped(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, i
   f.lb = lb;
   f.K = g->K;
   f.groups = groups;
+  f.room = group_room(N, lb);
   f.entries = g->group_entries.p;
   f.counts = g->group_counts.p;
   f.e_del_src = g->del_src.p;
@@ -3198,6 +3206,7 @@ void rows_grouped(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, i
   gp.entries = g->group_entries.p;
   gp.counts = g->group_counts.p;
   gp.groups = groups;
+  gp.room = f.room;
   gp.vbits = vbits;
   gp.ebits = f.ebits;
   gp.lb = lb;
@@ -3286,7 +3295,7 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
   if (g->group_pause > 0) g->group_pause -= 1;
   const int64_t P = ap.P = grouped ? N + (int64_t{1} << lb) : N;
   if (grouped) {
-    g->group_entries.reserve((size_t{2} << lb) * kGroupCap);
+    g->group_entries.reserve((size_t{2} << lb) * group_room(N, lb));
     g->group_counts.reserve(size_t{2} << lb);
   }
   reserve_ops(g, P);

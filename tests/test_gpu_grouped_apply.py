@@ -73,7 +73,7 @@ def test_more_operations_on_a_row_than_a_group_takes(dg, directed, parallel):
     op, og, hg, rng = _graph(dg, 6000, 20000, 1, directed, parallel, 0, 77)
     ot, _ = oracle.compute(og, 0)
     r = dg.sssp.compute(hg, 0)
-    for b, on_hub in enumerate([4096, 4097, 300, 5000, 4000]):
+    for b, on_hub in enumerate([4096, 4097, 300, 5000, 2000]):
         print(f"[groups] {on_hub} operations on row 7", flush=True)
         hub = rng.permutation(np.arange(8, og.n))[:on_hub]
         other = rng.integers(8, og.n, 200)
