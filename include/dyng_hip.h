@@ -229,7 +229,8 @@ typedef struct dyng_hip_counters {
   double pull_ms;         /* of which the pull pass */
   double relax_ms;        /* device time of the near-far propagation (the relax iterations) */
   int64_t blocks;         /* workgroups of the persistent launch */
-  double kernel_ms;       /* the persistent kernel's duration (HIP events on its stream) */
+  double kernel_ms;       /* the persistent kernel's duration (HIP events on its stream; of several runs
+                             in one launch, the run's own clock from its first to its last stamp) */
   double pack_ms;         /* Step 1 parts (s_memrealtime): packing the old tree and the roots, */
   double jump_ms;         /* the pointer-jumping rounds, */
   double unpack_ms;       /* and the final unpack */
