@@ -1453,7 +1453,7 @@ constexpr int kGroupBitsSome = 9, kGroupOpsSome = 128;
 constexpr int kGroupOps = 256;
 constexpr int64_t kGroupMost = int64_t{1} << 22;  ///< operations of a batch (1024 per group)
 constexpr int kGroupCap = 4096;   ///< most a group takes; one row with more operations sends the batch to the sort
-constexpr int kGroupLds = 1024;   ///< a group with fewer operations keeps them in LDS: 8 KB sorted segments, 28 KB of the rest
+constexpr int kGroupLds = 1024;   ///< a group with fewer operations keeps them in LDS (8 KB of segments, 24 KB of the rest)
 constexpr int kGroupPause = 15;   ///< batches sorted device-wide after one that a group could not take
 constexpr int kGroupBits = 12;    ///< at most 2^12 groups per direction
 constexpr uint32_t kGroupHash = 0x9E3779B1u;
@@ -2889,8 +2889,9 @@ void merges_exact(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s, dyng_h
 }
 
 /// The merges of a small batch queued behind its plan, with no read-back in between: the device
-/// checks that the arenas take what the plan asks (merges_fit) and holds the merges back otherwise; the grids are sized for the batch (every touched row is one of its at most N + 1 rows
-/// per store) and the merges loop over the rows the plan listed.
+/// checks that the arenas take what the plan asks (merges_fit) and holds the merges back otherwise;
+/// the grids are sized for the batch (every touched row is one of its at most N + 1 rows per store)
+/// and the merges loop over the rows the plan listed.
 void merges_queued(dyng_hip_graph* g, int64_t N, int vbits, hipStream_t s) {
   int rows[kModes];
   std::fill(rows, rows + kModes, static_cast<int>(N + 1));
