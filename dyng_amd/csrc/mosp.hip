@@ -10,6 +10,7 @@
 // does not depend on), no in-rows (a solve from the source never pulls), no slack. Its buffers live in a per-device cache
 // and are reused by the next call (they grow, never shrink, until the process ends).
 #include "internal.hpp"
+#include "path_costs.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -202,98 +203,13 @@ __global__ void k_tree_edge_costs(edge_rows out, edge_rows in, bool by_in_row, i
   }
 }
 
-/// What the path doubling tells the host (pinned memory).
-struct path_report {
-  int missing;  ///< the lowest vertex whose tree edge is not in the graph (INT32_MAX: none)
-  int ended;    ///< 1: every round ran
-};
-
-struct path_params {
-  int64_t* acc[2];   ///< sums of the even and odd rounds; acc[0] is the caller's
-  int32_t* jump[2];
-  int32_t n;
-  int columns;
-  grid_sync_state* bar;
-  unsigned long long limit;  ///< ticks a grid barrier waits at most
-  unsigned int rounds;       ///< at most: log2(n) rounded up, and one
-  const int* missing;
-  path_report* report;
-};
-
-constexpr int kPathBlock = 1024;
-constexpr int kPathSlots = 4;  ///< vertices of a thread in flight
-
-/// Clear the grid barrier and the missing vertex.
-__global__ void k_path_begin(grid_sync_state* bar, int* missing) {
+/// Clear the grid barrier, the missing vertex and the count of finished workgroups.
+__global__ void k_path_begin(grid_sync_state* bar, int* missing, int* finished) {
   u64* w = reinterpret_cast<u64*>(bar);
   for (unsigned int i = threadIdx.x; i < sizeof(grid_sync_state) / 8; i += blockDim.x) w[i] = 0;
-  if (threadIdx.x == 0) *missing = INT32_MAX;
-}
-
-/// Path doubling: in each round every vertex adds its ancestor's sum and jumps to the ancestor's
-/// ancestor, until none has one. A vertex's jump is -1 in the round after its sum became final (that
-/// round copies the sum to the other buffer) and -2 from then on (both buffers hold it: a round only
-/// passes the -2 on). One launch of resident workgroups with a grid barrier per round, at which each
-/// tells how many of its vertices go on: a launch per round had to queue log2(n) + 1 of them, 21 for
-/// 2^20 vertices whose trees are 5 rounds deep, and each empty one took 7 us with its gap. The rounds
-/// read what other workgroups wrote, so those accesses are at device scope.
-__global__ void __launch_bounds__(kPathBlock) k_path_costs(path_params p) {
-  const int threads = static_cast<int>(gridDim.x) * kPathBlock;
-  const int tid = static_cast<int>(blockIdx.x) * kPathBlock + static_cast<int>(threadIdx.x);
-  const grid_place at{blockIdx.x, gridDim.x};
-  int cur = 0;
-  for (unsigned int round = 1; round <= p.rounds; ++round) {
-    const int64_t* acc_in = p.acc[cur];
-    const int32_t* jump_in = p.jump[cur];
-    int64_t* acc_out = p.acc[cur ^ 1];
-    int32_t* jump_out = p.jump[cur ^ 1];
-    bool more = false;  // some vertex of this thread still has an ancestor
-    for (int64_t v0 = tid; v0 < p.n; v0 += int64_t{kPathSlots} * threads) {
-      int32_t j[kPathSlots], up[kPathSlots];
-#pragma unroll
-      for (int q = 0; q < kPathSlots; ++q) {
-        const int64_t v = v0 + int64_t{q} * threads;
-        j[q] = v < p.n ? ld(&jump_in[v]) : -2;
-      }
-#pragma unroll
-      for (int q = 0; q < kPathSlots; ++q) up[q] = j[q] >= 0 ? ld(&jump_in[j[q]]) : -2;
-      for (int c = 0; c < p.columns; ++c) {
-        int64_t a[kPathSlots], b[kPathSlots];
-#pragma unroll
-        for (int q = 0; q < kPathSlots; ++q) {
-          const int64_t v = v0 + int64_t{q} * threads;
-          a[q] = j[q] != -2 ? ld(&acc_in[v * p.columns + c]) : 0;
-          b[q] = j[q] >= 0 ? ld(&acc_in[static_cast<int64_t>(j[q]) * p.columns + c]) : 0;
-        }
-#pragma unroll
-        for (int q = 0; q < kPathSlots; ++q) {
-          const int64_t v = v0 + int64_t{q} * threads;
-          if (j[q] != -2) st(&acc_out[v * p.columns + c], a[q] + b[q]);
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < kPathSlots; ++q) {
-        const int64_t v = v0 + int64_t{q} * threads;
-        const int32_t next = j[q] < 0 ? -2 : up[q] < 0 ? -1 : up[q];
-        if (v < p.n) st(&jump_out[v], next);
-        more = more || next >= 0;
-      }
-    }
-    cur ^= 1;
-    const unsigned int mine = static_cast<unsigned int>(__syncthreads_count(more ? 1 : 0));
-    const grid_found found = grid_barrier<false>(p.bar, at, round, p.limit, [&] { grid_arrive(p.bar, at, round, mine); });
-    if (!found.ok) return;  // uniform: the host finds `ended` clear
-    if (found.published == 0) break;
-  }
-  if (cur == 1) {
-    // an odd number of rounds: the sums are in the other buffer, each vertex's written by this thread
-    for (int64_t v = tid; v < p.n; v += threads) {
-      for (int c = 0; c < p.columns; ++c) p.acc[0][v * p.columns + c] = ld(&p.acc[1][v * p.columns + c]);
-    }
-  }
-  if (tid == 0) {
-    p.report->missing = *p.missing;
-    p.report->ended = 1;
+  if (threadIdx.x == 0) {
+    *missing = INT32_MAX;
+    *finished = 0;
   }
 }
 
@@ -537,7 +453,7 @@ struct combined_cache {
   dbuf<unsigned long long> totals;
   dbuf<int64_t> acc;
   dbuf<int32_t> jump_a, jump_b;
-  dbuf<int> missing;  ///< the path costs' lowest vertex without its tree edge
+  dbuf<int> path_state;  ///< the path costs' lowest vertex without its tree edge, and the finished workgroups
   dbuf<grid_sync_state> bar;
   pinned<path_report> report;
   int cu_count = 0;
@@ -682,14 +598,15 @@ void mosp_path_costs(const dyng_hip_graph* g, const int32_t* parents, int64_t n,
   cc.acc.reserve(static_cast<size_t>(n) * columns);
   cc.jump_a.reserve(n);
   cc.jump_b.reserve(n);
-  cc.missing.reserve(1);
+  cc.path_state.reserve(2);
   cc.bar.reserve(1);
+  int* missing = cc.path_state.p;
   const edge_rows out{g->out.meta.p, g->out.base.p, g->out.nbr.p, g->out.w.p, g->out.slot_cap};
   const edge_rows in{g->in.meta.p, g->in.base.p, g->in.nbr.p, g->in.w.p, g->in.slot_cap};
   const bool by_in_row = g->props.allow_parallel == 0;
-  hipLaunchKernelGGL(k_path_begin, dim3(1), dim3(64), 0, s, cc.bar.p, cc.missing.p);
+  hipLaunchKernelGGL(k_path_begin, dim3(1), dim3(64), 0, s, cc.bar.p, missing, missing + 1);
   hipLaunchKernelGGL(k_tree_edge_costs, dim3(grid(n, 256)), dim3(256), 0, s, out, in, by_in_row, columns, parents,
-                     static_cast<int32_t>(n), source, costs, cc.jump_a.p, cc.missing.p);
+                     static_cast<int32_t>(n), source, costs, cc.jump_a.p, missing);
   DYNG_HIP_TRY(hipGetLastError());
   if (cc.cu_count == 0) {
     DYNG_HIP_TRY(hipDeviceGetAttribute(&cc.cu_count, hipDeviceAttributeMultiprocessorCount, g->device));
@@ -701,7 +618,7 @@ void mosp_path_costs(const dyng_hip_graph* g, const int32_t* parents, int64_t n,
   unsigned int rounds = 1;
   while ((int64_t{1} << rounds) < n) ++rounds;
   const path_params pp{{costs, cc.acc.p}, {cc.jump_a.p, cc.jump_b.p}, static_cast<int32_t>(n), columns, cc.bar.p,
-                       static_cast<unsigned long long>(kTimeoutUs) * 100ULL, rounds + 1, cc.missing.p, report};
+                       static_cast<unsigned long long>(kTimeoutUs) * 100ULL, rounds + 1, missing, missing + 1, report};
   // one workgroup per processor at most, so that all are resident
   const unsigned blocks = std::min(grid(n, kPathBlock), static_cast<unsigned>(cc.cu_count));
   hipLaunchKernelGGL(k_path_costs, dim3(blocks), dim3(kPathBlock), 0, s, pp);
