@@ -604,30 +604,29 @@ void mosp_path_costs(const dyng_hip_graph* g, const int32_t* parents, int64_t n,
   const edge_rows out{g->out.meta.p, g->out.base.p, g->out.nbr.p, g->out.w.p, g->out.slot_cap};
   const edge_rows in{g->in.meta.p, g->in.base.p, g->in.nbr.p, g->in.w.p, g->in.slot_cap};
   const bool by_in_row = g->props.allow_parallel == 0;
-  hipLaunchKernelGGL(k_path_begin, dim3(1), dim3(64), 0, s, cc.bar.p, missing, missing + 1);
-  hipLaunchKernelGGL(k_tree_edge_costs, dim3(grid(n, 256)), dim3(256), 0, s, out, in, by_in_row, columns, parents,
-                     static_cast<int32_t>(n), source, costs, cc.jump_a.p, missing);
-  DYNG_HIP_TRY(hipGetLastError());
   if (cc.cu_count == 0) {
     DYNG_HIP_TRY(hipDeviceGetAttribute(&cc.cu_count, hipDeviceAttributeMultiprocessorCount, g->device));
   }
   path_report* report = cc.report.p;
-  report->missing = INT32_MAX;
-  report->ended = 0;
   constexpr int64_t kTimeoutUs = 4000000;  // the engine's default for its barrier
   unsigned int rounds = 1;
   while ((int64_t{1} << rounds) < n) ++rounds;
   const path_params pp{{costs, cc.acc.p}, {cc.jump_a.p, cc.jump_b.p}, static_cast<int32_t>(n), columns, cc.bar.p,
                        static_cast<unsigned long long>(kTimeoutUs) * 100ULL, rounds + 1, missing, missing + 1, report};
   // one workgroup per processor at most, so that all are resident
-  const unsigned blocks = std::min(grid(n, kPathBlock), static_cast<unsigned>(cc.cu_count));
-  hipLaunchKernelGGL(k_path_costs, dim3(blocks), dim3(kPathBlock), 0, s, pp);
-  DYNG_HIP_TRY(hipGetLastError());
-  DYNG_HIP_TRY(hipStreamSynchronize(s));
-  if (report->ended == 0) {
-    fail(DYNG_HIP_RUNTIME_ERROR, "mosp: a grid barrier wait of the path costs ran past " + std::to_string(kTimeoutUs) +
-                                     " us");
-  }
+  const unsigned all = std::min(grid(n, kPathBlock), static_cast<unsigned>(cc.cu_count));
+  const bool ended = run_path_costs(all, [&](unsigned blocks) {
+    report->missing = INT32_MAX;
+    report->ended = 0;
+    hipLaunchKernelGGL(k_path_begin, dim3(1), dim3(64), 0, s, cc.bar.p, missing, missing + 1);
+    hipLaunchKernelGGL(k_tree_edge_costs, dim3(grid(n, 256)), dim3(256), 0, s, out, in, by_in_row, columns, parents,
+                       static_cast<int32_t>(n), source, costs, cc.jump_a.p, missing);
+    hipLaunchKernelGGL(k_path_costs, dim3(blocks), dim3(kPathBlock), 0, s, pp);
+    DYNG_HIP_TRY(hipGetLastError());
+    DYNG_HIP_TRY(hipStreamSynchronize(s));
+    return report->ended != 0;
+  });
+  if (!ended) fail(DYNG_HIP_RUNTIME_ERROR, "mosp: the path costs did not end");
   const int host_missing = report->missing;
   if (host_missing != INT32_MAX) {
     fail(DYNG_HIP_INVALID_ARGUMENT, "mosp: the MOSP tree edge (" + std::to_string(host_missing) +

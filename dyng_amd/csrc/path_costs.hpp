@@ -98,4 +98,13 @@ __global__ void __launch_bounds__(kPathBlock) k_path_costs(path_params p) {
   }
 }
 
+/// The doubling on `blocks` workgroups; if a wait gave up, again on one. Other work can hold enough of the
+/// device for the whole of the limit that the workgroups are not all resident; one workgroup waits for
+/// nobody, so the costs come late then and never not at all. `attempt(blocks)` starts from the tree
+/// edges' costs and says whether every workgroup ended.
+template <class Attempt>
+bool run_path_costs(unsigned int blocks, Attempt attempt) {
+  return attempt(blocks) || (blocks > 1 && attempt(1u));
+}
+
 }  // namespace dyng_hip

@@ -137,6 +137,18 @@ int main() {
         return 1;
       }
       ++checks;
+      // and the costs are there all the same, from a launch that waits for nobody
+      std::vector<unsigned int> tried;
+      const bool done = run_path_costs(blocks, [&](unsigned int on) {
+        tried.push_back(on);
+        quitter = on > 1 ? static_cast<int>(on) - 1 : -1;
+        return launch(t, on, on > 1 ? 1000 : 0, costs);
+      });
+      if (!done || tried != std::vector<unsigned int>{blocks, 1u} || costs != t.want) {
+        std::printf("chain of %d on %u workgroups, one gave up: no costs\n", n, blocks);
+        return 1;
+      }
+      ++checks;
     }
   }
   std::printf("ok %d\n", checks);
