@@ -2,6 +2,7 @@
 // result::from_arrays (cpp/src/algorithms/sssp/sssp.cpp) around the device graph and the engine,
 // exported as the API layer of include/dyng_hip.h (the calls python/bindings/sssp.cpp binds).
 #include "internal.hpp"
+#include "team_rule.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -115,6 +116,8 @@ struct dyng_hip_result {
   /// the token of the engine run that left this tree (its packed words may still be in the
   /// device's workspace); 0 for a tree the engine did not leave, or that changed since
   uint64_t tree_token = 0;
+  /// edges that the last repair scanned (0: none yet), by which repairs side by side are divided
+  int64_t repair_edges = 0;
   /// the work counters of the engine run that left this tree (compute, update or repair)
   dyng_hip_counters last{};
 };
@@ -338,6 +341,7 @@ void repair_core(dyng_hip_graph* g, dyng_hip_result* r, int64_t delta, int64_t m
       engine_finish(pend, &c);
     }
     r->tree_token = c.tree_token;
+    if (run.tuning.recompute == 0) r->repair_edges = c.pull_edges + c.relax_edges;
     r->last = c;
     engine_ms = c.kernel_ms;
   } catch (...) {
@@ -603,10 +607,11 @@ extern "C" int dyng_hip_api_update_each(dyng_hip_graph* g, const dyng_hip_batch*
     } else {
       // several results: result i runs on workspace slot i % kWorkspaceSlots, kWorkspaceSlots of them
       // side by side in one launch (four trees of RMAT-22, side by side against one after another: 0.22 and
-      // 0.50 ms with 1,000 operations, 0.83 and 1.47 with 65,000, 3.07 and 4.43 with 500,000). If one of them
-      // has a tuning that asks for a launch of its own, all are queued one after another on the caller's
-      // stream, kWorkspaceSlots runs ahead of the host (never two launches at once: their workgroups
-      // wait for each other at grid barriers and must all be resident)
+      // 0.50 ms with 1,000 operations, 0.83 and 1.47 with 65,000, 3.07 and 4.43 with 500,000), except those
+      // that are much heavier than the ones beside them (runs_alone). If one of them has a tuning that asks
+      // for a launch of its own, all are queued one after another on the caller's stream, kWorkspaceSlots
+      // runs ahead of the host (never two launches at once: their workgroups wait for each other at grid
+      // barriers and must all be resident)
       for (int64_t i = 0; i < count; ++i) grow_result(results[i], g->n, s);
       std::lock_guard<std::mutex> lk(pool().lock);
       std::vector<engine_pending> pend(static_cast<size_t>(count));
@@ -624,6 +629,7 @@ extern "C" int dyng_hip_api_update_each(dyng_hip_graph* g, const dyng_hip_batch*
           return;
         }
         r->tree_token = c.tree_token;
+        if (r->tuning.recompute == 0) r->repair_edges = c.pull_edges + c.relax_edges;
         r->version = g->version;
         r->trusted = true;
         r->engine_tree = true;
@@ -671,13 +677,26 @@ extern "C" int dyng_hip_api_update_each(dyng_hip_graph* g, const dyng_hip_batch*
             fail_result(j, std::current_exception());
           }
         }
-        if (m > 1) {
-          engine_launch_teams(group, m, s, queued, errors);
-        } else if (m == 1) {
+        int64_t edges[kWorkspaceSlots];
+        int order[kWorkspaceSlots];
+        for (int q = 0; q < m; ++q) edges[q] = results[of[q]]->repair_edges;
+        const int alone = runs_alone(edges, m, order);
+        for (int q = 0; q < alone; ++q) {
           try {
-            queued[0] = engine_launch(group[0], true, s);
+            queued[order[q]] = engine_launch(group[order[q]], true, s);
           } catch (...) {
-            errors[0] = std::current_exception();
+            errors[order[q]] = std::current_exception();
+          }
+        }
+        if (alone < m) {
+          const dyng_hip_sssp_run* sharing[kWorkspaceSlots];
+          engine_pending shared[kWorkspaceSlots];
+          std::exception_ptr failed[kWorkspaceSlots];
+          for (int q = alone; q < m; ++q) sharing[q - alone] = group[order[q]];
+          engine_launch_teams(sharing, m - alone, s, shared, failed);
+          for (int q = alone; q < m; ++q) {
+            queued[order[q]] = shared[q - alone];
+            errors[order[q]] = failed[q - alone];
           }
         }
         for (int q = 0; q < m; ++q) {
@@ -940,6 +959,7 @@ extern "C" int dyng_hip_result_clone(const dyng_hip_result* r, void* stream, dyn
     c->trusted = r->trusted;
     c->engine_tree = r->engine_tree;
     c->tuning = r->tuning;
+    c->repair_edges = r->repair_edges;
     c->n = r->n;
     c->distances.reserve(r->n);
     c->parents.reserve(r->n);
