@@ -42,6 +42,10 @@
 
 #include <algorithm>
 #include <cmath>
+#include <map>
+#include <memory>
+#include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace dyng_hip {
@@ -2773,19 +2777,19 @@ merge_params merge_setup(dyng_hip_graph* g, bool outs, int64_t N, int vbits) {
   mp.w = rs.w.p;
   mp.slot_cap = rs.slot_cap;
   mp.K = g->K;
-  mp.keys = outs ? g->keys_b.p : g->keys_b.p + N;
+  mp.keys = outs ? g->ops.keys_b : g->ops.keys_b + N;
   mp.N = N;
   mp.vbits = vbits;
-  mp.pend_alive = outs ? g->pend_alive.p : g->ipend_alive.p;
-  mp.pend_prefix = outs ? g->pend_prefix.p : g->ipend_prefix.p;
-  mp.kill_prefix = outs ? g->kill_prefix.p : g->ikill_prefix.p;
-  mp.pend_w = outs ? g->pend_w.p : g->ipend_w.p;
-  mp.touched = outs ? g->touched_out.p : g->touched_in.p;
+  mp.pend_alive = outs ? g->ops.pend_alive : g->ops.ipend_alive;
+  mp.pend_prefix = outs ? g->ops.pend_prefix : g->ops.ipend_prefix;
+  mp.kill_prefix = outs ? g->ops.kill_prefix : g->ops.ikill_prefix;
+  mp.pend_w = outs ? g->ops.pend_w : g->ops.ipend_w;
+  mp.touched = outs ? g->ops.touched_out : g->ops.touched_in;
   mp.touched_count = outs ? &dc->touched_out : &dc->touched_in;
   mp.row_a = outs ? g->row_a_out.p : g->row_a_in.p;
   mp.row_b = outs ? g->row_b_out.p : g->row_b_in.p;
-  mp.lane_rows = g->lane_rows.p + (outs ? 0 : 2 * (N + 1));
-  mp.lists = g->merge_lists.p + (outs ? 0 : kModes * (N + 1));
+  mp.lane_rows = g->ops.lane_rows + (outs ? 0 : 2 * (N + 1));
+  mp.lists = g->ops.merge_lists + (outs ? 0 : kModes * (N + 1));
   mp.list_count = outs ? dc->modes_out : dc->modes_in;
   mp.stage_nbr = g->stage_nbr.p;
   mp.stage_w = g->stage_w.p;
@@ -2945,32 +2949,82 @@ void begin_apply(dyng_hip_graph* g, const batch_scan& sc, int num_counts, hipStr
   b.tail_out = g->out.tail;
   b.tail_in = g->in.tail;
   for (int k = 0; k < g->K; ++k) b.col_max[k] = std::max<int64_t>(g->wmax[k], sc.wmax[k]);
-  b.counts = g->group_counts.p;
+  b.counts = g->ops.group_counts;
   b.num_counts = num_counts;
   hipLaunchKernelGGL(k_begin, dim3(1), dim3(1024), 0, s, g->ctl.p, b);
   DYNG_HIP_TRY(hipGetLastError());
 }
 
-/// Per-operation scratch for P places in sorted order.
-void reserve_ops(dyng_hip_graph* g, int64_t P) {
+scratch_pool& apply_scratch(int device) {
+  struct pools {
+    std::mutex lock;
+    std::map<int, std::unique_ptr<scratch_pool>> of;
+  };
+  static pools* all = new pools();  // lives until the process ends
+  std::lock_guard<std::mutex> hold(all->lock);
+  std::unique_ptr<scratch_pool>& pool = all->of[device];
+  if (!pool) {
+    pool = std::make_unique<scratch_pool>(
+        [](size_t bytes) -> void* {
+          void* p = nullptr;
+          if (hipMalloc(&p, bytes) == hipSuccess) return p;
+          (void)hipGetLastError();
+          return nullptr;
+        },
+        [](void* p) { (void)hipFree(p); });
+  }
+  return *pool;
+}
+
+/// Take the scratch of P places in sorted order, and of `groups` groups of both directions.
+void take_ops(dyng_hip_graph* g, int64_t P, size_t groups) {
   const int K = g->K;
-  g->keys_b.reserve(2 * P);  // out-row keys, then in-row keys
-  g->vals_b.reserve(2 * P);
-  g->pend_alive.reserve(P + 1);
-  g->kill.reserve(P + 1);
-  g->pend_prefix.reserve(P + 1);
-  g->kill_prefix.reserve(P + 1);
-  g->pend_w.reserve(P * K);
-  g->iop_type.reserve(P);
-  g->iop_wold.reserve(P * K);
-  g->iop_wnew.reserve(P * K);
-  g->ipend_alive.reserve(P + 1);
-  g->ikill.reserve(P + 1);
-  g->ipend_prefix.reserve(P + 1);
-  g->ikill_prefix.reserve(P + 1);
-  g->ipend_w.reserve(P * K);
-  g->merge_lists.reserve(2 * kModes * (P + 1));
-  g->lane_rows.reserve(4 * (P + 1));
+  op_scratch& o = g->ops;
+  // the arrays from `base` on, each from a 256-byte boundary; returns their size
+  auto lay_out = [&](unsigned char* base) {
+    size_t at = 0;
+    auto place = [&](auto*& p, size_t count) {
+      p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(base + at);
+      at += (count * sizeof(*p) + 255) / 256 * 256;
+    };
+    const size_t n = static_cast<size_t>(P);
+    place(o.keys_b, 2 * n);  // out-row keys, then in-row keys
+    place(o.vals_b, 2 * n);
+    place(o.group_entries, groups * kGroupCap);
+    place(o.group_counts, groups);
+    for (int32_t** p : {&o.pend_alive, &o.kill, &o.pend_prefix, &o.kill_prefix, &o.ipend_alive, &o.ikill,
+                        &o.ipend_prefix, &o.ikill_prefix}) {
+      place(*p, n + 1);
+    }
+    for (int32_t** p : {&o.pend_w, &o.ipend_w, &o.iop_wold, &o.iop_wnew}) place(*p, n * K);
+    place(o.iop_type, n);
+    place(o.touched_out, n + 1);
+    place(o.touched_in, n + 1);
+    place(o.lane_rows, 4 * (n + 1));
+    place(o.merge_lists, 2 * kModes * (n + 1));
+    return at;
+  };
+  const size_t bytes = lay_out(nullptr);
+  if (!g->pools_scratch) {
+    apply_scratch(g->device).join();
+    g->pools_scratch = true;
+  }
+  // a block that a failed apply left with the graph is used again: its work is on the graph's stream
+  if (o.block.bytes < bytes) {
+    if (o.block.p != nullptr) DYNG_HIP_TRY(hipFree(o.block.p));
+    o.block = {};
+    o.block = apply_scratch(g->device).take(bytes);
+    if (o.block.p == nullptr) {
+      throw status_error(DYNG_HIP_OUT_OF_MEMORY, "dyng: out of device memory (" + std::to_string(bytes) + " bytes)");
+    }
+  }
+  lay_out(static_cast<unsigned char*>(o.block.p));
+}
+
+/// The apply's work has ended: its scratch goes back.
+void give_ops(dyng_hip_graph* g) {
+  apply_scratch(g->device).give(g->ops.block);
+  g->ops = op_scratch{};
 }
 
 /// Groups per direction for N operations, as a power of two's exponent.
@@ -2982,12 +3036,6 @@ int group_bits(int64_t N, int vbits) {
     ++lb;
   }
   return lb;
-}
-
-/// Room per group: what one takes at most, or half of it where that is still eight times its share and
-/// a graph's first batch would pay for allocating the rest (100,000 operations: 34 MB, 0.6 ms).
-int group_room(int64_t N, int lb) {
-  return lb <= kGroupBitsFew || N > (int64_t{1} << 18) ? kGroupCap : kGroupCap / 2;
 }
 
 int op_bits(int64_t N) {
@@ -3008,8 +3056,8 @@ out_pair_params out_setup(dyng_hip_graph* g, const batch_scan& sc, const op_layo
                           int64_t n_before) {
   out_pair_params op{};
   op.L = L;
-  op.keys = g->keys_b.p;
-  op.vals = g->vals_b.p;
+  op.keys = g->ops.keys_b;
+  op.vals = g->ops.vals_b;
   op.N = N;
   op.stride = P;
   op.vbits = vbits;
@@ -3023,17 +3071,17 @@ out_pair_params out_setup(dyng_hip_graph* g, const batch_scan& sc, const op_layo
   op.nbr = g->out.nbr.p;
   op.w = g->out.w.p;
   op.slot_cap = g->out.slot_cap;
-  op.pend_alive = g->pend_alive.p;
-  op.kill = g->kill.p;
-  op.pend_w = g->pend_w.p;
+  op.pend_alive = g->ops.pend_alive;
+  op.kill = g->ops.kill;
+  op.pend_w = g->ops.pend_w;
   op.e_inc = g->ins_inc.p;
   op.e_fw = g->props.allow_parallel ? nullptr : g->ins_fw.p;
-  op.iop_type = g->iop_type.p;
-  op.iop_wold = g->iop_wold.p;
-  op.iop_wnew = g->iop_wnew.p;
+  op.iop_type = g->ops.iop_type;
+  op.iop_wold = g->ops.iop_wold;
+  op.iop_wnew = g->ops.iop_wnew;
   op.mark = g->mark_out.p;
   op.mark_gen = g->mark_generation;
-  op.touched = g->touched_out.p;
+  op.touched = g->ops.touched_out;
   op.row_a = g->row_a_out.p;
   op.row_b = g->row_b_out.p;
   op.ctl = g->ctl.p;
@@ -3045,27 +3093,27 @@ in_pair_params in_setup(dyng_hip_graph* g, const batch_scan& sc, const op_layout
   ip.L = L;
   ip.ins_w = sc.ins_w;
   ip.upsert = g->props.on_existing_insert == 0 ? 1 : 0;
-  ip.keys = g->keys_b.p + P;
-  ip.vals = g->vals_b.p + P;
+  ip.keys = g->ops.keys_b + P;
+  ip.vals = g->ops.vals_b + P;
   ip.N = N;
   ip.stride = P;
   ip.vbits = vbits;
   ip.K = g->K;
-  ip.iop_type = g->iop_type.p;
-  ip.iop_wold = g->iop_wold.p;
-  ip.iop_wnew = g->iop_wnew.p;
+  ip.iop_type = g->ops.iop_type;
+  ip.iop_wold = g->ops.iop_wold;
+  ip.iop_wnew = g->ops.iop_wnew;
   ip.meta = g->in.meta.p;
   ip.base = g->in.base.p;
   ip.dead = g->in.dead.p;
   ip.nbr = g->in.nbr.p;
   ip.w = g->in.w.p;
   ip.slot_cap = g->in.slot_cap;
-  ip.pend_alive = g->ipend_alive.p;
-  ip.kill = g->ikill.p;
-  ip.pend_w = g->ipend_w.p;
+  ip.pend_alive = g->ops.ipend_alive;
+  ip.kill = g->ops.ikill;
+  ip.pend_w = g->ops.ipend_w;
   ip.mark = g->mark_in.p;
   ip.mark_gen = g->mark_generation;
-  ip.touched = g->touched_in.p;
+  ip.touched = g->ops.touched_in;
   ip.row_a = g->row_a_in.p;
   ip.row_b = g->row_b_in.p;
   ip.ctl = g->ctl.p;
@@ -3102,13 +3150,13 @@ void rows_sorted(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, in
   mark_stage(g, 3, s);
   // one stable sort of both directions' keys (2N of them, 2 * vbits + 1 bits): one sort of 2N
   // keys costs little more than one of N, since rocPRIM's small-size path is launch-bound
-  sort_pairs(g->sort_tmp, g->keys_a.p, g->keys_b.p, g->vals_a.p, g->vals_b.p, 2 * N, 2 * vbits + 1, s);
-  hipLaunchKernelGGL(k_untag, dim3(std::min<unsigned>(blocks_for(2 * N), 1024)), dim3(kBlock), 0, s, g->keys_b.p,
+  sort_pairs(g->sort_tmp, g->keys_a.p, g->ops.keys_b, g->vals_a.p, g->ops.vals_b, 2 * N, 2 * vbits + 1, s);
+  hipLaunchKernelGGL(k_untag, dim3(std::min<unsigned>(blocks_for(2 * N), 1024)), dim3(kBlock), 0, s, g->ops.keys_b,
                      2 * N, vbits);
   if (g->props.on_missing_delete == 1 || g->props.on_existing_insert == 1) {
     // the error modes: every operation checked before anything changes (one more launch and
     // synchronization, only in these modes)
-    hipLaunchKernelGGL(k_check_pairs, dim3(blocks_for(N)), dim3(kBlock), 0, s, L, g->keys_b.p, g->vals_b.p, N,
+    hipLaunchKernelGGL(k_check_pairs, dim3(blocks_for(N)), dim3(kBlock), 0, s, L, g->ops.keys_b, g->ops.vals_b, N,
                        vbits, n_before, g->out.meta.p, g->out.base.p, g->out.nbr.p,
                        g->props.on_missing_delete == 1 ? 1 : 0, g->props.on_existing_insert == 1 ? 1 : 0, dc);
     DYNG_HIP_TRY(hipGetLastError());
@@ -3139,8 +3187,8 @@ void rows_sorted(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, in
     DYNG_HIP_TRY(hipGetLastError());
   }
   mark_stage(g, 8, s);
-  exclusive_scan4(g->scan_tmp, g->pend_alive.p, g->kill.p, g->ipend_alive.p, g->ikill.p, g->pend_prefix.p,
-                  g->kill_prefix.p, g->ipend_prefix.p, g->ikill_prefix.p, N + 1, s);
+  exclusive_scan4(g->scan_tmp, g->ops.pend_alive, g->ops.kill, g->ops.ipend_alive, g->ops.ikill, g->ops.pend_prefix,
+                  g->ops.kill_prefix, g->ops.ipend_prefix, g->ops.ikill_prefix, N + 1, s);
   mark_stage(g, 9, s);
   // ---- plan the merges: each row's mode, and the staging and tail slots they take ----
   if (wait != nullptr) DYNG_HIP_TRY(hipStreamWaitEvent(s, wait, 0));  // before the rows change
@@ -3183,9 +3231,9 @@ void rows_grouped(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, i
   f.lb = lb;
   f.K = g->K;
   f.groups = groups;
-  f.room = group_room(N, lb);
-  f.entries = g->group_entries.p;
-  f.counts = g->group_counts.p;
+  f.room = kGroupCap;
+  f.entries = g->ops.group_entries;
+  f.counts = g->ops.group_counts;
   f.e_del_src = g->del_src.p;
   f.e_del_dst = g->del_dst.p;
   f.e_ins_src = g->ins_src.p;
@@ -3204,8 +3252,8 @@ void rows_grouped(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, i
   mark_stage(g, 3, s);
   mark_stage(g, 4, s);
   group_params gp{};
-  gp.entries = g->group_entries.p;
-  gp.counts = g->group_counts.p;
+  gp.entries = g->ops.group_entries;
+  gp.counts = g->ops.group_counts;
   gp.groups = groups;
   gp.room = f.room;
   gp.vbits = vbits;
@@ -3214,17 +3262,17 @@ void rows_grouped(dyng_hip_graph* g, const batch_scan& sc, const op_layout& L, i
   uint32_t inverse = kGroupHash;  // Newton's iteration: right modulo 2^3, then 2^6, ... 2^48
   for (int i = 0; i < 4; ++i) inverse *= 2u - kGroupHash * inverse;
   gp.inverse = inverse;
-  gp.keys = g->keys_b.p;
-  gp.vals = g->vals_b.p;
+  gp.keys = g->ops.keys_b;
+  gp.vals = g->ops.vals_b;
   gp.P = P;
   gp.out = out_setup(g, sc, L, N, P, vbits, n_before);
   gp.in = in_setup(g, sc, L, N, P, vbits);
   gp.merge_out = merge_setup(g, true, P, vbits);
   gp.merge_in = merge_setup(g, false, P, vbits);
-  gp.pend_prefix_out = g->pend_prefix.p;
-  gp.kill_prefix_out = g->kill_prefix.p;
-  gp.pend_prefix_in = g->ipend_prefix.p;
-  gp.kill_prefix_in = g->ikill_prefix.p;
+  gp.pend_prefix_out = g->ops.pend_prefix;
+  gp.kill_prefix_out = g->ops.kill_prefix;
+  gp.pend_prefix_in = g->ops.ipend_prefix;
+  gp.kill_prefix_in = g->ops.ikill_prefix;
   gp.ctl = dc;
   mark_stage(g, 5, s);
   if (!g->props.allow_parallel) {
@@ -3295,13 +3343,7 @@ apply_pending apply_launch(dyng_hip_graph* g, const batch_scan& sc, hipStream_t 
   const bool grouped = group_eligible(g, N, vbits, lb) && g->group_pause == 0;
   if (g->group_pause > 0) g->group_pause -= 1;
   const int64_t P = ap.P = grouped ? N + (int64_t{1} << lb) : N;
-  if (grouped) {
-    g->group_entries.reserve((size_t{2} << lb) * group_room(N, lb));
-    g->group_counts.reserve(size_t{2} << lb);
-  }
-  reserve_ops(g, P);
-  g->touched_out.reserve(P + 1);
-  g->touched_in.reserve(P + 1);
+  take_ops(g, P, grouped ? size_t{2} << lb : 0);
   g->row_a_out.reserve(g->n_cap);
   g->row_b_out.reserve(g->n_cap);
   g->row_a_in.reserve(g->n_cap);
@@ -3352,6 +3394,7 @@ void apply_finish(dyng_hip_graph* g, const batch_scan& sc, apply_pending& ap, hi
     DYNG_HIP_TRY(hipStreamSynchronize(s));
     ap.replanned = true;
   }
+  give_ops(g);
   if (hc->error_bits != 0) {
     g->n = n_before;
     throw status_error(DYNG_HIP_DEVICE_ERROR, "dyng: the device apply reported an internal error",

@@ -3,6 +3,7 @@
 
 #include "../../include/dyng_hip.h"
 #include "common.hpp"
+#include "scratch_pool.hpp"
 
 #include <cstddef>
 #include <memory>
@@ -326,6 +327,27 @@ void apply_finish(dyng_hip_graph* g, const batch_scan& sc, apply_pending& ap, hi
                   dyng_hip_apply_summary* out);
 }  // namespace dyng_hip
 
+namespace dyng_hip {
+/// What an apply needs per operation, in one block of its device's pool from apply_launch to
+/// apply_finish: a dozen arrays of their own took a graph's first batch 0.25 to 0.45 ms each from 2 MB
+/// on, and stayed with every graph.
+struct op_scratch {
+  scratch_block block;
+  unsigned long long* keys_b;  ///< sorted operations: out-row keys, then in-row keys
+  uint32_t* vals_b;
+  unsigned long long* group_entries;  ///< the grouped apply's operations, a fixed room per group
+  int* group_counts;
+  int32_t *pend_alive, *kill, *pend_prefix, *kill_prefix, *pend_w;
+  int32_t *ipend_alive, *ikill, *ipend_prefix, *ikill_prefix, *ipend_w;
+  int32_t *iop_type, *iop_wold, *iop_wnew;
+  int4 *touched_out, *touched_in;
+  int4* lane_rows;       ///< the merge plan's rows of one thread each, per direction
+  int32_t* merge_lists;  ///< the merge plan's row lists, per direction and mode
+};
+/// The pool of a device's apply scratch.
+scratch_pool& apply_scratch(int device);
+}  // namespace dyng_hip
+
 /// The device graph behind the dyng_hip_graph handle.
 struct dyng_hip_graph {
   int device = 0;
@@ -357,20 +379,14 @@ struct dyng_hip_graph {
   int64_t num_del_slots = 0, num_ins_slots = 0;
 
   // apply scratch
-  dyng_hip::dbuf<unsigned long long> keys_a, keys_b;  ///< the apply's sort: out-row keys, then in-row keys
-  dyng_hip::dbuf<uint32_t> vals_a, vals_b;
+  dyng_hip::op_scratch ops;
+  bool pools_scratch = false;  ///< the graph is a user of its device's scratch pool
+  dyng_hip::dbuf<unsigned long long> keys_a;  ///< the device-wide sort's input: out-row keys, then in-row keys
+  dyng_hip::dbuf<uint32_t> vals_a;
   dyng_hip::dbuf<unsigned char> sort_tmp, scan_tmp;
-  dyng_hip::dbuf<unsigned long long> group_entries;  ///< the grouped apply's operations, a fixed room per group
-  dyng_hip::dbuf<int> group_counts;
   int group_pause = 0;  ///< batches left that are sorted device-wide (see resort)
-  dyng_hip::dbuf<int32_t> pend_alive, kill, pend_prefix, kill_prefix, pend_w;
-  dyng_hip::dbuf<int32_t> ipend_alive, ikill, ipend_prefix, ikill_prefix, ipend_w;
-  dyng_hip::dbuf<int32_t> iop_type, iop_wold, iop_wnew;
-  dyng_hip::dbuf<int4> touched_out, touched_in;
-  dyng_hip::dbuf<int4> lane_rows;  ///< the merge plan's rows of one thread each, per direction
   dyng_hip::dbuf<int32_t> mark_out, mark_in;
   dyng_hip::dbuf<int32_t> row_a_out, row_b_out, row_a_in, row_b_in;  ///< per vertex: its operations
-  dyng_hip::dbuf<int32_t> merge_lists;  ///< the merge plan's row lists, per direction and mode
   dyng_hip::dbuf<int32_t> stage_nbr, stage_w;
   int64_t stage_cap = 0;
   int mark_generation = 0;
@@ -387,6 +403,8 @@ struct dyng_hip_graph {
   dyng_hip_graph(const dyng_hip_graph&) = delete;
   dyng_hip_graph& operator=(const dyng_hip_graph&) = delete;
   ~dyng_hip_graph() {
+    if (ops.block.p != nullptr) (void)hipFree(ops.block.p);  // an apply failed half-way: its work may not have ended
+    if (pools_scratch) dyng_hip::apply_scratch(device).leave();
     for (hipEvent_t& e : apply_ev) {
       if (e != nullptr) (void)hipEventDestroy(e);
     }
