@@ -331,15 +331,16 @@ void repair_core(dyng_hip_graph* g, dyng_hip_result* r, int64_t delta, int64_t m
       }
     }
     engine_finish(pend, &c);
-    // the events that time the run are the workspace's, recorded around its kernel; the apply's time
-    // ends where the run's begins (each record is a packet that the stream waits at)
-    if (inflight != nullptr && pend.started != nullptr) *inflight->apply_ms = elapsed_ms(inflight->began, pend.started);
     if (pend.held) {
       // the apply's merges were planned again on the host (its arenas may have moved): the run now
       run = run_for();
       pend = engine_launch(&run, true, s);
       engine_finish(pend, &c);
     }
+    // the events that time the run are the workspace's, recorded around its kernel; the apply's time
+    // ends where the run's begins, the one that did something (each record is a packet that the stream
+    // waits at)
+    if (inflight != nullptr && pend.started != nullptr) *inflight->apply_ms = elapsed_ms(inflight->began, pend.started);
     r->tree_token = c.tree_token;
     if (run.tuning.recompute == 0) r->repair_edges = c.pull_edges + c.relax_edges;
     r->last = c;

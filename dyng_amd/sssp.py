@@ -114,7 +114,9 @@ class Stats:
     cost the caller no Python work it does not use): ``affected``, ``iterations``,
     ``frontier_visits``, ``fallback_used``, ``converged``, ``engine_used``, ``batch``
     (:class:`dyng_amd.ApplySummary`), ``invalidated``, ``epochs``, ``pushes``,
-    ``packed_parents``, ``device`` (:class:`DeviceCounters`), ``apply_ms``, ``engine_ms``.
+    ``packed_parents``, ``device`` (:class:`DeviceCounters`), ``apply_ms`` (stream time from behind
+    the batch scan to the start of the engine's kernel; of several results' update in the first one's
+    stats), ``engine_ms`` (that kernel, ``device.kernel_ms``).
     """
 
     __slots__ = ("_raw", "_batch", "_device")

@@ -284,7 +284,10 @@ typedef struct dyng_hip_stats { /* sssp::stats (sssp.hpp:100-117) + update_stats
   dyng_hip_apply_summary batch;
   int64_t invalidated, epochs, pushes;
   dyng_hip_counters device; /* the engine run's counters */
-  double apply_ms, engine_ms; /* stream time of the device apply and of the engine (events) */
+  /* apply_ms: stream time (events) from behind the batch scan to the start of the run's kernel (with
+   * several results: to the end of the apply, in the first result's stats): the apply, a second plan on
+   * the host if there was one, and the run's reset. engine_ms: the run's kernel (device.kernel_ms). */
+  double apply_ms, engine_ms;
 } dyng_hip_stats;
 
 typedef struct dyng_hip_result dyng_hip_result;
