@@ -126,13 +126,15 @@ def default_delta(graph: Graph, objective: int = 0) -> int:
 
 
 def candidate_tunings(delta: int) -> list[tuple[sssp.Tuning, int]]:
-    """The schedule grid the autotuner times: row-length thresholds for the edge-balanced tiles,
-    chunk sizes for the long rows and near-far widths around the default."""
+    """The schedule grid the autotuner times: near-far widths around the default, each with the engine's
+    own row-length thresholds (a phase each, which one number cannot give) and chunks, so that a tuned
+    result is not left with less than an untuned one, and with other thresholds and chunk sizes."""
     out = []
     for light in (256, 1024, 4096):
         for chunk in (128, 512):
             for scale in (0.25, 1.0, 4.0):
                 out.append((sssp.Tuning(light_degree=light, chunk_edges=chunk), max(1, int(delta * scale))))
+    out += [(sssp.Tuning(), max(1, int(delta * scale))) for scale in (0.25, 1.0, 4.0)]
     return out
 
 
