@@ -1,8 +1,8 @@
-"""The memory-ordering convention of the fused SSSP kernel, checked on its source text.
+"""The memory-ordering convention of the persistent kernels, checked on their source text.
 
-`sssp_fused_kernel` (dyng_amd/csrc/sssp.hip) separates its phases with a grid barrier that
-orders only agent-scope atomic operations (`DYNG_GRID_SYNC`): the barrier issues no cache
-write-back or invalidate, so a plain load or store of an array that other workgroups touch
+The engine's kernel (dyng_amd/csrc/sssp.hip) separates its phases with grid barriers that
+order only agent-scope atomic operations (`DYNG_GRID_SYNC`, `DYNG_GRID_SYNC_SENT`, the split
+`DYNG_FLUSH_AND_CHUNKS_WAIT`): they issue no cache write-back or invalidate, so a plain load or store of an array that other workgroups touch
 in the same launch may read a stale line or publish nothing.  The kernel therefore touches
 every such array only through the agent-scope helpers (`ld`, `st`, `ld_chunk`, `st_chunk`,
 `ld_int4`, the `atomic*` family).  The one exception is the distance-only unpack, whose
@@ -23,6 +23,8 @@ Rules:
    a plain load the previous one (or the kernel's start).
 2. `parents` and `distances` are the run's input tree until the unpack phase: nothing
    writes them before it (plain loads of them are fine anywhere).
+3. MOSP's path doubling (dyng_amd/csrc/path_costs.hpp) keeps rule 1 for its sums and jumps; its
+   plain store home comes after its last barrier.
 Text order stands in for control flow: a store at the end of a loop body whose back edge
 reaches an unfenced barrier would pass rule 1.  The kernel has no plain access in a loop
 that holds a barrier.
@@ -47,6 +49,9 @@ HELPER = re.compile(r"^(ld|st|ld_chunk|st_chunk|ld_int4|atomic[A-Za-z]+|__hip_at
 KERNEL_START = "sssp_fused_kernel(engine_params p)"
 KERNEL_END = "#undef DYNG_GRID_SYNC"
 UNPACK = "// ---- F: unpack ----"
+BARRIER = r"DYNG_GRID_SYNC(_FENCED)?\(\)|DYNG_GRID_SYNC_SENT\(|DYNG_FLUSH_AND_CHUNKS_WAIT\("
+PATHS = SOURCE.with_name("path_costs.hpp")
+PATH_ARRAYS = ("acc_in", "jump_in", "acc_out", "jump_out")
 
 
 def strip_comments(text: str) -> str:
@@ -121,7 +126,7 @@ def violations(text: str) -> list[str]:
     k1 = code.index(KERNEL_END, k0)
     unpack = text.index(UNPACK, k0)
     barriers = [(m.start(), m.group(1) is not None)
-                for m in re.finditer(r"DYNG_GRID_SYNC(_FENCED)?\(\)", code[k0:k1])]
+                for m in re.finditer(BARRIER, code[k0:k1])]
     barriers = [(k0 + at, fenced) for at, fenced in barriers]
 
     def fenced_window(pos: int, store: bool) -> bool:
@@ -159,6 +164,20 @@ def violations(text: str) -> list[str]:
     return found
 
 
+def path_violations(text: str) -> list[str]:
+    code = strip_comments(text)
+    k0 = code.index("k_path_costs(path_params p)")
+    last = code.rindex("grid_barrier<false>(")
+    found = []
+    for m in re.finditer(r"(?<![\w.>])({})\[|p\.(acc|jump)\[[^]]*\]\[".format("|".join(PATH_ARRAYS)), code[k0:]):
+        start = k0 + m.start()
+        wrapped = code[:start].rstrip().endswith("&") and bool(HELPER.match(enclosing_call(code, start) or ""))
+        home = m.group(2) is not None and start > last and is_store(code, k0 + m.end())
+        if not wrapped and not home:
+            found.append(f"line {line_of(code, start)}: plain access to {m.group(0)[:-1]}")
+    return found
+
+
 @pytest.fixture(scope="module")
 def source() -> str:
     return SOURCE.read_text()
@@ -192,6 +211,12 @@ def _plant(source: str, anchor: str, replacement: str) -> str:
     ("if (pred) st(&list[slot], v);", "if (pred) list[slot] = v;"),
     # a plain load through a local alias of a shared list
     ("v = ld(&cur[idx]);", "v = cur[idx];"),
+    # plain stores whose next barrier brings totals along
+    ("if (near) st(&p.in_far[v], 0);", "if (near) p.in_far[v] = 0;"),
+    ("if (tid == 0) st(&p.frontier[0], p.source);", "if (tid == 0) p.frontier[0] = p.source;"),
+    ("st(&p.packed[v], packed_inf);", "p.packed[v] = packed_inf;"),
+    # a plain load behind the split barrier
+    ("word = ld(&p.packed[v]);\n              du", "word = p.packed[v];\n              du"),
     # a shared flag written through a helper that is not agent-scope
     ("if (near) st(&p.in_far[v], 0);", "if (near) write_plain(&p.in_far[v], 0);"),
 ])
@@ -211,3 +236,27 @@ def test_a_tree_write_before_unpack_is_caught(source):
     planted = _plant(source, "for (int v = tid; v < n; v += threads) st(&p.ancestor[v], p.parents[v]);",
                      "for (int v = tid; v < n; v += threads) p.parents[v] = -1;")
     assert any("before the unpack" in v for v in violations(planted))
+
+
+def test_the_barriers_are_all_seen(source):
+    """Every use of a barrier in the kernel is one that the rules know."""
+    code = strip_comments(source)
+    k0 = code.index(KERNEL_START)
+    body = code[k0:code.index(KERNEL_END, k0)]
+    uses = re.findall(r"\b(DYNG_(?:GRID_SYNC|FLUSH)\w*|grid_barrier|grid_poll|stage_flush_wait)\b", body)
+    assert len(uses) == len(re.findall(BARRIER, body)) > 10
+    assert set(uses) == {"DYNG_GRID_SYNC", "DYNG_GRID_SYNC_FENCED", "DYNG_GRID_SYNC_SENT", "DYNG_FLUSH_AND_CHUNKS_WAIT"}
+
+
+def test_path_doubling_keeps_the_ordering_convention():
+    assert path_violations(PATHS.read_text()) == []
+
+
+@pytest.mark.parametrize("anchor, replacement", [
+    ("ld(&jump_in[j[q]])", "jump_in[j[q]]"),
+    ("ld(&acc_in[static_cast<int64_t>(j[q]) * p.columns + c])", "acc_in[static_cast<int64_t>(j[q]) * p.columns + c]"),
+    ("st(&jump_out[v], next)", "jump_out[v] = next"),
+    ("ld(&p.acc[1][v * p.columns + c])", "p.acc[1][v * p.columns + c]"),
+])
+def test_a_planted_plain_access_in_path_doubling_is_caught(anchor, replacement):
+    assert path_violations(_plant(PATHS.read_text(), anchor, replacement))
