@@ -18,8 +18,9 @@ struct alignas(16) row_quad {
 };
 
 /// First index in [lo, hi) whose neighbour (sign bit masked) is >= v, or hi. Each round probes
-/// seven evenly spaced entries with independent loads, so a long row costs about log8 of its
-/// length in dependent memory round trips instead of log2. The last 16 entries or fewer are read
+/// kProbes evenly spaced entries with independent loads: seven cost a long row about log8 of its
+/// length in dependent memory round trips instead of log2, and one reads the fewest lines (see
+/// find_runs in graph.hip, which says where those bound a search). The last 16 entries or fewer are read
 /// as the (at most five) aligned 16-byte words that hold them, all in flight together: one more
 /// round trip, and five load instructions where sixteen single entries would take sixteen (a
 /// wave's lanes usually search different rows, so each instruction fetches up to 64 lines). A

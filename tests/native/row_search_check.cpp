@@ -1,10 +1,10 @@
 // Host check of the row searches of dyng_amd/csrc/row_search.hpp against std::lower_bound and
-// std::upper_bound on the masked neighbour ids: random rows (runs of equal ids, dead marks in the
-// sign bit) starting at every offset within a 16-byte word, every sub-range of short rows and
-// random ranges of long ones, every probe value around the row's ids. Each row sits in an
-// allocation of whole 16-byte words, as device allocations are, so a build with AddressSanitizer
-// also shows that no load leaves the words that hold the row. Prints "ok <checks>" or the first
-// mismatch and exits nonzero.
+// std::upper_bound on the masked neighbour ids, with seven probes a round and with one: random rows
+// (runs of equal ids, dead marks in the sign bit) starting at every offset within a 16-byte word,
+// every sub-range of short rows and random ranges of long ones, every probe value around the row's
+// ids. Each row sits in an allocation of whole 16-byte words, as device allocations are, so a build
+// with AddressSanitizer also shows that no load leaves the words that hold the row. Prints
+// "ok <checks>" or the first mismatch and exits nonzero.
 #define DYNG_ROW_SEARCH_FN inline
 #include "../../dyng_amd/csrc/row_search.hpp"
 
@@ -42,7 +42,13 @@ bool check_range(placed_row& pr, int lo, int hi, int32_t v, long long& checks) {
   const int want_ub = static_cast<int>(std::upper_bound(a + lo, a + hi, v, id_less) - a);
   const int lb = row_lower_bound(a, lo, hi, v);
   const int ub = row_upper_bound_from(a, lb, hi, v);
+  const int lb1 = row_lower_bound<1>(a, lo, hi, v);  // the apply's and the path costs'
   ++checks;
+  if (lb1 != want_lb) {
+    std::printf("one probe: len %d skew %d lo %d hi %d v %d: lower %d (want %d)\n", pr.len, pr.skew, lo, hi, v, lb1,
+                want_lb);
+    return false;
+  }
   if (lb != want_lb || ub != want_ub) {
     std::printf("mismatch: len %d skew %d lo %d hi %d v %d: lower %d (want %d) upper %d (want %d)\n",
                 pr.len, pr.skew, lo, hi, v, lb, want_lb, ub, want_ub);
