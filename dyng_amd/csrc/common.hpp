@@ -147,18 +147,14 @@ struct op_sum {
   template <class T>
   DYNG_DEV T operator()(T a, T b) const { return a + b; }
 };
-struct op_min {
-  template <class T>
-  DYNG_DEV T operator()(T a, T b) const { return b < a ? b : a; }
-};
 struct op_max {
   template <class T>
   DYNG_DEV T operator()(T a, T b) const { return b > a ? b : a; }
 };
 
 
-/// Grid-wide barrier of a persistent kernel whose workgroups are all resident (the grid is sized
-/// to at most half of what the occupancy calculator says fits at once), in two halves.
+/// Grid-wide barrier of a persistent kernel whose workgroups are all resident (the grid is sized to at
+/// most what the occupancy calculator says fits at once), in two halves.
 ///
 /// Arrivals go up a two-level tree: workgroup b adds to the word of group b % G (G = min(16,
 /// workgroups)); the last member of a group to arrive adds the group's totals to the root's word,

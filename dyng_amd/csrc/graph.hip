@@ -16,22 +16,27 @@
 //
 // A batch (MOSP applyChangeBatch under upsert_last_wins, cpp/src/graph/apply_host.cpp:57-401) is
 // applied without leaving the device:
-//   1. Step 0 (apply_host.cpp:80-147): self-loops, vertex growth, undirected expansion; one key
-//      (u << b | v) per effective operation, in application order (deletions first).
-//   2. A stable radix sort by key groups the operations of each pair (u,v) in batch order.
-//   3. One thread per pair replays its operations on the runs of v in row u (binary searches in
-//      both runs): deletions mark the first alive match dead, insertions overwrite the first
-//      alive match (upsert) or add a pending entry; then the weight-increase flags of :348-394
-//      (final first (u,v) against the original first (u,v)). Each operation that changes an
-//      in-edge emits an in-operation for the in-rows.
-//   4. A planning pass sorts the touched rows into three merge modes (a short tail merged by one
-//      wave in registers, a longer tail by one workgroup, or the whole row into a new base) and
-//      sums the staging and relocation slots the full merges need, so the host can grow or
-//      compact the arena first; then one launch per mode merges the alive entries with the
-//      pending ones (positions from prefix sums and binary searches), in place, or at the arena's
-//      tail when the row outgrew its capacity.
-//   5. Steps 2-4 again for the in-rows with the in-operations (a deletion or a weight change
-//      matches the first alive in-entry of u with the old weights).
+//   1. k_batch_scan: ids, self-loops and weight ranges, before anything changes.
+//   2. k_group_front, Step 0 (apply_host.cpp:80-147): self-loops, vertex growth, undirected
+//      expansion; each effective operation goes to the group of its row, for the out-rows and for
+//      the in-rows. Rows are hashed into groups, so all of a row's operations are in one.
+//   3. k_group_pairs, a workgroup per group: the operations sorted by row, neighbour and application
+//      order (deletions first), then one thread per pair (u,v) replays its operations on the runs of
+//      v in row u (searches in both runs): deletions mark the first alive match dead, insertions
+//      overwrite the first alive match (upsert) or add a pending entry; then the weight-increase
+//      flags of :348-394 (final first (u,v) against the original first (u,v)). The in-rows replay
+//      the same operations; with parallel edges their groups come in a second launch, which matches
+//      the copy that each operation took by its old weights. Last, the group's touched rows are
+//      planned: a tail merged by a thread, a wave or a workgroup, or the whole row into a new base,
+//      and the staging and relocation slots that takes.
+//   4. k_tails and k_rows merge the alive entries with the pending ones (positions from prefix sums
+//      and searches), in place, or at the arena's tail when the row outgrew its capacity. For a small
+//      batch they are queued behind the plan and look for themselves whether the arenas take it; else
+//      the host reads the plan, and grows or compacts an arena first.
+// Batches that a group cannot take (more operations on a row than a workgroup sorts), past the
+// groups' number, or checked by an error mode before anything changes go through one device-wide
+// stable sort of both directions' keys (u << b | v) instead of steps 2 and 3, then a launch each for
+// the pairing, the scans and the plan (rows_sorted).
 #include "internal.hpp"
 
 #include <hip/hip_runtime.h>
@@ -1216,10 +1221,8 @@ struct merge_params {
   double headroom;
 };
 
-/// The in-place tail merges of one mode for both stores in one launch: workgroups [0, split)
-/// merge out-rows, the others in-rows. The two stores share nothing these merges write (the error
-/// bits aside, which they set atomically), so the halves run side by side.
-/// The merges of both stores in one launch: a workgroup's role and store by its place in the grid.
+/// The merges of both stores in one launch: a workgroup's role and store by its place in the grid. The
+/// stores share nothing that the merges write, the error bits aside, which they set atomically.
 struct merge_roles {
   merge_params side[2];
   int groups[4];        ///< workgroups per role and store: first role's out-rows, in-rows, second role's out-rows, in-rows
@@ -1446,10 +1449,11 @@ DYNG_DEV bool merges_fit(const apply_control* c, long long slot_cap_out, long lo
 /// RMAT-23), the untagging, the pairing, two scan launches and the plan: two launches for ten to
 /// seventeen, nothing between them through memory but the operations.
 constexpr int kGroupBlock = 256;
-/// Operations per group and direction (the groups hold 1 to 2 times this), by how many groups there are:
-/// few while processors are idle (2^7 groups per direction give every one of the 256 a workgroup),
-/// more up to the workgroups it holds at once (2^9), and beyond that what the front's reservations and
-/// the per-group work favour. 2,000 arcs of an undirected 64 K graph: 25 us with 32 each, 43 with
+/// Least operations of a group and direction on average before there are twice as many groups, by how
+/// many there are: few while processors are idle (2^7 groups per direction give every one of the 256 a
+/// workgroup), more up to the workgroups it holds at once (2^9), and beyond that what the front's
+/// reservations and the per-group work favour. So the groups of 4,096 to 32,767 operations hold 32 to 256
+/// each, of 65,536 to 262,143 operations 128 to 512, of more 256 to 512 (1,024 at 2^22 operations). 2,000 arcs of an undirected 64 K graph: 25 us with 32 each, 43 with
 /// 128; 100,000 operations on RMAT-22: 103 us with 128, 110 with 256; 1,000,000 on RMAT-23: 515 us with
 /// 256, 550 to 590 with 128.
 constexpr int kGroupBitsFew = 7, kGroupOpsFew = 32;
@@ -1838,65 +1842,65 @@ template <int KW, int T, int O>
 DYNG_DEV int merge_lane(const merge_params& p, int64_t at, int tl, int64_t a, int nops) {
   const u64 mask = (1ULL << p.vbits) - 1;
   const int K = p.K;
-      int32_t x[T];
-  #pragma unroll
-      for (int j = 0; j < T; ++j) x[j] = j < tl ? p.nbr[at + j] : -1;
-      int32_t ov[O];
-      bool pend[O];
-  #pragma unroll
-      for (int j = 0; j < O; ++j) {
-        pend[j] = j < nops && p.pend_alive[a + j] != 0;
-        ov[j] = pend[j] ? static_cast<int32_t>(p.keys[a + j] & mask) : 0;
+  int32_t x[T];
+#pragma unroll
+  for (int j = 0; j < T; ++j) x[j] = j < tl ? p.nbr[at + j] : -1;
+  int32_t ov[O];
+  bool pend[O];
+#pragma unroll
+  for (int j = 0; j < O; ++j) {
+    pend[j] = j < nops && p.pend_alive[a + j] != 0;
+    ov[j] = pend[j] ? static_cast<int32_t>(p.keys[a + j] & mask) : 0;
+  }
+  int alive = 0, pending = 0;
+  for (int k0 = 0; k0 == 0 || k0 < K; k0 += KW) {
+    int32_t wr[KW][T];
+    int32_t ow[KW][O];
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+#pragma unroll
+      for (int k = 0; k < KW; ++k) {
+        wr[k][j] = (j < tl && k0 + k < K) ? p.w[(k0 + k) * p.slot_cap + at + j] : 0;
       }
-      int alive = 0, pending = 0;
-      for (int k0 = 0; k0 == 0 || k0 < K; k0 += KW) {
-        int32_t wr[KW][T];
-        int32_t ow[KW][O];
-  #pragma unroll
-        for (int j = 0; j < T; ++j) {
-  #pragma unroll
-          for (int k = 0; k < KW; ++k) {
-            wr[k][j] = (j < tl && k0 + k < K) ? p.w[(k0 + k) * p.slot_cap + at + j] : 0;
-          }
+    }
+#pragma unroll
+    for (int j = 0; j < O; ++j) {
+#pragma unroll
+      for (int k = 0; k < KW; ++k) ow[k][j] = (pend[j] && k0 + k < K) ? p.pend_w[(k0 + k) * p.N + a + j] : 0;
+    }
+    // alive entries, at their places (the tail is sorted, dead entries carry the sign bit)
+    alive = 0;
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+      if (x[i] >= 0) {
+        int pos = alive;
+#pragma unroll
+        for (int j = 0; j < O; ++j) pos += (pend[j] && ov[j] < x[i]) ? 1 : 0;
+        if (k0 == 0) p.nbr[at + pos] = x[i];
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+          if (k0 + k < K) p.w[(k0 + k) * p.slot_cap + at + pos] = wr[k][i];
         }
-  #pragma unroll
-        for (int j = 0; j < O; ++j) {
-  #pragma unroll
-          for (int k = 0; k < KW; ++k) ow[k][j] = (pend[j] && k0 + k < K) ? p.pend_w[(k0 + k) * p.N + a + j] : 0;
-        }
-        // alive entries, at their places (the tail is sorted, dead entries carry the sign bit)
-        alive = 0;
-  #pragma unroll
-        for (int i = 0; i < T; ++i) {
-          if (x[i] >= 0) {
-            int pos = alive;
-  #pragma unroll
-            for (int j = 0; j < O; ++j) pos += (pend[j] && ov[j] < x[i]) ? 1 : 0;
-            if (k0 == 0) p.nbr[at + pos] = x[i];
-  #pragma unroll
-            for (int k = 0; k < KW; ++k) {
-              if (k0 + k < K) p.w[(k0 + k) * p.slot_cap + at + pos] = wr[k][i];
-            }
-            ++alive;
-          }
-        }
-        // pending entries (the operations are sorted by neighbour, then batch order)
-        pending = 0;
-  #pragma unroll
-        for (int j = 0; j < O; ++j) {
-          if (pend[j]) {
-            int pos = pending;
-  #pragma unroll
-            for (int i = 0; i < T; ++i) pos += (x[i] >= 0 && x[i] <= ov[j]) ? 1 : 0;
-            if (k0 == 0) p.nbr[at + pos] = ov[j];
-  #pragma unroll
-            for (int k = 0; k < KW; ++k) {
-              if (k0 + k < K) p.w[(k0 + k) * p.slot_cap + at + pos] = ow[k][j];
-            }
-            ++pending;
-          }
-        }
+        ++alive;
       }
+    }
+    // pending entries (the operations are sorted by neighbour, then batch order)
+    pending = 0;
+#pragma unroll
+    for (int j = 0; j < O; ++j) {
+      if (pend[j]) {
+        int pos = pending;
+#pragma unroll
+        for (int i = 0; i < T; ++i) pos += (x[i] >= 0 && x[i] <= ov[j]) ? 1 : 0;
+        if (k0 == 0) p.nbr[at + pos] = ov[j];
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+          if (k0 + k < K) p.w[(k0 + k) * p.slot_cap + at + pos] = ow[k][j];
+        }
+        ++pending;
+      }
+    }
+  }
   return alive + pending;
 }
 
@@ -2171,9 +2175,8 @@ DYNG_DEV int compact_alive(const merge_params& p, int64_t src, int len, int64_t 
   return carry;
 }
 
-/// One workgroup per row rewritten whole, staging from `stage_from` on (its tail or dead
-/// entries outgrew their limits, or the
-/// row its capacity): the alive base (A) and the alive tail (B) are compacted into the staging
+/// One workgroup per row rewritten whole, staging from `stage_from` on (its tail or dead entries
+/// outgrew their limits, or the row its capacity): the alive base (A) and the alive tail (B) are compacted into the staging
 /// arena, then A, B and the pending entries (C) are merged into one base run, in place or at the
 /// tail of the arena. An entry's place is its index in its run plus the entries of the other two
 /// runs before it: A before B before C among equal neighbours.

@@ -236,9 +236,9 @@ void scan_batch(dyng_hip_graph* g, const dyng_hip_batch* b, hipStream_t s, batch
 
 /// One engine run in flight: engine_launch queues it on `s` (the checks, the launch and the
 /// counters' read-back, nothing waited for), engine_finish waits for it and reports (or throws).
-/// dyng_hip_sssp_update / _compute are the two back to back. Runs on one device are queued on one
-/// stream, one after another: two persistent launches resident together gave wrong trees on
-/// MI355X (the kernel keeps a little per-lane state in scratch memory), so runs never overlap.
+/// dyng_hip_sssp_update / _compute are the two back to back. Launches on one device are queued one
+/// after another: a launch's workgroups wait for each other and must all be resident. Repairs that run
+/// side by side are teams of one launch (engine_launch_teams).
 struct apply_pending;
 struct engine_pending {
   dyng_hip_workspace* ws = nullptr;

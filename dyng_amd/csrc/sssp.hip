@@ -45,15 +45,16 @@ namespace dyng_hip {
 
 namespace {
 
-constexpr int kBlock = 1024;  ///< 16 waves per workgroup; 8 waves/SIMD fit two per CU, one is launched
+constexpr int kBlock = 1024;  ///< 16 waves per workgroup: two per CU in a solve, one in a repair
 constexpr int kWaves = kBlock / 64;
 constexpr int kWalkGlobal = 2;   ///< first rounds of the subtree walk: one level each
 constexpr int kWalkLocal = 16;   ///< later rounds: levels a workgroup walks on its own between grid barriers
 /// Grid rounds of the subtree walk before pointer jumping takes over: kWalkRounds and one more per
 /// kWalkRoundVertices vertices. A local round of 16 narrow levels takes about 38 us; pointer jumping
 /// reads every vertex a few times (1.87 ms over the 4096^2 grid's 16.8 M, about 0.11 ns per vertex
-/// and 0.1 ms of rounds), so the walk may spend about that before it gives up. With ten rounds for
-/// every size the grid's deep subtrees handed over (walk phase 1.35 ms on average); with 64 they
+/// and 0.1 ms of rounds), so the walk may spend about that before it gives up: a tree deeper than
+/// the limit pays for both, about twice what the jumping alone takes, and no tree more. With ten rounds
+/// for every size the grid's deep subtrees handed over (walk phase 1.35 ms on average); with 64 they
 /// finish in 11.5 rounds on average (0.59 ms).
 constexpr int kWalkRounds = kWalkGlobal + 8;
 constexpr int kWalkRoundVertices = 300000;
@@ -175,6 +176,7 @@ struct engine_params {
 
 /// Several runs in one launch, each on a team of workgroups with its own barrier and scratch.
 constexpr int kTeams = 4;
+static_assert(kTeams == kWorkspaceSlots, "a run of a launch has a workspace of its own");
 struct engine_teams {
   engine_params p[kTeams];
   int size;  ///< workgroups of a team
@@ -1053,7 +1055,7 @@ DYNG_DEV void engine_run(const engine_params& p) {
                   [&](const bool (&act)[kSlots], const int (&item)[kSlots], const int (&slot)[kSlots]) {
                     int32_t u[kSlots], w[kSlots];
                     bool add[kSlots];
-                int2 row[kSlots];
+                    int2 row[kSlots];
 #pragma unroll
                     for (int j = 0; j < kSlots; ++j) u[j] = act[j] ? L.vert[item[j]] : -1;
                     claim_children(act, u, slot, w, add, row);
@@ -1705,13 +1707,13 @@ struct dyng_hip_workspace {
   dyng_hip::dbuf<dyng_hip::grid_sync_state> bar;
   int grid_blocks = 0;
   int cu_count = 0;
-  int occupancy = 0;         ///< workgroups per CU of the 64-VGPR build
-  int occupancy_narrow = 0;
-  int occupancy_teams = 0;  ///< and of the 128-VGPR build
+  int occupancy = 0;         ///< workgroups per CU of the 64-VGPR builds
+  int occupancy_narrow = 0;  ///< of the 128-VGPR builds
+  int occupancy_teams = 0;   ///< and of the teams' kernel
   hipEvent_t ev_start = nullptr;
   hipEvent_t ev_stop = nullptr;
-  /// the launch as a hipGraph (control upload, barrier reset, events, the kernel, control
-  /// download), built once and replayed with the kernel node's arguments updated
+  /// the launch as a hipGraph (the reset, the events, the kernel), built once and replayed with both
+  /// kernel nodes' arguments updated
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
   hipGraphNode_t graph_reset = nullptr;
