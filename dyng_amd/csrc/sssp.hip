@@ -53,7 +53,8 @@ constexpr int kWalkLocal = 16;   ///< later rounds: levels a workgroup walks on 
 /// kWalkRoundVertices vertices. A local round of 16 narrow levels takes about 38 us; pointer jumping
 /// reads every vertex a few times (1.87 ms over the 4096^2 grid's 16.8 M, about 0.11 ns per vertex
 /// and 0.1 ms of rounds), so the walk may spend about that before it gives up: a tree deeper than
-/// the limit pays for both, about twice what the jumping alone takes, and no tree more. With ten rounds
+/// the limit pays for both, which is little beside its repair (64 chains of 32,768 vertices cut at
+/// their heads: 0.97 ms of 109). With ten rounds
 /// for every size the grid's deep subtrees handed over (walk phase 1.35 ms on average); with 64 they
 /// finish in 11.5 rounds on average (0.59 ms).
 constexpr int kWalkRounds = kWalkGlobal + 8;

@@ -77,3 +77,33 @@ def test_a_deep_solve_runs_in_local_rounds(dg, length, width):
     tree, _ = oracle.compute(og, 0)
     d, p = dg.sssp.compute(dg.Graph.from_edges(src, dst, w, num_vertices=n), 0).to_numpy()
     assert np.array_equal(d, tree.dist) and np.array_equal(p, tree.parent)
+
+
+@pytest.mark.parametrize("recompute", [False, True])
+def test_every_row_is_cut_into_chunks(dg, recompute):
+    """A frontier of all vertices whose rows are all past the limit, in the smallest chunks: as many as the
+    chunk list is made for, one per vertex and one per 16 slots of the long rows."""
+    rng = np.random.default_rng(16)
+    n, long_rows = 20_000, 40
+    rest = np.arange(2, n)
+    src = [np.array([0]), np.full(n - 2, 1), np.repeat(rest, 2), np.repeat(np.arange(2, 2 + long_rows), 1000)]
+    dst = [np.array([1]), rest, rng.integers(0, n, 2 * (n - 2)), rng.integers(0, n, 1000 * long_rows)]
+    src, dst = np.concatenate(src), np.concatenate(dst)
+    _, keep = np.unique(src * n + dst, return_index=True)
+    src, dst = src[keep], dst[keep]
+    w = rng.integers(1, 9, len(src))
+    og = oracle.build_from_edges(n, src, dst, w.reshape(-1, 1))
+    g = dg.Graph.from_edges(src, dst, w, num_vertices=n)
+    tree, _ = oracle.compute(og, 0)
+    r = dg.sssp.compute(g, 0)
+    r.set_tuning(dg.sssp.Tuning(light_degree=1, chunk_edges=16, recompute=recompute))
+    none = np.zeros(0, np.int64)
+    for b, (ins, dels) in enumerate([((0, 1, 7), (0, 1)), ((0, 1, 3), None), ((0, 2, 5), (0, 1))]):
+        ins = tuple(np.array([x]) for x in ins)
+        dels = tuple(np.array([x]) for x in dels) if dels else (none, none)
+        og, _, c = oracle.update(og, tree, ins[0], ins[1], ins[2].reshape(-1, 1), dels[0], dels[1])
+        st = dg.sssp.update(g, dg.EdgeBatch(insert=ins, delete=dels), r)
+        d, p = r.to_numpy()
+        assert np.array_equal(d, tree.dist) and np.array_equal(p, tree.parent), f"batch {b}"
+        if not recompute:
+            assert st.invalidated == c.invalidated and st.affected == c.affected, f"batch {b}"
