@@ -164,7 +164,7 @@ struct engine_params {
   int* far_b;
   int* touched;  ///< a repair's vertices whose words its claims may have changed (see claim_first)
   int4* chunks;
-  int64_t chunk_words;  ///< 8-byte words of the chunk list, two a chunk (as entries the repair kernel ran 1 % longer)
+  int64_t chunk_cap;
   control* ctl;
   grid_sync_state* bar;
   int32_t light;       ///< rows of more edges are cut into chunks (pull and relax)
@@ -866,7 +866,7 @@ DYNG_DEV void engine_run(const engine_params& p) {
   bool long_near = true;  // the next relax iteration's list holds a vertex with a row past `light`
   int step = 0, cstep = 0;  // ring positions (uniform across the grid)
   unsigned int round = 0;  // of the grid barrier (uniform over the grid)
-  const int64_t chunk_cap = p.chunk_words / 2;
+  const int64_t chunk_cap = p.chunk_cap;
   unsigned long long jump_items = 0;
   if (tid == 0) st(&c->t_phase[0], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
 
@@ -1917,7 +1917,7 @@ void attach_scratch(engine_params& p, const engine_scratch& sc) {
   p.far_b = sc.far_b;
   p.touched = sc.touched;
   p.chunks = sc.chunks;
-  p.chunk_words = 2 * sc.chunk_cap;
+  p.chunk_cap = sc.chunk_cap;
   p.ctl = sc.ctl;
   p.bar = sc.bar;
 }
