@@ -866,7 +866,7 @@ DYNG_DEV void engine_run(const engine_params& p) {
   bool long_near = true;  // the next relax iteration's list holds a vertex with a row past `light`
   int step = 0, cstep = 0;  // ring positions (uniform across the grid)
   unsigned int round = 0;  // of the grid barrier (uniform over the grid)
-  const int64_t chunk_cap = p.chunk_cap;
+  const int64_t chunk_cap = p.chunk_cap / 2;  // one phase's chunks: at most slots / 16 + n
   unsigned long long jump_items = 0;
   if (tid == 0) st(&c->t_phase[0], static_cast<u64>(__builtin_amdgcn_s_memrealtime()));
 
@@ -1752,9 +1752,10 @@ bool narrow_grid(int blocks, int occupancy_narrow, int cu_count) {
   return occupancy_narrow >= 1 && blocks <= occupancy_narrow * cu_count;
 }
 
-/// Chunk-list entries a run over n vertices and a row arena of `slots` slots may need: a phase
-/// lists every row at most once, in chunks of at least 16 edges: at most slots / 16 + n.
-int64_t chunks_for(int64_t n, int64_t slots) { return slots / 16 + n + 4096; }
+/// Chunk-list entries a run over n vertices and a row arena of `slots` slots may need: one pass
+/// over every row in chunks of at least 16 edges takes at most slots / 16 + n; the relax
+/// iterations keep two such lists (one iteration's chunks are relaxed during the next).
+int64_t chunks_for(int64_t n, int64_t slots) { return 2 * (slots / 16 + n + 4096); }
 
 void ws_reserve(dyng_hip_workspace* ws, int64_t n, int64_t slots, hipStream_t s) {
   const int64_t want_chunks = chunks_for(n, slots);
@@ -2295,7 +2296,7 @@ scratch_layout layout_for(int64_t n, int64_t slots) {
   L.far_a = take(4 * n);
   L.far_b = take(4 * n);
   L.touched = take(4 * n);
-  L.chunk_cap = 2 * chunks_for(n, slots);  // twice what a run needs: the published limit on the graph's size counts it
+  L.chunk_cap = chunks_for(n, slots);
   L.chunks = take(static_cast<int64_t>(sizeof(int4)) * L.chunk_cap);
   L.ctl = take(sizeof(control));
   L.bar = take(sizeof(grid_sync_state));
