@@ -2993,7 +2993,6 @@ void take_ops(dyng_hip_graph* g, int64_t P, size_t groups) {
     const size_t n = static_cast<size_t>(P);
     place(o.keys_b, 2 * n);  // out-row keys, then in-row keys
     place(o.vals_b, 2 * n);
-    place(o.group_entries, groups * kGroupCap);
     place(o.group_counts, groups);
     for (int32_t** p : {&o.pend_alive, &o.kill, &o.pend_prefix, &o.kill_prefix, &o.ipend_alive, &o.ikill,
                         &o.ipend_prefix, &o.ikill_prefix}) {
@@ -3005,18 +3004,20 @@ void take_ops(dyng_hip_graph* g, int64_t P, size_t groups) {
     place(o.touched_in, n + 1);
     place(o.lane_rows, 4 * (n + 1));
     place(o.merge_lists, 2 * kModes * (n + 1));
+    place(o.group_entries, groups * kGroupCap);  // last: a small batch fills few places of many
     return at;
   };
   const size_t bytes = lay_out(nullptr);
-  if (!g->pools_scratch) {
-    apply_scratch(g->device).join();
-    g->pools_scratch = true;
+  if (g->pool == nullptr) {
+    scratch_pool& pool = apply_scratch(g->device);
+    pool.join();
+    g->pool = &pool;
   }
   // a block that a failed apply left with the graph is used again: its work is on the graph's stream
   if (o.block.bytes < bytes) {
     if (o.block.p != nullptr) DYNG_HIP_TRY(hipFree(o.block.p));
     o.block = {};
-    o.block = apply_scratch(g->device).take(bytes);
+    o.block = g->pool->take(bytes);
     if (o.block.p == nullptr) {
       throw status_error(DYNG_HIP_OUT_OF_MEMORY, "dyng: out of device memory (" + std::to_string(bytes) + " bytes)");
     }
@@ -3026,7 +3027,7 @@ void take_ops(dyng_hip_graph* g, int64_t P, size_t groups) {
 
 /// The apply's work has ended: its scratch goes back.
 void give_ops(dyng_hip_graph* g) {
-  apply_scratch(g->device).give(g->ops.block);
+  g->pool->give(g->ops.block);
   g->ops = op_scratch{};
 }
 

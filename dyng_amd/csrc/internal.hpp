@@ -380,7 +380,7 @@ struct dyng_hip_graph {
 
   // apply scratch
   dyng_hip::op_scratch ops;
-  bool pools_scratch = false;  ///< the graph is a user of its device's scratch pool
+  dyng_hip::scratch_pool* pool = nullptr;  ///< its device's, once the graph uses it
   dyng_hip::dbuf<unsigned long long> keys_a;  ///< the device-wide sort's input: out-row keys, then in-row keys
   dyng_hip::dbuf<uint32_t> vals_a;
   dyng_hip::dbuf<unsigned char> sort_tmp, scan_tmp;
@@ -404,7 +404,7 @@ struct dyng_hip_graph {
   dyng_hip_graph& operator=(const dyng_hip_graph&) = delete;
   ~dyng_hip_graph() {
     if (ops.block.p != nullptr) (void)hipFree(ops.block.p);  // an apply failed half-way: its work may not have ended
-    if (pools_scratch) dyng_hip::apply_scratch(device).leave();
+    if (pool != nullptr) pool->leave();
     for (hipEvent_t& e : apply_ev) {
       if (e != nullptr) (void)hipEventDestroy(e);
     }
