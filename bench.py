@@ -577,20 +577,20 @@ def mosp_bench(args) -> int:
     p50 = statistics.median(wall)
     value = ops / (p50 / 1e3)
     log(f"[bench] gpu: p50 {p50:.3f} ms/update, {value:.3e} edges/s")
-    # the persistent kernel: three repair launches and the combined solve per step
+    # the persistent kernel: three repairs side by side in one launch (it ends with the slowest) and the
+    # combined tree's repair per step
     kbytes, kms = [], []
     for st in stats:
-        for o in st.objectives:
-            kbytes.append(fused_kernel_bytes(o.device, n, o.batch.deleted_edges + o.batch.ignored_deletions + ops,
-                                             ops))
-            kms.append(o.device.kernel_ms)
+        kbytes.append(sum(fused_kernel_bytes(o.device, n, o.batch.deleted_edges + o.batch.ignored_deletions + ops, ops)
+                          for o in st.objectives))
+        kms.append(max(o.device.kernel_ms for o in st.objectives))
         dels, ins = st.combined_batch
         kbytes.append(fused_kernel_bytes(st.combined_solve, n, dels + ins, ins))
         kms.append(st.combined_solve.kernel_ms)
     achieved = (sum(kbytes) / len(kbytes)) / (statistics.mean(kms) / 1e3) / 1e9
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic(args.workload),
-                "kernel": "sssp_fused_kernel (3 repairs + the combined tree's repair per step)",
+                "kernel": "sssp_teams_kernel (3 repairs side by side) and sssp_fused_kernel (the combined tree's)",
                 "kernel_ms_mean": round(statistics.mean(kms), 4), "algorithmic_bytes_mean": int(sum(kbytes) / len(kbytes))}
     cpu, exact = None, None
     if not args.no_cpu and args.cpu_sample > 0:
@@ -625,7 +625,7 @@ def mosp_bench(args) -> int:
         "config": {"workload": args.workload, "vertices": int(n), "edges": int(len(src)), "objectives": int(w.shape[1]),
                    "preferences": MOSP_PREFERENCES, "batch_ops": ops, "source": int(source),
                    "apply_ms_p50": round(statistics.median(s.objectives[0].apply_ms for s in stats), 4),
-                   "repairs_ms_p50": round(statistics.median(sum(o.engine_ms for o in s.objectives)
+                   "repairs_ms_p50": round(statistics.median(max(o.engine_ms for o in s.objectives)
                                                              for s in stats), 4),
                    "combined_repair_kernel_ms_p50": round(statistics.median(s.combined_solve.kernel_ms
                                                                             for s in stats), 4),
